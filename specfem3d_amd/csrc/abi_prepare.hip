@@ -18,6 +18,7 @@
 
 namespace sf {
 void free_checkpoints(Mesh* m);
+void flush_all(Mesh* m);
 
 Mesh* from_handle(long* p) {
   if (!p || !*p) fatal("Mesh_pointer", "null handle (prepare_constants_device not called?)");
@@ -471,7 +472,9 @@ extern "C" void FC_FUNC_(prepare_constants_device, PREPARE_CONSTANTS_DEVICE)(
 }
 
 namespace sf {
-static void build_elastic_assembly(Mesh* m);
+void ensure_gather_assembly(Mesh* m, int f);
+void ensure_element_colors(Mesh* m);
+static void prepare_acoustic_gather(Mesh* m);
 
 // Distinct (factor_common, factor_common_kappa) rows, compared bit for bit, and a 16-bit row index
 // per local point; gives up (planes only) beyond 65535 distinct rows.
@@ -585,13 +588,9 @@ extern "C" void FC_FUNC_(prepare_fields_elastic_device, PREPARE_FIELDS_ELASTIC_D
   const int64_t n = m->nglob;
   const int64_t nloc = (int64_t)m->nspec * 125;
   if (m->assembly < 0) {
-    // automatic assembly: coloured without attenuation, atomic with it (see Mesh::assembly)
-    m->assembly = *ATTENUATION ? 0 : 2;
-    if (m->assembly == 2 && m->nspec_acoustic > 0 && m->acoustic_elems && !m->ac_color_elems) {
-      std::vector<int> lst(m->nspec_acoustic);
-      SF_CHECK(hipMemcpy(lst.data(), m->acoustic_elems, sizeof(int) * lst.size(), hipMemcpyDeviceToHost));
-      build_colors(m, lst, m->ac_color_elems, m->ac_color_off, m->ac_ncolor);
-    }
+    // automatic assembly (see Mesh::assembly); the acoustic fields were prepared before it was known
+    m->assembly = *ATTENUATION ? 0 : 1;
+    if (m->assembly == 1) prepare_acoustic_gather(m);
   }
   {
     std::vector<realw> rm(3 * (size_t)n);
@@ -684,12 +683,8 @@ extern "C" void FC_FUNC_(prepare_fields_elastic_device, PREPARE_FIELDS_ELASTIC_D
       m->gammaval[s] = gammaval[s];
     }
   }
-  if (m->assembly == 1) build_elastic_assembly(m);
-  if (m->assembly == 2) {
-    std::vector<int> lst(m->nspec_elastic);
-    SF_CHECK(hipMemcpy(lst.data(), m->elastic_elems, sizeof(int) * lst.size(), hipMemcpyDeviceToHost));
-    build_colors(m, lst, m->el_color_elems, m->el_color_off, m->el_ncolor);
-  }
+  if (m->assembly == 2) ensure_element_colors(m);
+  ensure_gather_assembly(m, 0);
 }
 
 namespace sf {
@@ -754,40 +749,50 @@ static void build_colors(Mesh* m, const std::vector<int>& elems, int*& d_list, i
   d_list = lst.empty() ? nullptr : dupload(lst.data(), (int64_t)lst.size());
 }
 
-// CSR of local slots per global point sorted by the position of their element in the
-// processing list (ordered assembly); shared by the elastic and acoustic gathers.
-static void build_csr(Mesh* m, const std::vector<int>& elems, int*& ptr, int*& idx) {
-  HostSide* H = host_of(m);
-  const int n = m->nglob;
-  std::vector<int> cnt(n + 1, 0);
-  for (int e : elems)
-    for (int p = 0; p < 125; p++) cnt[H->ibool[(int64_t)e * 125 + p] + 1]++;
-  for (int g = 0; g < n; g++) cnt[g + 1] += cnt[g];
-  std::vector<int> id(cnt[n]);
-  std::vector<int> pos(cnt.begin(), cnt.end() - 1);
-  for (int e : elems)
-    for (int p = 0; p < 125; p++) {
-      const int g = H->ibool[(int64_t)e * 125 + p];
-      id[pos[g]++] = e * 125 + p;
-    }
-  ptr = dupload(cnt.data(), n + 1);
-  idx = dupload(id.data(), (int64_t)id.size());
-}
-
-static void build_elastic_assembly(Mesh* m) {
-  // the stiffness elements, then the C-PML elements (compute_forces_viscoelastic, then
-  // compute_forces_viscoelastic_PML: that is the order their contributions are summed in)
-  std::vector<int> lst(m->nspec_elastic + m->pml_n);
-  SF_CHECK(hipMemcpy(lst.data(), m->elastic_elems, sizeof(int) * m->nspec_elastic, hipMemcpyDeviceToHost));
+// Lists and buffers of the gather assembly for one field: the slots of each point in the processing
+// order, or in the colour order under assembly = 2 (the sums a coloured scatter makes, bit for bit),
+// those of the C-PML elements last (compute_forces_viscoelastic, then compute_forces_viscoelastic_PML).
+void ensure_gather_assembly(Mesh* m, int f) {
+  if (!m->asm_buf[f]) m->asm_buf[f] = dmalloc<realw>(3 * (int64_t)m->nspec * 125);
+  if (m->asm_ready) return;
+  if (m->assembly == 2) ensure_element_colors(m);
+  const int* first = m->assembly == 2 && m->el_color_elems ? m->el_color_elems : m->elastic_elems;
+  int* lst = dmalloc<int>(m->nspec_elastic + m->pml_n);
+  SF_CHECK(hipMemcpyAsync(lst, first, sizeof(int) * m->nspec_elastic, hipMemcpyDeviceToDevice, m->stream));
   if (m->pml_n)
-    SF_CHECK(hipMemcpy(lst.data() + m->nspec_elastic, m->pml_elems, sizeof(int) * m->pml_n, hipMemcpyDeviceToHost));
+    SF_CHECK(hipMemcpyAsync(lst + m->nspec_elastic, m->pml_elems, sizeof(int) * m->pml_n, hipMemcpyDeviceToDevice,
+                            m->stream));
   dfree(m->asm_ptr);
   dfree(m->asm_idx);
-  build_csr(m, lst, m->asm_ptr, m->asm_idx);
-  if (!m->asm_buf) m->asm_buf = dmalloc<realw>(3 * (int64_t)m->nspec * 125);
+  build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_elastic + m->pml_n, lst, m->ibool, m->asm_ptr, m->asm_idx);
+  dfree(lst);
+  if (!m->asm_flags) m->asm_flags = dmalloc<unsigned char>(m->nglob);
+  SF_CHECK(hipMemsetAsync(m->asm_flags, 0, (size_t)m->nglob, m->stream));
+  for (const FacePoints* fp : {&m->abs_el, &m->coupling, &m->src_pts, &m->adj_pts})
+    launch_mark_points(m->stream, fp->n, fp->iglob, AF_TERM, m->asm_flags);
+  launch_mark_points(m->stream, m->pml_nbc, m->pml_bc_pts, AF_EDGE, m->asm_flags);
   m->asm_ready = 1;
 }
 
+// give the lists and buffers back (the batched engine steps its own fields); a later stiffness call
+// on the mesh's fields builds them again
+void release_gather_assembly(Mesh* m) {
+  flush_all(m);
+  SF_CHECK(hipStreamSynchronize(m->stream));
+  dfree(m->asm_ptr);
+  dfree(m->asm_idx);
+  dfree(m->asm_buf[0]);
+  dfree(m->asm_buf[1]);
+  m->asm_ready = 0;
+}
+
+// the same for the fluid (ordered sums of the acoustic stiffness)
+static void prepare_acoustic_gather(Mesh* m) {
+  if (m->asm_ac_buf || m->nspec_acoustic <= 0 || !m->acoustic_elems) return;
+  build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_acoustic, m->acoustic_elems, m->ibool, m->asm_ac_ptr,
+                   m->asm_ac_idx);
+  m->asm_ac_buf = dmalloc<realw>((int64_t)m->nspec * 125);
+}
 
 }  // namespace sf
 
@@ -836,10 +841,7 @@ extern "C" void FC_FUNC_(prepare_fields_acoustic_device, PREPARE_FIELDS_ACOUSTIC
       }
     m->ac_g0 = gmax < 0 ? 0 : (gmin / 4) * 4;
     m->ac_n = gmax < 0 ? 0 : (int64_t)gmax + 1 - m->ac_g0;
-    if (m->assembly == 1) {
-      build_csr(m, lst, m->asm_ac_ptr, m->asm_ac_idx);
-      m->asm_ac_buf = dmalloc<realw>(nloc);
-    }
+    if (m->assembly == 1) prepare_acoustic_gather(m);
     if (m->assembly == 2) build_colors(m, lst, m->ac_color_elems, m->ac_color_off, m->ac_ncolor);
   }
   m->ac[0].pot = dmalloc<realw>(n);
@@ -1049,7 +1051,7 @@ extern "C" void FC_FUNC_(prepare_fields_elastic_pml, PREPARE_FIELDS_ELASTIC_PML)
     m->pml_bc_pts = bc.empty() ? nullptr : dupload(bc.data(), (int64_t)bc.size());
   }
   // the assembly structures follow the new lists
-  if (m->assembly == 1) build_elastic_assembly(m);
+  m->asm_ready = 0;
   if (m->assembly == 2) {
     std::vector<int> order = keep;
     if (m->elastic_launch) {
@@ -1058,6 +1060,7 @@ extern "C" void FC_FUNC_(prepare_fields_elastic_pml, PREPARE_FIELDS_ELASTIC_PML)
     }
     build_colors(m, order, m->el_color_elems, m->el_color_off, m->el_ncolor);
   }
+  ensure_gather_assembly(m, 0);
   prep_log("C-PML arrays prepared");
 }
 
@@ -1099,6 +1102,7 @@ extern "C" void FC_FUNC_(prepare_fields_elastic_adj_dev, PREPARE_FIELDS_ELASTIC_
       m->b_gammaval[s] = b_gammaval[s];
     }
   }
+  ensure_gather_assembly(m, 1);
   m->rho_kl = dmalloc<realw>(nloc);
   m->mu_kl = dmalloc<realw>(nloc);
   m->kappa_kl = dmalloc<realw>(nloc);
@@ -1174,6 +1178,7 @@ extern "C" void FC_FUNC_(prepare_sim2_or_3_const_device, PREPARE_SIM2_OR_3_CONST
     build_point_sets(own_ac, H->ibool, m->adj_ac_pts);
     remap_owner(m->adj_ac_pts, idx_ac);
   }
+  m->asm_ready = 0;  // the adjoint source points take terms
   m->adj_h = dupload(h.data(), (int64_t)h.size());
   m->adj_src = dmalloc<realw>(3 * (int64_t)m->nadj_rec_local);
 }
@@ -1206,7 +1211,7 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
   dfree(m->rec_ispec); dfree(m->rec_el_list); dfree(m->rec_ac_list);
   dfree(m->seismo_d); dfree(m->seismo_v); dfree(m->seismo_a); dfree(m->seismo_p);
   dfree(m->rho_kl); dfree(m->mu_kl); dfree(m->kappa_kl); dfree(m->rho_ac_kl); dfree(m->kappa_ac_kl);
-  dfree(m->asm_ptr); dfree(m->asm_idx); dfree(m->asm_buf);
+  dfree(m->asm_ptr); dfree(m->asm_idx); dfree(m->asm_flags); dfree(m->asm_buf[0]); dfree(m->asm_buf[1]);
   dfree(m->pml_elems); dfree(m->pml_cpml);
   dfree(m->pml_state); dfree(m->pml_coef); dfree(m->pml_masks); dfree(m->pml_off);
   dfree(m->pml_old); dfree(m->pml_pts); dfree(m->pml_bc_pts);
@@ -1228,23 +1233,17 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
 // Library extensions (no counterpart in the reference interface).
 
 // exact = 1: element kernels without fused multiply-add (the CPU reference's rounding);
-// assembly = 1: element contributions summed per global point in element order (deterministic,
-// the reference's serial order) instead of float atomics; assembly = 2: one launch per colour of
-// a greedy element colouring, plain read-modify-write scatter (deterministic, no atomics).
+// assembly: the order in which a global point's element contributions are summed. 1 = element order
+// (the reference's serial order), 2 = the colour order of a greedy element colouring, 0 = any order
+// (the solid takes element order; the fluid and its face terms use float atomics). All of them
+// store the solid's local forces and sum them in the next update (k_gather_update).
 extern "C" void sf_set_options(long* Mesh_pointer, int exact, int assembly) {
   Mesh* m = from_handle(Mesh_pointer);
   SF_CHECK(hipStreamSynchronize(m->stream));
   m->exact = exact ? 1 : 0;
   m->assembly = assembly;
-  if (assembly == 1) {
-    if (!m->asm_ready && m->nspec_elastic > 0 && m->kappamu) build_elastic_assembly(m);
-    if (!m->asm_ac_buf && m->nspec_acoustic > 0 && m->acoustic_elems) {
-      std::vector<int> lst(m->nspec_acoustic);
-      SF_CHECK(hipMemcpy(lst.data(), m->acoustic_elems, sizeof(int) * lst.size(), hipMemcpyDeviceToHost));
-      build_csr(m, lst, m->asm_ac_ptr, m->asm_ac_idx);
-      m->asm_ac_buf = dmalloc<realw>((int64_t)m->nspec * 125);
-    }
-  }
+  m->asm_ready = 0;  // rebuilt in the new order by the next stiffness call
+  if (assembly == 1) prepare_acoustic_gather(m);
   if (assembly == 2) {
     if (!m->el_color_elems) ensure_element_colors(m);
     if (!m->ac_color_elems && m->nspec_acoustic > 0 && m->acoustic_elems) {
@@ -1303,6 +1302,7 @@ extern "C" void sf_set_element_order(long* Mesh_pointer, int n, const int* order
   dfree(m->elastic_launch);
   m->elastic_launch = dupload(lst.data(), (int64_t)lst.size());
   if (m->el_color_elems) build_colors(m, lst, m->el_color_elems, m->el_color_off, m->el_ncolor);
+  if (m->assembly == 2) m->asm_ready = 0;  // the sums follow the colours
 }
 
 // Greedy element colouring used by assembly = 2 (host only, no device needed): colour[q] of

@@ -18,6 +18,7 @@
 namespace sf {
 realw* stage_to_device(Mesh* m, const realw* vals, int n, realw* dst);
 realw* stf_device_buffer(Mesh* m, int n);
+void ensure_gather_assembly(Mesh* m, int f);
 const std::vector<int>& host_ibool(Mesh* m);
 
 static inline int field_of(int foa) { return foa == 3 ? 1 : 0; }
@@ -31,13 +32,39 @@ static inline int field_of(int foa) { return foa == 3 ? 1 : 0; }
 // 18.9 / 19.2 / 18.7 us in rounds).
 static inline bool face_atomics(const Mesh* m) { return m->assembly == 0; }
 
+static GatherArgs gather_args(Mesh* m, int f) {
+  GatherArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.g0 = m->el_g0;  // only the elastic range changes (see Mesh::el_g0)
+  a.n = m->el_n;
+  a.ptr = m->asm_ptr;
+  a.idx = m->asm_idx;
+  a.local = m->asm_buf[f];
+  a.flags = m->asm_flags;
+  a.skip = m->gather_skip_el[f];
+  a.clean = m->accel_clean[f];
+  a.u = m->el[f].displ;
+  a.v = m->el[f].veloc;
+  a.a = m->el[f].accel;
+  a.rm = m->rmass;
+  a.dt2p = m->pending_dt2_el[f];
+  return a;
+}
+
+// sum the waiting local forces and run the pending corrector
 static void flush_el(Mesh* m, int f) {
-  if (m->pending_k3_el[f]) {
-    const int64_t o = 3 * m->el_g0;  // only the elastic range changes (see Mesh::el_g0)
+  if (m->pending_gather_el[f]) {
+    launch_gather_update(m->stream, gather_args(m, f), m->pending_k3_el[f] ? GATHER_CORRECT : GATHER_ONLY);
+    m->pending_gather_el[f] = 0;
+    m->gather_skip_el[f] = 0;
+    m->accel_clean[f] = 0;
+  } else if (m->pending_k3_el[f]) {
+    const int64_t o = 3 * m->el_g0;
     launch_corrector(m->stream, 3 * m->el_n, m->el[f].veloc + o, m->el[f].accel + o, m->rmass + o,
                      m->pending_dt2_el[f]);
-    m->pending_k3_el[f] = 0;
+    m->accel_clean[f] = 0;
   }
+  m->pending_k3_el[f] = 0;
 }
 static void flush_ac(Mesh* m, int f) {
   if (m->pending_k3_ac[f]) {
@@ -58,9 +85,8 @@ static ElasticArgs elastic_args(Mesh* m, int f, realw deltat) {
   ElasticArgs a;
   std::memset(&a, 0, sizeof(a));
   a.nelem = m->nspec_elastic;
-  // atomic launches may walk the elements in the host's locality order; the ordered assembly keeps
-  // the processing list (its gather sums in that order)
-  a.elems = (m->elastic_launch && m->assembly != 1) ? m->elastic_launch : m->elastic_elems;
+  // the launch may walk the elements in the host's locality order: the gather has its own
+  a.elems = m->elastic_launch ? m->elastic_launch : m->elastic_elems;
   a.ibool = m->ibool;
   a.irregular = m->irregular;
   a.xix_regular = m->xix_regular;
@@ -70,7 +96,6 @@ static ElasticArgs elastic_args(Mesh* m, int f, realw deltat) {
   a.kappamu = m->kappamu;
   a.displ = m->el[f].displ;
   a.veloc = m->el[f].veloc;
-  a.accel = m->el[f].accel;
   a.deltat = deltat;
   a.R = m->att[f].R;
   a.eps = m->att[f].eps;
@@ -86,27 +111,18 @@ static ElasticArgs elastic_args(Mesh* m, int f, realw deltat) {
     a.beta[s] = f ? m->b_betaval[s] : m->betaval[s];
     a.gamma[s] = f ? m->b_gammaval[s] : m->gammaval[s];
   }
-  a.local_out = m->asm_buf;
+  a.local_out = m->asm_buf[f];
   return a;
 }
 
 void elastic_forces(Mesh* m, int f, realw deltat, bool strain, bool att) {
+  ensure_gather_assembly(m, f);
   ElasticArgs a = elastic_args(m, f, deltat);
-  const bool ordered = m->assembly == 1 && m->asm_ready;
-  const bool colored = m->assembly == 2 && m->el_color_elems;
   const bool pml_call = f == 0 && m->pml_n > 0;
   const bool whole = m->timing_scope == 0;
   const bool timed = m->timing_count < m->timing_max && (whole || pml_call);
   if (timed && whole) SF_CHECK(hipEventRecord(m->timing_ev[2 * m->timing_count], m->stream));
-  if (colored) {
-    for (int c = 0; c < m->el_ncolor; c++) {
-      a.elems = m->el_color_elems + m->el_color_off[c];
-      a.nelem = m->el_color_off[c + 1] - m->el_color_off[c];
-      launch_elastic(m->stream, a, strain, att, m->exact != 0, 2, m->att_variant);
-    }
-  } else {
-    launch_elastic(m->stream, a, strain, att, m->exact != 0, ordered ? 1 : 0, m->att_variant);
-  }
+  launch_elastic(m->stream, a, strain, att, m->exact != 0, m->att_variant);
   if (pml_call) {
     // C-PML elements (pml_kernel_2_impl of compute_forces_viscoelastic_cuda), after the others: their
     // contributions are summed after those of the stiffness elements
@@ -124,7 +140,6 @@ void elastic_forces(Mesh* m, int f, realw deltat, bool strain, bool att) {
     P.kappamu = m->kappamu;
     P.displ = m->el[0].displ;
     P.veloc = m->el[0].veloc;
-    P.accel = m->el[0].accel;
     P.pml_old = m->pml_old;
     P.state = m->pml_state;
     P.coef = m->pml_coef;
@@ -132,20 +147,15 @@ void elastic_forces(Mesh* m, int f, realw deltat, bool strain, bool att) {
     P.off = m->pml_off;
     P.t1 = m->pml_t1;
     P.t2 = m->pml_t2;
-    P.local_out = m->asm_buf;
-    P.nloc = a.nloc;
-    // one launch, float atomics also under coloured assembly: split into its colours (about 1100
-    // elements each on the reference's C-PML example) the launches were too small to fill the chip
-    // (8 x 35 us against 240 us for one atomic launch before the dead-plane masks)
+    P.local_out = m->asm_buf[0];
     if (timed && !whole) SF_CHECK(hipEventRecord(m->timing_ev[2 * m->timing_count], m->stream));
-    launch_elastic_pml(m->stream, P, m->exact != 0, ordered ? 1 : 0);
+    launch_elastic_pml(m->stream, P, m->exact != 0);
   }
   if (timed) {
     SF_CHECK(hipEventRecord(m->timing_ev[2 * m->timing_count + 1], m->stream));
     m->timing_count++;
   }
-  if (ordered)
-    launch_ordered_gather(m->stream, m->nglob, 3, m->asm_ptr, m->asm_idx, m->asm_buf, a.nloc, m->el[f].accel);
+  m->pending_gather_el[f] = 1;
 }
 
 }  // namespace sf
@@ -165,6 +175,7 @@ extern "C" void FC_FUNC_(update_displacement_cuda, UPDATE_DISPLACMENT_CUDA)(long
   const int f = field_of(*FORWARD_OR_ADJOINT);
   check_field(m, f, "update_displacement_cuda");
   const int64_t n = 3 * m->el_n, o = 3 * m->el_g0;  // only the elastic range changes
+  if (!m->pending_k3_el[f]) flush_el(m, f);
   Wavefield& w = m->el[f];
   const bool pml = f == 0 && m->pml_n > 0;
   if (pml) {
@@ -177,15 +188,27 @@ extern "C" void FC_FUNC_(update_displacement_cuda, UPDATE_DISPLACMENT_CUDA)(long
       launch_pml_store_old(m->stream, m->pml_npts, m->pml_pts, w.displ, w.veloc, w.accel, m->rmass, 0, 0.f,
                            m->pml_t1, m->pml_t2, m->pml_old);
   }
-  if (m->pending_k3_el[f]) {
+  if (m->pending_gather_el[f]) {
+    GatherArgs a = gather_args(m, f);
+    a.dt = *deltat_F;
+    a.dt2 = *deltatover2_F;
+    a.dtsq2 = *deltatsqover2_F;
+    a.old = pml ? m->pml_old : nullptr;
+    a.t1 = m->pml_t1;
+    a.t2 = m->pml_t2;
+    launch_gather_update(m->stream, a, GATHER_STEP);
+  } else if (m->pending_k3_el[f]) {
     launch_corrector_predictor(m->stream, n, w.displ + o, w.veloc + o, w.accel + o, m->rmass + o,
                                m->pending_dt2_el[f], *deltat_F, *deltatover2_F, *deltatsqover2_F,
                                pml ? m->pml_old + o : nullptr, m->pml_t1, m->pml_t2);
-    m->pending_k3_el[f] = 0;
   } else {
     launch_predictor(m->stream, n, w.displ + o, w.veloc + o, w.accel + o, *deltat_F, *deltatover2_F,
                      *deltatsqover2_F);
   }
+  m->pending_gather_el[f] = 0;
+  m->gather_skip_el[f] = 0;
+  m->pending_k3_el[f] = 0;
+  m->accel_clean[f] = 1;  // zero, or at AF_TERM points about to take their terms
 }
 
 extern "C" void FC_FUNC_(update_displacement_ac_cuda, UPDATE_DISPLACEMENT_AC_CUDA)(long* Mesh_pointer,
@@ -218,7 +241,7 @@ extern "C" void FC_FUNC_(kernel_3_a_cuda, KERNEL_3_A_CUDA)(long* Mesh_pointer, r
     if (foa == 1 && f == 1) continue;
     if (foa == 3 && f == 0) continue;
     if (!m->el[f].displ) continue;
-    flush_el(m, f);
+    if (m->pending_k3_el[f]) flush_el(m, f);
     m->pending_k3_el[f] = 1;
     m->pending_dt2_el[f] = f ? *b_deltatover2_F : *deltatover2_F;
   }
@@ -336,7 +359,9 @@ extern "C" void FC_FUNC_(pml_impose_boundary_condition_elastic_cuda,
                          PML_IMPOSE_BOUNDARY_CONDITION_ELASTIC_CUDA)(long* Mesh_pointer) {
   Mesh* m = from_handle(Mesh_pointer);
   if (!m->pml_conditions || m->pml_nbc == 0) return;
-  flush_el(m, 0);
+  // local forces still to be summed are left out at these points, which gives them the same zeros
+  if (m->pending_gather_el[0] && !m->pending_k3_el[0]) m->gather_skip_el[0] |= AF_EDGE;
+  else flush_el(m, 0);
   launch_zero_points(m->stream, m->pml_nbc, m->pml_bc_pts, m->el[0].displ, m->el[0].veloc, m->el[0].accel);
 }
 
@@ -771,6 +796,7 @@ static void d2h(Mesh* m, realw* h, const realw* d, int64_t n) {
     DIR(m, m->el[F].displ, displ, *size);                                                                     \
     DIR(m, m->el[F].veloc, veloc, *size);                                                                     \
     DIR(m, m->el[F].accel, accel, *size);                                                                     \
+    m->accel_clean[F] = 0;                                                                                    \
   }
 #define SF_XFER1(NAME, F, MEMBER, DIR)                                                   \
   extern "C" void FC_FUNC_(NAME, X)(int* size, realw* arr, long* Mesh_pointer) {        \
@@ -778,6 +804,7 @@ static void d2h(Mesh* m, realw* h, const realw* d, int64_t n) {
     check_field(m, F, #NAME);                                                            \
     flush_el(m, F);                                                                      \
     DIR(m, m->el[F].MEMBER, arr, *size);                                                 \
+    m->accel_clean[F] = 0;                                                               \
   }
 #define H2D(m, d, h, n) h2d(m, d, h, n)
 #define D2H(m, d, h, n) d2h(m, h, d, n)

@@ -32,6 +32,7 @@
 
 namespace sf {
 void ensure_element_colors(Mesh* m);
+void release_gather_assembly(Mesh* m);
 void ensure_acoustic_colors(Mesh* m);
 bool element_is_elastic(Mesh* m, int e);
 
@@ -842,6 +843,7 @@ extern "C" long sf_batch_create(long* Mesh_pointer, int nshots, const int* nstep
   b->dt2 = deltatover2;
   b->dtsq2 = deltatsqover2;
   b->nshots = nshots;
+  release_gather_assembly(m);
   ensure_element_colors(m);
   if (m->nspec_acoustic > 0) {
     ensure_acoustic_colors(m);

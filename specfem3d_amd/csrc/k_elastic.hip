@@ -5,10 +5,11 @@
 //   * a 128-thread workgroup (two wave64s) processes one element; lane p owns the GLL point
 //     p = i + 5 j + 25 k (125 of the 128 lanes busy) and all three contractions read the element
 //     tile staged in LDS;
-//   * the element-to-global scatter is selected by MODE: 0 a float atomic add, 1 a store of
-//     the local contributions that a gather kernel later sums in the CPU's element order,
-//     2 a plain read-modify-write (the launch holds one colour of a greedy element colouring,
-//     so no two of its elements share a global point);
+//   * the local forces are stored, three floats per local point, and summed per global point by the
+//     update that follows (k_gather_update): one launch over all elements, no atomics, no colours.
+//     Against float atomics the viscoelastic launch on 64x64x32 elements (28 layers solid) went from
+//     854 to 620 us (the atomics' write-back was 15 % of its traffic), and against eight colour
+//     launches the elastic one from 277 to 187 us there and from 41 to 14 us on 20x20x20;
 //   * workgroup ids are remapped so each XCD (8 per chip, dispatched round-robin) walks one
 //     contiguous range of elements and keeps the shared points of neighbours in its own L2.
 // The arithmetic order of every sum follows the reference (the five terms of each
@@ -94,7 +95,7 @@ __device__ __forceinline__ void load_att_state(const ElasticArgs& A, int e, int 
 typedef __attribute__((address_space(3))) void* sf_lds_ptr;
 typedef __attribute__((address_space(1))) void* sf_global_ptr;
 
-template <bool STRAIN, bool ATT, int MODE, int AV>
+template <bool STRAIN, bool ATT, int AV>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(AV >= 2 ? 5 : 1)))
 k_elastic_pt(ElasticArgs A, GLLk G) {
   constexpr bool LATE = ATT && (AV == 1 || AV == 2);
@@ -235,25 +236,10 @@ k_elastic_pt(ElasticArgs A, GLLk G) {
 
   realw f[3];
   tile_divergence<1>(&sT[0][0], 128, gll_hpw(sG, irr != 0), sG + 50, i, j, k, f);
-  if (MODE == 1) {
-    A.local_out[ep] = f[0];
-    A.local_out[nl + ep] = f[1];
-    A.local_out[2 * nl + ep] = f[2];
-  } else if (MODE == 2) {
-    // coloured launch. (A plain update of the element-interior points inside atomic launches
-    // measured 1.9x slower on the 96x96x48 viscoelastic workload than atomics for all points.)
-    realw* a = A.accel + 3 * (int64_t)g;
-    a[0] = a[0] + (-f[0]);
-    a[1] = a[1] + (-f[1]);
-    a[2] = a[2] + (-f[2]);
-  } else {
-    // (plain stores of the 27 element-interior points, which belong to this element alone, measured
-    // 16 % slower on the 96x96x48 viscoelastic workload than atomics for all points)
-    realw* a = A.accel + 3 * (int64_t)g;
-    atomicAdd(a + 0, -f[0]);
-    atomicAdd(a + 1, -f[1]);
-    atomicAdd(a + 2, -f[2]);
-  }
+  realw* o = A.local_out + 3 * ep;
+  o[0] = f[0];
+  o[1] = f[1];
+  o[2] = f[2];
 }
 
 // element strain of a displacement field (compute_element_strain.F90:28-130); one lane per point
@@ -337,29 +323,23 @@ __global__ void __launch_bounds__(128) k_element_strain(ElasticArgs A, GLLk G, r
 }  // namespace SF_VNS
 using namespace SF_VNS;
 
-void SFX(launch_elastic)(hipStream_t s, const ElasticArgs& a, bool strain, bool att, int mode, int att_variant) {
+void SFX(launch_elastic)(hipStream_t s, const ElasticArgs& a, bool strain, bool att, int att_variant) {
   if (a.nelem <= 0) return;
   GLLk G = g_gll_host;
   if (SF_FOLD) fold_gll(G, a.xix_regular, a.jacobian_regular);
   dim3 grid(a.nelem), block(128);
-#define SF_K(S, T, O, V) hipLaunchKernelGGL((k_elastic_pt<S, T, O, V>), grid, block, 0, s, a, G)
-#define SF_KM(O)                                       \
-  if (att) {                                           \
-    if (att_variant == 1) SF_K(true, true, O, 1);      \
-    else if (att_variant == 2) SF_K(true, true, O, 2); \
-    else if (att_variant == 3) SF_K(true, true, O, 3); \
-    else if (att_variant == 4) SF_K(true, true, O, 4); \
-    else SF_K(true, true, O, 0);                       \
-  } else if (strain) SF_K(true, false, O, 0);          \
-  else SF_K(false, false, O, 0);
-  if (mode == 1) {
-    SF_KM(1)
-  } else if (mode == 2) {
-    SF_KM(2)
+#define SF_K(S, T, V) hipLaunchKernelGGL((k_elastic_pt<S, T, V>), grid, block, 0, s, a, G)
+  if (att) {
+    if (att_variant == 1) SF_K(true, true, 1);
+    else if (att_variant == 2) SF_K(true, true, 2);
+    else if (att_variant == 3) SF_K(true, true, 3);
+    else if (att_variant == 4) SF_K(true, true, 4);
+    else SF_K(true, true, 0);
+  } else if (strain) {
+    SF_K(true, false, 0);
   } else {
-    SF_KM(0)
+    SF_K(false, false, 0);
   }
-#undef SF_KM
 #undef SF_K
   SF_LAUNCH_CHECK("k_elastic_pt");
 }

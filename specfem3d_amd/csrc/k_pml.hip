@@ -12,9 +12,7 @@
 //     wavefront is one coalesced run. Per element, coefficient planes holding one value are read at
 //     one address, memory variables whose multiplier is zero over the element (most of them in
 //     face and edge regions) are not kept at all, and the remaining planes are packed;
-//   * the scatter is selected by MODE: 0 float atomics, 1 a local store for the ordered gather
-//     (one launch in both cases: the C-PML elements alone are too few to fill the chip colour by
-//     colour).
+//   * the local forces are stored for the gather assembly, like k_elastic_pt's.
 // Every sum keeps the reference's operand order; compiled twice (SF_EXACT = 1: no FMA contraction,
 // the CPU reference's rounding; SF_EXACT = 0: FMA, with the regular-element mapping folded into
 // the GLL tables as in k_elastic_pt).
@@ -51,7 +49,6 @@ __device__ __forceinline__ realw pml_conv(realw r, realw nw, realw od, realw c0,
 // dux_dyl_x, duy_dyl_y, duz_dyl_z, dux_dzl_x, duy_dzl_y, duz_dzl_z at 0..26; one-term ones at 27..38
 // (duz_dzl_y, duz_dyl_y, duy_dzl_z, duy_dyl_z | duz_dzl_x, duz_dxl_x, dux_dzl_z, dux_dxl_z |
 // duy_dyl_x, duy_dxl_x, dux_dyl_y, dux_dxl_y); displacement memory variables (c * 3 + s) at 39..47.
-template <int MODE>
 __global__ void __launch_bounds__(128) k_elastic_pml(PmlArgs A, GLLk G) {
   __shared__ realw sF[9][128];  // u (0..2), PML_displ_old (3..5), PML_displ_new (6..8)
   __shared__ realw sT[9][128];  // stress products t1 (0..2), t2 (3..5), t3 (6..8)
@@ -235,28 +232,21 @@ __global__ void __launch_bounds__(128) k_elastic_pml(PmlArgs A, GLLk G) {
   realw f[3];
   tile_divergence<1>(&sT[0][0], 128, gll_hpw(sG, irr != 0), sG + 50, i, j, k, f);
   const realw tot0 = f[0] + cpml[0], tot1 = f[1] + cpml[1], tot2 = f[2] + cpml[2];
-  if (MODE == 1) {
-    A.local_out[ep] = tot0;
-    A.local_out[A.nloc + ep] = tot1;
-    A.local_out[2 * A.nloc + ep] = tot2;
-  } else {
-    realw* a = A.accel + 3 * (int64_t)g;
-    atomicAdd(a + 0, -tot0);
-    atomicAdd(a + 1, -tot1);
-    atomicAdd(a + 2, -tot2);
-  }
+  realw* o = A.local_out + 3 * ep;
+  o[0] = tot0;
+  o[1] = tot1;
+  o[2] = tot2;
 }
 
 }  // namespace SF_VNS
 using namespace SF_VNS;
 
-void SFX(launch_elastic_pml)(hipStream_t s, const PmlArgs& a, int mode) {
+void SFX(launch_elastic_pml)(hipStream_t s, const PmlArgs& a) {
   if (a.nelem <= 0) return;
   GLLk G = g_gll_host;
   if (SF_FOLD) fold_gll(G, a.xix_regular, a.jacobian_regular);
   dim3 grid(a.nelem), block(128);
-  if (mode == 1) hipLaunchKernelGGL(k_elastic_pml<1>, grid, block, 0, s, a, G);
-  else hipLaunchKernelGGL(k_elastic_pml<0>, grid, block, 0, s, a, G);
+  hipLaunchKernelGGL(k_elastic_pml, grid, block, 0, s, a, G);
   SF_LAUNCH_CHECK("k_elastic_pml");
 }
 

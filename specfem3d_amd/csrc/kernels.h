@@ -41,6 +41,36 @@ void launch_corrector_predictor(hipStream_t s, int64_t n, realw* u, realw* v, re
                                 realw dt2_prev, realw dt, realw dt2, realw dtsq2, realw* old = nullptr,
                                 realw t1 = 0.f, realw t2 = 0.f);
 
+// Gather assembly: the stiffness launches store local forces (3 floats per slot e*125+p) and the pass
+// that needs the acceleration sums them, a point's slots in list order: a -= local[slot].
+enum : unsigned char {
+  AF_TERM = 1,  // boundary, coupling or source terms may have written the point's accel
+  AF_EDGE = 2   // point on the outer faces of the C-PML layers
+};
+struct GatherArgs {
+  int64_t g0, n;               // global points [g0, g0 + n)
+  const int* ptr;              // slot list of each global point: idx[ptr[g] .. ptr[g + 1])
+  const int* idx;
+  const realw* local;
+  const unsigned char* flags;  // AF_* per global point
+  int skip;                    // points with one of these flags take no contributions
+  int clean;                   // accel is zero at every point without AF_TERM (it need not be read)
+  realw *u, *v, *a;
+  const realw* rm;             // inverse mass, 3 per point
+  realw dt2p;                  // corrector: dt/2
+  realw dt, dt2, dtsq2;        // predictor
+  realw* old;                  // PML_displ_old = u + t1 v + t2 a of the corrected field, or null
+  realw t1, t2;
+};
+// what follows the sum: nothing (accel is left assembled), the corrector, or the corrector and the
+// predictor of the next step (accel left zero)
+enum { GATHER_ONLY = 0, GATHER_CORRECT = 1, GATHER_STEP = 2 };
+void launch_gather_update(hipStream_t s, const GatherArgs& a, int kind);
+// slot lists of the listed elements (k_assembly.hip); allocates ptr (nglob + 1) and idx (125 nelem)
+void build_slot_lists(hipStream_t s, int nglob, int nspec, int nelem, const int* list, const int* ibool, int*& ptr,
+                      int*& idx);
+void launch_mark_points(hipStream_t s, int n, const int* ig, unsigned char bit, unsigned char* flags);
+
 // element stiffness (k_elastic.hip / k_acoustic.hip)
 struct ElasticArgs {
   int nelem;
@@ -53,7 +83,6 @@ struct ElasticArgs {
   const float2* kappamu;
   const realw* displ;
   const realw* veloc;
-  realw* accel;
   realw deltat;
   realw* R;                // 18 planes of nloc
   realw* eps;              // 6 planes of nloc
@@ -65,12 +94,10 @@ struct ElasticArgs {
   realw* eps_tr3;          // nloc or null
   int64_t nloc;            // nspec*125
   realw alpha[3], beta[3], gamma[3];
-  realw* local_out;        // ordered assembly: 3 planes of nloc
+  realw* local_out;        // local forces, 3 per local point
 };
-// mode: 0 atomic scatter, 1 store local contributions (ordered gather), 2 plain read-modify-write
-// (the element list is one colour: its elements share no global point)
 // att_variant: scheduling of the attenuation state in the point kernel (k_elastic_pt's AV)
-void launch_elastic(hipStream_t s, const ElasticArgs& a, bool strain, bool att, bool exact, int mode,
+void launch_elastic(hipStream_t s, const ElasticArgs& a, bool strain, bool att, bool exact,
                     int att_variant);
 // deviatoric strain planes 0..4 and trace/3 of A.displ; with_trace also writes plane 5 = 3 * trace/3
 void launch_element_strain(hipStream_t s, const ElasticArgs& a, realw* eps, realw* eps_tr3, bool with_trace,
@@ -92,7 +119,6 @@ struct PmlArgs {
   const float2* kappamu;
   const realw* displ;
   const realw* veloc;
-  realw* accel;
   const realw* pml_old;    // 3*nglob
   // per C-PML element: [2 ic] bit m set if coefficient plane m is one value over the element,
   // [2 ic + 1] bit m set if state plane m is live (its multiplier plane is not all zero; dead planes
@@ -102,11 +128,9 @@ struct PmlArgs {
   realw* state;            // live state planes, 125 values each, packed per element in plane order
   const realw* coef;       // coefficient planes packed per element in plane order: 1 value if uniform, else 125
   realw t1, t2;            // deltatover2 (1 - 2 theta), deltatsqover2 (1 - theta)
-  realw* local_out;        // ordered assembly: 3 planes of nloc
-  int64_t nloc;
+  realw* local_out;        // local forces, 3 per local point
 };
-// mode: 0 atomic scatter, 1 store local contributions (ordered gather)
-void launch_elastic_pml(hipStream_t s, const PmlArgs& a, bool exact, int mode);
+void launch_elastic_pml(hipStream_t s, const PmlArgs& a, bool exact);
 // PML_displ_old at the listed points: u + t1 v + t2 a, with the pending corrector (a *= rmass,
 // v += dt2p a) applied first when dt2p_pending != 0
 void launch_pml_store_old(hipStream_t s, int n, const int* pts, const realw* u, const realw* v, const realw* a,

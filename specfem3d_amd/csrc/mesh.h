@@ -197,12 +197,11 @@ struct Mesh {
   // execution
   hipStream_t stream = nullptr;
   // Defaults for a host that never calls sf_set_options (the Fortran drop-in): the FMA build and,
-  // once prepare_fields_elastic_device knows whether attenuation is on, coloured assembly without it
-  // (float atomics are the limit of the light elastic kernel) and atomic assembly with it (the
-  // colour launches re-read more state than the atomics write back).
+  // once prepare_fields_elastic_device knows whether attenuation is on, element-order sums (fluid
+  // atomics with it).
   int exact = 0;                   // 1: kernels built without fused multiply-add (oracle order)
-  int assembly = -1;               // 0 atomic scatter-add, 1 ordered gather (oracle order), 2 coloured,
-                                   // -1 automatic (resolved at prepare_fields_elastic_device)
+  int assembly = -1;               // order of the element sums: 1 element order (oracle order), 2 colour
+                                   // order, 0 any (sf_set_options), -1 automatic
   int att_variant = 4;             // attenuation-state scheduling of the point kernel (0..4)
   int ac_kernel_dd = 0;            // 1: fluid kernels read the adjoint potential_dot_dot (misfit gradient)
   // deferred corrector (kernel_3) per field, fused into the next predictor when possible
@@ -210,11 +209,18 @@ struct Mesh {
   realw pending_dt2_el[2] = {0.f, 0.f};
   int pending_k3_ac[2] = {0, 0};
   realw pending_dt2_ac[2] = {0.f, 0.f};
-  // ordered-assembly structures (CSR of contributions per global point, sorted by element)
+  // gather assembly of the solid: slots e*125+p of each global point in list order (the processing
+  // order, or the colour order under assembly = 2), the C-PML elements last
   int* asm_ptr = nullptr;          // nglob+1
-  int* asm_idx = nullptr;          // slots e*125+p
-  realw* asm_buf = nullptr;        // 3*nspec*125 per-element local forces
-  int asm_ready = 0;
+  int* asm_idx = nullptr;
+  unsigned char* asm_flags = nullptr;          // AF_* per global point
+  realw* asm_buf[2] = {nullptr, nullptr};      // local forces of each field, 3 per local point
+  int asm_ready = 0;               // lists and flags match the element lists and terms
+  // local forces of a field wait to be summed: by the next update together with the corrector, or
+  // by whichever entry point reads or writes accel first
+  int pending_gather_el[2] = {0, 0};
+  int gather_skip_el[2] = {0, 0};  // AF_* of the points that the pending sum leaves out
+  int accel_clean[2] = {0, 0};     // accel is zero at every point without AF_TERM
   int* asm_ac_ptr = nullptr;       // same for the acoustic elements (1 component)
   int* asm_ac_idx = nullptr;
   realw* asm_ac_buf = nullptr;

@@ -1,0 +1,44 @@
+"""Gather assembly fused with the Newmark update: fields read and written between the steps, where the
+sum is taken early, the acceleration is not known to be zero, or both. Without FMA contraction every
+path sums in the oracle's order, so the fields equal its bit for bit."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from conftest import small_elastic_box, smooth_warp
+
+pytestmark = pytest.mark.gpu
+
+
+def put_fields(g, u, v, a):
+    n = C.c_int(u.size)
+    p = [x.ctypes.data_as(C.c_void_p) for x in (u, v, a)]
+    g.L.transfer_fields_el_to_device_(C.byref(n), *p, g.MP)
+
+
+@pytest.mark.parametrize("assembly", [0, 1])
+@pytest.mark.parametrize("n,warp", [(1, False), (2, True), (5, False)])
+def test_fields_between_steps(oracle_mod, n, warp, assembly):
+    from specfem3d_amd.solver import GPUSolver
+    db, src, rec = small_elastic_box(n=n, warp=smooth_warp(500.0 * n) if warp else None)
+    o = oracle_mod.OracleSolver(db, src, rec, "f32")
+    o.stf_table = src.stf_table(40)
+    o.run(6)
+    g = GPUSolver(db, src, rec, nstep=40, exact=True, assembly=assembly)
+    print(f"[gpu] gather n={n} warp={warp} assembly={assembly}", flush=True)
+    for _ in range(6):
+        g.step()
+    rng = np.random.default_rng(n)
+    u, v, a = (rng.normal(size=3 * db.nglob).astype(np.float32) * s for s in (1e-3, 1e-1, 1e1))
+    put_fields(g, u, v, a)            # an acceleration that is nonzero everywhere
+    o.displ[:], o.veloc[:], o.accel[:] = u, v, a
+    for k in range(6):
+        g.step()
+        o.run(1)
+        if k % 2:                     # sum and corrector before the next update
+            for x, y in zip(g.fields(), (o.displ, o.veloc, o.accel)):
+                assert np.array_equal(x, y), k
+    for x, y in zip(g.fields(), (o.displ, o.veloc, o.accel)):
+        assert np.array_equal(x, y)
+    g.close()
