@@ -84,6 +84,7 @@ struct Du9 {
   realw xx, xy, xz, yx, yy, yz, zx, zy, zz;
 };
 
+template <bool FOLD = SF_FOLD>
 __device__ __forceinline__ Du9 map_gradient(const Grad9& t, bool irr, const JacPt& J, realw xr) {
   Du9 d;
   if (irr) {
@@ -96,7 +97,7 @@ __device__ __forceinline__ Du9 map_gradient(const Grad9& t, bool irr, const JacP
     d.zx = J.xix * t.z1 + J.etax * t.z2 + J.gax * t.z3;
     d.zy = J.xiy * t.z1 + J.etay * t.z2 + J.gay * t.z3;
     d.zz = J.xiz * t.z1 + J.etaz * t.z2 + J.gaz * t.z3;
-  } else if (SF_FOLD) {
+  } else if (FOLD) {
     d.xx = t.x1; d.xy = t.x2; d.xz = t.x3;
     d.yx = t.y1; d.yy = t.y2; d.yz = t.y3;
     d.zx = t.z1; d.zy = t.z2; d.zz = t.z3;
@@ -128,6 +129,7 @@ __device__ __forceinline__ Sigma6 iso_stress(const Du9& d, realw kappal, realw m
 }
 
 // jacobian * sigma . (dxi/dx), (deta/dx), (dgamma/dx): t[0..2] xi, t[3..5] eta, t[6..8] gamma
+template <bool FOLD = SF_FOLD>
 __device__ __forceinline__ void stress_products(const Sigma6& s, bool irr, const JacPt& J, realw jacl, realw xr,
                                                 realw t[9]) {
   const realw syx = s.xy, szx = s.xz, szy = s.yz;
@@ -141,7 +143,7 @@ __device__ __forceinline__ void stress_products(const Sigma6& s, bool irr, const
     t[6] = jacl * (s.xx * J.gax + syx * J.gay + szx * J.gaz);
     t[7] = jacl * (s.xy * J.gax + s.yy * J.gay + szy * J.gaz);
     t[8] = jacl * (s.xz * J.gax + s.yz * J.gay + s.zz * J.gaz);
-  } else if (SF_FOLD) {
+  } else if (FOLD) {
     t[0] = s.xx; t[1] = s.xy; t[2] = s.xz;
     t[3] = syx;  t[4] = s.yy; t[5] = s.yz;
     t[6] = szx;  t[7] = szy;  t[8] = s.zz;
@@ -212,6 +214,28 @@ __device__ __forceinline__ void stage_gll(realw* sG, const GLLk& G, int lane) {
 __device__ __forceinline__ const realw* gll_hp(const realw* sG, bool irr) { return (SF_FOLD && !irr) ? sG + 75 : sG; }
 __device__ __forceinline__ const realw* gll_hpw(const realw* sG, bool irr) {
   return (SF_FOLD && !irr) ? sG + 100 : sG + 25;
+}
+
+// One line of five GLL points against the derivative tables, held by one lane: the coefficients have
+// constant indices and come from scalar registers, and each point of the line is read once instead
+// of once per output. Sums left to right, as tile_gradient and tile_divergence.
+__device__ __forceinline__ void line_gradient(const realw* hp, const realw in[5], realw out[5]) {
+#pragma unroll
+  for (int m = 0; m < 5; m++) {
+    realw r = hp[m * 5] * in[0];
+#pragma unroll
+    for (int l = 1; l < 5; l++) r = r + hp[m * 5 + l] * in[l];
+    out[m] = r;
+  }
+}
+__device__ __forceinline__ void line_divergence(const realw* hpw, const realw in[5], realw out[5]) {
+#pragma unroll
+  for (int m = 0; m < 5; m++) {
+    realw r = hpw[m] * in[0];
+#pragma unroll
+    for (int l = 1; l < 5; l++) r = r + hpw[l * 5 + m] * in[l];
+    out[m] = r;
+  }
 }
 
 __device__ __forceinline__ JacPt load_jac(const realw* J, int64_t P, int64_t q) {

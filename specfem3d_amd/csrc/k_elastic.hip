@@ -1,7 +1,8 @@
 // k_elastic.hip -- isotropic elastic / viscoelastic (3 SLS) element stiffness for NGLL=5.
 //
 // Restates compute_forces_viscoelastic.F90:33-962 (with the memory update of
-// compute_element_att_memory.f90:28-156) as one gfx950 kernel, k_elastic_pt:
+// compute_element_att_memory.f90:28-156) as two gfx950 kernels: k_elastic_line without attenuation
+// (described there) and k_elastic_pt with it:
 //   * a 128-thread workgroup (two wave64s) processes one element; lane p owns the GLL point
 //     p = i + 5 j + 25 k (125 of the 128 lanes busy) and all three contractions read the element
 //     tile staged in LDS;
@@ -9,7 +10,8 @@
 //     update that follows (k_gather_update): one launch over all elements, no atomics, no colours.
 //     Against float atomics the viscoelastic launch on 64x64x32 elements (28 layers solid) went from
 //     854 to 620 us (the atomics' write-back was 15 % of its traffic), and against eight colour
-//     launches the elastic one from 277 to 187 us there and from 41 to 14 us on 20x20x20;
+//     launches the elastic one from 277 to 187 us there and from 41 to 14 us on 20x20x20 (both of
+//     them this kernel without attenuation, which k_elastic_line has replaced);
 //   * workgroup ids are remapped so each XCD (8 per chip, dispatched round-robin) walks one
 //     contiguous range of elements and keeps the shared points of neighbours in its own L2.
 // The arithmetic order of every sum follows the reference (the five terms of each
@@ -95,11 +97,11 @@ __device__ __forceinline__ void load_att_state(const ElasticArgs& A, int e, int 
 typedef __attribute__((address_space(3))) void* sf_lds_ptr;
 typedef __attribute__((address_space(1))) void* sf_global_ptr;
 
-template <bool STRAIN, bool ATT, int AV>
+template <int AV>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(AV >= 2 ? 5 : 1)))
 k_elastic_pt(ElasticArgs A, GLLk G) {
-  constexpr bool LATE = ATT && (AV == 1 || AV == 2);
-  constexpr bool DL = ATT && AV == 4;
+  constexpr bool LATE = AV == 1 || AV == 2;
+  constexpr bool DL = AV == 4;
   __shared__ realw sU[6][128];            // u (0..2) and dt*v (3..5)
   __shared__ realw sX[DL ? 24 : 9][128];  // stress products (planes 0..8); with DL first the state
   realw(*const sT)[128] = sX;             // t1 (0..2), t2 (3..5), t3 (6..8)
@@ -123,7 +125,7 @@ k_elastic_pt(ElasticArgs A, GLLk G) {
   }
   const float2 km = A.kappamu[ep];
   realw Rv[6][3], Sn[6], fcv[3], fckv[3];
-  if (ATT && !DL) {
+  if (!DL) {
 #pragma unroll
     for (int cc = 0; cc < 6; cc++)
 #pragma unroll
@@ -134,15 +136,10 @@ k_elastic_pt(ElasticArgs A, GLLk G) {
   {
     const realw* d = A.displ + 3 * (int64_t)g;
     const realw u0 = d[0], u1 = d[1], u2 = d[2];
-    realw v0 = 0, v1 = 0, v2 = 0;
-    if (ATT) {
-      const realw* v = A.veloc + 3 * (int64_t)g;
-      v0 = v[0]; v1 = v[1]; v2 = v[2];
-    }
+    const realw* v = A.veloc + 3 * (int64_t)g;
+    const realw v0 = v[0], v1 = v[1], v2 = v[2];
     sU[0][p] = u0; sU[1][p] = u1; sU[2][p] = u2;
-    if (ATT) {
-      sU[3][p] = A.deltat * v0; sU[4][p] = A.deltat * v1; sU[5][p] = A.deltat * v2;
-    }
+    sU[3][p] = A.deltat * v0; sU[4][p] = A.deltat * v1; sU[5][p] = A.deltat * v2;
   }
   __syncthreads();
   if (DL) {
@@ -166,20 +163,16 @@ k_elastic_pt(ElasticArgs A, GLLk G) {
   const Grad9 tg = tile_gradient<1>(sU[0], sU[1], sU[2], hpg, i, j, k);
   const Du9 du = map_gradient(tg, irr != 0, J, A.xix_regular);
 
-  realw e_xx = 0, e_yy = 0, e_xy = 0, e_xz = 0, e_yz = 0, e_tr = 0;
-  if (STRAIN) {
-    Du9 st = du;
-    if (ATT) st = map_gradient(tile_gradient_continue<1>(tg, sU[3], sU[4], sU[5], hpg, i, j, k), irr != 0, J,
-                               A.xix_regular);
-    e_tr = (st.xx + st.yy + st.zz);
-    const realw templ = ONE_THIRD * (st.xx + st.yy + st.zz);
-    if (A.eps_tr3 && active) A.eps_tr3[ep] = templ;
-    e_xx = st.xx - templ;
-    e_yy = st.yy - templ;
-    e_xy = (realw)0.5 * (st.xy + st.yx);
-    e_xz = (realw)0.5 * (st.zx + st.xz);
-    e_yz = (realw)0.5 * (st.zy + st.yz);
-  }
+  const Du9 st = map_gradient(tile_gradient_continue<1>(tg, sU[3], sU[4], sU[5], hpg, i, j, k), irr != 0, J,
+                              A.xix_regular);
+  const realw e_tr = (st.xx + st.yy + st.zz);
+  const realw templ = ONE_THIRD * (st.xx + st.yy + st.zz);
+  if (A.eps_tr3 && active) A.eps_tr3[ep] = templ;
+  const realw e_xx = st.xx - templ;
+  const realw e_yy = st.yy - templ;
+  const realw e_xy = (realw)0.5 * (st.xy + st.yx);
+  const realw e_xz = (realw)0.5 * (st.zx + st.xz);
+  const realw e_yz = (realw)0.5 * (st.zy + st.yz);
 
   const realw kappal = km.x, mul = km.y;
   Sigma6 sg = iso_stress(du, kappal, mul);
@@ -193,36 +186,34 @@ k_elastic_pt(ElasticArgs A, GLLk G) {
 #pragma unroll
     for (int c = 0; c < 6; c++) Sn[c] = sX[18 + c][p];
   }
-  if (ATT) {
-    const realw rxx = (Rv[0][0] + Rv[0][1]) + Rv[0][2];
-    const realw ryy = (Rv[1][0] + Rv[1][1]) + Rv[1][2];
-    const realw rtr = (Rv[5][0] + Rv[5][1]) + Rv[5][2];
-    sg.xx = sg.xx - rxx - rtr;
-    sg.yy = sg.yy - ryy - rtr;
-    sg.zz = sg.zz + rxx + ryy - rtr;
-    sg.xy = sg.xy - ((Rv[2][0] + Rv[2][1]) + Rv[2][2]);
-    sg.xz = sg.xz - ((Rv[3][0] + Rv[3][1]) + Rv[3][2]);
-    sg.yz = sg.yz - ((Rv[4][0] + Rv[4][1]) + Rv[4][2]);
-    if (active) {
-      // memory-variable update (second-order RK) with old strain Sn and new strain Snp1
-      if (LATE) load_att_state(A, e, q, ep, nl, Sn, fcv, fckv);
-      const realw Snp1[6] = {e_xx, e_yy, e_xy, e_xz, e_yz, e_tr};
+  const realw rxx = (Rv[0][0] + Rv[0][1]) + Rv[0][2];
+  const realw ryy = (Rv[1][0] + Rv[1][1]) + Rv[1][2];
+  const realw rtr = (Rv[5][0] + Rv[5][1]) + Rv[5][2];
+  sg.xx = sg.xx - rxx - rtr;
+  sg.yy = sg.yy - ryy - rtr;
+  sg.zz = sg.zz + rxx + ryy - rtr;
+  sg.xy = sg.xy - ((Rv[2][0] + Rv[2][1]) + Rv[2][2]);
+  sg.xz = sg.xz - ((Rv[3][0] + Rv[3][1]) + Rv[3][2]);
+  sg.yz = sg.yz - ((Rv[4][0] + Rv[4][1]) + Rv[4][2]);
+  if (active) {
+    // memory-variable update (second-order RK) with old strain Sn and new strain Snp1
+    if (LATE) load_att_state(A, e, q, ep, nl, Sn, fcv, fckv);
+    const realw Snp1[6] = {e_xx, e_yy, e_xy, e_xz, e_yz, e_tr};
 #pragma unroll
-      for (int s = 0; s < 3; s++) {
-        const realw flk = kappal * fckv[s];
-        A.R[r_idx(e, 5 * 3 + s, q)] = A.alpha[s] * Rv[5][s] + flk * (A.beta[s] * Sn[5] + A.gamma[s] * Snp1[5]);
-        const realw flm = mul * fcv[s];
+    for (int s = 0; s < 3; s++) {
+      const realw flk = kappal * fckv[s];
+      A.R[r_idx(e, 5 * 3 + s, q)] = A.alpha[s] * Rv[5][s] + flk * (A.beta[s] * Sn[5] + A.gamma[s] * Snp1[5]);
+      const realw flm = mul * fcv[s];
 #pragma unroll
-        for (int cc = 0; cc < 5; cc++)
-          A.R[r_idx(e, cc * 3 + s, q)] = A.alpha[s] * Rv[cc][s] + flm * (A.beta[s] * Sn[cc] + A.gamma[s] * Snp1[cc]);
-      }
+      for (int cc = 0; cc < 5; cc++)
+        A.R[r_idx(e, cc * 3 + s, q)] = A.alpha[s] * Rv[cc][s] + flm * (A.beta[s] * Sn[cc] + A.gamma[s] * Snp1[cc]);
     }
   }
-  if (STRAIN && active) {
+  if (active) {
     realw* Ep = A.eps;
     Ep[eps_idx(e, 0, q)] = e_xx; Ep[eps_idx(e, 1, q)] = e_yy; Ep[eps_idx(e, 2, q)] = e_xy;
     Ep[eps_idx(e, 3, q)] = e_xz; Ep[eps_idx(e, 4, q)] = e_yz;
-    if (ATT) Ep[eps_idx(e, 5, q)] = e_tr;
+    Ep[eps_idx(e, 5, q)] = e_tr;
   }
 
   {
@@ -240,6 +231,165 @@ k_elastic_pt(ElasticArgs A, GLLk G) {
   o[0] = f[0];
   o[1] = f[1];
   o[2] = f[2];
+}
+
+// Elastic stiffness without attenuation: a 128-lane workgroup takes five elements, a lane one line of
+// five GLL points at a time (line_gradient, line_divergence). Lane (el, c) of 125 holds the gamma column
+// of c = i + 5 j, whose contraction stays in its registers, and for the other two directions the xi row
+// 5 c .. 5 c + 4 and the eta row (c % 5) + 25 (c / 5) + 5 l, read from and written back to LDS.
+//
+// k_elastic_pt reads 45 tile values and 15 coefficients from LDS per point and contraction stage,
+// 123 reads in all; here it is 33 reads and 12 writes per point, and the coefficients sit in scalar
+// registers. Planes A (u, then the xi derivatives, the xi products and their divergence) and B (the
+// same for eta) are reused in place: a row is read and written by one lane, and a point's values are
+// read and replaced by the lane of its column; only the xi derivatives need a barrier before they
+// replace u. 15 KB of LDS per workgroup, 61 to 80 VGPRs, 5 waves per SIMD. Per launch against
+// k_elastic_pt storing the same forces: 64x64x32 elements 187 -> 100 us (0.50 GB: the rate of a large
+// copy), 20x20x20 14.3 -> 12.5, 24^3 with strain 22.2 -> 19.5, irregular 43x37x29 89 -> 87 (its 40 B of
+// Jacobian terms per point were already the limit).
+// REG: no irregular element in the mesh (FMA build: the mapping is folded into the tables).
+template <bool STRAIN, bool REG>
+__global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk G) {
+  constexpr bool FOLD = REG && SF_FOLD;
+  constexpr int PL = 626;
+  __shared__ realw sA[3][PL], sB[3][PL];
+  __shared__ realw sW[25];
+  const int t = threadIdx.x;
+  const bool lane = t < 125;                       // lanes 125..127 shadow the last element's first points
+  const int el = lane ? t / 25 : 4, c = lane ? t - 25 * el : t - 125;
+  const int i = c % 5, j = c / 5;
+  const int ie = xcd_remap(blockIdx.x, gridDim.x) * 5 + el;
+  const bool active = lane && ie < A.nelem;
+  const int e = A.elems[ie < A.nelem ? ie : A.nelem - 1];
+  const int64_t ep = (int64_t)e * 125 + c;         // local point of k = 0
+  const int irr = REG ? 0 : A.irregular[e];
+  const int64_t jp = REG ? 0 : (int64_t)(irr ? irr - 1 : 0) * 125 + c;
+  if (t < 25) sW[t] = G.wxy[t];
+  float2 km[5];
+  realw d3[5][3];
+  {
+    realw u[3][5];
+    int g[5];
+#pragma unroll
+    for (int k = 0; k < 5; k++) g[k] = A.ibool[ep + 25 * k];
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+      const realw* d = A.displ + 3 * (int64_t)g[k];
+      u[0][k] = d[0]; u[1][k] = d[1]; u[2][k] = d[2];
+    }
+#pragma unroll
+    for (int k = 0; k < 5; k++) km[k] = A.kappamu[ep + 25 * k];
+    const int b = el * 125 + c;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      if (lane) {
+#pragma unroll
+        for (int k = 0; k < 5; k++) sA[a][b + 25 * k] = u[a][k];
+      }
+      realw r[5];
+      line_gradient(G.hp, u[a], r);
+#pragma unroll
+      for (int k = 0; k < 5; k++) d3[k][a] = r[k];
+    }
+  }
+  lds_barrier();
+  const int bx = el * 125 + 5 * c, by = el * 125 + i + 25 * j;  // first points of the lane's two rows
+  realw x[3][5];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    realw r[5], y[5];
+#pragma unroll
+    for (int l = 0; l < 5; l++) {
+      r[l] = sA[a][bx + l];
+      y[l] = sA[a][by + 5 * l];
+    }
+    line_gradient(G.hp, r, x[a]);
+    line_gradient(G.hp, y, r);
+    if (lane) {
+#pragma unroll
+      for (int l = 0; l < 5; l++) sB[a][by + 5 * l] = r[l];
+    }
+  }
+  lds_barrier();                                   // every row of u has been read
+  if (lane) {
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+      for (int l = 0; l < 5; l++) sA[a][bx + l] = x[a][l];
+  }
+  lds_barrier();
+  const realw ONE_THIRD = (realw)1 / (realw)3;
+#pragma unroll
+  for (int k = 0; k < 5; k++) {
+    const int b = el * 125 + c + 25 * k;
+    const Grad9 tg = {sA[0][b], sA[1][b], sA[2][b], sB[0][b], sB[1][b], sB[2][b], d3[k][0], d3[k][1], d3[k][2]};
+    JacPt J = {};
+    realw jacl = A.jacobian_regular;
+    if (!REG && irr) {
+      J = load_jac(A.jac, A.jac_plane, jp + 25 * k);
+      jacl = J.jac;
+    }
+    const Du9 du = map_gradient<FOLD>(tg, irr != 0, J, A.xix_regular);
+    if (STRAIN) {
+      const realw templ = ONE_THIRD * (du.xx + du.yy + du.zz);
+      if (active) {
+        if (A.eps_tr3) A.eps_tr3[ep + 25 * k] = templ;
+        const int p = c + 25 * k;
+        A.eps[eps_idx(e, 0, p)] = du.xx - templ;
+        A.eps[eps_idx(e, 1, p)] = du.yy - templ;
+        A.eps[eps_idx(e, 2, p)] = (realw)0.5 * (du.xy + du.yx);
+        A.eps[eps_idx(e, 3, p)] = (realw)0.5 * (du.zx + du.xz);
+        A.eps[eps_idx(e, 4, p)] = (realw)0.5 * (du.zy + du.yz);
+      }
+    }
+    const Sigma6 sg = iso_stress(du, km[k].x, km[k].y);
+    realw s[9];
+    stress_products<FOLD>(sg, irr != 0, J, jacl, A.xix_regular, s);
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      if (lane) {
+        sA[a][b] = s[a];
+        sB[a][b] = s[3 + a];
+      }
+      d3[k][a] = s[6 + a];
+    }
+  }
+  lds_barrier();
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    realw r[5], y[5], o[5];
+#pragma unroll
+    for (int l = 0; l < 5; l++) {
+      r[l] = sA[a][bx + l];
+      y[l] = sB[a][by + 5 * l];
+    }
+    line_divergence(G.hpw, r, o);
+    if (lane) {
+#pragma unroll
+      for (int l = 0; l < 5; l++) sA[a][bx + l] = o[l];
+    }
+    line_divergence(G.hpw, y, o);
+    if (lane) {
+#pragma unroll
+      for (int l = 0; l < 5; l++) sB[a][by + 5 * l] = o[l];
+    }
+#pragma unroll
+    for (int k = 0; k < 5; k++) r[k] = d3[k][a];
+    line_divergence(G.hpw, r, o);
+#pragma unroll
+    for (int k = 0; k < 5; k++) d3[k][a] = o[k];
+  }
+  lds_barrier();
+  if (!active) return;
+  const realw w3 = sW[i * 5 + j];
+#pragma unroll
+  for (int k = 0; k < 5; k++) {
+    const int b = el * 125 + c + 25 * k;
+    const realw w1 = sW[j * 5 + k], w2 = sW[i * 5 + k];
+    realw* o = A.local_out + 3 * (ep + 25 * k);
+#pragma unroll
+    for (int a = 0; a < 3; a++) o[a] = w1 * sA[a][b] + w2 * sB[a][b] + w3 * d3[k][a];
+  }
 }
 
 // element strain of a displacement field (compute_element_strain.F90:28-130); one lane per point
@@ -328,17 +478,31 @@ void SFX(launch_elastic)(hipStream_t s, const ElasticArgs& a, bool strain, bool 
   GLLk G = g_gll_host;
   if (SF_FOLD) fold_gll(G, a.xix_regular, a.jacobian_regular);
   dim3 grid(a.nelem), block(128);
-#define SF_K(S, T, V) hipLaunchKernelGGL((k_elastic_pt<S, T, V>), grid, block, 0, s, a, G)
+#define SF_K(V) hipLaunchKernelGGL((k_elastic_pt<V>), grid, block, 0, s, a, G)
   if (att) {
-    if (att_variant == 1) SF_K(true, true, 1);
-    else if (att_variant == 2) SF_K(true, true, 2);
-    else if (att_variant == 3) SF_K(true, true, 3);
-    else if (att_variant == 4) SF_K(true, true, 4);
-    else SF_K(true, true, 0);
-  } else if (strain) {
-    SF_K(true, false, 0);
+    if (att_variant == 1) SF_K(1);
+    else if (att_variant == 2) SF_K(2);
+    else if (att_variant == 3) SF_K(3);
+    else if (att_variant == 4) SF_K(4);
+    else SF_K(0);
   } else {
-    SF_K(false, false, 0);
+    const bool reg = a.jac_plane == 0;  // no irregular element in the mesh
+    if (reg && SF_FOLD) {
+      for (int q = 0; q < 25; q++) {
+        G.hp[q] = G.hpr[q];
+        G.hpw[q] = G.hpwr[q];
+      }
+    }
+    const dim3 grid5((a.nelem + 4) / 5);
+#define SF_L(S, R) hipLaunchKernelGGL((k_elastic_line<S, R>), grid5, block, 0, s, a, G)
+    if (strain) {
+      if (reg) SF_L(true, true);
+      else SF_L(true, false);
+    } else {
+      if (reg) SF_L(false, true);
+      else SF_L(false, false);
+    }
+#undef SF_L
   }
 #undef SF_K
   SF_LAUNCH_CHECK("k_elastic_pt");

@@ -42,3 +42,29 @@ def test_fields_between_steps(oracle_mod, n, warp, assembly):
     for x, y in zip(g.fields(), (o.displ, o.veloc, o.accel)):
         assert np.array_equal(x, y)
     g.close()
+
+
+@pytest.mark.parametrize("n", [2, 3, 6])
+def test_mixed_elements(oracle_mod, n):
+    """Cubes and irregular elements in one workgroup (five elements, a lane one line of points), element
+    counts with every remainder: 8, 27, 216."""
+    from specfem3d_amd.solver import GPUSolver
+    L = 500.0 * n
+
+    def bend(x, y, z):                # the element corners inside x < 3L/4, y < 3L/4 move, the others stay
+        d = 30.0 * ((x > 0) & (x < 0.75 * L) & (y > 0) & (y < 0.75 * L) & (z < 0) & (z > -L))
+        return x + d, y - 0.5 * d, z + 0.7 * d
+
+    db, src, rec = small_elastic_box(n=n, warp=bend)
+    print(f"[gpu] mixed n={n} irregular={db.nspec_irregular} of {db.nspec}", flush=True)
+    assert db.nspec_irregular > 0 and (n < 3 or db.nspec_irregular < db.nspec)
+    ref = oracle_mod.OracleSolver(db, src, rec, "f32").run(60)
+    g = GPUSolver(db, src, rec, nstep=60, exact=True, assembly=1)
+    out = g.run().copy()
+    g.close()
+    assert np.abs(ref).max() > 0 and np.array_equal(out, ref)
+    g = GPUSolver(db, src, rec, nstep=60, exact=False, assembly=-1)
+    fast = g.run().copy()
+    g.close()
+    e = np.linalg.norm((fast - ref).astype(np.float64)) / np.linalg.norm(ref.astype(np.float64))
+    assert e < 1e-5, e
