@@ -753,8 +753,11 @@ static void build_colors(Mesh* m, const std::vector<int>& elems, int*& d_list, i
 // order, or in the colour order under assembly = 2 (the sums a coloured scatter makes, bit for bit),
 // those of the C-PML elements last (compute_forces_viscoelastic, then compute_forces_viscoelastic_PML).
 void ensure_gather_assembly(Mesh* m, int f) {
-  if (!m->asm_buf[f]) m->asm_buf[f] = dmalloc<realw>(3 * (int64_t)m->nspec * 125);
+  const int eb = 20;  // elements per block of slots: a multiple of the five of a k_elastic_line workgroup
+  const int first_pml = (m->nspec_elastic + eb - 1) / eb * eb;
+  if (!m->asm_buf[f]) m->asm_buf[f] = dmalloc<realw>(3 * 125 * ((int64_t)m->nspec + 2 * eb));  // both lists, rounded up
   if (m->asm_ready) return;
+  flush_all(m);       // local forces in the old slots
   if (m->assembly == 2) ensure_element_colors(m);
   const int* first = m->assembly == 2 && m->el_color_elems ? m->el_color_elems : m->elastic_elems;
   int* lst = dmalloc<int>(m->nspec_elastic + m->pml_n);
@@ -762,15 +765,23 @@ void ensure_gather_assembly(Mesh* m, int f) {
   if (m->pml_n)
     SF_CHECK(hipMemcpyAsync(lst + m->nspec_elastic, m->pml_elems, sizeof(int) * m->pml_n, hipMemcpyDeviceToDevice,
                             m->stream));
-  dfree(m->asm_ptr);
   dfree(m->asm_idx);
-  build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_elastic + m->pml_n, lst, m->ibool, m->asm_ptr, m->asm_idx);
+  int* ptr = nullptr;
+  m->asm_pos0 = first_pml;
+  m->asm_eb = build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_elastic + m->pml_n, lst,
+                               m->elastic_launch ? m->elastic_launch : m->elastic_elems, m->nspec_elastic, first_pml,
+                               eb, m->ibool, ptr, m->asm_idx);
   dfree(lst);
-  if (!m->asm_flags) m->asm_flags = dmalloc<unsigned char>(m->nglob);
-  SF_CHECK(hipMemsetAsync(m->asm_flags, 0, (size_t)m->nglob, m->stream));
+  if (!m->asm_info) {
+    m->asm_info = dmalloc<uint16_t>(m->nglob);
+    m->asm_base = dmalloc<int>((m->el_n + 63) / 64);
+    m->rmass1 = dmalloc<realw>(m->nglob);
+  }
+  launch_gather_info(m->stream, m->el_g0, m->el_n, ptr, m->rmass, m->asm_info, m->asm_base, m->rmass1);
   for (const FacePoints* fp : {&m->abs_el, &m->coupling, &m->src_pts, &m->adj_pts})
-    launch_mark_points(m->stream, fp->n, fp->iglob, AF_TERM, m->asm_flags);
-  launch_mark_points(m->stream, m->pml_nbc, m->pml_bc_pts, AF_EDGE, m->asm_flags);
+    launch_mark_points(m->stream, fp->n, fp->iglob, AF_TERM, m->asm_info);
+  launch_mark_points(m->stream, m->pml_nbc, m->pml_bc_pts, AF_EDGE, m->asm_info);
+  dfree(ptr);
   m->asm_ready = 1;
 }
 
@@ -779,8 +790,10 @@ void ensure_gather_assembly(Mesh* m, int f) {
 void release_gather_assembly(Mesh* m) {
   flush_all(m);
   SF_CHECK(hipStreamSynchronize(m->stream));
-  dfree(m->asm_ptr);
   dfree(m->asm_idx);
+  dfree(m->asm_info);
+  dfree(m->asm_base);
+  dfree(m->rmass1);
   dfree(m->asm_buf[0]);
   dfree(m->asm_buf[1]);
   m->asm_ready = 0;
@@ -789,8 +802,8 @@ void release_gather_assembly(Mesh* m) {
 // the same for the fluid (ordered sums of the acoustic stiffness)
 static void prepare_acoustic_gather(Mesh* m) {
   if (m->asm_ac_buf || m->nspec_acoustic <= 0 || !m->acoustic_elems) return;
-  build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_acoustic, m->acoustic_elems, m->ibool, m->asm_ac_ptr,
-                   m->asm_ac_idx);
+  (void)build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_acoustic, m->acoustic_elems, nullptr, 0, 0, 1,
+                         m->ibool, m->asm_ac_ptr, m->asm_ac_idx);
   m->asm_ac_buf = dmalloc<realw>((int64_t)m->nspec * 125);
 }
 
@@ -1211,7 +1224,7 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
   dfree(m->rec_ispec); dfree(m->rec_el_list); dfree(m->rec_ac_list);
   dfree(m->seismo_d); dfree(m->seismo_v); dfree(m->seismo_a); dfree(m->seismo_p);
   dfree(m->rho_kl); dfree(m->mu_kl); dfree(m->kappa_kl); dfree(m->rho_ac_kl); dfree(m->kappa_ac_kl);
-  dfree(m->asm_ptr); dfree(m->asm_idx); dfree(m->asm_flags); dfree(m->asm_buf[0]); dfree(m->asm_buf[1]);
+  dfree(m->asm_idx); dfree(m->asm_info); dfree(m->asm_base); dfree(m->rmass1); dfree(m->asm_buf[0]); dfree(m->asm_buf[1]);
   dfree(m->pml_elems); dfree(m->pml_cpml);
   dfree(m->pml_state); dfree(m->pml_coef); dfree(m->pml_masks); dfree(m->pml_off);
   dfree(m->pml_old); dfree(m->pml_pts); dfree(m->pml_bc_pts);
@@ -1302,7 +1315,7 @@ extern "C" void sf_set_element_order(long* Mesh_pointer, int n, const int* order
   dfree(m->elastic_launch);
   m->elastic_launch = dupload(lst.data(), (int64_t)lst.size());
   if (m->el_color_elems) build_colors(m, lst, m->el_color_elems, m->el_color_off, m->el_ncolor);
-  if (m->assembly == 2) m->asm_ready = 0;  // the sums follow the colours
+  m->asm_ready = 0;  // the slots follow the launch order (and the sums the colours)
 }
 
 // Greedy element colouring used by assembly = 2 (host only, no device needed): colour[q] of

@@ -37,16 +37,17 @@ static GatherArgs gather_args(Mesh* m, int f) {
   std::memset(&a, 0, sizeof(a));
   a.g0 = m->el_g0;  // only the elastic range changes (see Mesh::el_g0)
   a.n = m->el_n;
-  a.ptr = m->asm_ptr;
+  a.info = m->asm_info;
+  a.base = m->asm_base;
   a.idx = m->asm_idx;
   a.local = m->asm_buf[f];
-  a.flags = m->asm_flags;
   a.skip = m->gather_skip_el[f];
   a.clean = m->accel_clean[f];
   a.u = m->el[f].displ;
   a.v = m->el[f].veloc;
   a.a = m->el[f].accel;
   a.rm = m->rmass;
+  a.rm1 = m->rmass1;
   a.dt2p = m->pending_dt2_el[f];
   return a;
 }
@@ -112,6 +113,7 @@ static ElasticArgs elastic_args(Mesh* m, int f, realw deltat) {
     a.gamma[s] = f ? m->b_gammaval[s] : m->gammaval[s];
   }
   a.local_out = m->asm_buf[f];
+  a.eb = m->asm_eb;
   return a;
 }
 
@@ -148,6 +150,8 @@ void elastic_forces(Mesh* m, int f, realw deltat, bool strain, bool att) {
     P.t1 = m->pml_t1;
     P.t2 = m->pml_t2;
     P.local_out = m->asm_buf[0];
+    P.eb = m->asm_eb;
+    P.pos0 = m->asm_pos0;
     if (timed && !whole) SF_CHECK(hipEventRecord(m->timing_ev[2 * m->timing_count], m->stream));
     launch_elastic_pml(m->stream, P, m->exact != 0);
   }

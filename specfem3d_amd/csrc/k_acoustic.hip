@@ -108,7 +108,7 @@ __global__ void __launch_bounds__(128) k_acoustic(AcousticArgs A, GLLk G) {
     }
     const realw f = G.wxy[j * 5 + k] * n1 + G.wxy[i * 5 + k] * n2 + G.wxy[i * 5 + j] * n3;
     if (MODE == 1) {
-      A.local_out[(int64_t)e * 125 + c + 25 * k] = f;
+      A.local_out[(int64_t)ie * 125 + c + 25 * k] = f;
     } else if (MODE == 2) {
       A.potdd[g[k]] = A.potdd[g[k]] + (-f);
     } else {

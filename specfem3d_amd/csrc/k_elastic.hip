@@ -227,7 +227,7 @@ k_elastic_pt(ElasticArgs A, GLLk G) {
 
   realw f[3];
   tile_divergence<1>(&sT[0][0], 128, gll_hpw(sG, irr != 0), sG + 50, i, j, k, f);
-  realw* o = A.local_out + 3 * ep;
+  realw* o = A.local_out + 3 * (int64_t)gather_slot(ie, q / 5, i, A.eb);
   o[0] = f[0];
   o[1] = f[1];
   o[2] = f[2];
@@ -382,11 +382,12 @@ __global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk G) {
   lds_barrier();
   if (!active) return;
   const realw w3 = sW[i * 5 + j];
+  const int slot = gather_slot(ie, j, i, A.eb);    // of k = 0
 #pragma unroll
   for (int k = 0; k < 5; k++) {
     const int b = el * 125 + c + 25 * k;
     const realw w1 = sW[j * 5 + k], w2 = sW[i * 5 + k];
-    realw* o = A.local_out + 3 * (ep + 25 * k);
+    realw* o = A.local_out + 3 * (int64_t)(slot + k * 25 * A.eb);
 #pragma unroll
     for (int a = 0; a < 3; a++) o[a] = w1 * sA[a][b] + w2 * sB[a][b] + w3 * d3[k][a];
   }

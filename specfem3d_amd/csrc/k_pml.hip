@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(128) k_elastic_pml(PmlArgs A, GLLk G) {
   realw f[3];
   tile_divergence<1>(&sT[0][0], 128, gll_hpw(sG, irr != 0), sG + 50, i, j, k, f);
   const realw tot0 = f[0] + cpml[0], tot1 = f[1] + cpml[1], tot2 = f[2] + cpml[2];
-  realw* o = A.local_out + 3 * ep;
+  realw* o = A.local_out + 3 * (int64_t)gather_slot(A.pos0 + ie, q / 5, i, A.eb);
   o[0] = tot0;
   o[1] = tot1;
   o[2] = tot2;

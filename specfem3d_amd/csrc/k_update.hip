@@ -138,37 +138,70 @@ __global__ void k_zero_points(int n, const int* __restrict__ pts, realw* __restr
 // read-modify-write launch per element colour. A store of the local forces and this pass move 24 B
 // per local point plus 4 B of slot index; a colour launch reads and writes 24 B of accel for each of
 // the point's elements, and eight small launches leave most of the chip idle on small meshes.
-// Stiffness and update per step, before (colours without attenuation, atomics with it) and after:
-// 20x20x20 elastic 50 -> 25 us, 43x37x29 irregular 193 -> 152, 64x64x32 elastic 383 -> 381 (this pass
-// 194 us, 0.81 GB: bound by HBM), 64x64x32 fluid over viscoelastic 958 -> 817.
+// Stiffness and update per step, before (colours without attenuation, atomics with it) and after,
+// with the point-per-lane stiffness: 20x20x20 elastic 50 -> 25 us, 43x37x29 irregular 193 -> 152,
+// 64x64x32 fluid over viscoelastic 958 -> 817.
 //
-// The slots of 64 consecutive points lie in neighbouring elements, and consecutive blocks of one XCD
-// take consecutive points, so the rest of a fetched line is used from that XCD's L2.
+// The pass is bound by HBM: 0.72 GB and 150 us on 64x64x32 elements. It took 194 us with three
+// masses per point and a pointer array (0.81 GB) and 185 us without; the rest of the way came from
+// the slots' order. Consecutive points run through consecutive elements (a structured numbering) or
+// through one element (points numbered element by element): with one element's forces after the
+// other's, a wave over a structured mesh takes 48 B out of each of 16 lines. build_slot_lists counts
+// the lines of both orders and takes blocks of 20 elements (gather_slot) where those are fewer: 150
+// us, and 99 -> 104 us for the stiffness launch that writes them (621 -> 643 with attenuation, one
+// element per workgroup); blocks of 5, 10 and 40 elements: 156, 152, 149 us.
 // `clean`: accel is known to be zero away from AF_TERM points (the previous pass left it so), and is
 // neither read nor cleared there.
+// The number of slots comes with the flags, 2 B per point, and the position of a point's first slot
+// from a scan over the wave's 64 points. The three inverse masses of a point are equal away from the
+// absorbing faces and read as one value there. Each XCD takes its blocks backwards: the element
+// launches before and after go forwards, so both ends of this pass meet what the other pass left in
+// the caches (188 -> 185 us forwards to backwards on 64x64x32).
+
+// inclusive prefix sum over a wave64 (row shifts by 1, 2, 4, 8, then the last lanes of rows 0 / 0..1
+// broadcast into the rows behind)
+__device__ __forceinline__ int wave_prefix(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+  return x;
+}
+
 template <int KIND, bool OLD>
 __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
   const int nb = (int)gridDim.x, b = (int)blockIdx.x;
-  const int q = nb >> 3, r = nb & 7, x = b & 7;  // contiguous blocks per XCD
-  const int64_t t = (int64_t)(x * q + (x < r ? x : r) + (b >> 3)) * 256 + threadIdx.x;
-  if (t >= A.n) return;
+  const int q = nb >> 3, r = nb & 7, x = b & 7;  // contiguous blocks per XCD, last one first
+  const int last = x < r ? q : q - 1;
+  const int64_t t = (int64_t)(x * q + (x < r ? x : r) + last - (b >> 3)) * 256 + threadIdx.x;
   const int64_t g = A.g0 + t;
-  const int p0 = A.ptr[g];
-  int p1 = A.ptr[g + 1];
-  const int fl = A.flags[g];
+  const int fl = t < A.n ? A.info[g] : 0;
+  const int cnt = fl >> AF_COUNT;
+  const int p1w = wave_prefix(cnt);               // every lane of the wave takes part
+  if (t >= A.n) return;
+  int p1 = A.base[t >> 6] + p1w;
+  const int p0 = p1 - cnt;
   const bool full = !A.clean || (fl & AF_TERM);
   realw u[3], v[3], m[3], a[3] = {0.f, 0.f, 0.f};
+  if (KIND != GATHER_ONLY) {
+    m[0] = A.rm1[g];
+    m[1] = m[0];
+    m[2] = m[0];
+  }
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    if (KIND != GATHER_ONLY) {
-      v[c] = A.v[3 * g + c];
-      m[c] = A.rm[3 * g + c];
-    }
+    if (KIND != GATHER_ONLY) v[c] = A.v[3 * g + c];
     if (KIND == GATHER_STEP) u[c] = A.u[3 * g + c];
   }
   if (full) {
 #pragma unroll
     for (int c = 0; c < 3; c++) a[c] = A.a[3 * g + c];
+  }
+  if (KIND != GATHER_ONLY && (fl & AF_MASS3)) {
+    m[1] = A.rm[3 * g + 1];
+    m[2] = A.rm[3 * g + 2];
   }
   if (fl & A.skip) p1 = p0;
   for (int s = p0; s < p1; s += 4) {  // four slots in flight (an interior face point has two)

@@ -41,22 +41,32 @@ void launch_corrector_predictor(hipStream_t s, int64_t n, realw* u, realw* v, re
                                 realw dt2_prev, realw dt, realw dt2, realw dtsq2, realw* old = nullptr,
                                 realw t1 = 0.f, realw t2 = 0.f);
 
-// Gather assembly: the stiffness launches store local forces (3 floats per slot e*125+p) and the pass
-// that needs the acceleration sums them, a point's slots in list order: a -= local[slot].
-enum : unsigned char {
-  AF_TERM = 1,  // boundary, coupling or source terms may have written the point's accel
-  AF_EDGE = 2   // point on the outer faces of the C-PML layers
+// Gather assembly: the stiffness launches store local forces, 3 floats per slot, and the pass that
+// needs the acceleration sums them, a point's slots in list order: a -= local[slot].
+// The slot of point p = 5 row + i of the element at launch position pos: blocks of `eb` elements hold
+// row by row the elements' five points, so that a row of points that runs through the elements of a
+// block is contiguous (eb = 1: one element after the other).
+__host__ __device__ __forceinline__ int gather_slot(int pos, int row, int i, int eb) {
+  const int b = pos / eb;
+  return b * eb * 125 + (row * eb + (pos - b * eb)) * 5 + i;
+}
+enum : uint16_t {
+  AF_TERM = 1,   // boundary, coupling or source terms may have written the point's accel
+  AF_EDGE = 2,   // point on the outer faces of the C-PML layers
+  AF_MASS3 = 4,  // the point's three inverse masses differ (implicit Stacey term)
+  AF_COUNT = 3   // shift of the number of slots
 };
 struct GatherArgs {
   int64_t g0, n;               // global points [g0, g0 + n)
-  const int* ptr;              // slot list of each global point: idx[ptr[g] .. ptr[g + 1])
-  const int* idx;
+  const uint16_t* info;        // AF_* and the number of slots << AF_COUNT, per global point
+  const int* base;             // first slot entry of each 64 points from g0 on
+  const int* idx;              // slots of every point, one point after the other
   const realw* local;
-  const unsigned char* flags;  // AF_* per global point
   int skip;                    // points with one of these flags take no contributions
   int clean;                   // accel is zero at every point without AF_TERM (it need not be read)
   realw *u, *v, *a;
-  const realw* rm;             // inverse mass, 3 per point
+  const realw* rm;             // inverse mass, 3 per point (read at AF_MASS3 points)
+  const realw* rm1;            // ... and 1 per point (the others)
   realw dt2p;                  // corrector: dt/2
   realw dt, dt2, dtsq2;        // predictor
   realw* old;                  // PML_displ_old = u + t1 v + t2 a of the corrected field, or null
@@ -66,10 +76,16 @@ struct GatherArgs {
 // predictor of the next step (accel left zero)
 enum { GATHER_ONLY = 0, GATHER_CORRECT = 1, GATHER_STEP = 2 };
 void launch_gather_update(hipStream_t s, const GatherArgs& a, int kind);
-// slot lists of the listed elements (k_assembly.hip); allocates ptr (nglob + 1) and idx (125 nelem)
-void build_slot_lists(hipStream_t s, int nglob, int nspec, int nelem, const int* list, const int* ibool, int*& ptr,
-                      int*& idx);
-void launch_mark_points(hipStream_t s, int n, const int* ig, unsigned char bit, unsigned char* flags);
+// slot lists (k_assembly.hip): the elements of `order` give the order of the sums, those of `launch`
+// (nelem_launch of them) the slots, `pos0` launch positions on for the elements behind; allocates ptr
+// (nglob + 1) and idx (125 nelem). lines: cache lines that the waves of a pass over all points touch
+// with eb = 1 and with `eb`; idx holds slots for the returned one of the two.
+int build_slot_lists(hipStream_t s, int nglob, int nspec, int nelem, const int* order, const int* launch, int nlaunch,
+                     int pos0, int eb, const int* ibool, int*& ptr, int*& idx);
+void launch_mark_points(hipStream_t s, int n, const int* ig, uint16_t bit, uint16_t* info);
+// info (flags to be marked afterwards), base and rm1 of GatherArgs from the slot lists and the masses
+void launch_gather_info(hipStream_t s, int64_t g0, int64_t n, const int* ptr, const realw* rm, uint16_t* info,
+                        int* base, realw* rm1);
 
 // element stiffness (k_elastic.hip / k_acoustic.hip)
 struct ElasticArgs {
@@ -94,7 +110,8 @@ struct ElasticArgs {
   realw* eps_tr3;          // nloc or null
   int64_t nloc;            // nspec*125
   realw alpha[3], beta[3], gamma[3];
-  realw* local_out;        // local forces, 3 per local point
+  realw* local_out;        // local forces, 3 per slot (gather_slot)
+  int eb;
 };
 // att_variant: scheduling of the attenuation state in the point kernel (k_elastic_pt's AV)
 void launch_elastic(hipStream_t s, const ElasticArgs& a, bool strain, bool att, bool exact,
@@ -128,7 +145,8 @@ struct PmlArgs {
   realw* state;            // live state planes, 125 values each, packed per element in plane order
   const realw* coef;       // coefficient planes packed per element in plane order: 1 value if uniform, else 125
   realw t1, t2;            // deltatover2 (1 - 2 theta), deltatsqover2 (1 - theta)
-  realw* local_out;        // local forces, 3 per local point
+  realw* local_out;        // local forces, 3 per slot (gather_slot)
+  int eb, pos0;            // ... pos0: launch position of the first listed element
 };
 void launch_elastic_pml(hipStream_t s, const PmlArgs& a, bool exact);
 // PML_displ_old at the listed points: u + t1 v + t2 a, with the pending corrector (a *= rmass,

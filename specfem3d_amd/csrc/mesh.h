@@ -209,12 +209,15 @@ struct Mesh {
   realw pending_dt2_el[2] = {0.f, 0.f};
   int pending_k3_ac[2] = {0, 0};
   realw pending_dt2_ac[2] = {0.f, 0.f};
-  // gather assembly of the solid: slots e*125+p of each global point in list order (the processing
-  // order, or the colour order under assembly = 2), the C-PML elements last
-  int* asm_ptr = nullptr;          // nglob+1
+  // gather assembly of the solid: slots of each global point in list order (the processing order, or
+  // the colour order under assembly = 2), the C-PML elements last
   int* asm_idx = nullptr;
-  unsigned char* asm_flags = nullptr;          // AF_* per global point
-  realw* asm_buf[2] = {nullptr, nullptr};      // local forces of each field, 3 per local point
+  int asm_eb = 1;                  // elements per block of slots (gather_slot)
+  int asm_pos0 = 0;                // launch position of the first C-PML element
+  uint16_t* asm_info = nullptr;    // AF_* and the number of slots, per global point
+  int* asm_base = nullptr;         // first slot entry of each 64 points of the elastic range
+  realw* rmass1 = nullptr;         // inverse mass of the points whose three are equal (nglob)
+  realw* asm_buf[2] = {nullptr, nullptr};      // local forces of each field, 3 per slot
   int asm_ready = 0;               // lists and flags match the element lists and terms
   // local forces of a field wait to be summed: by the next update together with the corrector, or
   // by whichever entry point reads or writes accel first

@@ -44,10 +44,11 @@ def test_fields_between_steps(oracle_mod, n, warp, assembly):
     g.close()
 
 
+@pytest.mark.parametrize("order", [None, "morton"])
 @pytest.mark.parametrize("n", [2, 3, 6])
-def test_mixed_elements(oracle_mod, n):
+def test_mixed_elements(oracle_mod, n, order):
     """Cubes and irregular elements in one workgroup (five elements, a lane one line of points), element
-    counts with every remainder: 8, 27, 216."""
+    counts with every remainder: 8, 27, 216; the launch order moves the slots, not the sums."""
     from specfem3d_amd.solver import GPUSolver
     L = 500.0 * n
 
@@ -59,7 +60,7 @@ def test_mixed_elements(oracle_mod, n):
     print(f"[gpu] mixed n={n} irregular={db.nspec_irregular} of {db.nspec}", flush=True)
     assert db.nspec_irregular > 0 and (n < 3 or db.nspec_irregular < db.nspec)
     ref = oracle_mod.OracleSolver(db, src, rec, "f32").run(60)
-    g = GPUSolver(db, src, rec, nstep=60, exact=True, assembly=1)
+    g = GPUSolver(db, src, rec, nstep=60, exact=True, assembly=1, element_order=order)
     out = g.run().copy()
     g.close()
     assert np.abs(ref).max() > 0 and np.array_equal(out, ref)
