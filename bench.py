@@ -164,7 +164,7 @@ def batched_measurement(args) -> dict:
     finite = all(bool(np.isfinite(b.seismograms(i)).all()) for i in range(len(w.shots)))
     b.close()
     value = db.nglob * float(sum(nsteps)) / wall
-    kbytes = batch_stiffness_bytes(db, len(w.shots), fused=choice["assembly"] == 3)
+    kbytes = batch_stiffness_bytes(db, len(w.shots), fused=False)
     ach = kbytes / (kms / 1e3) / 1e9
     run_gbs = batch_step_bytes(db, sum(nsteps), max(nsteps)) / wall / 1e9
     # plain single-shot path on the same mesh (first shot), timed the same way
@@ -195,8 +195,7 @@ def batched_measurement(args) -> dict:
                              "frac": round(run_gbs / HBM_PEAK_GBS, 4),
                              "bytes_per_update": round(batch_step_bytes(db, sum(nsteps), max(nsteps))
                                                        / (db.nglob * float(sum(nsteps))), 2)},
-            "roofline": {"bound": "hbm", "kernel": "k_elastic_batch (all shots live"
-                         + (", Newmark update fused)" if choice["assembly"] == 3 else ")"), "achieved": round(ach, 1),
+            "roofline": {"bound": "hbm", "kernel": "k_elastic_batch (all shots live)", "achieved": round(ach, 1),
                          "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                          "bytes_per_launch": kbytes, "avg_pass_ms": round(kms, 4), "step_ms": round(sms, 4)}}
 
@@ -229,7 +228,7 @@ def batched_visco_measurement(args) -> dict:
     finite = all(bool(np.isfinite(b.seismograms(i)).all()) for i in range(len(shots)))
     b.close()
     value = db.nglob * float(n * len(shots)) / wall
-    kbytes = batch_stiffness_bytes(db, len(shots), fused=choice["assembly"] == 3, attenuation=att)
+    kbytes = batch_stiffness_bytes(db, len(shots), fused=False, attenuation=att)
     ach = kbytes / (kms / 1e3) / 1e9
     src, rec, _ = shots[0]
     ps = min(args.plain_steps, n)
@@ -249,8 +248,7 @@ def batched_visco_measurement(args) -> dict:
     return {"workload": f"{w.name.split(',')[0]} viscoelastic Q_mu=100, {len(shots)} shots x {n} steps",
             "value": value, "unit": "GLL-point updates/s", "wall_s": round(wall, 3), "plain_single_shot": plain,
             "ratio_vs_plain": value / plain, "autotuned": choice, "seismograms_finite": finite,
-            "roofline": {"bound": "hbm", "kernel": "k_visco_batch (all shots live"
-                         + (", Newmark update fused)" if choice["assembly"] == 3 else ")"), "achieved": round(ach, 1),
+            "roofline": {"bound": "hbm", "kernel": "k_visco_batch (all shots live" + ")", "achieved": round(ach, 1),
                          "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                          "bytes_per_launch": kbytes, "avg_pass_ms": round(kms, 4), "step_ms": round(sms, 4)}}
 

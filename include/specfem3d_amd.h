@@ -377,13 +377,14 @@ void sf_batch_add_source(long batch, int shot, int ispec, const realw* sourcearr
 void sf_batch_add_receiver(long batch, int shot, int ispec, const double* hxi, const double* heta,
                            const double* hgamma, const double* nu);
 void sf_batch_finalize(long batch);
-/* shots per workgroup 4 or 8; assembly 0 = atomic scatter, 2 = one launch per element colour,
-   3 = coloured with the Newmark update fused into the colour launches (same results as 2); only
-   at step 1 (a new batch or after sf_batch_reset) */
+/* shots per workgroup 4 or 8; assembly 0, 2 or 3: one code path, which sums every point's element
+   contributions in the colour order of a greedy element colouring; only at step 1 (a new batch or
+   after sf_batch_reset) */
 void sf_batch_set_options(long batch, int shots_per_group, int assembly);
 void sf_batch_get_options(long batch, int* shots_per_group, int* assembly);
-/* kernel variants with the same results: "lds_overlay" 0/1 (displacement tile and stress products
-   share LDS); unknown names are fatal */
+/* same results for every value: "local_groups" >= 1, groups of eight shots whose local forces are held
+   at a time (default: as many as the card has room for); "lds_overlay" 0/1, accepted without effect;
+   unknown names are fatal */
 void sf_batch_set_tuning(long batch, const char* name, int value);
 int sf_batch_get_tuning(long batch, const char* name);
 double sf_batch_autotune(long batch, int trial_steps);

@@ -4,25 +4,23 @@
 // The reference runs one shot per process (one Mesh_pointer, one source set, iterate_time.F90).
 // Here a Batch borrows a prepared elastic Mesh (ibool, moduli, Jacobians, inverse mass, Stacey
 // face points, element colours) and steps S interleaved wavefields together:
-//   * layout: value (g, c, s) at ((int64_t)g * 3 + c) * S + s (shot-fastest rows, see k_batch.hip);
+//   * layout: groups of eight shots, each a field of its own with rows of eight (batch_idx);
 //   * shots are placed in decreasing order of record length, so the live shots at any step are
-//     a prefix of the row and finished shots cost no memory traffic;
-//   * a mesh with fluid elements also steps S interleaved potentials over its acoustic range of
-//     global points (value (g, s) at (g - g0) * S + s): per step the potential predictor, free
+//     a prefix and a finished group costs no memory traffic;
+//   * a mesh with fluid elements also steps S potentials over its acoustic range of global points
+//     in the same layout: per step the potential predictor, free
 //     surface, acoustic stiffness, fluid Stacey and fluid side of the coupling, the corrector and
 //     the free surface again come first, then the solid side of the coupling with the elastic
 //     boundary terms (the single-shot call order of iterate_time.F90);
-//   * one step = fused corrector/predictor, Stacey rounds, source rounds, stiffness (one launch per
-//     element colour with plain read-modify-writes, or one atomic launch), receivers, and a
-//     one-lane kernel that advances the device step counter. Assembly mode 3 instead records the
-//     receivers first and folds the corrector/predictor into the coloured stiffness launches
-//     (k_batch.hip), which removes the separate pass over u, v, a. Every kernel reads the counter,
-//     so a group of steps is captured once into a hipGraph and replayed;
+//   * one step = sum of the local forces with the corrector and predictor (k_batch_gather), Stacey
+//     rounds, source rounds, stiffness (one launch that stores local forces), receivers, and a one-lane
+//     kernel that advances the device step counter. Every kernel reads the counter, so a group of
+//     steps is captured once into a hipGraph and replayed;
 //   * the per-point arithmetic and the order of every sum equal the single-shot path (same
 //     kernels' expressions, same colour order, same face rounds), so each shot of a batch is
 //     bit-identical to its single-shot run with the same options.
-// Shots-per-workgroup and the assembly mode are chosen by an autotuner that times each candidate
-// for a few steps from rest and then resets the batch.
+// Shots-per-workgroup are chosen by an autotuner that times each candidate for a few steps from rest
+// and then resets the batch.
 #include <algorithm>
 #include <cstring>
 #include <numeric>
@@ -39,9 +37,8 @@ bool element_is_elastic(Mesh* m, int e);
 struct Batch {
   Mesh* m = nullptr;
   int nshots = 0, S = 0;
-  int S0 = 0;                    // padded shot count at creation; S shrinks as shots finish
-  int sc = 4, mode = 2;          // shots per workgroup, assembly (0 atomic, 2 coloured, 3 fused)
-  int overlay = 0;               // 1: displacement tile and stress products share LDS
+  int sc = 4, mode = 2;          // shots per workgroup; assembly, kept for callers (no effect)
+  int overlay = 0;               // "lds_overlay", kept for callers that set it (no effect)
   int max_nstep = 0;
   realw dt = 0.f, dt2 = 0.f, dtsq2 = 0.f;  // deltat, deltatover2, deltatsqover2
   std::vector<int> nstep_user;   // per user shot
@@ -50,16 +47,18 @@ struct Batch {
   int* d_it = nullptr;
   int h_it = 1;                  // host mirror of the step counter
   realw *u = nullptr, *v = nullptr, *a = nullptr;
-  realw* u_last = nullptr;       // final displacement of slots dropped by compaction (stride S0)
-  std::vector<int> h_nstep;      // per slot (S0 entries, decreasing, padding 0)
   bool att = false;              // 3-SLS attenuation: per-shot memory variables and strain
   bool ac = false;               // fluid elements: per-shot potentials over the acoustic range
   int64_t ac_g0 = 0, ac_n = 0;   // acoustic range [ac_g0, ac_g0 + ac_n) of global points
   realw *pot = nullptr, *potd = nullptr, *potdd = nullptr;
-  realw* p_last = nullptr;       // final potential of slots dropped by compaction (stride S0)
   realw *R = nullptr, *eps = nullptr;
-  unsigned char* flags = nullptr;  // fused mode: BF_* per local point (first/last colour, cleared)
-  int flags_version = -1;        // Mesh::color_version the flags were built for (-1: stale)
+  // gather assembly: slots of each global point in colour order, AF_TERM per global point, local forces
+  // of `loc_groups` groups of eight shots (all of them unless the card has no room)
+  int *asm_ptr = nullptr, *asm_idx = nullptr, *ac_ptr = nullptr, *ac_idx = nullptr;
+  uint16_t* info = nullptr;
+  realw *local = nullptr, *ac_local = nullptr;
+  int loc_groups = 0, ac_loc_groups = 0;
+  int max_groups = 1 << 20;      // "local_groups"
   // sources: (source, point) entries sorted into rounds (the k-th source of each shot)
   struct Src { int shot, ispec; std::vector<realw> arr, stf; };
   std::vector<Src> srcs;
@@ -95,37 +94,32 @@ static __device__ __forceinline__ int load_it(const int* it) {
   return __hip_atomic_load(it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Newmark update of every live (row, shot): predictor only on the first step, otherwise the
-// deferred corrector of the previous step fused with the predictor (k_update.hip arithmetic).
-// A lane takes four consecutive shots of one row (a float4); a workgroup takes 256 / (S/4) rows,
-// so the row and quad of a lane come from 32-bit arithmetic on threadIdx. Finished shots keep
-// their values (their lanes store what they loaded).
-__global__ void __launch_bounds__(256) k_batch_update(int64_t nrow, int S, int rows_per_block,
-                                                      const int* __restrict__ nstep, const int* __restrict__ itp,
-                                                      realw* __restrict__ u, realw* __restrict__ v,
-                                                      realw* __restrict__ a, const realw* __restrict__ rm, realw dt2p,
-                                                      realw dt, realw dt2, realw dtsq2, int first) {
-  const int nq = S >> 2;
-  const int rl = (int)threadIdx.x / nq;
-  const int qd = (int)threadIdx.x - rl * nq;
-  if (rl >= rows_per_block) return;
-  const int64_t row = (int64_t)blockIdx.x * rows_per_block + rl;
+// Newmark update of every live (row, shot) from an assembled accel: the corrector of the previous step
+// fused with the predictor (k_update.hip arithmetic), where the local forces have no room for all
+// groups (see enqueue_stiffness).
+// A lane takes four consecutive shots of one row (a float4), blockIdx.y is the group of eight.
+// Finished shots keep their values (their lanes store what they loaded).
+__global__ void __launch_bounds__(256) k_batch_update(int64_t nrow, const int* __restrict__ nstep,
+                                                      const int* __restrict__ itp, realw* __restrict__ u,
+                                                      realw* __restrict__ v, realw* __restrict__ a,
+                                                      const realw* __restrict__ rm, realw dt2p, realw dt, realw dt2,
+                                                      realw dtsq2) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = t >> 1;
   if (row >= nrow) return;
   const int it = load_it(itp);
-  const int s = 4 * qd;
+  const int s = 8 * (int)blockIdx.y + 4 * (int)(t & 1);
   if (nstep[s] < it) return;                       // shots are sorted: the whole quad has finished
   const bool l1 = nstep[s + 1] >= it, l2 = nstep[s + 2] >= it, l3 = nstep[s + 3] >= it;
-  const int64_t o = row * S + s;
+  const int64_t o = batch_idx(nrow, row, s);
   const float4 U0 = *reinterpret_cast<const float4*>(u + o);
   const float4 V0 = *reinterpret_cast<const float4*>(v + o);
   const float4 A0 = *reinterpret_cast<const float4*>(a + o);
-  const realw M = first ? (realw)0 : rm[row];
+  const realw M = rm[row];
   float4 U = U0, V = V0, A = A0;
 #define SF_BU(c)                           \
-  if (!first) {                            \
-    A.c = A.c * M;                         \
-    V.c = V.c + dt2p * A.c;                \
-  }                                        \
+  A.c = A.c * M;                           \
+  V.c = V.c + dt2p * A.c;                  \
   U.c = U.c + dt * V.c + dtsq2 * A.c;      \
   V.c = V.c + dt2 * A.c;                   \
   A.c = 0.f;
@@ -139,8 +133,138 @@ __global__ void __launch_bounds__(256) k_batch_update(int64_t nrow, int S, int r
   *reinterpret_cast<float4*>(a + o) = A;
 }
 
+// Sum of the local forces of every live (row, quad of shots) in list order, a = a - local, and with STEP
+// the corrector of the finished step and the predictor of the next one (the arithmetic of
+// k_batch_update; a: read and cleared at AF_TERM points, zero elsewhere).
+//
+// The element colours with the Newmark update folded in, which this replaced, moved fewer bytes but
+// scattered their accel, u and v stores over parts of cache lines: on 64x64x32 elements x 32 shots
+// the element pass without its arithmetic took 7.3 of 7.4 ms, of which the stores 4.4 ms (9.5 GB, 2.2
+// TB/s), and the shared points' u was read once per colour (6.3 instead of 3.3 GB). Here both passes
+// store whole lines, the element pass is bound by its arithmetic (3.45 ms there: VALU 2.4 ms, HBM 2.1,
+// LDS 1.6) and this one by HBM (3.96 ms, 19.3 GB, 4.9 TB/s). Steps before and after: 32x32x16 x 16
+// shots 598 -> 500 us, 64x64x32 x 32 8.53 -> 7.56 ms, viscoelastic 18x18x12 x 8 319 -> 233 us and
+// 40x40x20 x 16 4.02 -> 3.41 ms.
+struct BatchGatherArgs {
+  int64_t g0, n, nrow;           // global points [g0, g0 + n), rows of a group
+  const int *ptr, *idx;
+  const realw* local;
+  int64_t loc_group;
+  int first_group;               // group of blockIdx.y = 0 (and of the buffer's first block)
+  const uint16_t* info;
+  const int *nstep, *it;
+  realw *u, *v, *a;
+  const realw* rm;
+  realw dt2p, dt, dt2, dtsq2;
+};
+
+__device__ __forceinline__ void sub4(float4& a, const float4& l) {
+  a.x = a.x + (-l.x);
+  a.y = a.y + (-l.y);
+  a.z = a.z + (-l.z);
+  a.w = a.w + (-l.w);
+}
+
+// a -= the local forces of slots ptr[g] .. ptr[g + 1], `unit` floats per slot, four slots in flight
+__device__ __forceinline__ void gather4(float4& a, const int* ptr, const int* idx, int64_t g, const realw* local,
+                                        int unit) {
+  const int p0 = ptr[g], p1 = ptr[g + 1];
+  for (int p = p0; p < p1; p += 4) {
+    int k[4];
+    float4 l[4];
+#pragma unroll
+    for (int w = 0; w < 4; w++) k[w] = p + w < p1 ? idx[p + w] : -1;
+#pragma unroll
+    for (int w = 0; w < 4; w++)
+      if (k[w] >= 0) l[w] = *reinterpret_cast<const float4*>(local + (int64_t)k[w] * unit);
+#pragma unroll
+    for (int w = 0; w < 4; w++)
+      if (k[w] >= 0) sub4(a, l[w]);
+  }
+}
+
+// contiguous blocks of points per XCD
+__device__ __forceinline__ int64_t xcd_block() {
+  const int nb = (int)gridDim.x, b = (int)blockIdx.x;
+  const int q = nb >> 3, r = nb & 7, x = b & 7;
+  return (int64_t)x * q + (x < r ? x : r) + (b >> 3);
+}
+
+template <bool STEP>
+__global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs A) {
+  const int64_t t = xcd_block() * 256 + threadIdx.x;
+  const int64_t pt = t / 6;
+  if (pt >= A.n) return;
+  const int cq = (int)(t - 6 * pt), c = cq >> 1;
+  const int it = load_it(A.it);
+  const int s = 8 * (A.first_group + (int)blockIdx.y) + 4 * (cq & 1);
+  if (A.nstep[s] < it) return;                       // shots are sorted: the whole quad has finished
+  const int64_t g = A.g0 + pt;
+  const int64_t o = batch_idx(A.nrow, 3 * g + c, s);
+  const bool term = (A.info[g] & AF_TERM) != 0;
+  float4 U0, V0, Ac = make_float4(0.f, 0.f, 0.f, 0.f);
+  realw M = 0.f;
+  if (STEP) {
+    U0 = *reinterpret_cast<const float4*>(A.u + o);
+    V0 = *reinterpret_cast<const float4*>(A.v + o);
+    M = A.rm[3 * g + c];
+  }
+  if (term) Ac = *reinterpret_cast<const float4*>(A.a + o);
+  gather4(Ac, A.ptr, A.idx, g, A.local + (int64_t)blockIdx.y * A.loc_group + 8 * c + 4 * (cq & 1), 24);
+  if (!STEP) {
+    *reinterpret_cast<float4*>(A.a + o) = Ac;
+    return;
+  }
+  const bool l1 = A.nstep[s + 1] >= it, l2 = A.nstep[s + 2] >= it, l3 = A.nstep[s + 3] >= it;
+  float4 U = U0, V = V0;
+#define SF_BG(c)                              \
+  Ac.c = Ac.c * M;                            \
+  V.c = V.c + A.dt2p * Ac.c;                  \
+  U.c = U.c + A.dt * V.c + A.dtsq2 * Ac.c;    \
+  V.c = V.c + A.dt2 * Ac.c;
+  SF_BG(x) SF_BG(y) SF_BG(z) SF_BG(w)
+#undef SF_BG
+  if (!l1) { U.y = U0.y; V.y = V0.y; }
+  if (!l2) { U.z = U0.z; V.z = V0.z; }
+  if (!l3) { U.w = U0.w; V.w = V0.w; }
+  *reinterpret_cast<float4*>(A.u + o) = U;
+  *reinterpret_cast<float4*>(A.v + o) = V;
+  if (term) *reinterpret_cast<float4*>(A.a + o) = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+// the same for the potentials: chi'' -= local forces, then the corrector chi'' *= rmass, chi' += dt/2 chi''
+// (rows g - g0; the boundary terms are in chi'' already)
+__global__ void __launch_bounds__(256) k_batch_ac_gather(int64_t nrow, int64_t g0, const int* __restrict__ ptr,
+                                                         const int* __restrict__ idx, const realw* __restrict__ local,
+                                                         int64_t loc_group, int first_group,
+                                                         const int* __restrict__ nstep, const int* __restrict__ itp,
+                                                         realw* __restrict__ potd, realw* __restrict__ potdd,
+                                                         const realw* __restrict__ rm, realw dt2) {
+  const int64_t t = xcd_block() * 256 + threadIdx.x;
+  const int64_t row = t >> 1;
+  if (row >= nrow) return;
+  const int it = load_it(itp);
+  const int s = 8 * (first_group + (int)blockIdx.y) + 4 * (int)(t & 1);
+  if (nstep[s] < it) return;
+  const int64_t o = batch_idx(nrow, row, s);
+  float4 V = *reinterpret_cast<const float4*>(potd + o);
+  float4 Ac = *reinterpret_cast<const float4*>(potdd + o);
+  const float4 V0 = V, A0 = Ac;
+  const realw M = rm[row];
+  gather4(Ac, ptr, idx, g0 + row, local + (int64_t)blockIdx.y * loc_group + 4 * (int)(t & 1), 8);
+  const bool l1 = nstep[s + 1] >= it, l2 = nstep[s + 2] >= it, l3 = nstep[s + 3] >= it;
+#define SF_AG(c) Ac.c = Ac.c * M; V.c = V.c + dt2 * Ac.c;
+  SF_AG(x) SF_AG(y) SF_AG(z) SF_AG(w)
+#undef SF_AG
+  if (!l1) { V.y = V0.y; Ac.y = A0.y; }
+  if (!l2) { V.z = V0.z; Ac.z = A0.z; }
+  if (!l3) { V.w = V0.w; Ac.w = A0.w; }
+  *reinterpret_cast<float4*>(potd + o) = V;
+  *reinterpret_cast<float4*>(potdd + o) = Ac;
+}
+
 // Stacey (k_stacey_el arithmetic) for every (face point of one round, live shot)
-__global__ void k_batch_stacey(int n, int S, const int* __restrict__ ig, const realw* __restrict__ nrm,
+__global__ void k_batch_stacey(int n, int S, int64_t nrow, const int* __restrict__ ig, const realw* __restrict__ nrm,
                                const realw* __restrict__ jw, const realw* __restrict__ rvp,
                                const realw* __restrict__ rvs, const int* __restrict__ nstep,
                                const int* __restrict__ itp, const realw* __restrict__ veloc, realw* accel) {
@@ -149,8 +273,8 @@ __global__ void k_batch_stacey(int n, int S, const int* __restrict__ ig, const r
   const int s = t - q * S;
   if (q >= n) return;
   if (nstep[s] < load_it(itp)) return;
-  const int64_t b = (int64_t)ig[q] * 3 * S + s;
-  const realw vx = veloc[b], vy = veloc[b + S], vz = veloc[b + 2 * S];
+  const int64_t b = batch_idx(nrow, 3 * (int64_t)ig[q], s);
+  const realw vx = veloc[b], vy = veloc[b + 8], vz = veloc[b + 16];
   const realw nx = nrm[3 * q], ny = nrm[3 * q + 1], nz = nrm[3 * q + 2];
   const realw vn = vx * nx + vy * ny + vz * nz;
   const realw p = rvp[q], sv = rvs[q];
@@ -160,12 +284,12 @@ __global__ void k_batch_stacey(int n, int S, const int* __restrict__ ig, const r
   const realw w = jw[q];
   const realw fx = tx * w, fy = ty * w, fz = tz * w;
   accel[b] = accel[b] - fx;
-  accel[b + S] = accel[b + S] - fy;
-  accel[b + 2 * S] = accel[b + 2 * S] - fz;
+  accel[b + 8] = accel[b + 8] - fy;
+  accel[b + 16] = accel[b + 16] - fz;
 }
 
 // source entries of one round: accel += sourcearray * stf(it) (k_add_sources_el arithmetic)
-__global__ void k_batch_sources(int n, int S, int max_nstep, const int* __restrict__ ig, const int* __restrict__ slot,
+__global__ void k_batch_sources(int n, int64_t nrow, int max_nstep, const int* __restrict__ ig, const int* __restrict__ slot,
                                 const int* __restrict__ sid, const int* __restrict__ ploc,
                                 const realw* __restrict__ arr, const realw* __restrict__ stf,
                                 const int* __restrict__ nstep, const int* __restrict__ itp, realw* accel) {
@@ -176,14 +300,14 @@ __global__ void k_batch_sources(int n, int S, int max_nstep, const int* __restri
   if (nstep[s] < it) return;
   const realw* sa = arr + ((int64_t)sid[t] * 125 + ploc[t]) * 3;
   const realw st = stf[(int64_t)sid[t] * max_nstep + it - 1];
-  const int64_t b = (int64_t)ig[t] * 3 * S + s;
+  const int64_t b = batch_idx(nrow, 3 * (int64_t)ig[t], s);
   accel[b] = accel[b] + sa[0] * st;
-  accel[b + S] = accel[b + S] + sa[1] * st;
-  accel[b + 2 * S] = accel[b + 2 * S] + sa[2] * st;
+  accel[b + 8] = accel[b + 8] + sa[1] * st;
+  accel[b + 16] = accel[b + 16] + sa[2] * st;
 }
 
 // receivers (k_seismo_el arithmetic): one wave64 per receiver, FP64 sums, rotation by nu
-__global__ void __launch_bounds__(64) k_batch_seismo(int nrec, int S, const int* __restrict__ slot,
+__global__ void __launch_bounds__(64) k_batch_seismo(int nrec, int64_t nrow, const int* __restrict__ slot,
                                                      const int* __restrict__ ig, const double* __restrict__ h,
                                                      const double* __restrict__ nu, const int* __restrict__ nstep,
                                                      const int* __restrict__ itp, const realw* __restrict__ u,
@@ -196,11 +320,11 @@ __global__ void __launch_bounds__(64) k_batch_seismo(int nrec, int S, const int*
   const int lane = threadIdx.x;
   double sx = 0.0, sy = 0.0, sz = 0.0;
   for (int p = lane; p < 125; p += 64) {
-    const int64_t b = (int64_t)ig[(int64_t)r * 125 + p] * 3 * S + s;
+    const int64_t b = batch_idx(nrow, 3 * (int64_t)ig[(int64_t)r * 125 + p], s);
     const double hl = h[(int64_t)r * 125 + p];
     sx += (double)u[b] * hl;
-    sy += (double)u[b + S] * hl;
-    sz += (double)u[b + 2 * S] * hl;
+    sy += (double)u[b + 8] * hl;
+    sz += (double)u[b + 16] * hl;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -217,43 +341,25 @@ __global__ void __launch_bounds__(64) k_batch_seismo(int nrec, int S, const int*
   }
 }
 
-// ---- fluid domain: potentials over the acoustic range, value (g, s) at (g - g0) * S + s
-// Newmark on the potential rows of live shots (k_update.hip arithmetic): correct = 0 the
-// predictor chi += dt chi' + dt^2/2 chi'', chi' += dt/2 chi'', chi'' = 0; correct = 1 the corrector
-// chi'' *= rmass, chi' += dt/2 chi''. A lane takes four consecutive shots of one row.
-__global__ void __launch_bounds__(256) k_batch_ac_newmark(int64_t nrow, int S, int rows_per_block,
-                                                          const int* __restrict__ nstep, const int* __restrict__ itp,
-                                                          realw* __restrict__ pot, realw* __restrict__ potd,
-                                                          realw* __restrict__ potdd, const realw* __restrict__ rm,
-                                                          realw dt, realw dt2, realw dtsq2, int correct) {
-  const int nq = S >> 2;
-  const int rl = (int)threadIdx.x / nq;
-  const int qd = (int)threadIdx.x - rl * nq;
-  if (rl >= rows_per_block) return;
-  const int64_t row = (int64_t)blockIdx.x * rows_per_block + rl;
+// ---- fluid domain: potentials over the acoustic range, rows g - g0
+// Predictor on the potential rows of live shots (k_update.hip arithmetic): chi += dt chi' + dt^2/2 chi'',
+// chi' += dt/2 chi'', chi'' = 0. A lane takes four consecutive shots of one row.
+__global__ void __launch_bounds__(256) k_batch_ac_predictor(int64_t nrow, const int* __restrict__ nstep,
+                                                            const int* __restrict__ itp, realw* __restrict__ pot,
+                                                            realw* __restrict__ potd, realw* __restrict__ potdd,
+                                                            realw dt, realw dt2, realw dtsq2) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = t >> 1;
   if (row >= nrow) return;
   const int it = load_it(itp);
-  const int s = 4 * qd;
+  const int s = 8 * (int)blockIdx.y + 4 * (int)(t & 1);
   if (nstep[s] < it) return;
   const bool l1 = nstep[s + 1] >= it, l2 = nstep[s + 2] >= it, l3 = nstep[s + 3] >= it;
-  const int64_t o = row * S + s;
+  const int64_t o = batch_idx(nrow, row, s);
   const float4 V0 = *reinterpret_cast<const float4*>(potd + o);
   const float4 A0 = *reinterpret_cast<const float4*>(potdd + o);
-  float4 V = V0, A = A0;
-  if (correct) {
-    const realw M = rm[row];
-#define SF_AC(c) A.c = A.c * M; V.c = V.c + dt2 * A.c;
-    SF_AC(x) SF_AC(y) SF_AC(z) SF_AC(w)
-#undef SF_AC
-    if (!l1) { V.y = V0.y; A.y = A0.y; }
-    if (!l2) { V.z = V0.z; A.z = A0.z; }
-    if (!l3) { V.w = V0.w; A.w = A0.w; }
-    *reinterpret_cast<float4*>(potd + o) = V;
-    *reinterpret_cast<float4*>(potdd + o) = A;
-    return;
-  }
   const float4 U0 = *reinterpret_cast<const float4*>(pot + o);
-  float4 U = U0;
+  float4 U = U0, V = V0, A = A0;
 #define SF_AP(c) U.c = U.c + dt * V.c + dtsq2 * A.c; V.c = V.c + dt2 * A.c; A.c = 0.f;
   SF_AP(x) SF_AP(y) SF_AP(z) SF_AP(w)
 #undef SF_AP
@@ -266,7 +372,7 @@ __global__ void __launch_bounds__(256) k_batch_ac_newmark(int64_t nrow, int S, i
 }
 
 // free surface (k_free_surface): zero chi, chi', chi'' of every (free-surface point, live shot)
-__global__ void k_batch_free_surface(int n, int S, int64_t g0, const int* __restrict__ ig,
+__global__ void k_batch_free_surface(int n, int S, int64_t nrow, int64_t g0, const int* __restrict__ ig,
                                      const int* __restrict__ nstep, const int* __restrict__ itp, realw* pot,
                                      realw* potd, realw* potdd) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;  // n * S < 2^31 (checked by the caller)
@@ -274,14 +380,14 @@ __global__ void k_batch_free_surface(int n, int S, int64_t g0, const int* __rest
   const int s = t - q * S;
   if (q >= n) return;
   if (nstep[s] < load_it(itp)) return;
-  const int64_t b = ((int64_t)ig[q] - g0) * S + s;
+  const int64_t b = batch_idx(nrow, (int64_t)ig[q] - g0, s);
   pot[b] = 0.f;
   potd[b] = 0.f;
   potdd[b] = 0.f;
 }
 
 // fluid Stacey (k_stacey_ac arithmetic) for every (face point of one round, live shot)
-__global__ void k_batch_stacey_ac(int n, int S, int64_t g0, const int* __restrict__ ig, const realw* __restrict__ jw,
+__global__ void k_batch_stacey_ac(int n, int S, int64_t nrow, int64_t g0, const int* __restrict__ ig, const realw* __restrict__ jw,
                                   const realw* __restrict__ rho, const realw* __restrict__ cp,
                                   const int* __restrict__ nstep, const int* __restrict__ itp,
                                   const realw* __restrict__ potd, realw* potdd) {
@@ -290,13 +396,13 @@ __global__ void k_batch_stacey_ac(int n, int S, int64_t g0, const int* __restric
   const int s = t - q * S;
   if (q >= n) return;
   if (nstep[s] < load_it(itp)) return;
-  const int64_t b = ((int64_t)ig[q] - g0) * S + s;
+  const int64_t b = batch_idx(nrow, (int64_t)ig[q] - g0, s);
   const realw absorbl = potd[b] * jw[q] / cp[q] / rho[q];
   potdd[b] = potdd[b] - absorbl;
 }
 
 // fluid side of the coupling (k_coupling_ac_el arithmetic, forward field): chi'' += w (u . n)
-__global__ void k_batch_coupling_ac_el(int n, int S, int64_t g0, const int* __restrict__ ig,
+__global__ void k_batch_coupling_ac_el(int n, int S, int64_t nrow, int64_t nrow_ac, int64_t g0, const int* __restrict__ ig,
                                        const realw* __restrict__ nrm, const realw* __restrict__ jw,
                                        const int* __restrict__ nstep, const int* __restrict__ itp,
                                        const realw* __restrict__ u, realw* potdd) {
@@ -306,15 +412,15 @@ __global__ void k_batch_coupling_ac_el(int n, int S, int64_t g0, const int* __re
   if (q >= n) return;
   if (nstep[s] < load_it(itp)) return;
   const int64_t g = ig[q];
-  const int64_t e = g * 3 * S + s;
-  const realw ux = u[e], uy = u[e + S], uz = u[e + 2 * S];
+  const int64_t e = batch_idx(nrow, 3 * g, s);
+  const realw ux = u[e], uy = u[e + 8], uz = u[e + 16];
   const realw un = ux * nrm[3 * q] + uy * nrm[3 * q + 1] + uz * nrm[3 * q + 2];
-  const int64_t b = (g - g0) * S + s;
+  const int64_t b = batch_idx(nrow_ac, g - g0, s);
   potdd[b] = potdd[b] + jw[q] * un;
 }
 
 // solid side of the coupling (k_coupling_el_ac arithmetic, forward field): a += w n (-chi'')
-__global__ void k_batch_coupling_el_ac(int n, int S, int64_t g0, const int* __restrict__ ig,
+__global__ void k_batch_coupling_el_ac(int n, int S, int64_t nrow, int64_t nrow_ac, int64_t g0, const int* __restrict__ ig,
                                        const realw* __restrict__ nrm, const realw* __restrict__ jw,
                                        const int* __restrict__ nstep, const int* __restrict__ itp,
                                        const realw* __restrict__ potdd, realw* accel) {
@@ -324,12 +430,12 @@ __global__ void k_batch_coupling_el_ac(int n, int S, int64_t g0, const int* __re
   if (q >= n) return;
   if (nstep[s] < load_it(itp)) return;
   const int64_t g = ig[q];
-  const realw pr = -potdd[(g - g0) * S + s];
+  const realw pr = -potdd[batch_idx(nrow_ac, g - g0, s)];
   const realw w = jw[q];
-  const int64_t e = g * 3 * S + s;
+  const int64_t e = batch_idx(nrow, 3 * g, s);
   accel[e] = accel[e] + w * nrm[3 * q] * pr;
-  accel[e + S] = accel[e + S] + w * nrm[3 * q + 1] * pr;
-  accel[e + 2 * S] = accel[e + 2 * S] + w * nrm[3 * q + 2] * pr;
+  accel[e + 8] = accel[e + 8] + w * nrm[3 * q + 1] * pr;
+  accel[e + 16] = accel[e + 16] + w * nrm[3 * q + 2] * pr;
 }
 
 __global__ void k_batch_tick(int* itp) {
@@ -339,51 +445,6 @@ __global__ void k_batch_tick(int* itp) {
 __global__ void k_batch_fill(int64_t n, realw* p) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n) p[t] = 0.f;
-}
-
-// Compaction of shot-interleaved rows (grid-stride loops over int64 counts; launched with at most
-// 2^20 workgroups): dst[r * S2 + s] = src[r * S + s] for s < S2 (S2 <= S, multiples of 8; float4)
-__global__ void k_batch_restride(int64_t nrow, int S, int S2, const realw* __restrict__ src,
-                                 realw* __restrict__ dst) {
-  const int nq = S2 >> 2;
-  const int64_t total = nrow * nq;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = t / nq;
-    const int k = (int)(t - r * nq);
-    *reinterpret_cast<float4*>(dst + r * S2 + 4 * k) = *reinterpret_cast<const float4*>(src + r * S + 4 * k);
-  }
-}
-
-// per-(element, shot) blocks of `blk` values: dst block (e, s) at (e * S2 + s) * blk = src block at
-// (e * S + s) * blk, for s < S2
-__global__ void k_batch_restride_blocks(int64_t nspec, int S, int S2, int blk, const realw* __restrict__ src,
-                                        realw* __restrict__ dst) {
-  const int64_t per_e = (int64_t)S2 * blk;
-  const int64_t total = nspec * per_e;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t e = t / per_e;
-    const int64_t w = t - e * per_e;  // s * blk + j
-    dst[t] = src[e * (int64_t)S * blk + w];
-  }
-}
-
-// final displacement of the slots [S2, S) that compaction drops: arch[r * S0 + s] = u[r * S + s]
-__global__ void k_batch_archive(int64_t nrow, int S, int S2, int S0, const realw* __restrict__ u,
-                                realw* __restrict__ arch) {
-  const int nd = S - S2;
-  const int64_t total = nrow * nd;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = t / nd;
-    const int s = S2 + (int)(t - r * nd);
-    arch[r * S0 + s] = u[r * S + s];
-  }
-}
-
-static dim3 stride_grid(int64_t n) {
-  int64_t b = (n + 255) / 256;
-  if (b < 1) b = 1;
-  if (b > (1 << 20)) b = 1 << 20;
-  return dim3((unsigned)b);
 }
 
 // ------------------------------------------------------------------------------ host side
@@ -416,92 +477,7 @@ static void drop_graph(Batch* b) {
   b->graph_steps = 0;
 }
 
-// Give the live shots (a prefix of the slots, which are sorted by decreasing record length) rows
-// of their own width once at least 8 slots have finished: with S = 32 and 8 live shots, every row
-// read would fetch four times the bytes it uses. Slots [S2, S) are finished; their final
-// displacement is kept for sf_batch_displ. Kernel arguments change, so captured graphs are dropped.
-static void compact(Batch* b, int S2) {
-  Mesh* m = b->m;
-  hipStream_t st = m->stream;
-  drop_graph(b);
-  const int64_t nrow = 3 * (int64_t)m->nglob;
-  if (!b->u_last) b->u_last = balloc<realw>(nrow * b->S0);
-  hipLaunchKernelGGL(k_batch_archive, stride_grid(nrow * (b->S - S2)), dim3(256), 0, st, nrow, b->S, S2, b->S0,
-                     b->u, b->u_last);
-  SF_LAUNCH_CHECK("k_batch_archive");
-  for (realw** f : {&b->u, &b->v, &b->a}) {
-    realw* d = balloc<realw>(nrow * S2);
-    hipLaunchKernelGGL(k_batch_restride, stride_grid(nrow * (S2 / 4)), dim3(256), 0, st, nrow, b->S, S2, *f, d);
-    SF_LAUNCH_CHECK("k_batch_restride");
-    SF_CHECK(hipStreamSynchronize(st));
-    bfree(*f);
-    *f = d;
-  }
-  if (b->ac) {
-    const int64_t na = b->ac_n;
-    if (!b->p_last) b->p_last = balloc<realw>(na * b->S0);
-    hipLaunchKernelGGL(k_batch_archive, stride_grid(na * (b->S - S2)), dim3(256), 0, st, na, b->S, S2, b->S0,
-                       b->pot, b->p_last);
-    SF_LAUNCH_CHECK("k_batch_archive");
-    for (realw** f : {&b->pot, &b->potd, &b->potdd}) {
-      realw* d = balloc<realw>(na * S2);
-      hipLaunchKernelGGL(k_batch_restride, stride_grid(na * (S2 / 4)), dim3(256), 0, st, na, b->S, S2, *f, d);
-      SF_LAUNCH_CHECK("k_batch_restride");
-      SF_CHECK(hipStreamSynchronize(st));
-      bfree(*f);
-      *f = d;
-    }
-  }
-  if (b->att) {
-    const int64_t ne = m->nspec;
-    for (auto fb : {std::make_pair(&b->R, 18 * 125), std::make_pair(&b->eps, 6 * 125)}) {
-      realw* d = balloc<realw>(ne * S2 * fb.second);
-      hipLaunchKernelGGL(k_batch_restride_blocks, stride_grid(ne * S2 * fb.second), dim3(256), 0, st, ne, b->S, S2,
-                         fb.second, *fb.first, d);
-      SF_LAUNCH_CHECK("k_batch_restride_blocks");
-      SF_CHECK(hipStreamSynchronize(st));
-      bfree(*fb.first);
-      *fb.first = d;
-    }
-  }
-  b->S = S2;
-}
-
-static void maybe_compact(Batch* b) {
-  int nlive = 0;
-  for (int s = 0; s < b->S; s++) nlive += b->h_nstep[s] >= b->h_it ? 1 : 0;
-  const int S2 = std::max(8, (nlive + 7) / 8 * 8);
-  if (S2 < b->S) compact(b, S2);
-}
-
-// back to rows of the full width (a rewind after compaction); the contents are zeroed next
-static void restore_width(Batch* b) {
-  if (b->S == b->S0) return;
-  Mesh* m = b->m;
-  drop_graph(b);
-  SF_CHECK(hipStreamSynchronize(m->stream));
-  const int64_t n = 3 * (int64_t)m->nglob * b->S0;
-  for (realw** f : {&b->u, &b->v, &b->a}) {
-    bfree(*f);
-    *f = balloc<realw>(n);
-  }
-  if (b->ac) {
-    for (realw** f : {&b->pot, &b->potd, &b->potdd}) {
-      bfree(*f);
-      *f = balloc<realw>(b->ac_n * b->S0);
-    }
-  }
-  if (b->att) {
-    bfree(b->R);
-    bfree(b->eps);
-    b->R = balloc<realw>(18 * (int64_t)m->nspec * 125 * b->S0);
-    b->eps = balloc<realw>(6 * (int64_t)m->nspec * 125 * b->S0);
-  }
-  b->S = b->S0;
-}
-
 static void zero_state(Batch* b) {
-  restore_width(b);
   Mesh* m = b->m;
   const int64_t n = 3 * (int64_t)m->nglob * b->S;
   for (realw* p : {b->u, b->v, b->a})
@@ -556,43 +532,72 @@ static int point_flags(int nglob, int nelem, const int* ibool0, const int* elems
   return 0;
 }
 
-static void build_point_flags(Batch* b) {
+// room for the local forces of as many groups as the card takes, at least one
+static realw* local_room(int64_t per_group, int groups, int* got) {
+  for (int n = groups; n > 0; n /= 2) {
+    void* p = nullptr;
+    if (hipMalloc(&p, sizeof(realw) * (size_t)(per_group * n)) == hipSuccess) {
+      *got = n;
+      return reinterpret_cast<realw*>(p);
+    }
+    (void)hipGetLastError();
+  }
+  fatal("sf_batch", "out of device memory for the batched wavefields");
+}
+
+// slot lists in the colour order of the single-shot run, points that take boundary or source terms,
+// buffers of the local forces
+static void build_gather(Batch* b) {
   Mesh* m = b->m;
-  ensure_element_colors(m);
-  const int ne = m->nspec_elastic;
-  std::vector<int> lst(ne), hib((size_t)m->nspec * 125), col(ne);
-  SF_CHECK(hipMemcpy(lst.data(), m->el_color_elems, sizeof(int) * ne, hipMemcpyDeviceToHost));
-  SF_CHECK(hipMemcpy(hib.data(), m->ibool, sizeof(int) * hib.size(), hipMemcpyDeviceToHost));
-  for (int c = 0; c < m->el_ncolor; c++)
-    for (int q = m->el_color_off[c]; q < m->el_color_off[c + 1]; q++) col[q] = c;
-  std::vector<unsigned char> forced((size_t)m->nglob, 0);
-  if (m->stacey && m->abs_el.n > 0) {
-    std::vector<int> ig(m->abs_el.n);
-    SF_CHECK(hipMemcpy(ig.data(), m->abs_el.iglob, sizeof(int) * ig.size(), hipMemcpyDeviceToHost));
-    for (int g : ig) forced[g] = 1;
-  }
-  if (b->ac && m->coupling.n > 0) {
-    // the solid side of the coupling adds to these points before the colours
-    std::vector<int> ig(m->coupling.n);
-    SF_CHECK(hipMemcpy(ig.data(), m->coupling.iglob, sizeof(int) * ig.size(), hipMemcpyDeviceToHost));
-    for (int g : ig) forced[g] = 1;
-  }
-  for (const Batch::Src& q : b->srcs)
-    for (int p = 0; p < 125; p++) forced[hib[(size_t)q.ispec * 125 + p]] = 1;
-  std::vector<unsigned char> fl((size_t)m->nspec * 125, 0);
-  if (point_flags(m->nglob, ne, hib.data(), lst.data(), col.data(), forced.data(), fl.data()) != 0)
-    fatal("sf_batch", "element colouring shares a point inside a colour");
-  bfree(b->flags);
-  b->flags = bupload(fl.data(), (int64_t)fl.size());
-  b->flags_version = m->color_version;
+  if (!b->asm_ptr)
+    (void)build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_elastic, m->el_color_elems, m->elastic_elems,
+                           m->nspec_elastic, 0, 1, m->ibool, b->asm_ptr, b->asm_idx);
+  if (!b->local) b->local = local_room((int64_t)m->nspec_elastic * 3000, std::min(b->S / 8, b->max_groups), &b->loc_groups);
+  if (b->ac && !b->ac_ptr)
+    (void)build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_acoustic, m->ac_color_elems, m->acoustic_elems,
+                           m->nspec_acoustic, 0, 1, m->ibool, b->ac_ptr, b->ac_idx);
+  if (b->ac && !b->ac_local)
+    b->ac_local = local_room((int64_t)m->nspec_acoustic * 1000, std::min(b->S / 8, b->max_groups), &b->ac_loc_groups);
+  if (!b->info) b->info = balloc<uint16_t>(m->nglob);
+  SF_CHECK(hipMemsetAsync(b->info, 0, sizeof(uint16_t) * (size_t)m->nglob, m->stream));
+  if (m->stacey) launch_mark_points(m->stream, m->abs_el.n, m->abs_el.iglob, AF_TERM, b->info);
+  if (b->ac) launch_mark_points(m->stream, m->coupling.n, m->coupling.iglob, AF_TERM, b->info);
+  launch_mark_points(m->stream, b->src_n, b->src_ig, AF_TERM, b->info);
+}
+
+static BatchGatherArgs gather_args(Batch* b) {
+  Mesh* m = b->m;
+  BatchGatherArgs A;
+  A.g0 = m->el_g0;
+  A.n = m->el_n;
+  A.nrow = 3 * (int64_t)m->nglob;
+  A.ptr = b->asm_ptr;
+  A.idx = b->asm_idx;
+  A.local = b->local;
+  A.loc_group = (int64_t)m->nspec_elastic * 3000;
+  A.first_group = 0;
+  A.info = b->info;
+  A.nstep = b->d_nstep;
+  A.it = b->d_it;
+  A.u = b->u;
+  A.v = b->v;
+  A.a = b->a;
+  A.rm = m->rmass;
+  A.dt2p = b->dt2;
+  A.dt = b->dt;
+  A.dt2 = b->dt2;
+  A.dtsq2 = b->dtsq2;
+  return A;
 }
 
 static void enqueue_stiffness(Batch* b, hipStream_t st) {
   Mesh* m = b->m;
   BatchArgs A;
   std::memset(&A, 0, sizeof(A));
-  A.ngroups = b->S / b->sc;
+  A.elems = m->elastic_elems;
+  A.nelem = m->nspec_elastic;
   A.S = b->S;
+  A.nrow = 3 * (int64_t)m->nglob;
   A.ibool = m->ibool;
   A.irregular = m->irregular;
   A.xix_regular = m->xix_regular;
@@ -601,15 +606,11 @@ static void enqueue_stiffness(Batch* b, hipStream_t st) {
   A.jac_plane = (int64_t)m->nspec_irregular * 125;
   A.kappamu = m->kappamu;
   A.u = b->u;
-  A.a = b->a;
+  A.v = b->v;
+  A.dt = b->dt;
+  A.loc_group = (int64_t)m->nspec_elastic * 3000;
   A.nstep = b->d_nstep;
   A.it = b->d_it;
-  A.v = b->v;
-  A.rmass = m->rmass;
-  A.flags = b->flags;
-  A.dt = b->dt;
-  A.dt2 = b->dt2;
-  A.dtsq2 = b->dtsq2;
   if (b->att) {
     A.R = b->R;
     A.eps = b->eps;
@@ -624,28 +625,28 @@ static void enqueue_stiffness(Batch* b, hipStream_t st) {
       A.beta[s] = m->betaval[s];
       A.gamma[s] = m->gammaval[s];
     }
-    for (int c = 0; c < m->el_ncolor; c++) {
-      A.elems = m->el_color_elems + m->el_color_off[c];
-      A.nelem = m->el_color_off[c + 1] - m->el_color_off[c];
-      launch_visco_batch(st, A, b->sc, b->mode, m->exact != 0);
+  }
+  const int groups = b->S / 8;
+  for (int g = 0; g < groups; g += b->loc_groups) {
+    const int n = std::min(b->loc_groups, groups - g);
+    A.s_first = 8 * g;
+    A.ngroups = 8 * n / b->sc;
+    A.local = b->local - g * A.loc_group;            // indexed by the shot's own group
+    if (b->att) launch_visco_batch(st, A, b->sc, m->exact != 0);
+    else launch_elastic_batch(st, A, b->sc, m->exact != 0);
+    if (b->loc_groups < groups) {
+      // no room for the local forces of all groups: sum them into accel before the next ones
+      BatchGatherArgs ga = gather_args(b);
+      ga.first_group = g;
+      hipLaunchKernelGGL(k_batch_gather<false>, dim3(sf_grid(6 * ga.n, 256).x, (unsigned)n), dim3(256), 0, st, ga);
+      SF_LAUNCH_CHECK("k_batch_gather");
     }
-  } else if (b->mode == 2 || b->mode == 3) {
-    for (int c = 0; c < m->el_ncolor; c++) {
-      A.elems = m->el_color_elems + m->el_color_off[c];
-      A.nelem = m->el_color_off[c + 1] - m->el_color_off[c];
-      launch_elastic_batch(st, A, b->sc, b->mode, b->overlay, m->exact != 0);
-    }
-  } else {
-    A.elems = m->elastic_elems;
-    A.nelem = m->nspec_elastic;
-    launch_elastic_batch(st, A, b->sc, 0, b->overlay, m->exact != 0);
   }
 }
 
-// one time step; `first` selects the plain predictor (no pending corrector)
 static void enqueue_seismo(Batch* b, hipStream_t st) {
   if (b->nrec <= 0) return;
-  hipLaunchKernelGGL(k_batch_seismo, dim3(b->nrec), dim3(64), 0, st, b->nrec, b->S, b->rec_slot, b->rec_ig,
+  hipLaunchKernelGGL(k_batch_seismo, dim3(b->nrec), dim3(64), 0, st, b->nrec, 3 * (int64_t)b->m->nglob, b->rec_slot, b->rec_ig,
                      b->rec_h, b->rec_nu, b->d_nstep, b->d_it, b->u, b->seis);
   SF_LAUNCH_CHECK("k_batch_seismo");
 }
@@ -663,23 +664,22 @@ static dim3 pair_grid(int cnt, int S, const char* what) {
 static void enqueue_fluid(Batch* b, hipStream_t st) {
   Mesh* m = b->m;
   const int S = b->S;
-  const int rpb = 256 / (S / 4);
-  const int64_t na = b->ac_n;
-  const dim3 rows = sf_grid((na + rpb - 1) / rpb, 1);
-  hipLaunchKernelGGL(k_batch_ac_newmark, rows, dim3(256), 0, st, na, S, rpb, b->d_nstep, b->d_it, b->pot, b->potd,
-                     b->potdd, m->rmass_ac + b->ac_g0, b->dt, b->dt2, b->dtsq2, 0);
-  SF_LAUNCH_CHECK("k_batch_ac_newmark");
+  const int64_t na = b->ac_n, nrow = 3 * (int64_t)m->nglob;
+  const dim3 rows(sf_grid(2 * na, 256).x, (unsigned)(S / 8));
+  hipLaunchKernelGGL(k_batch_ac_predictor, rows, dim3(256), 0, st, na, b->d_nstep, b->d_it, b->pot, b->potd,
+                     b->potdd, b->dt, b->dt2, b->dtsq2);
+  SF_LAUNCH_CHECK("k_batch_ac_predictor");
   const FacePoints& fs = m->free_ac;
   if (fs.n > 0)
     hipLaunchKernelGGL(k_batch_free_surface, pair_grid(fs.n, S, "too many free-surface points x shots"), dim3(256),
-                       0, st, fs.n, S, b->ac_g0, fs.iglob, b->d_nstep, b->d_it, b->pot, b->potd, b->potdd);
+                       0, st, fs.n, S, na, b->ac_g0, fs.iglob, b->d_nstep, b->d_it, b->pot, b->potd, b->potdd);
   if (m->stacey) {
     const FacePoints& f = m->abs_ac;
     for (int r = 0; r < f.nrounds; r++) {
       const int o = f.round_off[r], cnt = f.round_off[r + 1] - o;
       if (cnt <= 0) continue;
       hipLaunchKernelGGL(k_batch_stacey_ac, pair_grid(cnt, S, "too many fluid Stacey points x shots"), dim3(256), 0,
-                         st, cnt, S, b->ac_g0, f.iglob + o, f.jacw + o, f.imp_p + o, f.imp_s + o, b->d_nstep,
+                         st, cnt, S, na, b->ac_g0, f.iglob + o, f.jacw + o, f.imp_p + o, f.imp_s + o, b->d_nstep,
                          b->d_it, b->potd, b->potdd);
     }
     SF_LAUNCH_CHECK("k_batch_stacey_ac");
@@ -689,14 +689,15 @@ static void enqueue_fluid(Batch* b, hipStream_t st) {
     const int o = cf.round_off[r], cnt = cf.round_off[r + 1] - o;
     if (cnt <= 0) continue;
     hipLaunchKernelGGL(k_batch_coupling_ac_el, pair_grid(cnt, S, "too many coupling points x shots"), dim3(256), 0,
-                       st, cnt, S, b->ac_g0, cf.iglob + o, cf.normal + 3 * o, cf.jacw + o, b->d_nstep, b->d_it, b->u,
+                       st, cnt, S, nrow, na, b->ac_g0, cf.iglob + o, cf.normal + 3 * o, cf.jacw + o, b->d_nstep, b->d_it, b->u,
                        b->potdd);
   }
   SF_LAUNCH_CHECK("k_batch_coupling_ac_el");
   BatchAcArgs A;
   std::memset(&A, 0, sizeof(A));
-  A.ngroups = S / b->sc;
-  A.S = S;
+  A.elems = m->acoustic_elems;
+  A.nelem = m->nspec_acoustic;
+  A.nrow = na;
   A.g0 = b->ac_g0;
   A.ibool = m->ibool;
   A.irregular = m->irregular;
@@ -706,41 +707,42 @@ static void enqueue_fluid(Batch* b, hipStream_t st) {
   A.jac_plane = (int64_t)m->nspec_irregular * 125;
   A.rho = m->rho;
   A.pot = b->pot;
-  A.potdd = b->potdd;
+  A.loc_group = (int64_t)m->nspec_acoustic * 1000;
   A.nstep = b->d_nstep;
   A.it = b->d_it;
-  if (b->mode == 0) {
-    A.elems = m->acoustic_elems;
-    A.nelem = m->nspec_acoustic;
-    launch_acoustic_batch(st, A, b->sc, 0, m->exact != 0);
-  } else {
-    for (int c = 0; c < m->ac_ncolor; c++) {
-      A.elems = m->ac_color_elems + m->ac_color_off[c];
-      A.nelem = m->ac_color_off[c + 1] - m->ac_color_off[c];
-      launch_acoustic_batch(st, A, b->sc, 2, m->exact != 0);
-    }
+  for (int g = 0; g < S / 8; g += b->ac_loc_groups) {
+    const int n = std::min(b->ac_loc_groups, S / 8 - g);
+    A.s_first = 8 * g;
+    A.ngroups = 8 * n / b->sc;
+    A.local = b->ac_local - g * A.loc_group;
+    launch_acoustic_batch(st, A, b->sc, m->exact != 0);
+    hipLaunchKernelGGL(k_batch_ac_gather, dim3(rows.x, (unsigned)n), dim3(256), 0, st, na, b->ac_g0, b->ac_ptr,
+                       b->ac_idx, b->ac_local, A.loc_group, g, b->d_nstep, b->d_it, b->potd, b->potdd,
+                       m->rmass_ac + b->ac_g0, b->dt2);
+    SF_LAUNCH_CHECK("k_batch_ac_gather");
   }
-  hipLaunchKernelGGL(k_batch_ac_newmark, rows, dim3(256), 0, st, na, S, rpb, b->d_nstep, b->d_it, b->pot, b->potd,
-                     b->potdd, m->rmass_ac + b->ac_g0, b->dt, b->dt2, b->dtsq2, 1);
-  SF_LAUNCH_CHECK("k_batch_ac_newmark");
   if (fs.n > 0)
     hipLaunchKernelGGL(k_batch_free_surface, pair_grid(fs.n, S, "too many free-surface points x shots"), dim3(256),
-                       0, st, fs.n, S, b->ac_g0, fs.iglob, b->d_nstep, b->d_it, b->pot, b->potd, b->potdd);
+                       0, st, fs.n, S, na, b->ac_g0, fs.iglob, b->d_nstep, b->d_it, b->pot, b->potd, b->potdd);
   SF_LAUNCH_CHECK("k_batch_free_surface");
 }
 
+// one time step; `first`: the wavefields are zero
 static void enqueue_step(Batch* b, hipStream_t st, bool first) {
   Mesh* m = b->m;
-  const bool fused = b->mode == 3;
-  if (fused) {
-    enqueue_seismo(b, st);  // u already holds this step's predicted displacement
-  } else {
-    const int64_t nrow = 3 * (int64_t)m->nglob;
-    const realw dt = b->dt, dt2 = b->dt2, dtsq2 = b->dtsq2;
-    const int rpb = 256 / (b->S / 4);
-    hipLaunchKernelGGL(k_batch_update, sf_grid((nrow + rpb - 1) / rpb, 1), dim3(256), 0, st, nrow, b->S, rpb,
-                       b->d_nstep, b->d_it, b->u, b->v, b->a, m->rmass, dt2, dt, dt2, dtsq2, first ? 1 : 0);
-    SF_LAUNCH_CHECK("k_batch_update");
+  if (!first) {
+    // sums, corrector and predictor (at rest before the first step: nothing to do)
+    if (b->loc_groups == b->S / 8) {
+      const BatchGatherArgs ga = gather_args(b);
+      hipLaunchKernelGGL(k_batch_gather<true>, dim3(sf_grid(6 * ga.n, 256).x, (unsigned)(b->S / 8)), dim3(256), 0, st,
+                         ga);
+      SF_LAUNCH_CHECK("k_batch_gather");
+    } else {
+      const int64_t nrow = 3 * (int64_t)m->nglob;
+      hipLaunchKernelGGL(k_batch_update, dim3(sf_grid(2 * nrow, 256).x, (unsigned)(b->S / 8)), dim3(256), 0, st, nrow,
+                         b->d_nstep, b->d_it, b->u, b->v, b->a, m->rmass, b->dt2, b->dt, b->dt2, b->dtsq2);
+      SF_LAUNCH_CHECK("k_batch_update");
+    }
   }
   if (b->ac) enqueue_fluid(b, st);
   if (m->stacey) {
@@ -750,7 +752,7 @@ static void enqueue_step(Batch* b, hipStream_t st, bool first) {
       if (cnt <= 0) continue;
       if ((int64_t)cnt * b->S >= 0x7fffffff) fatal("sf_batch", "too many Stacey points x shots");
       hipLaunchKernelGGL(k_batch_stacey, sf_grid((int64_t)cnt * b->S, 256), dim3(256), 0, st, cnt, b->S,
-                         f.iglob + o, f.normal + 3 * o, f.jacw + o, f.imp_p + o, f.imp_s + o, b->d_nstep, b->d_it,
+                         3 * (int64_t)m->nglob, f.iglob + o, f.normal + 3 * o, f.jacw + o, f.imp_p + o, f.imp_s + o, b->d_nstep, b->d_it,
                          b->v, b->a);
     }
     SF_LAUNCH_CHECK("k_batch_stacey");
@@ -761,7 +763,7 @@ static void enqueue_step(Batch* b, hipStream_t st, bool first) {
       const int o = cf.round_off[r], cnt = cf.round_off[r + 1] - o;
       if (cnt <= 0) continue;
       hipLaunchKernelGGL(k_batch_coupling_el_ac, pair_grid(cnt, b->S, "too many coupling points x shots"), dim3(256),
-                         0, st, cnt, b->S, b->ac_g0, cf.iglob + o, cf.normal + 3 * o, cf.jacw + o, b->d_nstep,
+                         0, st, cnt, b->S, 3 * (int64_t)m->nglob, b->ac_n, b->ac_g0, cf.iglob + o, cf.normal + 3 * o, cf.jacw + o, b->d_nstep,
                          b->d_it, b->potdd, b->a);
     }
     SF_LAUNCH_CHECK("k_batch_coupling_el_ac");
@@ -769,7 +771,7 @@ static void enqueue_step(Batch* b, hipStream_t st, bool first) {
   for (int r = 0; r < b->src_nrounds; r++) {
     const int o = b->src_round_off[r], cnt = b->src_round_off[r + 1] - o;
     if (cnt <= 0) continue;
-    hipLaunchKernelGGL(k_batch_sources, sf_grid(cnt, 128), dim3(128), 0, st, cnt, b->S, b->max_nstep, b->src_ig + o,
+    hipLaunchKernelGGL(k_batch_sources, sf_grid(cnt, 128), dim3(128), 0, st, cnt, 3 * (int64_t)m->nglob, b->max_nstep, b->src_ig + o,
                        b->src_slot + o, b->src_id + o, b->src_ploc + o, b->src_arr, b->src_stf, b->d_nstep, b->d_it,
                        b->a);
     SF_LAUNCH_CHECK("k_batch_sources");
@@ -781,7 +783,7 @@ static void enqueue_step(Batch* b, hipStream_t st, bool first) {
     SF_CHECK(hipEventRecord(b->ev[b->ev_used + 1], st));
     b->ev_used += 2;
   }
-  if (!fused) enqueue_seismo(b, st);
+  enqueue_seismo(b, st);
   hipLaunchKernelGGL(k_batch_tick, dim3(1), dim3(64), 0, st, b->d_it);
   SF_LAUNCH_CHECK("k_batch_tick");
 }
@@ -790,12 +792,7 @@ static void enqueue_step(Batch* b, hipStream_t st, bool first) {
 static void run_steps(Batch* b, int n, int graph_steps) {
   Mesh* m = b->m;
   n = std::min(n, b->max_nstep - b->h_it + 1);
-  if (b->mode == 3 && (!b->flags || b->flags_version != m->color_version)) {
-    drop_graph(b);
-    build_point_flags(b);
-  }
   while (n > 0) {
-    maybe_compact(b);
     if (b->h_it == 1 || graph_steps <= 1 || n < graph_steps) {
       enqueue_step(b, m->stream, b->h_it == 1);
       b->h_it++;
@@ -867,8 +864,6 @@ extern "C" long sf_batch_create(long* Mesh_pointer, int nshots, const int* nstep
     ns[k] = nstep[order[k]];
   }
   b->d_nstep = bupload(ns.data(), b->S);
-  b->h_nstep = ns;
-  b->S0 = b->S;
   b->d_it = balloc<int>(1);
   const int64_t n = 3 * (int64_t)m->nglob * b->S;
   b->u = balloc<realw>(n);
@@ -993,14 +988,14 @@ extern "C" void sf_batch_finalize(long h) {
     b->rec_nu = bupload(nu.data(), (int64_t)nu.size());
     b->seis = balloc<realw>((int64_t)b->max_nstep * std::max(1, b->nrec) * 3);
   }
-  b->flags_version = -1;  // sources changed: the fused mode's cleared points change
+  build_gather(b);
   b->ready = true;
   zero_state(b);
 }
 
-// shots per workgroup (4 or 8; divides the padded shot count) and assembly (0 atomic, 2 coloured,
-// 3 coloured with the Newmark update fused). The modes keep different intermediate states, so the
-// batch must be at step 1 (new, or after sf_batch_reset).
+// shots per workgroup (4 or 8; divides the padded shot count) and assembly (0, 2 or 3, as
+// sf_set_options: every value sums in the colour order). The batch must be at step 1 (new, or after
+// sf_batch_reset).
 extern "C" void sf_batch_set_options(long h, int shots_per_group, int assembly) {
   Batch* b = batch_of(h);
   if (shots_per_group != 4 && shots_per_group != 8)
@@ -1015,8 +1010,10 @@ extern "C" void sf_batch_set_options(long h, int shots_per_group, int assembly) 
   b->mode = assembly;
 }
 
-// Kernel variants that give the same results: "lds_overlay" 0/1 (the displacement tile shares LDS
-// with the stress products). Unknown names are fatal.
+// "local_groups": groups of eight shots whose local forces are held at a time (at most all of them, the
+// default where the card has the room; fewer save 24 B per local point and shot and take an extra pass
+// over accel; same results). "lds_overlay" 0/1 is accepted and read back without effect: the elastic
+// kernel's rows always share their LDS with the stress products. Unknown names are fatal.
 extern "C" void sf_batch_set_tuning(long h, const char* name, int value) {
   Batch* b = batch_of(h);
   if (std::strcmp(name, "lds_overlay") == 0) {
@@ -1024,6 +1021,15 @@ extern "C" void sf_batch_set_tuning(long h, const char* name, int value) {
     SF_CHECK(hipStreamSynchronize(b->m->stream));
     drop_graph(b);
     b->overlay = value;
+  } else if (std::strcmp(name, "local_groups") == 0) {
+    if (value < 1) fatal("sf_batch_set_tuning", "local_groups must be positive");
+    if (b->h_it != 1) fatal("sf_batch_set_tuning", "local_groups changes only at step 1 (call sf_batch_reset first)");
+    SF_CHECK(hipStreamSynchronize(b->m->stream));
+    drop_graph(b);
+    bfree(b->local);
+    bfree(b->ac_local);
+    b->max_groups = value;
+    if (b->ready) build_gather(b);
   } else {
     fatal("sf_batch_set_tuning", "unknown tuning switch");
   }
@@ -1032,6 +1038,7 @@ extern "C" void sf_batch_set_tuning(long h, const char* name, int value) {
 extern "C" int sf_batch_get_tuning(long h, const char* name) {
   Batch* b = batch_of(h);
   if (std::strcmp(name, "lds_overlay") == 0) return b->overlay;
+  if (std::strcmp(name, "local_groups") == 0) return b->loc_groups;
   fatal("sf_batch_get_tuning", "unknown tuning switch");
   return 0;
 }
@@ -1078,11 +1085,9 @@ extern "C" void sf_batch_displ(long h, int shot, realw* out) {
   SF_CHECK(hipStreamSynchronize(b->m->stream));
   const int64_t n = 3 * (int64_t)b->m->nglob;
   const int s = b->slot_of[shot];
-  const bool dropped = s >= b->S;  // finished and compacted away: its final state was archived
-  const int stride = dropped ? b->S0 : b->S;
-  std::vector<realw> all((size_t)n * stride);
-  SF_CHECK(hipMemcpy(all.data(), dropped ? b->u_last : b->u, sizeof(realw) * all.size(), hipMemcpyDeviceToHost));
-  for (int64_t q = 0; q < n; q++) out[q] = all[(size_t)q * stride + s];
+  std::vector<realw> all((size_t)n * 8);           // the shot's group
+  SF_CHECK(hipMemcpy(all.data(), b->u + batch_idx(n, 0, s & ~7), sizeof(realw) * all.size(), hipMemcpyDeviceToHost));
+  for (int64_t q = 0; q < n; q++) out[q] = all[(size_t)q * 8 + (s & 7)];
 }
 
 // Potential of one shot over all global points (zero outside the acoustic range; all zero on a mesh
@@ -1095,11 +1100,10 @@ extern "C" void sf_batch_potential(long h, int shot, realw* out) {
   for (int64_t q = 0; q < n; q++) out[q] = 0.f;
   if (!b->ac) return;
   const int s = b->slot_of[shot];
-  const bool dropped = s >= b->S;
-  const int stride = dropped ? b->S0 : b->S;
-  std::vector<realw> all((size_t)b->ac_n * stride);
-  SF_CHECK(hipMemcpy(all.data(), dropped ? b->p_last : b->pot, sizeof(realw) * all.size(), hipMemcpyDeviceToHost));
-  for (int64_t q = 0; q < b->ac_n; q++) out[b->ac_g0 + q] = all[(size_t)q * stride + s];
+  std::vector<realw> all((size_t)b->ac_n * 8);
+  SF_CHECK(hipMemcpy(all.data(), b->pot + batch_idx(b->ac_n, 0, s & ~7), sizeof(realw) * all.size(),
+                     hipMemcpyDeviceToHost));
+  for (int64_t q = 0; q < b->ac_n; q++) out[b->ac_g0 + q] = all[(size_t)q * 8 + (s & 7)];
 }
 
 // Rewind to step 1 with zero wavefields and seismograms (keeps sources, receivers and options).
@@ -1144,39 +1148,30 @@ extern "C" void sf_batch_time(long h, int nsteps, double* stiffness_ms, double* 
   b->ev_used = 0;
 }
 
-// Autotuner: times every (assembly, shots per workgroup, LDS overlay) candidate for `trial_steps`
-// eager steps from rest (after a warm-up; a candidate whose first step takes over twice the best
-// so far is dropped), keeps the fastest and rewinds the batch. Returns the chosen step time in ms.
+// Autotuner: times every shots-per-workgroup candidate for `trial_steps` eager steps from rest (after a
+// warm-up; a candidate whose first step takes over twice the best so far is dropped), keeps the
+// fastest and rewinds the batch. Returns the chosen step time in ms.
 extern "C" double sf_batch_autotune(long h, int trial_steps) {
   Batch* b = batch_of(h);
   if (!b->ready) fatal("sf_batch_autotune", "sf_batch_finalize first");
   double best = 1e300;
-  int best_sc = b->sc, best_mode = b->mode, best_ov = b->overlay;
-  for (int mode : {3, 2, 0})
-    for (int sc : {4, 8})
-    for (int ov : {1, 0}) {
-      if (b->S % sc) continue;
-      if (b->att && (mode == 0 || ov != 1)) continue;  // coloured only; no overlay switch
-      b->sc = sc;
-      b->mode = mode;
-      b->overlay = ov;
-      drop_graph(b);
-      zero_state(b);
-      run_steps(b, 2, 1);  // warm-up (first step runs the plain predictor)
-      double ks = 0.0, st = 0.0;
-      sf_batch_time(h, 1, &ks, &st);
-      if (st > 2.0 * best) continue;  // far behind the best so far: not worth the full trial
-      sf_batch_time(h, trial_steps, &ks, &st);
-      if (st < best) {
-        best = st;
-        best_sc = sc;
-        best_mode = mode;
-        best_ov = ov;
-      }
+  int best_sc = b->sc;
+  for (int sc : {4, 8}) {
+    if (b->S % sc) continue;
+    b->sc = sc;
+    drop_graph(b);
+    zero_state(b);
+    run_steps(b, 2, 1);  // warm-up (the first step has no update)
+    double ks = 0.0, st = 0.0;
+    sf_batch_time(h, 1, &ks, &st);
+    if (st > 2.0 * best) continue;  // far behind the best so far: not worth the full trial
+    sf_batch_time(h, trial_steps, &ks, &st);
+    if (st < best) {
+      best = st;
+      best_sc = sc;
     }
+  }
   b->sc = best_sc;
-  b->mode = best_mode;
-  b->overlay = best_ov;
   drop_graph(b);
   zero_state(b);
   return best;
@@ -1187,9 +1182,9 @@ extern "C" void sf_batch_destroy(long h) {
   SF_CHECK(hipStreamSynchronize(b->m->stream));
   drop_graph(b);
   bfree(b->d_nstep); bfree(b->d_it); bfree(b->u); bfree(b->v); bfree(b->a); bfree(b->R); bfree(b->eps);
-  bfree(b->u_last);
-  bfree(b->pot); bfree(b->potd); bfree(b->potdd); bfree(b->p_last);
-  bfree(b->flags);
+  bfree(b->pot); bfree(b->potd); bfree(b->potdd);
+  bfree(b->asm_ptr); bfree(b->asm_idx); bfree(b->ac_ptr); bfree(b->ac_idx); bfree(b->info);
+  bfree(b->local); bfree(b->ac_local);
   bfree(b->src_ig); bfree(b->src_slot); bfree(b->src_id); bfree(b->src_ploc); bfree(b->src_arr); bfree(b->src_stf);
   bfree(b->rec_slot); bfree(b->rec_ig); bfree(b->rec_h); bfree(b->rec_nu); bfree(b->seis);
   delete b;

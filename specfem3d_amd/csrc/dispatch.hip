@@ -19,8 +19,8 @@ void launch_elastic_exact(hipStream_t, const ElasticArgs&, bool, bool, int);
 void launch_elastic_fast(hipStream_t, const ElasticArgs&, bool, bool, int);
 void launch_element_strain_exact(hipStream_t, const ElasticArgs&, realw*, realw*, bool);
 void launch_element_strain_fast(hipStream_t, const ElasticArgs&, realw*, realw*, bool);
-void launch_elastic_batch_exact(hipStream_t, const BatchArgs&, int, int, int);
-void launch_elastic_batch_fast(hipStream_t, const BatchArgs&, int, int, int);
+void launch_elastic_batch_exact(hipStream_t, const BatchArgs&, int);
+void launch_elastic_batch_fast(hipStream_t, const BatchArgs&, int);
 void launch_elastic_pml_exact(hipStream_t, const PmlArgs&);
 void launch_elastic_pml_fast(hipStream_t, const PmlArgs&);
 void launch_acoustic_exact(hipStream_t, const AcousticArgs&, int);
@@ -48,29 +48,29 @@ void launch_elastic_pml(hipStream_t s, const PmlArgs& a, bool exact) {
     launch_elastic_pml_fast(s, a);
 }
 
-void launch_visco_batch_exact(hipStream_t, const BatchArgs&, int, int);
-void launch_visco_batch_fast(hipStream_t, const BatchArgs&, int, int);
-void launch_visco_batch(hipStream_t s, const BatchArgs& a, int sc, int mode, bool exact) {
+void launch_visco_batch_exact(hipStream_t, const BatchArgs&, int);
+void launch_visco_batch_fast(hipStream_t, const BatchArgs&, int);
+void launch_visco_batch(hipStream_t s, const BatchArgs& a, int sc, bool exact) {
   if (exact)
-    launch_visco_batch_exact(s, a, sc, mode);
+    launch_visco_batch_exact(s, a, sc);
   else
-    launch_visco_batch_fast(s, a, sc, mode);
+    launch_visco_batch_fast(s, a, sc);
 }
 
-void launch_elastic_batch(hipStream_t s, const BatchArgs& a, int sc, int mode, int overlay, bool exact) {
+void launch_elastic_batch(hipStream_t s, const BatchArgs& a, int sc, bool exact) {
   if (exact)
-    launch_elastic_batch_exact(s, a, sc, mode, overlay);
+    launch_elastic_batch_exact(s, a, sc);
   else
-    launch_elastic_batch_fast(s, a, sc, mode, overlay);
+    launch_elastic_batch_fast(s, a, sc);
 }
 
-void launch_acoustic_batch_exact(hipStream_t, const BatchAcArgs&, int, int);
-void launch_acoustic_batch_fast(hipStream_t, const BatchAcArgs&, int, int);
-void launch_acoustic_batch(hipStream_t s, const BatchAcArgs& a, int sc, int mode, bool exact) {
+void launch_acoustic_batch_exact(hipStream_t, const BatchAcArgs&, int);
+void launch_acoustic_batch_fast(hipStream_t, const BatchAcArgs&, int);
+void launch_acoustic_batch(hipStream_t s, const BatchAcArgs& a, int sc, bool exact) {
   if (exact)
-    launch_acoustic_batch_exact(s, a, sc, mode);
+    launch_acoustic_batch_exact(s, a, sc);
   else
-    launch_acoustic_batch_fast(s, a, sc, mode);
+    launch_acoustic_batch_fast(s, a, sc);
 }
 
 void launch_acoustic(hipStream_t s, const AcousticArgs& a, bool exact, int mode) {

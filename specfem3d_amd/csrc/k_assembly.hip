@@ -117,11 +117,12 @@ __global__ void k_csr_sort(int nglob, const int* __restrict__ ptr, const int* __
   }
 }
 
-// 128-byte lines of the local forces that a wave over 64 consecutive points reads: lanes whose w-th
-// slot lies in another line than that of the lane before
+// 128-byte lines of the local forces that a wave over 64 consecutive points reads (one wave in 16 is
+// counted): lanes whose w-th slot lies in another line than that of the lane before
 __global__ void k_count_lines(int nglob, const int* __restrict__ ptr, const int* __restrict__ idx,
                               const int* __restrict__ pos, int eb, unsigned long long* lines) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int g = (t >> 6) * 1024 + (t & 63);
   const int b = g < nglob ? ptr[g] : 0, e = g < nglob ? ptr[g + 1] : 0;
   int n1 = 0, n2 = 0;
   for (int w = 0; w < 4; w++) {
@@ -209,7 +210,7 @@ int build_slot_lists(hipStream_t s, int nglob, int nspec, int nelem, const int* 
     if (nelem > nlaunch)
       hipLaunchKernelGGL(k_list_position, sf_grid(nelem - nlaunch, 256), dim3(256), 0, s, nelem - nlaunch,
                          order + nlaunch, pos, pos0);
-    hipLaunchKernelGGL(k_count_lines, sf_grid(nglob, 256), dim3(256), 0, s, nglob, ptr, idx, pos, eb, lines);
+    hipLaunchKernelGGL(k_count_lines, sf_grid((nglob + 1023) / 1024 * 64, 256), dim3(256), 0, s, nglob, ptr, idx, pos, eb, lines);
     SF_CHECK(hipMemcpyAsync(h, lines, sizeof(h), hipMemcpyDeviceToHost, s));
     SF_CHECK(hipStreamSynchronize(s));
     if (h[0] <= h[1]) eb = 1;

@@ -1,30 +1,21 @@
 // k_batch.hip -- element stiffness of the batched many-shot engine (elastic, isotropic).
 //
-// Many independent shots share one mesh. Their wavefields are interleaved shot-fastest: the value
-// (global point g, component c, shot s) lives at ((int64_t)g * 3 + c) * S + s, S = padded shot
-// count. A workgroup takes one element and a group of SC shots (SC = 4 or 8): the element's ibool,
-// moduli and Jacobian terms are loaded once for the SC shots, and workgroups of one element's shot
-// groups are adjacent in the grid, so the groups share the L2 lines of each row. The per-point arithmetic is elastic_point.h, the
-// same code as the single-shot kernel, so a batched shot reproduces its single-shot run.
+// Many independent shots share one mesh. Their wavefields are kept in groups of eight shots
+// (batch_idx): a point's three rows of a group are 96 contiguous bytes, and a run of points is a run
+// of full cache lines that no other group touches, so a finished group costs nothing and leaves no
+// holes in the rows of the others. A workgroup takes one element and SC
+// shots (SC = 4 or 8): the element's ibool, moduli and Jacobian terms are loaded once for them, and
+// the workgroups of one element's shots are adjacent in the grid, so they share those. The per-point
+// arithmetic is elastic_point.h, the same code as the single-shot kernel, so a batched shot reproduces
+// its single-shot run.
 //
 // Shots are stored in decreasing order of record length; a shot is live at step `it` while
 // nstep[s] >= it, and a group whose first shot has finished exits at once (uneven record
 // lengths cost nothing after a shot ends). `it` is read from device memory so a captured graph
 // of the step can be replayed.
 //
-// MODE 3 fuses the Newmark update into the coloured stiffness launches. Within a colour no two
-// elements share a point, and the colours of a step run in order, so for every global point the
-// element of its highest colour (flag BF_LAST) holds the last contribution: it finishes the
-// point there -- a *= rmass, v += dt/2 a (corrector), then the next step's predictor
-// u += dt v + dt^2/2 a, v += dt/2 a -- because every other element containing the point has
-// already gathered u in an earlier colour. The element of the lowest colour (BF_FIRST) writes its
-// contribution instead of adding it, so `a` is never cleared except at points that the Stacey and
-// source passes add to before the colours (BF_ZERO: cleared by the finisher, never BF_FIRST). A
-// point of a single element is gathered, computed and finished in one workgroup with no `a`
-// traffic. The sums run in the same order as the separate update path (Stacey, sources, colours
-// in order, then the corrector), so the results are the same bits. At a shot's last step the
-// finisher applies the corrector only, leaving the state of the last step as the single-shot run
-// does.
+// The stiffness stores the local forces, and the update that starts the next step sums them per point
+// (k_batch_gather in batch.hip), in the element order of the single-shot run.
 //
 // Compiled twice like k_elastic.hip: SF_EXACT=1 without FMA contraction, SF_EXACT=0 with it.
 #include "elastic_point.h"
@@ -43,20 +34,6 @@
 namespace sf {
 namespace SF_VNS {
 
-// corrector of the finished step, then (cont) the predictor of the next one; never contracted, so
-// the fast build rounds like the separate update kernel (k_update.hip)
-__device__ __forceinline__ void newmark_finish(realw& u, realw& v, realw& a, realw M, realw dt, realw dt2, realw dtsq2,
-                                               bool cont) {
-#pragma clang fp contract(off)
-  a = a * M;
-  v = v + dt2 * a;
-  if (cont) {
-    u = u + dt * v + dtsq2 * a;
-    v = v + dt2 * a;
-  }
-}
-
-__device__ __forceinline__ realw& q4(float4& x, int r) { return r == 0 ? x.x : r == 1 ? x.y : r == 2 ? x.z : x.w; }
 __device__ __forceinline__ realw c4(const float4& x, int r) { return r == 0 ? x.x : r == 1 ? x.y : r == 2 ? x.z : x.w; }
 
 __device__ __forceinline__ int xcd_remap_b(int b, int nb) {
@@ -64,162 +41,164 @@ __device__ __forceinline__ int xcd_remap_b(int b, int nb) {
   return x * q + (x < r ? x : r) + (b >> 3);
 }
 
-// OV = 1 overlays the displacement tile on the stress-product planes (9 instead of 12 planes of
-// LDS, one more barrier; the lane keeps its own displacement in registers for the fused update),
-// which lets more workgroups share a CU.
-template <int NQ, int MODE, int OV>
-__global__ void __launch_bounds__(128 * NQ) __attribute__((amdgpu_waves_per_eu(OV ? 4 : 3)))
-k_elastic_batch(BatchArgs B, GLLk G) {
-  constexpr int SC = 4 * NQ;
-  // LDS tile rows (component or stress product, shot) of PST floats, point fastest. PST = 132:
-  // the rows of a lane's two quads start 16 banks apart (4 * 132 = 16 mod 32), so the 32 lanes of
-  // an LDS pass (16 consecutive points, two quads) read 32 different banks.
-  constexpr int PST = 132;
-  constexpr int CPL = SC * PST;                   // one component / product plane
-  __shared__ realw sBuf[(OV ? 9 : 12) * CPL];
-  realw* const sT = sBuf;                         // stress products   [m][s][p]
-  // displacement tile [c][s][p]; with OV it shares the planes of the products t3 (m = 6..8),
-  // which are written last
-  realw* const sU = OV ? sBuf + 6 * CPL : sBuf + 9 * CPL;
-  __shared__ realw sG[SF_NGLL_TABLE];                        // hprime, hprimewgll, wgllwgll
-  stage_gll(sG, G, threadIdx.x);
+// One element and SC = 4 or 8 shots per workgroup of 32 SC lanes, in two lane roles:
+//   * global memory: lane = three units of 4 consecutive shots of one point and component, unit n =
+//     (point, component, quad) with the quad fastest: with SC = 8 the units of a row of five points are
+//     480 contiguous bytes, and the element's local forces one run of 12 KB;
+//   * contractions: lane = (line of five points, shot), shot fastest, 25 SC lanes: the line scheme of
+//     k_elastic_line (k_elastic.hip). The lane's gamma column stays in its registers, its xi and eta
+//     rows go through LDS once each way, the coefficients sit in scalar registers.
+// Both meet in LDS planes of the same order (point, component, shot). 61 VGPRs, 24 KB of LDS, six
+// workgroups per CU. Two or three elements per workgroup fill the lanes better (25 SC of 32 SC work
+// here) and are slower all the same (572 and 700 us against 523 for the whole step of 16 shots on
+// 32x32x16 elements, same source otherwise): seven or ten waves wait for each other at each barrier.
+// REG: no irregular element in the mesh (FMA build: the mapping is folded into the tables).
+template <int SC, bool REG>
+__global__ void __launch_bounds__(32 * SC) k_elastic_batch(BatchArgs B, GLLk G) {
+  constexpr bool FOLD = REG && SF_FOLD;
+  constexpr int NQ = SC / 4, NU = 375 * NQ, NT = 32 * SC, PS = 3 * SC;
+  __shared__ __attribute__((aligned(16))) realw sA[375 * SC], sB[375 * SC];  // (p, a, s) at p PS + a SC + s
+  __shared__ realw sW[25];
+  const int t = threadIdx.x;
   const int it = __hip_atomic_load(B.it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const int b = xcd_remap_b(blockIdx.x, gridDim.x);
   const int ie = b / B.ngroups;
-  const int s0 = (b - ie * B.ngroups) * SC;
+  const int s0 = B.s_first + (b - ie * B.ngroups) * SC;
   if (B.nstep[s0] < it) return;                   // every shot of this group has finished
-  const int q = threadIdx.x % NQ, p = threadIdx.x / NQ;
-  const int sq = s0 + 4 * q;                      // first shot of this lane's quad
-  const bool live0 = B.nstep[sq] >= it;           // shots sorted: later ones finish first
-  bool live[4];
-#pragma unroll
-  for (int r = 0; r < 4; r++) live[r] = B.nstep[sq + r] >= it;
-  const bool active = p < 125;
-  const int pp = active ? p : 124;
+  if (t < 25) sW[t] = G.wxy[t];
   const int e = B.elems[ie];
-  const int irr = B.irregular[e];
-  const int64_t S = B.S;
-  const int g = B.ibool[(int64_t)e * 125 + pp];
-  const int64_t row = (int64_t)g * 3 * S + sq;
-  const int ts = 4 * q;                           // tile slot of the quad
-  // Load order matters (the vector-memory counter retires in order): point flags, displacement,
-  // moduli and Jacobian terms first, then the lane's accumulator and velocity rows, which are
-  // only needed after the element computation and stay in flight across the LDS-only barriers
-  // (a: unless this lane writes first; v: only where it finishes the update).
-  const unsigned fl = MODE == 3 ? (unsigned)B.flags[(int64_t)e * 125 + pp] : 0u;
-  float4 u0 = make_float4(0.f, 0.f, 0.f, 0.f), u1 = u0, u2 = u0;  // staged into LDS below
-  if (live0) {
-    u0 = *reinterpret_cast<const float4*>(B.u + row);
-    u1 = *reinterpret_cast<const float4*>(B.u + row + S);
-    u2 = *reinterpret_cast<const float4*>(B.u + row + 2 * S);
-  }
-  const float2 km = B.kappamu[(int64_t)e * 125 + pp];
-  JacPt J = {};
-  realw jacl = B.jacobian_regular;
-  if (irr) {
-    J = load_jac(B.jac, B.jac_plane, (int64_t)(irr - 1) * 125 + pp);
-    jacl = J.jac;
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  const bool first = MODE == 3 && (fl & BF_FIRST) != 0;
-  const bool last = MODE == 3 && (fl & BF_LAST) != 0;
-  const bool mine = active && live0;
-  float4 A[3], V[3];
+  const int irr = REG ? 0 : B.irregular[e];
+  // memory role: units t, t + NT, t + 2 NT of 375 NQ
+  const int q4 = t % NQ, sq = s0 + 4 * q4;        // NT is a multiple of NQ: one quad for all three
+  const bool live0 = B.nstep[sq] >= it;           // shots sorted: later ones finish first
+  int64_t row[3];
+  bool mine[3];
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
-    A[c] = make_float4(0.f, 0.f, 0.f, 0.f);
-    V[c] = A[c];
-    if (MODE != 0 && mine && (!first || !live[3])) A[c] = *reinterpret_cast<const float4*>(B.a + row + c * S);
-    if (last && mine) V[c] = *reinterpret_cast<const float4*>(B.v + row + c * S);
+  for (int m = 0; m < 3; m++) {
+    const int n = t + m * NT, p = n < NU ? n / (3 * NQ) : 124;
+    mine[m] = n < NU && live0;
+    row[m] = batch_idx(B.nrow, 3 * (int64_t)B.ibool[(int64_t)e * 125 + p] + n / NQ % 3, sq);
   }
-  __builtin_amdgcn_sched_barrier(0);
-  if (active) {
+  // line role: column / rows of c, shot s (25 SC of the lanes; the rest shadow the first ones)
+  const bool lane = t < 25 * SC;
+  const int tt = lane ? t : t - 25 * SC;
+  const int s = tt % SC, c = tt / SC;
+  const int i = c % 5, j = c / 5;
+  const int64_t ep = (int64_t)e * 125 + c;
+  float2 km[5];
+  {
+    float4 u[3];
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      sU[(0 * SC + ts + r) * PST + p] = c4(u0, r);
-      sU[(1 * SC + ts + r) * PST + p] = c4(u1, r);
-      sU[(2 * SC + ts + r) * PST + p] = c4(u2, r);
+    for (int m = 0; m < 3; m++) {
+      u[m] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (mine[m]) u[m] = *reinterpret_cast<const float4*>(B.u + row[m]);
+    }
+#pragma unroll
+    for (int k = 0; k < 5; k++) km[k] = B.kappamu[ep + 25 * k];
+#pragma unroll
+    for (int m = 0; m < 3; m++)
+      if (t + m * NT < NU) *reinterpret_cast<float4*>(&sA[4 * (t + m * NT)]) = u[m];
+  }
+  lds_barrier();
+  const int bp = c * PS + s;                      // point k of the column at bp + 25 PS k
+  const int bx = 5 * c * PS + s, by = (i + 25 * j) * PS + s;
+  realw d3[5][3];
+  {
+    realw x[3][5];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      realw r[5], y[5], z[5];
+#pragma unroll
+      for (int l = 0; l < 5; l++) {
+        r[l] = sA[bx + PS * l + SC * a];
+        y[l] = sA[by + 5 * PS * l + SC * a];
+        z[l] = sA[bp + 25 * PS * l + SC * a];
+      }
+      line_gradient(G.hp, r, x[a]);
+      line_gradient(G.hp, y, r);
+      if (lane) {
+#pragma unroll
+        for (int l = 0; l < 5; l++) sB[by + 5 * PS * l + SC * a] = r[l];
+      }
+      line_gradient(G.hp, z, r);
+#pragma unroll
+      for (int k = 0; k < 5; k++) d3[k][a] = r[k];
+    }
+    lds_barrier();                                // every row of u has been read
+    if (lane) {
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int l = 0; l < 5; l++) sA[bx + PS * l + SC * a] = x[a][l];
     }
   }
   lds_barrier();
-
-  const int k = pp / 25, j = (pp / 5) % 5, i = pp % 5;
-  realw t3[4][3];                                 // products t3 of each shot (written last with OV)
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const realw* su = sU + (ts + r) * PST;
-    const Grad9 tg = tile_gradient<1>(su, su + SC * PST, su + 2 * SC * PST, gll_hp(sG, irr != 0), i, j, k);
-    const Du9 du = map_gradient(tg, irr != 0, J, B.xix_regular);
-    const Sigma6 sg = iso_stress(du, km.x, km.y);
-    realw t[9];
-    stress_products(sg, irr != 0, J, jacl, B.xix_regular, t);
-    if (active) {
-#pragma unroll
-      for (int m = 0; m < (OV ? 6 : 9); m++) sT[(m * SC + ts + r) * PST + p] = t[m];
+  for (int k = 0; k < 5; k++) {
+    const int q = bp + 25 * PS * k;
+    const Grad9 tg = {sA[q], sA[q + SC], sA[q + 2 * SC], sB[q], sB[q + SC], sB[q + 2 * SC], d3[k][0], d3[k][1], d3[k][2]};
+    JacPt J = {};
+    realw jacl = B.jacobian_regular;
+    if (!REG && irr) {
+      J = load_jac(B.jac, B.jac_plane, (int64_t)(irr - 1) * 125 + c + 25 * k);
+      jacl = J.jac;
     }
-    t3[r][0] = t[6]; t3[r][1] = t[7]; t3[r][2] = t[8];
-  }
-  if (OV) {
-    lds_barrier();                                // every lane is done with the displacement tile
-    if (active) {
+    const Du9 du = map_gradient<FOLD>(tg, irr != 0, J, B.xix_regular);
+    const Sigma6 sg = iso_stress(du, km[k].x, km[k].y);
+    realw pr[9];
+    stress_products<FOLD>(sg, irr != 0, J, jacl, B.xix_regular, pr);
 #pragma unroll
-      for (int r = 0; r < 4; r++)
-#pragma unroll
-        for (int m = 6; m < 9; m++) sT[(m * SC + ts + r) * PST + p] = t3[r][m - 6];
+    for (int a = 0; a < 3; a++) {
+      if (lane) {
+        sA[q + SC * a] = pr[a];
+        sB[q + SC * a] = pr[3 + a];
+      }
+      d3[k][a] = pr[6 + a];
     }
   }
   lds_barrier();
-  if (!mine) return;
-
-  // one force component at a time for the lane's four shots (keeps few values live)
-  realw* a = B.a + row;
-  const realw* hpw = gll_hpw(sG, irr != 0);
-  const realw* wxy = sG + 50;
-  bool cont[4], ends = false;
 #pragma unroll
-  for (int r = 0; r < 4; r++) {
-    cont[r] = live[r] && B.nstep[sq + r] > it;
-    ends = ends || (live[r] && !cont[r]);
+  for (int a = 0; a < 3; a++) {
+    realw r[5], y[5], o[5];
+#pragma unroll
+    for (int l = 0; l < 5; l++) {
+      r[l] = sA[bx + PS * l + SC * a];
+      y[l] = sB[by + 5 * PS * l + SC * a];
+    }
+    line_divergence(G.hpw, r, o);
+    if (lane) {
+#pragma unroll
+      for (int l = 0; l < 5; l++) sA[bx + PS * l + SC * a] = o[l];
+    }
+    line_divergence(G.hpw, y, o);
+    if (lane) {
+#pragma unroll
+      for (int l = 0; l < 5; l++) sB[by + 5 * PS * l + SC * a] = o[l];
+    }
+#pragma unroll
+    for (int k = 0; k < 5; k++) r[k] = d3[k][a];
+    line_divergence(G.hpw, r, o);
+#pragma unroll
+    for (int k = 0; k < 5; k++) d3[k][a] = o[k];
   }
+  lds_barrier();
+  if (lane) {
+    const realw w3 = sW[i * 5 + j];
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
-    realw f[4];
+    for (int k = 0; k < 5; k++) {
+      const int q = bp + 25 * PS * k;
+      const realw w1 = sW[j * 5 + k], w2 = sW[i * 5 + k];
 #pragma unroll
-    for (int r = 0; r < 4; r++) f[r] = tile_divergence_c<1>(sT + (ts + r) * PST, CPL, hpw, wxy, i, j, k, c);
-    if (MODE == 0) {
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-        if (live[r]) atomicAdd(a + c * S + r, -f[r]);
-      continue;
+      for (int a = 0; a < 3; a++) sA[q + SC * a] = w1 * sA[q + SC * a] + w2 * sB[q + SC * a] + w3 * d3[k][a];
     }
-    float4 Ac = A[c];
+  }
+  lds_barrier();
+  // finished shots of a live quad store what their last displacement gives; nothing reads it
+  realw* o = B.local + (int64_t)(sq >> 3) * B.loc_group + (int64_t)ie * 3000 + (sq & 7);
 #pragma unroll
-    for (int r = 0; r < 4; r++)
-      if (live[r]) q4(Ac, r) = (first ? 0.f : q4(Ac, r)) + (-f[r]);
-    if (MODE == 2 || !last) {
-      *reinterpret_cast<float4*>(a + c * S) = Ac;
-      continue;
-    }
-    // fused mode, last colour of this point: finish the Newmark update of component c
-    const realw M = B.rmass[(int64_t)g * 3 + c];
-    float4 Vc = V[c];
-    // this step's displacement: the LDS tile without overlay, else the row again (still in cache)
-    float4 U;
-    if (OV) {
-      U = *reinterpret_cast<const float4*>(B.u + row + c * S);
-    } else {
-      const realw* su = sU + (c * SC + ts) * PST + p;
-      U = make_float4(su[0], su[PST], su[2 * PST], su[3 * PST]);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      if (!live[r]) continue;
-      newmark_finish(q4(U, r), q4(Vc, r), q4(Ac, r), M, B.dt, B.dt2, B.dtsq2, cont[r]);
-      if (cont[r]) q4(Ac, r) = 0.f;
-    }
-    if (cont[0]) *reinterpret_cast<float4*>(B.u + row + c * S) = U;
-    *reinterpret_cast<float4*>(B.v + row + c * S) = Vc;
-    if ((fl & BF_ZERO) || ends) *reinterpret_cast<float4*>(a + c * S) = Ac;
+  for (int m = 0; m < 3; m++) {
+    const int n = t + m * NT;
+    if (mine[m]) *reinterpret_cast<float4*>(o + 8 * (n / NQ)) = *reinterpret_cast<const float4*>(&sA[4 * n]);
   }
 }
 
@@ -227,8 +206,7 @@ k_elastic_batch(BatchArgs B, GLLk G) {
 // (one block per element and shot: plane, point). The tile holds u and dt*v (6 rows per shot; they share the
 // LDS of the stress products t2, t3, written after a barrier). Per shot, the arithmetic and its
 // order are the single-shot point kernel's (k_elastic_pt): strain at u + dt v, isotropic stress
-// minus the memory-variable sums, memory update, stress products. Assembly as k_elastic_batch
-// (MODE 2 coloured read-modify-write, 3 coloured with the Newmark update fused).
+// minus the memory-variable sums, memory update, stress products.
 // Per-shot state is one block per (element, shot), point-fastest within each plane: the lanes of a
 // wave that read one shot read consecutive words (a shot-fastest row would spread a wave's reads
 // of one shot over S times as many cache lines), and the planes of a block sit at fixed offsets
@@ -240,7 +218,7 @@ __device__ __forceinline__ int64_t eb_idx(int64_t e, int c, int p, int64_t S, in
   return ((e * S + s) * 6 + c) * 125 + p;
 }
 
-template <int NQ, int MODE>
+template <int NQ>
 __global__ void __launch_bounds__(128 * NQ) k_visco_batch(BatchArgs B, GLLk G) {
   constexpr int SC = 4 * NQ;
   constexpr int PST = 132;                        // see k_elastic_batch
@@ -253,7 +231,7 @@ __global__ void __launch_bounds__(128 * NQ) k_visco_batch(BatchArgs B, GLLk G) {
   const int it = __hip_atomic_load(B.it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const int b = xcd_remap_b(blockIdx.x, gridDim.x);
   const int ie = b / B.ngroups;
-  const int s0 = (b - ie * B.ngroups) * SC;
+  const int s0 = B.s_first + (b - ie * B.ngroups) * SC;
   if (B.nstep[s0] < it) return;
   const int q = threadIdx.x % NQ, p = threadIdx.x / NQ;
   const int sq = s0 + 4 * q;
@@ -268,7 +246,7 @@ __global__ void __launch_bounds__(128 * NQ) k_visco_batch(BatchArgs B, GLLk G) {
   const int64_t S = B.S;
   const int64_t ep = (int64_t)e * 125 + pp;
   const int g = B.ibool[ep];
-  const int64_t row = (int64_t)g * 3 * S + sq;
+  const int64_t row = batch_idx(B.nrow, 3 * (int64_t)g, sq);
   const int ts = 4 * q;
   float4 u[3], V[3];                              // staged into the tile below
 #pragma unroll
@@ -276,13 +254,10 @@ __global__ void __launch_bounds__(128 * NQ) k_visco_batch(BatchArgs B, GLLk G) {
     u[c] = make_float4(0.f, 0.f, 0.f, 0.f);
     V[c] = u[c];
     if (live0) {
-      u[c] = *reinterpret_cast<const float4*>(B.u + row + c * S);
-      V[c] = *reinterpret_cast<const float4*>(B.v + row + c * S);
+      u[c] = *reinterpret_cast<const float4*>(B.u + row + c * 8);
+      V[c] = *reinterpret_cast<const float4*>(B.v + row + c * 8);
     }
   }
-  const unsigned fl = MODE == 3 ? (unsigned)B.flags[ep] : 0u;
-  const bool first = MODE == 3 && (fl & BF_FIRST) != 0;
-  const bool last = MODE == 3 && (fl & BF_LAST) != 0;
   const bool mine = active && live0;
   JacPt J = {};
   realw jacl = B.jacobian_regular;
@@ -402,42 +377,17 @@ __global__ void __launch_bounds__(128 * NQ) k_visco_batch(BatchArgs B, GLLk G) {
   lds_barrier();
   if (!mine) return;
 
-  realw* a = B.a + row;
   const realw* hpw = gll_hpw(sG, irr != 0);
   const realw* wxy = sG + 50;
-  bool cont[4], ends = false;
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    cont[r] = live[r] && B.nstep[sq + r] > it;
-    ends = ends || (live[r] && !cont[r]);
-  }
+  realw* o = B.local + (int64_t)(sq >> 3) * B.loc_group + ((int64_t)ie * 125 + p) * 24 + (sq & 7);
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    realw f[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) f[r] = tile_divergence_c<1>(sT + (ts + r) * PST, CPL, hpw, wxy, i, j, k, c);
-    float4 Ac = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (!first || !live[3]) Ac = *reinterpret_cast<const float4*>(a + c * S);
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-      if (live[r]) q4(Ac, r) = (first ? 0.f : q4(Ac, r)) + (-f[r]);
-    if (MODE == 2 || !last) {
-      *reinterpret_cast<float4*>(a + c * S) = Ac;
-      continue;
-    }
-    const realw M = B.rmass[(int64_t)g * 3 + c];
-    // this step's u and v rows again (read at the start for the tile; kept out of registers)
-    float4 Vc = *reinterpret_cast<const float4*>(B.v + row + c * S);
-    float4 U = *reinterpret_cast<const float4*>(B.u + row + c * S);
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      if (!live[r]) continue;
-      newmark_finish(q4(U, r), q4(Vc, r), q4(Ac, r), M, B.dt, B.dt2, B.dtsq2, cont[r]);
-      if (cont[r]) q4(Ac, r) = 0.f;
-    }
-    if (cont[0]) *reinterpret_cast<float4*>(B.u + row + c * S) = U;
-    *reinterpret_cast<float4*>(B.v + row + c * S) = Vc;
-    if ((fl & BF_ZERO) || ends) *reinterpret_cast<float4*>(a + c * S) = Ac;
+    float4 f;
+    f.x = tile_divergence_c<1>(sT + ts * PST, CPL, hpw, wxy, i, j, k, c);
+    f.y = tile_divergence_c<1>(sT + (ts + 1) * PST, CPL, hpw, wxy, i, j, k, c);
+    f.z = tile_divergence_c<1>(sT + (ts + 2) * PST, CPL, hpw, wxy, i, j, k, c);
+    f.w = tile_divergence_c<1>(sT + (ts + 3) * PST, CPL, hpw, wxy, i, j, k, c);
+    *reinterpret_cast<float4*>(o + 8 * c) = f;
   }
 }
 
@@ -447,9 +397,8 @@ __global__ void __launch_bounds__(128 * NQ) k_visco_batch(BatchArgs B, GLLk G) {
 // potential tile and the three products (rho^-1 jacobian grad chi . grad xi, eta, gamma) go through
 // LDS, one row of PST floats per (plane, shot). Every sum runs in k_acoustic's order (the gamma
 // contraction reads the same values the column kernel holds in registers), so a batched shot
-// reproduces the single-shot run with the same assembly. MODE 0 atomic scatter, 2 plain
-// read-modify-write (the launch holds one colour).
-template <int NQ, int MODE>
+// reproduces the single-shot run with the same order of sums.
+template <int NQ>
 __global__ void __launch_bounds__(128 * NQ) k_acoustic_batch(BatchAcArgs B, GLLk G) {
   constexpr int SC = 4 * NQ;
   constexpr int PST = 132;
@@ -460,23 +409,20 @@ __global__ void __launch_bounds__(128 * NQ) k_acoustic_batch(BatchAcArgs B, GLLk
   const int it = __hip_atomic_load(B.it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const int b = xcd_remap_b(blockIdx.x, gridDim.x);
   const int ie = b / B.ngroups;
-  const int s0 = (b - ie * B.ngroups) * SC;
+  const int s0 = B.s_first + (b - ie * B.ngroups) * SC;
   if (B.nstep[s0] < it) return;
   const int q = threadIdx.x % NQ, p = threadIdx.x / NQ;
   const int sq = s0 + 4 * q;
-  bool live[4];
-#pragma unroll
-  for (int r = 0; r < 4; r++) live[r] = B.nstep[sq + r] >= it;
+  const bool live0 = B.nstep[sq] >= it;
   const bool active = p < 125;
   const int pp = active ? p : 124;
   const int e = B.elems[ie];
   const int irr = B.irregular[e];
-  const int64_t S = B.S;
   const int g = B.ibool[(int64_t)e * 125 + pp];
-  const int64_t row = ((int64_t)g - B.g0) * S + sq;
+  const int64_t row = batch_idx(B.nrow, (int64_t)g - B.g0, sq);
   const int ts = 4 * q;
   float4 c0 = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (live[0]) c0 = *reinterpret_cast<const float4*>(B.pot + row);
+  if (live0) c0 = *reinterpret_cast<const float4*>(B.pot + row);
   const realw rho_invl = (realw)1 / B.rho[(int64_t)e * 125 + pp];
   JacPt J = {};
   if (irr) J = load_jac(B.jac, B.jac_plane, (int64_t)(irr - 1) * 125 + pp);
@@ -521,11 +467,10 @@ __global__ void __launch_bounds__(128 * NQ) k_acoustic_batch(BatchAcArgs B, GLLk
     }
   }
   lds_barrier();
-  if (!active || !live[0]) return;
+  if (!active || !live0) return;
   const realw* hpw = sG + 25;
   const realw* wxy = sG + 50;
-  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (MODE == 2) acc = *reinterpret_cast<const float4*>(B.potdd + row);
+  float f[4];
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const realw* s1 = sBuf + (1 * SC + ts + r) * PST;
@@ -540,85 +485,65 @@ __global__ void __launch_bounds__(128 * NQ) k_acoustic_batch(BatchAcArgs B, GLLk
       n2 = n2 + hpw[l * 5 + j] * s2[b2 + 5 * l];
       n3 = n3 + hpw[l * 5 + k] * s3[b3 + 25 * l];
     }
-    const realw f = wxy[j * 5 + k] * n1 + wxy[i * 5 + k] * n2 + wxy[i * 5 + j] * n3;
-    if (!live[r]) continue;
-    if (MODE == 0) atomicAdd(B.potdd + row + r, -f);
-    else q4(acc, r) = q4(acc, r) + (-f);
+    f[r] = wxy[j * 5 + k] * n1 + wxy[i * 5 + k] * n2 + wxy[i * 5 + j] * n3;
   }
-  if (MODE == 2) *reinterpret_cast<float4*>(B.potdd + row) = acc;
+  realw* o = B.local + (int64_t)(sq >> 3) * B.loc_group + ((int64_t)ie * 125 + p) * 8 + (sq & 7);
+  *reinterpret_cast<float4*>(o) = make_float4(f[0], f[1], f[2], f[3]);
 }
 
 }  // namespace SF_VNS
 using namespace SF_VNS;
 
-void SFX(launch_elastic_batch)(hipStream_t st, const BatchArgs& a, int sc, int mode, int overlay) {
+void SFX(launch_elastic_batch)(hipStream_t st, const BatchArgs& a, int sc) {
   if (a.nelem <= 0 || a.ngroups <= 0) return;
+  const bool reg = a.jac_plane == 0;
+  GLLk G = g_gll_host;
+  if (reg && SF_FOLD) {
+    fold_gll(G, a.xix_regular, a.jacobian_regular);
+    for (int q = 0; q < 25; q++) {
+      G.hp[q] = G.hpr[q];
+      G.hpw[q] = G.hpwr[q];
+    }
+  }
   const int64_t nb = (int64_t)a.nelem * a.ngroups;
   if (nb > 0x7fffffff) fatal("launch_elastic_batch", "grid too large");
-  GLLk G = g_gll_host;
-  if (SF_FOLD) fold_gll(G, a.xix_regular, a.jacobian_regular);
-  dim3 grid((unsigned)nb);
-#define SF_KB(NQ, M)                                                                           \
-  if (overlay) hipLaunchKernelGGL((k_elastic_batch<NQ, M, 1>), grid, dim3(128 * NQ), 0, st, a, G); \
-  else hipLaunchKernelGGL((k_elastic_batch<NQ, M, 0>), grid, dim3(128 * NQ), 0, st, a, G)
-#define SF_KBM(M)                  \
-  if (sc == 4) SF_KB(1, M);        \
-  else if (sc == 8) SF_KB(2, M);   \
-  else fatal("launch_elastic_batch", "shots per workgroup must be 4 or 8");
-  if (mode == 3) {
-    if (!a.v || !a.rmass || !a.flags) fatal("launch_elastic_batch", "fused update needs v, rmass and point flags");
-    SF_KBM(3)
-  } else if (mode == 2) {
-    SF_KBM(2)
+#define SF_KB(SC, R) hipLaunchKernelGGL((k_elastic_batch<SC, R>), dim3((unsigned)nb), dim3(32 * SC), 0, st, a, G)
+  if (sc == 4) {
+    if (reg) SF_KB(4, true);
+    else SF_KB(4, false);
+  } else if (sc == 8) {
+    if (reg) SF_KB(8, true);
+    else SF_KB(8, false);
   } else {
-    SF_KBM(0)
+    fatal("launch_elastic_batch", "shots per workgroup must be 4 or 8");
   }
-#undef SF_KBM
 #undef SF_KB
   SF_LAUNCH_CHECK("k_elastic_batch");
 }
 
-void SFX(launch_visco_batch)(hipStream_t st, const BatchArgs& a, int sc, int mode) {
+void SFX(launch_visco_batch)(hipStream_t st, const BatchArgs& a, int sc) {
   if (a.nelem <= 0 || a.ngroups <= 0) return;
   const int64_t nb = (int64_t)a.nelem * a.ngroups;
   if (nb > 0x7fffffff) fatal("launch_visco_batch", "grid too large");
   if (!a.R || !a.eps || !a.v) fatal("launch_visco_batch", "memory variables, strain and velocity are needed");
-  if (mode == 3 && (!a.rmass || !a.flags)) fatal("launch_visco_batch", "fused update needs rmass and point flags");
-  dim3 grid((unsigned)nb);
+  const dim3 grid((unsigned)nb);
   GLLk G = g_gll_host;
   if (SF_FOLD) fold_gll(G, a.xix_regular, a.jacobian_regular);
-#define SF_KV(NQ, M) hipLaunchKernelGGL((k_visco_batch<NQ, M>), grid, dim3(128 * NQ), 0, st, a, G)
-  if (mode == 3) {
-    if (sc == 4) SF_KV(1, 3);
-    else if (sc == 8) SF_KV(2, 3);
-    else fatal("launch_visco_batch", "shots per workgroup must be 4 or 8");
-  } else if (mode == 2) {
-    if (sc == 4) SF_KV(1, 2);
-    else if (sc == 8) SF_KV(2, 2);
-    else fatal("launch_visco_batch", "shots per workgroup must be 4 or 8");
-  } else {
-    fatal("launch_visco_batch", "viscoelastic batches use coloured assembly (2 or 3)");
-  }
-#undef SF_KV
+  if (sc == 4) hipLaunchKernelGGL(k_visco_batch<1>, grid, dim3(128), 0, st, a, G);
+  else if (sc == 8) hipLaunchKernelGGL(k_visco_batch<2>, grid, dim3(256), 0, st, a, G);
+  else fatal("launch_visco_batch", "shots per workgroup must be 4 or 8");
   SF_LAUNCH_CHECK("k_visco_batch");
 }
 
-void SFX(launch_acoustic_batch)(hipStream_t st, const BatchAcArgs& a, int sc, int mode) {
+void SFX(launch_acoustic_batch)(hipStream_t st, const BatchAcArgs& a, int sc) {
   if (a.nelem <= 0 || a.ngroups <= 0) return;
   const int64_t nb = (int64_t)a.nelem * a.ngroups;
   if (nb > 0x7fffffff) fatal("launch_acoustic_batch", "grid too large");
-  dim3 grid((unsigned)nb);
+  const dim3 grid((unsigned)nb);
   const GLLk G = g_gll_host;
-#define SF_KA(NQ, M) hipLaunchKernelGGL((k_acoustic_batch<NQ, M>), grid, dim3(128 * NQ), 0, st, a, G)
-  if (sc != 4 && sc != 8) fatal("launch_acoustic_batch", "shots per workgroup must be 4 or 8");
-  if (mode == 0) {
-    if (sc == 4) SF_KA(1, 0);
-    else SF_KA(2, 0);
-  } else {
-    if (sc == 4) SF_KA(1, 2);
-    else SF_KA(2, 2);
-  }
-#undef SF_KA
+  if (sc == 4) hipLaunchKernelGGL(k_acoustic_batch<1>, grid, dim3(128), 0, st, a, G);
+  else if (sc == 8) hipLaunchKernelGGL(k_acoustic_batch<2>, grid, dim3(256), 0, st, a, G);
+  else fatal("launch_acoustic_batch", "shots per workgroup must be 4 or 8");
   SF_LAUNCH_CHECK("k_acoustic_batch");
 }
 

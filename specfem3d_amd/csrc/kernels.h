@@ -156,28 +156,34 @@ void launch_pml_store_old(hipStream_t s, int n, const int* pts, const realw* u, 
 // zero u, v, a at the listed points (Dirichlet condition of the C-PML outer faces)
 void launch_zero_points(hipStream_t s, int n, const int* pts, realw* u, realw* v, realw* a);
 
-// batched many-shot stiffness (k_batch.hip): fields interleaved shot-fastest,
-// value (g, c, s) at ((int64_t)g * 3 + c) * S + s
+// Batched wavefields (k_batch.hip, batch.hip): groups of eight shots, each group a field of its own
+// with rows of eight values: value (row r, shot s) of nrow rows at batch_idx, the next row of the same
+// shot 8 further on. Rows are 3 g + c for the solid and g - g0 for the potentials.
+__host__ __device__ __forceinline__ int64_t batch_idx(int64_t nrow, int64_t r, int s) {
+  return (((int64_t)(s >> 3) * nrow + r) << 3) + (s & 7);
+}
 struct BatchArgs {
   int nelem;
   const int* elems;
-  int ngroups;             // S / shots-per-workgroup
-  int S;                   // padded shot count (row stride)
+  int ngroups;             // shot groups of the launch: of 4 or 8 shots (launch_*_batch)
+  int s_first;             // first shot of the launch, a multiple of 8
+  int S;                   // padded shot count
+  int64_t nrow;            // rows of a group: 3 nglob
   const int* ibool;
   const int* irregular;
   realw xix_regular, jacobian_regular;
   const realw* jac;
   int64_t jac_plane;
   const float2* kappamu;
-  realw* u;
-  realw* a;
+  const realw* u;
+  const realw* v;          // viscoelastic: strain at u + dt v
+  realw dt;
+  // local forces: slot 125 ie + p of the launch, three rows of eight shots each; a block of loc_group
+  // floats per group of eight
+  realw* local;
+  int64_t loc_group;
   const int* nstep;        // per shot slot, decreasing (padding slots 0)
   const int* it;           // device step counter, 1-based current step
-  // fused Newmark update (mode 3 only)
-  realw* v;
-  const realw* rmass;      // inverse mass, 3 per global point
-  const unsigned char* flags;  // per local point e*125+p: BF_FIRST | BF_LAST | BF_ZERO
-  realw dt, dt2, dtsq2;
   // 3-SLS attenuation (k_visco_batch): per-shot memory variables and strain, one block per
   // (element, shot): value (e, shot, plane, p) at ((e * S + shot) * 18 + plane) * 125 + p
   // (strain: 6 planes)
@@ -191,21 +197,20 @@ struct BatchArgs {
   int64_t nloc;
   realw alpha[3], beta[3], gamma[3];
 };
+// per-local-point flags of sf_batch_point_flags
 enum : unsigned char { BF_FIRST = 1, BF_LAST = 2, BF_ZERO = 4 };
-// sc = shots per workgroup (4, 8); mode 0 atomic scatter, 2 plain read-modify-write (one colour),
-// 3 one colour with the Newmark update fused (see k_batch.hip); overlay 1 shares the LDS of the
-// displacement tile and the stress products
-void launch_elastic_batch(hipStream_t s, const BatchArgs& a, int sc, int mode, int overlay, bool exact);
-// viscoelastic (3 SLS) batched stiffness; mode 2 or 3
-void launch_visco_batch(hipStream_t s, const BatchArgs& a, int sc, int mode, bool exact);
+// sc = shots per workgroup (4, 8)
+void launch_elastic_batch(hipStream_t s, const BatchArgs& a, int sc, bool exact);
+// viscoelastic (3 SLS) batched stiffness
+void launch_visco_batch(hipStream_t s, const BatchArgs& a, int sc, bool exact);
 
-// batched acoustic stiffness (k_batch.hip): potentials interleaved shot-fastest over the acoustic
-// range of global points, value (g, s) at (g - g0) * S + s
+// batched acoustic stiffness (k_batch.hip): potentials over the acoustic range of global points
 struct BatchAcArgs {
   int nelem;
   const int* elems;
-  int ngroups;             // S / shots-per-workgroup
-  int S;                   // padded shot count (row stride)
+  int ngroups;             // shot groups of the launch, of 4 or 8 shots
+  int s_first;             // first shot of the launch, a multiple of 8
+  int64_t nrow;            // rows of a group: points of the acoustic range
   int64_t g0;              // first global point of the acoustic range
   const int* ibool;
   const int* irregular;
@@ -214,12 +219,13 @@ struct BatchAcArgs {
   int64_t jac_plane;
   const realw* rho;        // rhostore, nspec*125
   const realw* pot;
-  realw* potdd;
+  realw* local;            // slot 125 ie + p: a row of eight shots; loc_group floats per group of eight
+  int64_t loc_group;
   const int* nstep;        // per shot slot, decreasing (padding slots 0)
   const int* it;           // device step counter, 1-based current step
 };
-// sc = shots per workgroup (4, 8); mode 0 atomic scatter, 2 plain read-modify-write (one colour)
-void launch_acoustic_batch(hipStream_t s, const BatchAcArgs& a, int sc, int mode, bool exact);
+// sc = shots per workgroup (4, 8)
+void launch_acoustic_batch(hipStream_t s, const BatchAcArgs& a, int sc, bool exact);
 
 struct AcousticArgs {
   int nelem;
