@@ -55,7 +55,8 @@ static GatherArgs gather_args(Mesh* m, int f) {
 // sum the waiting local forces and run the pending corrector
 static void flush_el(Mesh* m, int f) {
   if (m->pending_gather_el[f]) {
-    launch_gather_update(m->stream, gather_args(m, f), m->pending_k3_el[f] ? GATHER_CORRECT : GATHER_ONLY);
+    launch_gather_update(m->stream, gather_args(m, f), m->pending_k3_el[f] ? GATHER_CORRECT : GATHER_ONLY,
+                         m->exact != 0);
     m->pending_gather_el[f] = 0;
     m->gather_skip_el[f] = 0;
     m->accel_clean[f] = 0;
@@ -200,7 +201,7 @@ extern "C" void FC_FUNC_(update_displacement_cuda, UPDATE_DISPLACMENT_CUDA)(long
     a.old = pml ? m->pml_old : nullptr;
     a.t1 = m->pml_t1;
     a.t2 = m->pml_t2;
-    launch_gather_update(m->stream, a, GATHER_STEP);
+    launch_gather_update(m->stream, a, GATHER_STEP, m->exact != 0);
   } else if (m->pending_k3_el[f]) {
     launch_corrector_predictor(m->stream, n, w.displ + o, w.veloc + o, w.accel + o, m->rmass + o,
                                m->pending_dt2_el[f], *deltat_F, *deltatover2_F, *deltatsqover2_F,

@@ -158,15 +158,9 @@ struct BatchGatherArgs {
   realw dt2p, dt, dt2, dtsq2;
 };
 
-__device__ __forceinline__ void sub4(float4& a, const float4& l) {
-  a.x = a.x + (-l.x);
-  a.y = a.y + (-l.y);
-  a.z = a.z + (-l.z);
-  a.w = a.w + (-l.w);
-}
-
 // a -= the local forces of slots ptr[g] .. ptr[g + 1], `unit` floats per slot, four slots in flight
-__device__ __forceinline__ void gather4(float4& a, const int* ptr, const int* idx, int64_t g, const realw* local,
+template <typename T>
+__device__ __forceinline__ void gather4(T a[4], const int* ptr, const int* idx, int64_t g, const realw* local,
                                         int unit) {
   const int p0 = ptr[g], p1 = ptr[g + 1];
   for (int p = p0; p < p1; p += 4) {
@@ -178,8 +172,13 @@ __device__ __forceinline__ void gather4(float4& a, const int* ptr, const int* id
     for (int w = 0; w < 4; w++)
       if (k[w] >= 0) l[w] = *reinterpret_cast<const float4*>(local + (int64_t)k[w] * unit);
 #pragma unroll
-    for (int w = 0; w < 4; w++)
-      if (k[w] >= 0) sub4(a, l[w]);
+    for (int w = 0; w < 4; w++) {
+      if (k[w] < 0) continue;
+      a[0] = a[0] + (-(T)l[w].x);
+      a[1] = a[1] + (-(T)l[w].y);
+      a[2] = a[2] + (-(T)l[w].z);
+      a[3] = a[3] + (-(T)l[w].w);
+    }
   }
 }
 
@@ -190,7 +189,8 @@ __device__ __forceinline__ int64_t xcd_block() {
   return (int64_t)x * q + (x < r ? x : r) + (b >> 3);
 }
 
-template <bool STEP>
+// T: float follows the reference's operations (exact builds), double rounds once per stored value
+template <bool STEP, typename T>
 __global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs A) {
   const int64_t t = xcd_block() * 256 + threadIdx.x;
   const int64_t pt = t / 6;
@@ -202,31 +202,32 @@ __global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs A) {
   const int64_t g = A.g0 + pt;
   const int64_t o = batch_idx(A.nrow, 3 * g + c, s);
   const bool term = (A.info[g] & AF_TERM) != 0;
-  float4 U0, V0, Ac = make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 U, V;
+  T a[4] = {0, 0, 0, 0};
   realw M = 0.f;
   if (STEP) {
-    U0 = *reinterpret_cast<const float4*>(A.u + o);
-    V0 = *reinterpret_cast<const float4*>(A.v + o);
+    U = *reinterpret_cast<const float4*>(A.u + o);
+    V = *reinterpret_cast<const float4*>(A.v + o);
     M = A.rm[3 * g + c];
   }
-  if (term) Ac = *reinterpret_cast<const float4*>(A.a + o);
-  gather4(Ac, A.ptr, A.idx, g, A.local + (int64_t)blockIdx.y * A.loc_group + 8 * c + 4 * (cq & 1), 24);
+  if (term) {
+    const float4 a0 = *reinterpret_cast<const float4*>(A.a + o);
+    a[0] = a0.x; a[1] = a0.y; a[2] = a0.z; a[3] = a0.w;
+  }
+  gather4<T>(a, A.ptr, A.idx, g, A.local + (int64_t)blockIdx.y * A.loc_group + 8 * c + 4 * (cq & 1), 24);
   if (!STEP) {
-    *reinterpret_cast<float4*>(A.a + o) = Ac;
+    *reinterpret_cast<float4*>(A.a + o) = make_float4((realw)a[0], (realw)a[1], (realw)a[2], (realw)a[3]);
     return;
   }
-  const bool l1 = A.nstep[s + 1] >= it, l2 = A.nstep[s + 2] >= it, l3 = A.nstep[s + 3] >= it;
-  float4 U = U0, V = V0;
-#define SF_BG(c)                              \
-  Ac.c = Ac.c * M;                            \
-  V.c = V.c + A.dt2p * Ac.c;                  \
-  U.c = U.c + A.dt * V.c + A.dtsq2 * Ac.c;    \
-  V.c = V.c + A.dt2 * Ac.c;
-  SF_BG(x) SF_BG(y) SF_BG(z) SF_BG(w)
+#define SF_BG(c, r)                                             \
+  if (r == 0 || A.nstep[s + r] >= it) {                         \
+    const T ac = a[r] * (T)M;                                   \
+    T vc = (T)V.c + (T)A.dt2p * ac;                             \
+    U.c = (realw)((T)U.c + (T)A.dt * vc + (T)A.dtsq2 * ac);     \
+    V.c = (realw)(vc + (T)A.dt2 * ac);                          \
+  }
+  SF_BG(x, 0) SF_BG(y, 1) SF_BG(z, 2) SF_BG(w, 3)
 #undef SF_BG
-  if (!l1) { U.y = U0.y; V.y = V0.y; }
-  if (!l2) { U.z = U0.z; V.z = V0.z; }
-  if (!l3) { U.w = U0.w; V.w = V0.w; }
   *reinterpret_cast<float4*>(A.u + o) = U;
   *reinterpret_cast<float4*>(A.v + o) = V;
   if (term) *reinterpret_cast<float4*>(A.a + o) = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -234,6 +235,7 @@ __global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs A) {
 
 // the same for the potentials: chi'' -= local forces, then the corrector chi'' *= rmass, chi' += dt/2 chi''
 // (rows g - g0; the boundary terms are in chi'' already)
+template <typename T>
 __global__ void __launch_bounds__(256) k_batch_ac_gather(int64_t nrow, int64_t g0, const int* __restrict__ ptr,
                                                          const int* __restrict__ idx, const realw* __restrict__ local,
                                                          int64_t loc_group, int first_group,
@@ -248,17 +250,19 @@ __global__ void __launch_bounds__(256) k_batch_ac_gather(int64_t nrow, int64_t g
   if (nstep[s] < it) return;
   const int64_t o = batch_idx(nrow, row, s);
   float4 V = *reinterpret_cast<const float4*>(potd + o);
-  float4 Ac = *reinterpret_cast<const float4*>(potdd + o);
-  const float4 V0 = V, A0 = Ac;
+  const float4 a0 = *reinterpret_cast<const float4*>(potdd + o);
   const realw M = rm[row];
-  gather4(Ac, ptr, idx, g0 + row, local + (int64_t)blockIdx.y * loc_group + 4 * (int)(t & 1), 8);
-  const bool l1 = nstep[s + 1] >= it, l2 = nstep[s + 2] >= it, l3 = nstep[s + 3] >= it;
-#define SF_AG(c) Ac.c = Ac.c * M; V.c = V.c + dt2 * Ac.c;
-  SF_AG(x) SF_AG(y) SF_AG(z) SF_AG(w)
+  T a[4] = {a0.x, a0.y, a0.z, a0.w};
+  gather4<T>(a, ptr, idx, g0 + row, local + (int64_t)blockIdx.y * loc_group + 4 * (int)(t & 1), 8);
+  float4 Ac = a0;
+#define SF_AG(c, r)                          \
+  if (r == 0 || nstep[s + r] >= it) {        \
+    const T ac = a[r] * (T)M;                \
+    Ac.c = (realw)ac;                        \
+    V.c = (realw)((T)V.c + (T)dt2 * ac);     \
+  }
+  SF_AG(x, 0) SF_AG(y, 1) SF_AG(z, 2) SF_AG(w, 3)
 #undef SF_AG
-  if (!l1) { V.y = V0.y; Ac.y = A0.y; }
-  if (!l2) { V.z = V0.z; Ac.z = A0.z; }
-  if (!l3) { V.w = V0.w; Ac.w = A0.w; }
   *reinterpret_cast<float4*>(potd + o) = V;
   *reinterpret_cast<float4*>(potdd + o) = Ac;
 }
@@ -638,7 +642,9 @@ static void enqueue_stiffness(Batch* b, hipStream_t st) {
       // no room for the local forces of all groups: sum them into accel before the next ones
       BatchGatherArgs ga = gather_args(b);
       ga.first_group = g;
-      hipLaunchKernelGGL(k_batch_gather<false>, dim3(sf_grid(6 * ga.n, 256).x, (unsigned)n), dim3(256), 0, st, ga);
+      const dim3 grid(sf_grid(6 * ga.n, 256).x, (unsigned)n);
+      if (m->exact) hipLaunchKernelGGL((k_batch_gather<false, float>), grid, dim3(256), 0, st, ga);
+      else hipLaunchKernelGGL((k_batch_gather<false, double>), grid, dim3(256), 0, st, ga);
       SF_LAUNCH_CHECK("k_batch_gather");
     }
   }
@@ -716,9 +722,10 @@ static void enqueue_fluid(Batch* b, hipStream_t st) {
     A.ngroups = 8 * n / b->sc;
     A.local = b->ac_local - g * A.loc_group;
     launch_acoustic_batch(st, A, b->sc, m->exact != 0);
-    hipLaunchKernelGGL(k_batch_ac_gather, dim3(rows.x, (unsigned)n), dim3(256), 0, st, na, b->ac_g0, b->ac_ptr,
-                       b->ac_idx, b->ac_local, A.loc_group, g, b->d_nstep, b->d_it, b->potd, b->potdd,
-                       m->rmass_ac + b->ac_g0, b->dt2);
+    auto* gather = m->exact ? &k_batch_ac_gather<float> : &k_batch_ac_gather<double>;
+    hipLaunchKernelGGL(gather, dim3(rows.x, (unsigned)n), dim3(256), 0, st, na, b->ac_g0, b->ac_ptr, b->ac_idx,
+                       b->ac_local, A.loc_group, g, b->d_nstep, b->d_it, b->potd, b->potdd, m->rmass_ac + b->ac_g0,
+                       b->dt2);
     SF_LAUNCH_CHECK("k_batch_ac_gather");
   }
   if (fs.n > 0)
@@ -734,8 +741,9 @@ static void enqueue_step(Batch* b, hipStream_t st, bool first) {
     // sums, corrector and predictor (at rest before the first step: nothing to do)
     if (b->loc_groups == b->S / 8) {
       const BatchGatherArgs ga = gather_args(b);
-      hipLaunchKernelGGL(k_batch_gather<true>, dim3(sf_grid(6 * ga.n, 256).x, (unsigned)(b->S / 8)), dim3(256), 0, st,
-                         ga);
+      const dim3 grid(sf_grid(6 * ga.n, 256).x, (unsigned)(b->S / 8));
+      if (m->exact) hipLaunchKernelGGL((k_batch_gather<true, float>), grid, dim3(256), 0, st, ga);
+      else hipLaunchKernelGGL((k_batch_gather<true, double>), grid, dim3(256), 0, st, ga);
       SF_LAUNCH_CHECK("k_batch_gather");
     } else {
       const int64_t nrow = 3 * (int64_t)m->nglob;

@@ -150,6 +150,12 @@ __global__ void k_zero_points(int n, const int* __restrict__ pts, realw* __restr
 // the lines of both orders and takes blocks of 20 elements (gather_slot) where those are fewer: 150
 // us, and 99 -> 104 us for the stiffness launch that writes them (621 -> 643 with attenuation, one
 // element per workgroup); blocks of 5, 10 and 40 elements: 156, 152, 149 us.
+// T: float follows the reference's operations one by one (exact builds); double keeps the sum, the
+// corrector and the predictor of a step in registers and rounds u, v (and a) once each. The pass waits
+// for memory either way (150 -> 154 us on 64x64x32 elements), and the rounding of v in every step is
+// the largest error of a run: against the same loop in 64 bits, displacement and records of 20x20x20
+// elements and 100 steps are off by 0.76 times, kernels of 24^3 by 0.79 times what they were.
+//
 // `clean`: accel is known to be zero away from AF_TERM points (the previous pass left it so), and is
 // neither read nor cleared there.
 // The number of slots comes with the flags, 2 B per point, and the position of a point's first slot
@@ -170,7 +176,7 @@ __device__ __forceinline__ int wave_prefix(int x) {
   return x;
 }
 
-template <int KIND, bool OLD>
+template <int KIND, bool OLD, typename T>
 __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
   const int nb = (int)gridDim.x, b = (int)blockIdx.x;
   const int q = nb >> 3, r = nb & 7, x = b & 7;  // contiguous blocks per XCD, last one first
@@ -184,7 +190,8 @@ __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
   int p1 = A.base[t >> 6] + p1w;
   const int p0 = p1 - cnt;
   const bool full = !A.clean || (fl & AF_TERM);
-  realw u[3], v[3], m[3], a[3] = {0.f, 0.f, 0.f};
+  T a[3] = {0, 0, 0};
+  realw u[3], v[3], m[3];
   if (KIND != GATHER_ONLY) {
     m[0] = A.rm1[g];
     m[1] = m[0];
@@ -221,40 +228,47 @@ __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
     for (int w = 0; w < 4; w++) {
       if (k[w] < 0) continue;
 #pragma unroll
-      for (int c = 0; c < 3; c++) a[c] = a[c] + (-l[w][c]);
+      for (int c = 0; c < 3; c++) a[c] = a[c] + (-(T)l[w][c]);
     }
   }
   if (KIND == GATHER_ONLY) {
     if (p1 > p0) {
 #pragma unroll
-      for (int c = 0; c < 3; c++) A.a[3 * g + c] = a[c];
+      for (int c = 0; c < 3; c++) A.a[3 * g + c] = (realw)a[c];
     }
     return;
   }
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    a[c] = a[c] * m[c];
-    v[c] = v[c] + A.dt2p * a[c];
+    a[c] = a[c] * (T)m[c];
+    T vc = (T)v[c] + (T)A.dt2p * a[c];
     if (KIND == GATHER_STEP) {
-      if (OLD) A.old[3 * g + c] = u[c] + A.t1 * v[c] + A.t2 * a[c];
-      u[c] = u[c] + A.dt * v[c] + A.dtsq2 * a[c];
-      v[c] = v[c] + A.dt2 * a[c];
-      A.u[3 * g + c] = u[c];
+      T uc = u[c];
+      if (OLD) A.old[3 * g + c] = (realw)(uc + (T)A.t1 * vc + (T)A.t2 * a[c]);
+      uc = uc + (T)A.dt * vc + (T)A.dtsq2 * a[c];
+      vc = vc + (T)A.dt2 * a[c];
+      A.u[3 * g + c] = (realw)uc;
       if (full) A.a[3 * g + c] = 0.f;
     } else {
-      A.a[3 * g + c] = a[c];
+      A.a[3 * g + c] = (realw)a[c];
     }
-    A.v[3 * g + c] = v[c];
+    A.v[3 * g + c] = (realw)vc;
   }
 }
 
-void launch_gather_update(hipStream_t s, const GatherArgs& a, int kind) {
+void launch_gather_update(hipStream_t s, const GatherArgs& a, int kind, bool exact) {
   if (a.n <= 0) return;
   const dim3 grid = sf_grid(a.n, 256), block(256);
-  if (kind == GATHER_ONLY) hipLaunchKernelGGL((k_gather_update<GATHER_ONLY, false>), grid, block, 0, s, a);
-  else if (kind == GATHER_CORRECT) hipLaunchKernelGGL((k_gather_update<GATHER_CORRECT, false>), grid, block, 0, s, a);
-  else if (a.old) hipLaunchKernelGGL((k_gather_update<GATHER_STEP, true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((k_gather_update<GATHER_STEP, false>), grid, block, 0, s, a);
+#define SF_GU(K, OLD)                                                                        \
+  do {                                                                                      \
+    if (exact) hipLaunchKernelGGL((k_gather_update<K, OLD, float>), grid, block, 0, s, a);  \
+    else hipLaunchKernelGGL((k_gather_update<K, OLD, double>), grid, block, 0, s, a);       \
+  } while (0)
+  if (kind == GATHER_ONLY) SF_GU(GATHER_ONLY, false);
+  else if (kind == GATHER_CORRECT) SF_GU(GATHER_CORRECT, false);
+  else if (a.old) SF_GU(GATHER_STEP, true);
+  else SF_GU(GATHER_STEP, false);
+#undef SF_GU
   SF_LAUNCH_CHECK("k_gather_update");
 }
 

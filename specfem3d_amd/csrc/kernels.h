@@ -75,7 +75,9 @@ struct GatherArgs {
 // what follows the sum: nothing (accel is left assembled), the corrector, or the corrector and the
 // predictor of the next step (accel left zero)
 enum { GATHER_ONLY = 0, GATHER_CORRECT = 1, GATHER_STEP = 2 };
-void launch_gather_update(hipStream_t s, const GatherArgs& a, int kind);
+// exact: the reference's single-precision operations; else sums, corrector and predictor in double
+// precision, rounded once per stored value
+void launch_gather_update(hipStream_t s, const GatherArgs& a, int kind, bool exact);
 // slot lists (k_assembly.hip): the elements of `order` give the order of the sums, those of `launch`
 // (nelem_launch of them) the slots, `pos0` launch positions on for the elements behind; allocates ptr
 // (nglob + 1) and idx (125 nelem). lines: cache lines that the waves of a pass over all points touch
