@@ -474,7 +474,6 @@ extern "C" void FC_FUNC_(prepare_constants_device, PREPARE_CONSTANTS_DEVICE)(
 namespace sf {
 void ensure_gather_assembly(Mesh* m, int f);
 void ensure_element_colors(Mesh* m);
-static void prepare_acoustic_gather(Mesh* m);
 
 // Distinct (factor_common, factor_common_kappa) rows, compared bit for bit, and a 16-bit row index
 // per local point; gives up (planes only) beyond 65535 distinct rows.
@@ -588,9 +587,8 @@ extern "C" void FC_FUNC_(prepare_fields_elastic_device, PREPARE_FIELDS_ELASTIC_D
   const int64_t n = m->nglob;
   const int64_t nloc = (int64_t)m->nspec * 125;
   if (m->assembly < 0) {
-    // automatic assembly (see Mesh::assembly); the acoustic fields were prepared before it was known
+    // automatic assembly (see Mesh::assembly)
     m->assembly = *ATTENUATION ? 0 : 1;
-    if (m->assembly == 1) prepare_acoustic_gather(m);
   }
   {
     std::vector<realw> rm(3 * (size_t)n);
@@ -770,7 +768,7 @@ void ensure_gather_assembly(Mesh* m, int f) {
   m->asm_pos0 = first_pml;
   m->asm_eb = build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_elastic + m->pml_n, lst,
                                m->elastic_launch ? m->elastic_launch : m->elastic_elems, m->nspec_elastic, first_pml,
-                               eb, m->ibool, ptr, m->asm_idx);
+                               3, eb, m->ibool, ptr, m->asm_idx);
   dfree(lst);
   if (!m->asm_info) {
     m->asm_info = dmalloc<uint16_t>(m->nglob);
@@ -797,14 +795,36 @@ void release_gather_assembly(Mesh* m) {
   dfree(m->asm_buf[0]);
   dfree(m->asm_buf[1]);
   m->asm_ready = 0;
+  dfree(m->asm_ac_idx);
+  dfree(m->asm_ac_info);
+  dfree(m->asm_ac_base);
+  dfree(m->asm_ac_buf[0]);
+  dfree(m->asm_ac_buf[1]);
+  m->asm_ac_ready = 0;
 }
 
-// the same for the fluid (ordered sums of the acoustic stiffness)
-static void prepare_acoustic_gather(Mesh* m) {
-  if (m->asm_ac_buf || m->nspec_acoustic <= 0 || !m->acoustic_elems) return;
-  (void)build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_acoustic, m->acoustic_elems, nullptr, 0, 0, 1,
-                         m->ibool, m->asm_ac_ptr, m->asm_ac_idx);
-  m->asm_ac_buf = dmalloc<realw>((int64_t)m->nspec * 125);
+// the same for the fluid; the points of its free surface are marked AF_EDGE
+void ensure_gather_acoustic(Mesh* m, int f) {
+  const int eb = 20;
+  if (!m->asm_ac_buf[f]) m->asm_ac_buf[f] = dmalloc<realw>(125 * ((int64_t)m->nspec_acoustic + eb));
+  if (m->asm_ac_ready) return;
+  flush_all(m);
+  if (m->assembly == 2) ensure_acoustic_colors(m);
+  const int* order = m->assembly == 2 && m->ac_color_elems ? m->ac_color_elems : m->acoustic_elems;
+  dfree(m->asm_ac_idx);
+  int* ptr = nullptr;
+  m->asm_ac_eb = build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_acoustic, order, m->acoustic_elems,
+                                  m->nspec_acoustic, 0, 1, eb, m->ibool, ptr, m->asm_ac_idx);
+  if (!m->asm_ac_info) {
+    m->asm_ac_info = dmalloc<uint16_t>(m->nglob);
+    m->asm_ac_base = dmalloc<int>((m->ac_n + 63) / 64);
+  }
+  launch_gather_info(m->stream, m->ac_g0, m->ac_n, ptr, nullptr, m->asm_ac_info, m->asm_ac_base, nullptr);
+  for (const FacePoints* fp : {&m->abs_ac, &m->coupling, &m->src_ac_pts, &m->adj_ac_pts})
+    launch_mark_points(m->stream, fp->n, fp->iglob, AF_TERM, m->asm_ac_info);
+  launch_mark_points(m->stream, m->free_ac.n, m->free_ac.iglob, AF_EDGE, m->asm_ac_info);
+  dfree(ptr);
+  m->asm_ac_ready = 1;
 }
 
 }  // namespace sf
@@ -854,8 +874,6 @@ extern "C" void FC_FUNC_(prepare_fields_acoustic_device, PREPARE_FIELDS_ACOUSTIC
       }
     m->ac_g0 = gmax < 0 ? 0 : (gmin / 4) * 4;
     m->ac_n = gmax < 0 ? 0 : (int64_t)gmax + 1 - m->ac_g0;
-    if (m->assembly == 1) prepare_acoustic_gather(m);
-    if (m->assembly == 2) build_colors(m, lst, m->ac_color_elems, m->ac_color_off, m->ac_ncolor);
   }
   m->ac[0].pot = dmalloc<realw>(n);
   m->ac[0].potd = dmalloc<realw>(n);
@@ -1191,7 +1209,7 @@ extern "C" void FC_FUNC_(prepare_sim2_or_3_const_device, PREPARE_SIM2_OR_3_CONST
     build_point_sets(own_ac, H->ibool, m->adj_ac_pts);
     remap_owner(m->adj_ac_pts, idx_ac);
   }
-  m->asm_ready = 0;  // the adjoint source points take terms
+  m->asm_ready = m->asm_ac_ready = 0;  // the adjoint source points take terms
   m->adj_h = dupload(h.data(), (int64_t)h.size());
   m->adj_src = dmalloc<realw>(3 * (int64_t)m->nadj_rec_local);
 }
@@ -1228,7 +1246,7 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
   dfree(m->pml_elems); dfree(m->pml_cpml);
   dfree(m->pml_state); dfree(m->pml_coef); dfree(m->pml_masks); dfree(m->pml_off);
   dfree(m->pml_old); dfree(m->pml_pts); dfree(m->pml_bc_pts);
-  dfree(m->asm_ac_ptr); dfree(m->asm_ac_idx); dfree(m->asm_ac_buf);
+  dfree(m->asm_ac_idx); dfree(m->asm_ac_info); dfree(m->asm_ac_base); dfree(m->asm_ac_buf[0]); dfree(m->asm_ac_buf[1]);
   dfree(m->d_norm);
   if (m->h_norm) (void)hipHostFree(m->h_norm);
   if (m->timing_ev) {
@@ -1248,23 +1266,14 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
 // exact = 1: element kernels without fused multiply-add (the CPU reference's rounding);
 // assembly: the order in which a global point's element contributions are summed. 1 = element order
 // (the reference's serial order), 2 = the colour order of a greedy element colouring, 0 = any order
-// (the solid takes element order; the fluid and its face terms use float atomics). All of them
-// store the solid's local forces and sum them in the next update (k_gather_update).
+// (element order; the face terms of the fluid and the coupling use float atomics). All of them store
+// the local forces and sum them in the next update (k_gather_update).
 extern "C" void sf_set_options(long* Mesh_pointer, int exact, int assembly) {
   Mesh* m = from_handle(Mesh_pointer);
   SF_CHECK(hipStreamSynchronize(m->stream));
   m->exact = exact ? 1 : 0;
   m->assembly = assembly;
-  m->asm_ready = 0;  // rebuilt in the new order by the next stiffness call
-  if (assembly == 1) prepare_acoustic_gather(m);
-  if (assembly == 2) {
-    if (!m->el_color_elems) ensure_element_colors(m);
-    if (!m->ac_color_elems && m->nspec_acoustic > 0 && m->acoustic_elems) {
-      std::vector<int> lst(m->nspec_acoustic);
-      SF_CHECK(hipMemcpy(lst.data(), m->acoustic_elems, sizeof(int) * lst.size(), hipMemcpyDeviceToHost));
-      build_colors(m, lst, m->ac_color_elems, m->ac_color_off, m->ac_ncolor);
-    }
-  }
+  m->asm_ready = m->asm_ac_ready = 0;  // rebuilt in the new order by the next stiffness call
 }
 
 // Tuning switches read by the step calls: "att_variant" (0..4: attenuation-state scheduling of the

@@ -19,6 +19,7 @@ namespace sf {
 realw* stage_to_device(Mesh* m, const realw* vals, int n, realw* dst);
 realw* stf_device_buffer(Mesh* m, int n);
 void ensure_gather_assembly(Mesh* m, int f);
+void ensure_gather_acoustic(Mesh* m, int f);
 const std::vector<int>& host_ibool(Mesh* m);
 
 static inline int field_of(int foa) { return foa == 3 ? 1 : 0; }
@@ -55,7 +56,7 @@ static GatherArgs gather_args(Mesh* m, int f) {
 // sum the waiting local forces and run the pending corrector
 static void flush_el(Mesh* m, int f) {
   if (m->pending_gather_el[f]) {
-    launch_gather_update(m->stream, gather_args(m, f), m->pending_k3_el[f] ? GATHER_CORRECT : GATHER_ONLY,
+    launch_gather_update(m->stream, gather_args(m, f), 3, m->pending_k3_el[f] ? GATHER_CORRECT : GATHER_ONLY,
                          m->exact != 0);
     m->pending_gather_el[f] = 0;
     m->gather_skip_el[f] = 0;
@@ -68,13 +69,49 @@ static void flush_el(Mesh* m, int f) {
   }
   m->pending_k3_el[f] = 0;
 }
+
+static GatherArgs gather_args_ac(Mesh* m, int f) {
+  GatherArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.g0 = m->ac_g0;
+  a.n = m->ac_n;
+  a.info = m->asm_ac_info;
+  a.base = m->asm_ac_base;
+  a.idx = m->asm_ac_idx;
+  a.local = m->asm_ac_buf[f];
+  a.skip = m->gather_skip_ac[f];
+  a.clean = m->potdd_clean[f];
+  a.u = m->ac[f].pot;
+  a.v = m->ac[f].potd;
+  a.a = m->ac[f].potdd;
+  a.rm1 = m->rmass_ac;
+  a.dt2p = m->pending_dt2_ac[f];
+  return a;
+}
+
 static void flush_ac(Mesh* m, int f) {
-  if (m->pending_k3_ac[f]) {
+  int& fz = m->free_zero[f];
+  if (m->pending_gather_ac[f]) {
+    launch_gather_update(m->stream, gather_args_ac(m, f), 1, m->pending_k3_ac[f] ? GATHER_CORRECT : GATHER_ONLY,
+                         m->exact != 0);
+    if (m->gather_skip_ac[f]) fz |= FREE_DD;
+    else fz = m->pending_k3_ac[f] ? 0 : fz & FREE_POT;
+    m->pending_gather_ac[f] = 0;
+    m->gather_skip_ac[f] = 0;
+    m->potdd_clean[f] = 0;
+  } else if (m->pending_k3_ac[f]) {
     const int64_t g0 = m->ac_g0;
     launch_corrector(m->stream, m->ac_n, m->ac[f].potd + g0, m->ac[f].potdd + g0, m->rmass_ac + g0,
                      m->pending_dt2_ac[f]);
-    m->pending_k3_ac[f] = 0;
+    if (!(fz & FREE_DD)) fz = 0;
+    m->potdd_clean[f] = 0;
   }
+  m->pending_k3_ac[f] = 0;
+}
+// before boundary, coupling or source terms are added to chi''
+static void flush_ac_terms(Mesh* m, int f) {
+  flush_ac(m, f);
+  m->free_zero[f] &= FREE_POT;
 }
 void flush_all(Mesh* m) {
   for (int f = 0; f < 2; f++) {
@@ -201,7 +238,7 @@ extern "C" void FC_FUNC_(update_displacement_cuda, UPDATE_DISPLACMENT_CUDA)(long
     a.old = pml ? m->pml_old : nullptr;
     a.t1 = m->pml_t1;
     a.t2 = m->pml_t2;
-    launch_gather_update(m->stream, a, GATHER_STEP, m->exact != 0);
+    launch_gather_update(m->stream, a, 3, GATHER_STEP, m->exact != 0);
   } else if (m->pending_k3_el[f]) {
     launch_corrector_predictor(m->stream, n, w.displ + o, w.veloc + o, w.accel + o, m->rmass + o,
                                m->pending_dt2_el[f], *deltat_F, *deltatover2_F, *deltatsqover2_F,
@@ -226,14 +263,27 @@ extern "C" void FC_FUNC_(update_displacement_ac_cuda, UPDATE_DISPLACEMENT_AC_CUD
   AcField& a = m->ac[f];
   if (!a.pot) fatal("update_displacement_ac_cuda", "acoustic field not prepared");
   const int64_t g0 = m->ac_g0;  // only the acoustic range changes (see Mesh::ac_g0)
-  if (m->pending_k3_ac[f]) {
+  if (!m->pending_k3_ac[f]) flush_ac(m, f);
+  bool dd = m->free_zero[f] & FREE_DD;  // chi'' enters the update as zero on the free surface
+  if (m->pending_gather_ac[f]) {
+    GatherArgs ga = gather_args_ac(m, f);
+    ga.dt = *deltat_F;
+    ga.dt2 = *deltatover2_F;
+    ga.dtsq2 = *deltatsqover2_F;
+    launch_gather_update(m->stream, ga, 1, GATHER_STEP, m->exact != 0);
+    dd = m->gather_skip_ac[f] != 0;
+  } else if (m->pending_k3_ac[f]) {
     launch_corrector_predictor(m->stream, m->ac_n, a.pot + g0, a.potd + g0, a.potdd + g0, m->rmass_ac + g0,
                                m->pending_dt2_ac[f], *deltat_F, *deltatover2_F, *deltatsqover2_F);
-    m->pending_k3_ac[f] = 0;
   } else {
     launch_predictor(m->stream, m->ac_n, a.pot + g0, a.potd + g0, a.potdd + g0, *deltat_F, *deltatover2_F,
                      *deltatsqover2_F);
   }
+  m->free_zero[f] = FREE_DD | (dd ? m->free_zero[f] & FREE_POT : 0);
+  m->pending_gather_ac[f] = 0;
+  m->gather_skip_ac[f] = 0;
+  m->pending_k3_ac[f] = 0;
+  m->potdd_clean[f] = 1;
 }
 
 extern "C" void FC_FUNC_(kernel_3_a_cuda, KERNEL_3_A_CUDA)(long* Mesh_pointer, realw* deltatover2_F,
@@ -267,7 +317,7 @@ extern "C" void FC_FUNC_(kernel_3_acoustic_cuda, KERNEL_3_ACOUSTIC_CUDA)(long* M
     if (foa == 1 && f == 1) continue;
     if (foa == 3 && f == 0) continue;
     if (!m->ac[f].pot) continue;
-    flush_ac(m, f);
+    if (m->pending_k3_ac[f]) flush_ac(m, f);
     m->pending_k3_ac[f] = 1;
     m->pending_dt2_ac[f] = f ? *b_deltatover2_F : *deltatover2_F;
   }
@@ -311,7 +361,9 @@ extern "C" void FC_FUNC_(compute_forces_acoustic_cuda, COMPUTE_FORCES_ACOUSTIC_C
     if (foa == 1 && f == 1) continue;
     if (foa == 3 && f == 0) continue;
     if (!m->ac[f].pot) continue;
+    if (m->nspec_acoustic <= 0) continue;
     flush_ac(m, f);
+    ensure_gather_acoustic(m, f);
     AcousticArgs a;
     a.nelem = m->nspec_acoustic;
     a.elems = m->acoustic_elems;
@@ -323,26 +375,17 @@ extern "C" void FC_FUNC_(compute_forces_acoustic_cuda, COMPUTE_FORCES_ACOUSTIC_C
     a.jac_plane = (int64_t)m->nspec_irregular * 125;
     a.rho = m->rho;
     a.pot = m->ac[f].pot;
-    a.potdd = m->ac[f].potdd;
-    a.local_out = m->asm_ac_buf;
-    const bool ordered = m->assembly == 1 && m->asm_ac_buf;
-    if (m->assembly == 2 && m->ac_color_elems) {
-      for (int c = 0; c < m->ac_ncolor; c++) {
-        a.elems = m->ac_color_elems + m->ac_color_off[c];
-        a.nelem = m->ac_color_off[c + 1] - m->ac_color_off[c];
-        launch_acoustic(m->stream, a, m->exact != 0, 2);
-      }
-    } else {
-      launch_acoustic(m->stream, a, m->exact != 0, ordered ? 1 : 0);
-    }
-    if (ordered)
-      launch_ordered_gather(m->stream, m->nglob, 1, m->asm_ac_ptr, m->asm_ac_idx, m->asm_ac_buf,
-                            (int64_t)m->nspec * 125, m->ac[f].potdd);
+    a.local_out = m->asm_ac_buf[f];
+    a.eb = m->asm_ac_eb;
+    launch_acoustic(m->stream, a, m->exact != 0);
+    m->pending_gather_ac[f] = 1;
   }
 }
 
 // compute_forces_acoustic_cuda.cu:334 -- zero chi, chi', chi'' on the fluid free surface. It
-// commutes with a deferred acoustic corrector (zeroed points stay zero through it).
+// commutes with a deferred acoustic corrector (zeroed points stay zero through it), a waiting sum leaves
+// these points out, and where the three are zero already (Mesh::free_zero: the call before the forces
+// of a step follows an update that kept the zeros of the call after the last) nothing is launched.
 extern "C" void FC_FUNC_(acoustic_enforce_free_surf_cuda, ACOUSTIC_ENFORCE_FREE_SURF_CUDA)(
     long* Mesh_pointer, int* ABSORB_INSTEAD_OF_FREE_SURFACE, int* FORWARD_OR_ADJOINT) {
   Mesh* m = from_handle(Mesh_pointer);
@@ -352,7 +395,11 @@ extern "C" void FC_FUNC_(acoustic_enforce_free_surf_cuda, ACOUSTIC_ENFORCE_FREE_
     if (foa == 1 && f == 1) continue;
     if (foa == 3 && f == 0) continue;
     if (!m->ac[f].pot) continue;
-    launch_free_surface(m->stream, m->free_ac, m->ac[f].pot, m->ac[f].potd, m->ac[f].potdd);
+    const int known = m->pending_gather_ac[f] ? FREE_POT : FREE_POT | FREE_DD;
+    if ((m->free_zero[f] & known) != known)
+      launch_free_surface(m->stream, m->free_ac, m->ac[f].pot, m->ac[f].potd, m->ac[f].potdd);
+    if (m->pending_gather_ac[f]) m->gather_skip_ac[f] |= AF_EDGE;
+    m->free_zero[f] |= known;
   }
 }
 
@@ -488,7 +535,7 @@ extern "C" void FC_FUNC_(compute_stacey_acoustic_cuda, COMPUTE_STACEY_ACOUSTIC_C
   const int foa = *FORWARD_OR_ADJOINT_f;
   const int64_t rec_len = 25 * (int64_t)m->num_abs_boundary_faces;
   if (foa == 0 || foa == 1) {
-    flush_ac(m, 0);
+    flush_ac_terms(m, 0);
     const bool store = m->simulation_type == 1 && m->save_forward && h_b_absorb_potential;
     launch_stacey_acoustic(m->stream, m->abs_ac, m->ac[0].potd, m->ac[0].potdd, m->b_absorb_potential, store ? 1 : 0,
                            face_atomics(m));
@@ -499,7 +546,7 @@ extern "C" void FC_FUNC_(compute_stacey_acoustic_cuda, COMPUTE_STACEY_ACOUSTIC_C
     }
   }
   if ((foa == 0 || foa == 3) && m->simulation_type == 3 && m->ac[1].pot) {
-    flush_ac(m, 1);
+    flush_ac_terms(m, 1);
     SF_CHECK(hipMemcpyAsync(m->b_absorb_potential, h_b_absorb_potential, sizeof(realw) * rec_len,
                             hipMemcpyHostToDevice, m->stream));
     launch_stacey_acoustic_replay(m->stream, m->abs_ac, m->b_absorb_potential, m->ac[1].potdd);
@@ -516,7 +563,7 @@ extern "C" void FC_FUNC_(compute_stacey_acoustic_undoatt_cuda, COMPUTE_STACEY_AC
     if (foa == 1 && f == 1) continue;
     if (foa == 3 && f == 0) continue;
     if (!m->ac[f].pot) continue;
-    flush_ac(m, f);
+    flush_ac_terms(m, f);
     launch_stacey_acoustic(m->stream, m->abs_ac, m->ac[f].potd, m->ac[f].potdd, nullptr, 0, face_atomics(m));
   }
 }
@@ -532,7 +579,7 @@ extern "C" void FC_FUNC_(compute_coupling_ac_el_cuda, COMPUTE_COUPLING_AC_EL_CUD
     if (foa == 1 && f == 1) continue;
     if (foa == 3 && f == 0) continue;
     if (!m->ac[f].pot || !m->el[f].displ) continue;
-    flush_ac(m, f);
+    flush_ac_terms(m, f);
     const int flip = (m->simulation_type != 1 && f == 0) ? 1 : 0;
     launch_coupling_ac_el(m->stream, m->coupling, m->el[f].displ, m->ac[f].potdd, flip, face_atomics(m));
   }
@@ -615,7 +662,7 @@ static void add_sources_ac(Mesh* m, int f, const double* h_stf, int nsrc, const 
   if (nsrc < m->nsources) fatal(where, "NSOURCES smaller than the number of prepared sources");
   std::vector<realw> s(m->nsources);
   for (int i = 0; i < m->nsources; i++) s[i] = (realw)h_stf[i];
-  flush_ac(m, f);
+  flush_ac_terms(m, f);
   realw* d = stf_device_buffer(m, m->nsources);
   stage_to_device(m, s.data(), m->nsources, d);
   launch_add_sources_ac(m->stream, m->src_ac_pts, m->src_array, m->src_kappa, d, m->ac[f].potdd);
@@ -653,7 +700,7 @@ extern "C" void FC_FUNC_(add_sources_ac_sim_2_or_3_cuda, ADD_SOURCES_AC_SIM_2_OR
   const int nt = *NTSTEP_BETWEEN_READ_ADJSRC;
   const int isample = nt - ((*it - 1) % nt);  // 1-based
   const realw* src = h_source_adjoint + (int64_t)3 * nadj * (isample - 1);
-  flush_ac(m, 0);
+  flush_ac_terms(m, 0);
   stage_to_device(m, src, 3 * nadj, m->adj_src);
   launch_adjoint_sources_ac(m->stream, m->adj_ac_pts, m->adj_h, m->adj_src, m->ac[0].potdd);
 }
@@ -839,6 +886,7 @@ SF_XFER1(transfer_b_accel_from_device, 1, accel, D2H)
     DIR(m, m->ac[F].pot, p, *size);                                                                            \
     DIR(m, m->ac[F].potd, pd, *size);                                                                          \
     DIR(m, m->ac[F].potdd, pdd, *size);                                                                        \
+    m->potdd_clean[F] = m->free_zero[F] = 0;                                                                   \
   }
 #define SF_XFERAC1(NAME, F, MEMBER, DIR)                                          \
   extern "C" void FC_FUNC_(NAME, X)(int* size, realw* arr, long* Mesh_pointer) { \
@@ -846,6 +894,7 @@ SF_XFER1(transfer_b_accel_from_device, 1, accel, D2H)
     if (!m->ac[F].pot) fatal(#NAME, "acoustic field not prepared");               \
     flush_ac(m, F);                                                               \
     DIR(m, m->ac[F].MEMBER, arr, *size);                                          \
+    m->potdd_clean[F] = m->free_zero[F] = 0;                                      \
   }
 SF_XFERAC3(transfer_fields_ac_to_device, 0, H2D)
 SF_XFERAC3(transfer_fields_ac_from_device, 0, D2H)

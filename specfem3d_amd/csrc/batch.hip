@@ -555,11 +555,11 @@ static void build_gather(Batch* b) {
   Mesh* m = b->m;
   if (!b->asm_ptr)
     (void)build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_elastic, m->el_color_elems, m->elastic_elems,
-                           m->nspec_elastic, 0, 1, m->ibool, b->asm_ptr, b->asm_idx);
+                           m->nspec_elastic, 0, 3, 1, m->ibool, b->asm_ptr, b->asm_idx);
   if (!b->local) b->local = local_room((int64_t)m->nspec_elastic * 3000, std::min(b->S / 8, b->max_groups), &b->loc_groups);
   if (b->ac && !b->ac_ptr)
     (void)build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_acoustic, m->ac_color_elems, m->acoustic_elems,
-                           m->nspec_acoustic, 0, 1, m->ibool, b->ac_ptr, b->ac_idx);
+                           m->nspec_acoustic, 0, 1, 1, m->ibool, b->ac_ptr, b->ac_idx);
   if (b->ac && !b->ac_local)
     b->ac_local = local_room((int64_t)m->nspec_acoustic * 1000, std::min(b->S / 8, b->max_groups), &b->ac_loc_groups);
   if (!b->info) b->info = balloc<uint16_t>(m->nglob);

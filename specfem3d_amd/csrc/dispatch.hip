@@ -23,8 +23,8 @@ void launch_elastic_batch_exact(hipStream_t, const BatchArgs&, int);
 void launch_elastic_batch_fast(hipStream_t, const BatchArgs&, int);
 void launch_elastic_pml_exact(hipStream_t, const PmlArgs&);
 void launch_elastic_pml_fast(hipStream_t, const PmlArgs&);
-void launch_acoustic_exact(hipStream_t, const AcousticArgs&, int);
-void launch_acoustic_fast(hipStream_t, const AcousticArgs&, int);
+void launch_acoustic_exact(hipStream_t, const AcousticArgs&);
+void launch_acoustic_fast(hipStream_t, const AcousticArgs&);
 
 void launch_elastic(hipStream_t s, const ElasticArgs& a, bool strain, bool att, bool exact, int att_variant) {
   if (exact)
@@ -73,11 +73,11 @@ void launch_acoustic_batch(hipStream_t s, const BatchAcArgs& a, int sc, bool exa
     launch_acoustic_batch_fast(s, a, sc);
 }
 
-void launch_acoustic(hipStream_t s, const AcousticArgs& a, bool exact, int mode) {
+void launch_acoustic(hipStream_t s, const AcousticArgs& a, bool exact) {
   if (exact)
-    launch_acoustic_exact(s, a, mode);
+    launch_acoustic_exact(s, a);
   else
-    launch_acoustic_fast(s, a, mode);
+    launch_acoustic_fast(s, a);
 }
 
 static std::string g_last_error;

@@ -1,10 +1,9 @@
 // k_acoustic.hip -- acoustic (fluid potential) element stiffness for NGLL=5.
 //
-// Restates compute_forces_acoustic.F90:35-726: chi'' -= div((1/rho) grad chi) in weak form.
-// Same tiling as the elastic kernel (5 elements per 128-lane workgroup, one GLL column per
-// lane, gamma contractions in registers, xi/eta through LDS). Compiled twice like
+// Restates compute_forces_acoustic.F90:35-726: chi'' -= div((1/rho) grad chi) in weak form. The lane
+// layout is that of k_elastic_line (k_elastic.hip), for one component. Compiled twice like
 // k_elastic.hip (SF_EXACT = 1: no fused multiply-add, the reference's rounding).
-#include "kernels.h"
+#include "elastic_point.h"
 
 #ifndef SF_EXACT
 #define SF_EXACT 1
@@ -20,115 +19,137 @@
 namespace sf {
 namespace SF_VNS {
 
-template <int MODE>
+// The local forces are stored, one float per slot (gather_slot), and summed per global point by the
+// update that follows (k_gather_update<1>). A 128-lane workgroup takes five elements, a lane one line
+// of five points at a time: lane (el, c) holds the gamma column of c = i + 5 j in registers and the xi
+// row 5 c .. 5 c + 4 and the eta row (c % 5) + 25 (c / 5) + 5 l in LDS, the coefficients in scalar
+// registers. Plane A holds chi, then the xi derivatives, the xi products and their divergence, plane
+// B the same for eta.
+// Bound by HBM: 28 B per local point with the index and the density, 96 MB on 40x40x30 elements, 22 us
+// (4.3 TB/s, near the rate of a large copy) where a lane per column with float atomics took 82 us;
+// on 64x64x4 36 -> 12 us, on 19x17x4, in eight colour launches before, 53 -> 5. The sum, fused with the
+// corrector, takes 18.6 us on 40x40x30 (20.9 with one element's slots after the other's); a corrector
+// alone took 10.
 __global__ void __launch_bounds__(128) k_acoustic(AcousticArgs A, GLLk G) {
-  __shared__ realw s_buf[5][2][128];
-  const int tid = threadIdx.x;
-  const int el = tid / 25;
-  const int c = tid - el * 25;
+  constexpr int PL = 626;
+  __shared__ realw sA[PL], sB[PL];
+  __shared__ realw sW[25];
+  const int t = threadIdx.x;
+  const bool lane = t < 125;                       // lanes 125..127 shadow the last element's first points
+  const int el = lane ? t / 25 : 4, c = lane ? t - 25 * el : t - 125;
   const int i = c % 5, j = c / 5;
-  const int ie = blockIdx.x * 5 + el;
-  const bool active = (tid < 125) && (ie < A.nelem);
-  const int e = active ? A.elems[ie] : 0;
-  const int elx = el < 5 ? el : 4;
-
-  int g[5];
-  realw chi[5];
-  if (active) {
+  // blocks b, b + 8, ... (one XCD) take one contiguous range of elements
+  const int nb = gridDim.x, q = nb >> 3, r8 = nb & 7, xc = blockIdx.x & 7;
+  const int ie = (xc * q + (xc < r8 ? xc : r8) + (int)(blockIdx.x >> 3)) * 5 + el;
+  const bool active = lane && ie < A.nelem;
+  const int e = A.elems[ie < A.nelem ? ie : A.nelem - 1];
+  const int64_t ep = (int64_t)e * 125 + c;         // local point of k = 0
+  const int irr = A.irregular[e];
+  const int64_t jp = (int64_t)(irr ? irr - 1 : 0) * 125 + c;
+  if (t < 25) sW[t] = G.wxy[t];
+  realw rho[5], d3[5];
+  {
+    int g[5];
+    realw chi[5];
 #pragma unroll
-    for (int k = 0; k < 5; k++) {
-      g[k] = A.ibool[(int64_t)e * 125 + c + 25 * k];
-      chi[k] = A.pot[g[k]];
-      s_buf[el][0][c + 25 * k] = chi[k];
+    for (int k = 0; k < 5; k++) g[k] = A.ibool[ep + 25 * k];
+#pragma unroll
+    for (int k = 0; k < 5; k++) chi[k] = A.pot[g[k]];
+#pragma unroll
+    for (int k = 0; k < 5; k++) rho[k] = A.rho[ep + 25 * k];
+    if (lane) {
+#pragma unroll
+      for (int k = 0; k < 5; k++) sA[el * 125 + c + 25 * k] = chi[k];
+    }
+    line_gradient(G.hp, chi, d3);
+  }
+  lds_barrier();
+  const int bx = el * 125 + 5 * c, by = el * 125 + i + 25 * j;  // first points of the lane's two rows
+  realw x[5];
+  {
+    realw r[5], y[5];
+#pragma unroll
+    for (int l = 0; l < 5; l++) {
+      r[l] = sA[bx + l];
+      y[l] = sA[by + 5 * l];
+    }
+    line_gradient(G.hp, r, x);
+    line_gradient(G.hp, y, r);
+    if (lane) {
+#pragma unroll
+      for (int l = 0; l < 5; l++) sB[by + 5 * l] = r[l];
     }
   }
-  __syncthreads();
-  const int irr = active ? A.irregular[e] : 0;
-  realw t1[5], t2[5], t3[5];
+  lds_barrier();                                   // every row of chi has been read
+  if (lane) {
+#pragma unroll
+    for (int l = 0; l < 5; l++) sA[bx + l] = x[l];
+  }
+  lds_barrier();
 #pragma unroll
   for (int k = 0; k < 5; k++) {
-    if (!active) continue;
-    const int p = c + 25 * k;
-    const realw* s = s_buf[elx][0];
-    const int b1 = 5 * j + 25 * k, b2 = i + 25 * k;
-    realw a1 = G.hp[i * 5] * s[b1];
-    realw a2 = G.hp[j * 5] * s[b2];
-    realw a3 = G.hp[k * 5] * chi[0];
-#pragma unroll
-    for (int l = 1; l < 5; l++) {
-      a1 = a1 + G.hp[i * 5 + l] * s[b1 + l];
-      a2 = a2 + G.hp[j * 5 + l] * s[b2 + 5 * l];
-      a3 = a3 + G.hp[k * 5 + l] * chi[l];
-    }
-    const int64_t ep = (int64_t)e * 125 + p;
-    const realw rho_invl = (realw)1 / A.rho[ep];
+    const int b = el * 125 + c + 25 * k;
+    const realw a1 = sA[b], a2 = sB[b], a3 = d3[k];
+    const realw rho_invl = (realw)1 / rho[k];
+    realw t1, t2;
     if (irr) {
-      const int64_t q = (int64_t)(irr - 1) * 125 + p;
-      const int64_t P = A.jac_plane;
-      const realw* J = A.jac;
-      const realw xixl = J[q], xiyl = J[P + q], xizl = J[2 * P + q], etaxl = J[3 * P + q], etayl = J[4 * P + q];
-      const realw etazl = J[5 * P + q], gaxl = J[6 * P + q], gayl = J[7 * P + q], gazl = J[8 * P + q];
-      const realw jl = J[9 * P + q];
-      const realw dpdx = xixl * a1 + etaxl * a2 + gaxl * a3;
-      const realw dpdy = xiyl * a1 + etayl * a2 + gayl * a3;
-      const realw dpdz = xizl * a1 + etazl * a2 + gazl * a3;
-      t1[k] = rho_invl * jl * (xixl * dpdx + xiyl * dpdy + xizl * dpdz);
-      t2[k] = rho_invl * jl * (etaxl * dpdx + etayl * dpdy + etazl * dpdz);
-      t3[k] = rho_invl * jl * (gaxl * dpdx + gayl * dpdy + gazl * dpdz);
+      const JacPt J = load_jac(A.jac, A.jac_plane, jp + 25 * k);
+      const realw dpdx = J.xix * a1 + J.etax * a2 + J.gax * a3;
+      const realw dpdy = J.xiy * a1 + J.etay * a2 + J.gay * a3;
+      const realw dpdz = J.xiz * a1 + J.etaz * a2 + J.gaz * a3;
+      t1 = rho_invl * J.jac * (J.xix * dpdx + J.xiy * dpdy + J.xiz * dpdz);
+      t2 = rho_invl * J.jac * (J.etax * dpdx + J.etay * dpdy + J.etaz * dpdz);
+      d3[k] = rho_invl * J.jac * (J.gax * dpdx + J.gay * dpdy + J.gaz * dpdz);
     } else {
       const realw jl = A.jacobian_regular, xr = A.xix_regular;
-      t1[k] = rho_invl * jl * xr * xr * a1;
-      t2[k] = rho_invl * jl * xr * xr * a2;
-      t3[k] = rho_invl * jl * xr * xr * a3;
+      t1 = rho_invl * jl * xr * xr * a1;
+      t2 = rho_invl * jl * xr * xr * a2;
+      d3[k] = rho_invl * jl * xr * xr * a3;
+    }
+    if (lane) {
+      sA[b] = t1;
+      sB[b] = t2;
     }
   }
-  __syncthreads();
-  if (active) {
+  lds_barrier();
+  {
+    realw r[5], y[5], o[5];
 #pragma unroll
-    for (int k = 0; k < 5; k++) {
-      s_buf[el][0][c + 25 * k] = t1[k];
-      s_buf[el][1][c + 25 * k] = t2[k];
+    for (int l = 0; l < 5; l++) {
+      r[l] = sA[bx + l];
+      y[l] = sB[by + 5 * l];
     }
+    line_divergence(G.hpw, r, o);
+    if (lane) {
+#pragma unroll
+      for (int l = 0; l < 5; l++) sA[bx + l] = o[l];
+    }
+    line_divergence(G.hpw, y, o);
+    if (lane) {
+#pragma unroll
+      for (int l = 0; l < 5; l++) sB[by + 5 * l] = o[l];
+    }
+    line_divergence(G.hpw, d3, o);
+#pragma unroll
+    for (int k = 0; k < 5; k++) d3[k] = o[k];
   }
-  __syncthreads();
+  lds_barrier();
   if (!active) return;
+  const realw w3 = sW[i * 5 + j];
+  const int slot = gather_slot(ie, j, i, A.eb);    // of k = 0
 #pragma unroll
   for (int k = 0; k < 5; k++) {
-    const int b1 = 5 * j + 25 * k, b2 = i + 25 * k;
-    const realw* s1 = s_buf[el][0];
-    const realw* s2 = s_buf[el][1];
-    realw n1 = G.hpw[0 * 5 + i] * s1[b1];
-    realw n2 = G.hpw[0 * 5 + j] * s2[b2];
-    realw n3 = G.hpw[0 * 5 + k] * t3[0];
-#pragma unroll
-    for (int l = 1; l < 5; l++) {
-      n1 = n1 + G.hpw[l * 5 + i] * s1[b1 + l];
-      n2 = n2 + G.hpw[l * 5 + j] * s2[b2 + 5 * l];
-      n3 = n3 + G.hpw[l * 5 + k] * t3[l];
-    }
-    const realw f = G.wxy[j * 5 + k] * n1 + G.wxy[i * 5 + k] * n2 + G.wxy[i * 5 + j] * n3;
-    if (MODE == 1) {
-      A.local_out[(int64_t)ie * 125 + c + 25 * k] = f;
-    } else if (MODE == 2) {
-      A.potdd[g[k]] = A.potdd[g[k]] + (-f);
-    } else {
-      atomicAdd(A.potdd + g[k], -f);
-    }
+    const int b = el * 125 + c + 25 * k;
+    A.local_out[slot + k * 25 * A.eb] = sW[j * 5 + k] * sA[b] + sW[i * 5 + k] * sB[b] + w3 * d3[k];
   }
 }
 
 }  // namespace SF_VNS
 using namespace SF_VNS;
 
-void SFX(launch_acoustic)(hipStream_t s, const AcousticArgs& a, int mode) {
+void SFX(launch_acoustic)(hipStream_t s, const AcousticArgs& a) {
   if (a.nelem <= 0) return;
-  dim3 grid((a.nelem + 4) / 5), block(128);
-  if (mode == 1)
-    hipLaunchKernelGGL(k_acoustic<1>, grid, block, 0, s, a, g_gll_host);
-  else if (mode == 2)
-    hipLaunchKernelGGL(k_acoustic<2>, grid, block, 0, s, a, g_gll_host);
-  else
-    hipLaunchKernelGGL(k_acoustic<0>, grid, block, 0, s, a, g_gll_host);
+  hipLaunchKernelGGL(k_acoustic, dim3((a.nelem + 4) / 5), dim3(128), 0, s, a, g_gll_host);
   SF_LAUNCH_CHECK("k_acoustic");
 }
 

@@ -1,7 +1,7 @@
 // k_assembly.hip -- structures of the gather assembly, built on the device.
 //
-// The element stiffness stores its local forces, three floats per local point, and the pass that
-// needs the assembled acceleration sums them (k_gather_update in k_update.hip). The sums need, per
+// The element stiffness stores its local forces, three floats per local point (one in the fluid), and
+// the pass that needs the assembled acceleration sums them (k_gather_update in k_update.hip). The sums need, per
 // global point, the list of its local points in a fixed element order: a CSR, each point's entries
 // sorted by the position of their element in a list. It is built here (count, scan, fill, sort each
 // point's few entries) instead of on the host: 131072 elements take about a millisecond, a host
@@ -120,7 +120,7 @@ __global__ void k_csr_sort(int nglob, const int* __restrict__ ptr, const int* __
 // 128-byte lines of the local forces that a wave over 64 consecutive points reads (one wave in 16 is
 // counted): lanes whose w-th slot lies in another line than that of the lane before
 __global__ void k_count_lines(int nglob, const int* __restrict__ ptr, const int* __restrict__ idx,
-                              const int* __restrict__ pos, int eb, unsigned long long* lines) {
+                              const int* __restrict__ pos, int ncomp, int eb, unsigned long long* lines) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   const int g = (t >> 6) * 1024 + (t & 63);
   const int b = g < nglob ? ptr[g] : 0, e = g < nglob ? ptr[g + 1] : 0;
@@ -129,8 +129,8 @@ __global__ void k_count_lines(int nglob, const int* __restrict__ ptr, const int*
     int l1 = -1, l2 = -1;
     if (b + w < e) {
       const int p = idx[b + w] % 125, q = pos[idx[b + w] / 125];
-      l1 = (int)((int64_t)gather_slot(q, p / 5, p % 5, 1) * 3 / 32);
-      l2 = (int)((int64_t)gather_slot(q, p / 5, p % 5, eb) * 3 / 32);
+      l1 = (int)((int64_t)gather_slot(q, p / 5, p % 5, 1) * ncomp / 32);
+      l2 = (int)((int64_t)gather_slot(q, p / 5, p % 5, eb) * ncomp / 32);
     }
     const int o1 = __shfl_up(l1, 1), o2 = __shfl_up(l2, 1);
     const bool head = (threadIdx.x & 63) == 0;
@@ -167,10 +167,13 @@ __global__ void k_gather_info(int64_t g0, int64_t n, const int* __restrict__ ptr
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t g = g0 + t;
-  const realw x = rm[3 * g], y = rm[3 * g + 1], z = rm[3 * g + 2];
-  const bool same = x == y && x == z;
+  bool same = true;
+  if (rm) {
+    const realw x = rm[3 * g], y = rm[3 * g + 1], z = rm[3 * g + 2];
+    same = x == y && x == z;
+    rm1[g] = x;
+  }
   info[g] = (uint16_t)(((ptr[g + 1] - ptr[g]) << AF_COUNT) | (same ? 0 : AF_MASS3));
-  rm1[g] = x;
   if (t % 64 == 0) base[t / 64] = ptr[g];
 }
 
@@ -182,7 +185,7 @@ static T* alloc_dev(int64_t n) {
 }
 
 int build_slot_lists(hipStream_t s, int nglob, int nspec, int nelem, const int* order, const int* launch, int nlaunch,
-                     int pos0, int eb, const int* ibool, int*& ptr, int*& idx) {
+                     int pos0, int ncomp, int eb, const int* ibool, int*& ptr, int*& idx) {
   const int64_t nl = (int64_t)nelem * 125, np = (int64_t)nglob + 1;
   const int64_t ntile = (np + SCAN_TILE - 1) / SCAN_TILE;
   ptr = alloc_dev<int>(np);
@@ -210,7 +213,8 @@ int build_slot_lists(hipStream_t s, int nglob, int nspec, int nelem, const int* 
     if (nelem > nlaunch)
       hipLaunchKernelGGL(k_list_position, sf_grid(nelem - nlaunch, 256), dim3(256), 0, s, nelem - nlaunch,
                          order + nlaunch, pos, pos0);
-    hipLaunchKernelGGL(k_count_lines, sf_grid((nglob + 1023) / 1024 * 64, 256), dim3(256), 0, s, nglob, ptr, idx, pos, eb, lines);
+    hipLaunchKernelGGL(k_count_lines, sf_grid((nglob + 1023) / 1024 * 64, 256), dim3(256), 0, s, nglob, ptr, idx, pos, ncomp,
+                       eb, lines);
     SF_CHECK(hipMemcpyAsync(h, lines, sizeof(h), hipMemcpyDeviceToHost, s));
     SF_CHECK(hipStreamSynchronize(s));
     if (h[0] <= h[1]) eb = 1;

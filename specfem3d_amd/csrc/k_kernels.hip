@@ -155,22 +155,6 @@ __global__ void __launch_bounds__(128) k_seismo_ac(AcReceiverArgs A, GLLk G, con
   }
 }
 
-// ordered assembly: for each global point, subtract its element contributions in increasing
-// element order (the order of the reference's serial element loop). ptr/idx is a CSR list of
-// local slots e*125+p per global point, sorted by element.
-__global__ void k_ordered_gather(int nglob, int ncomp, const int* __restrict__ ptr, const int* __restrict__ idx,
-                                 const realw* __restrict__ local, int64_t nl, realw* out) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= nglob) return;
-  const int b = ptr[g], e = ptr[g + 1];
-  if (b == e) return;
-  for (int c = 0; c < ncomp; c++) {
-    realw a = out[(int64_t)g * ncomp + c];
-    for (int q = b; q < e; q++) a = a - local[c * nl + idx[q]];
-    out[(int64_t)g * ncomp + c] = a;
-  }
-}
-
 // max over points of the vector norm (check_stability.f90); NaN propagates as +inf bits
 __global__ void k_max_norm(int64_t npts, int ncomp, const realw* __restrict__ f, unsigned int* out) {
   __shared__ realw sm[256];
@@ -222,13 +206,6 @@ void launch_seismo_ac(hipStream_t s, const AcReceiverArgs& a, const realw* field
   if (a.n <= 0) return;
   hipLaunchKernelGGL(k_seismo_ac, dim3((unsigned)a.n), dim3(128), 0, s, a, g_gll_host, field, pressure, out);
   SF_LAUNCH_CHECK("k_seismo_ac");
-}
-
-void launch_ordered_gather(hipStream_t s, int nglob, int ncomp, const int* ptr, const int* idx, const realw* local,
-                           int64_t nloc, realw* out) {
-  hipLaunchKernelGGL(k_ordered_gather, sf_grid(nglob, 256), dim3(256), 0, s, nglob, ncomp, ptr, idx, local, nloc,
-                     out);
-  SF_LAUNCH_CHECK("k_ordered_gather");
 }
 
 void launch_max_norm(hipStream_t s, int64_t npts, int ncomp, const realw* f, realw* out) {

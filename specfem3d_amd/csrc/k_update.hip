@@ -176,7 +176,7 @@ __device__ __forceinline__ int wave_prefix(int x) {
   return x;
 }
 
-template <int KIND, bool OLD, typename T>
+template <int NC, int KIND, bool OLD, typename T>
 __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
   const int nb = (int)gridDim.x, b = (int)blockIdx.x;
   const int q = nb >> 3, r = nb & 7, x = b & 7;  // contiguous blocks per XCD, last one first
@@ -190,85 +190,91 @@ __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
   int p1 = A.base[t >> 6] + p1w;
   const int p0 = p1 - cnt;
   const bool full = !A.clean || (fl & AF_TERM);
-  T a[3] = {0, 0, 0};
-  realw u[3], v[3], m[3];
-  if (KIND != GATHER_ONLY) {
-    m[0] = A.rm1[g];
-    m[1] = m[0];
-    m[2] = m[0];
+  T a[NC];
+  realw u[NC], v[NC], m[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    a[c] = 0;
+    if (KIND != GATHER_ONLY) m[c] = A.rm1[g];
   }
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
-    if (KIND != GATHER_ONLY) v[c] = A.v[3 * g + c];
-    if (KIND == GATHER_STEP) u[c] = A.u[3 * g + c];
+  for (int c = 0; c < NC; c++) {
+    if (KIND != GATHER_ONLY) v[c] = A.v[NC * g + c];
+    if (KIND == GATHER_STEP) u[c] = A.u[NC * g + c];
   }
-  if (full) {
+  const bool zero = fl & A.skip;
+  if (full && !zero) {
 #pragma unroll
-    for (int c = 0; c < 3; c++) a[c] = A.a[3 * g + c];
+    for (int c = 0; c < NC; c++) a[c] = A.a[NC * g + c];
   }
-  if (KIND != GATHER_ONLY && (fl & AF_MASS3)) {
-    m[1] = A.rm[3 * g + 1];
-    m[2] = A.rm[3 * g + 2];
+  if (NC == 3 && KIND != GATHER_ONLY && (fl & AF_MASS3)) {
+#pragma unroll
+    for (int c = 1; c < NC; c++) m[c] = A.rm[NC * g + c];
   }
-  if (fl & A.skip) p1 = p0;
+  if (zero) p1 = p0;
   for (int s = p0; s < p1; s += 4) {  // four slots in flight (an interior face point has two)
     int k[4];
-    realw l[4][3];
+    realw l[4][NC];
 #pragma unroll
     for (int w = 0; w < 4; w++) k[w] = s + w < p1 ? A.idx[s + w] : -1;
 #pragma unroll
     for (int w = 0; w < 4; w++) {
       if (k[w] < 0) continue;
-      const realw* o = A.local + 3 * (int64_t)k[w];
-      l[w][0] = o[0];
-      l[w][1] = o[1];
-      l[w][2] = o[2];
+      const realw* o = A.local + NC * (int64_t)k[w];
+#pragma unroll
+      for (int c = 0; c < NC; c++) l[w][c] = o[c];
     }
 #pragma unroll
     for (int w = 0; w < 4; w++) {
       if (k[w] < 0) continue;
 #pragma unroll
-      for (int c = 0; c < 3; c++) a[c] = a[c] + (-(T)l[w][c]);
+      for (int c = 0; c < NC; c++) a[c] = a[c] + (-(T)l[w][c]);
     }
   }
   if (KIND == GATHER_ONLY) {
-    if (p1 > p0) {
+    if (p1 > p0 || zero) {
 #pragma unroll
-      for (int c = 0; c < 3; c++) A.a[3 * g + c] = (realw)a[c];
+      for (int c = 0; c < NC; c++) A.a[NC * g + c] = (realw)a[c];
     }
     return;
   }
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
+  for (int c = 0; c < NC; c++) {
     a[c] = a[c] * (T)m[c];
     T vc = (T)v[c] + (T)A.dt2p * a[c];
     if (KIND == GATHER_STEP) {
       T uc = u[c];
-      if (OLD) A.old[3 * g + c] = (realw)(uc + (T)A.t1 * vc + (T)A.t2 * a[c]);
+      if (OLD) A.old[NC * g + c] = (realw)(uc + (T)A.t1 * vc + (T)A.t2 * a[c]);
       uc = uc + (T)A.dt * vc + (T)A.dtsq2 * a[c];
       vc = vc + (T)A.dt2 * a[c];
-      A.u[3 * g + c] = (realw)uc;
-      if (full) A.a[3 * g + c] = 0.f;
+      A.u[NC * g + c] = (realw)uc;
+      if (full) A.a[NC * g + c] = 0.f;
     } else {
-      A.a[3 * g + c] = (realw)a[c];
+      A.a[NC * g + c] = (realw)a[c];
     }
-    A.v[3 * g + c] = (realw)vc;
+    A.v[NC * g + c] = (realw)vc;
   }
 }
 
-void launch_gather_update(hipStream_t s, const GatherArgs& a, int kind, bool exact) {
-  if (a.n <= 0) return;
+template <int NC, int KIND, bool OLD>
+static void launch_gather(hipStream_t s, const GatherArgs& a, bool exact) {
   const dim3 grid = sf_grid(a.n, 256), block(256);
-#define SF_GU(K, OLD)                                                                        \
-  do {                                                                                      \
-    if (exact) hipLaunchKernelGGL((k_gather_update<K, OLD, float>), grid, block, 0, s, a);  \
-    else hipLaunchKernelGGL((k_gather_update<K, OLD, double>), grid, block, 0, s, a);       \
-  } while (0)
-  if (kind == GATHER_ONLY) SF_GU(GATHER_ONLY, false);
-  else if (kind == GATHER_CORRECT) SF_GU(GATHER_CORRECT, false);
-  else if (a.old) SF_GU(GATHER_STEP, true);
-  else SF_GU(GATHER_STEP, false);
-#undef SF_GU
+  if (exact) hipLaunchKernelGGL((k_gather_update<NC, KIND, OLD, float>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((k_gather_update<NC, KIND, OLD, double>), grid, block, 0, s, a);
+}
+
+void launch_gather_update(hipStream_t s, const GatherArgs& a, int ncomp, int kind, bool exact) {
+  if (a.n <= 0) return;
+  if (ncomp == 1) {
+    if (kind == GATHER_ONLY) launch_gather<1, GATHER_ONLY, false>(s, a, exact);
+    else if (kind == GATHER_CORRECT) launch_gather<1, GATHER_CORRECT, false>(s, a, exact);
+    else launch_gather<1, GATHER_STEP, false>(s, a, exact);
+  } else {
+    if (kind == GATHER_ONLY) launch_gather<3, GATHER_ONLY, false>(s, a, exact);
+    else if (kind == GATHER_CORRECT) launch_gather<3, GATHER_CORRECT, false>(s, a, exact);
+    else if (a.old) launch_gather<3, GATHER_STEP, true>(s, a, exact);
+    else launch_gather<3, GATHER_STEP, false>(s, a, exact);
+  }
   SF_LAUNCH_CHECK("k_gather_update");
 }
 

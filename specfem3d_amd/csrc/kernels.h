@@ -41,8 +41,9 @@ void launch_corrector_predictor(hipStream_t s, int64_t n, realw* u, realw* v, re
                                 realw dt2_prev, realw dt, realw dt2, realw dtsq2, realw* old = nullptr,
                                 realw t1 = 0.f, realw t2 = 0.f);
 
-// Gather assembly: the stiffness launches store local forces, 3 floats per slot, and the pass that
-// needs the acceleration sums them, a point's slots in list order: a -= local[slot].
+// Gather assembly: the stiffness launches store local forces, 3 floats per slot in the solid and 1 in
+// the fluid, and the pass that needs the acceleration (chi'' in the fluid) sums them, a point's slots in
+// list order: a -= local[slot].
 // The slot of point p = 5 row + i of the element at launch position pos: blocks of `eb` elements hold
 // row by row the elements' five points, so that a row of points that runs through the elements of a
 // block is contiguous (eb = 1: one element after the other).
@@ -52,7 +53,7 @@ __host__ __device__ __forceinline__ int gather_slot(int pos, int row, int i, int
 }
 enum : uint16_t {
   AF_TERM = 1,   // boundary, coupling or source terms may have written the point's accel
-  AF_EDGE = 2,   // point on the outer faces of the C-PML layers
+  AF_EDGE = 2,   // point on the outer faces of the C-PML layers, or on the free surface of the fluid
   AF_MASS3 = 4,  // the point's three inverse masses differ (implicit Stacey term)
   AF_COUNT = 3   // shift of the number of slots
 };
@@ -62,11 +63,11 @@ struct GatherArgs {
   const int* base;             // first slot entry of each 64 points from g0 on
   const int* idx;              // slots of every point, one point after the other
   const realw* local;
-  int skip;                    // points with one of these flags take no contributions
+  int skip;                    // points with one of these flags end with zero: no contributions, no terms
   int clean;                   // accel is zero at every point without AF_TERM (it need not be read)
   realw *u, *v, *a;
   const realw* rm;             // inverse mass, 3 per point (read at AF_MASS3 points)
-  const realw* rm1;            // ... and 1 per point (the others)
+  const realw* rm1;            // ... and 1 per point (the others; every point of the fluid)
   realw dt2p;                  // corrector: dt/2
   realw dt, dt2, dtsq2;        // predictor
   realw* old;                  // PML_displ_old = u + t1 v + t2 a of the corrected field, or null
@@ -77,15 +78,16 @@ struct GatherArgs {
 enum { GATHER_ONLY = 0, GATHER_CORRECT = 1, GATHER_STEP = 2 };
 // exact: the reference's single-precision operations; else sums, corrector and predictor in double
 // precision, rounded once per stored value
-void launch_gather_update(hipStream_t s, const GatherArgs& a, int kind, bool exact);
+void launch_gather_update(hipStream_t s, const GatherArgs& a, int ncomp, int kind, bool exact);
 // slot lists (k_assembly.hip): the elements of `order` give the order of the sums, those of `launch`
 // (nelem_launch of them) the slots, `pos0` launch positions on for the elements behind; allocates ptr
 // (nglob + 1) and idx (125 nelem). lines: cache lines that the waves of a pass over all points touch
 // with eb = 1 and with `eb`; idx holds slots for the returned one of the two.
 int build_slot_lists(hipStream_t s, int nglob, int nspec, int nelem, const int* order, const int* launch, int nlaunch,
-                     int pos0, int eb, const int* ibool, int*& ptr, int*& idx);
+                     int pos0, int ncomp, int eb, const int* ibool, int*& ptr, int*& idx);
 void launch_mark_points(hipStream_t s, int n, const int* ig, uint16_t bit, uint16_t* info);
-// info (flags to be marked afterwards), base and rm1 of GatherArgs from the slot lists and the masses
+// info (flags to be marked afterwards), base and rm1 of GatherArgs from the slot lists and the masses;
+// rm null: one mass per point, rm1 is not written
 void launch_gather_info(hipStream_t s, int64_t g0, int64_t n, const int* ptr, const realw* rm, uint16_t* info,
                         int* base, realw* rm1);
 
@@ -239,14 +241,11 @@ struct AcousticArgs {
   int64_t jac_plane;
   const realw* rho;
   const realw* pot;
-  realw* potdd;
-  realw* local_out;        // ordered assembly: 1 plane of nloc
+  realw* local_out;        // local forces, 1 per slot (gather_slot)
+  int eb;
 };
-void launch_acoustic(hipStream_t s, const AcousticArgs& a, bool exact, int mode);
+void launch_acoustic(hipStream_t s, const AcousticArgs& a, bool exact);
 
-// ordered assembly: out[g*ncomp + c] -= contributions in element order
-void launch_ordered_gather(hipStream_t s, int nglob, int ncomp, const int* ptr, const int* idx,
-                           const realw* local, int64_t nloc, realw* out);
 
 // boundary terms (k_boundary.hip)
 // atomic: one launch with float atomics instead of one launch per round (used when the element

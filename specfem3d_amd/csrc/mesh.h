@@ -40,6 +40,8 @@ struct AttField {            // memory variables + stored strain of one elastic 
   realw* eps = nullptr;      // 6 * nloc: per-element blocks of 6 planes xx,yy,xy,xz,yz,trace (eps_idx)
 };
 
+enum { FREE_POT = 1, FREE_DD = 2 };
+
 struct FacePoints {          // flattened boundary/coupling face points
   int n = 0;                 // number of face points (faces * 25)
   int* iglob = nullptr;
@@ -224,9 +226,19 @@ struct Mesh {
   int pending_gather_el[2] = {0, 0};
   int gather_skip_el[2] = {0, 0};  // AF_* of the points that the pending sum leaves out
   int accel_clean[2] = {0, 0};     // accel is zero at every point without AF_TERM
-  int* asm_ac_ptr = nullptr;       // same for the acoustic elements (1 component)
+  // the same for the fluid (1 component; the inverse mass is rmass_ac)
   int* asm_ac_idx = nullptr;
-  realw* asm_ac_buf = nullptr;
+  int asm_ac_eb = 1;
+  uint16_t* asm_ac_info = nullptr;
+  int* asm_ac_base = nullptr;
+  realw* asm_ac_buf[2] = {nullptr, nullptr};
+  int asm_ac_ready = 0;
+  int pending_gather_ac[2] = {0, 0};
+  int gather_skip_ac[2] = {0, 0};
+  int potdd_clean[2] = {0, 0};
+  // points of the fluid's free surface: FREE_POT = chi and chi' are zero there, FREE_DD = chi'' is (as
+  // stored: a waiting sum and a deferred corrector not counted)
+  int free_zero[2] = {0, 0};
   // coloured assembly (assembly = 2): element lists regrouped by colour; elements of one
   // colour share no global point, colour c is elems[off[c] .. off[c+1])
   int el_ncolor = 0, ac_ncolor = 0;

@@ -69,3 +69,44 @@ def test_mixed_elements(oracle_mod, n, order):
     g.close()
     e = np.linalg.norm((fast - ref).astype(np.float64)) / np.linalg.norm(ref.astype(np.float64))
     assert e < 1e-5, e
+
+
+@pytest.mark.parametrize("n,warp", [(2, False), (3, True), (5, False)])
+def test_potentials_between_steps(oracle_mod, n, warp):
+    """The fluid's sums, fused with its update and free surface, under a solid bottom layer: potentials put
+    between the steps (nonzero on the free surface too) and read back after every step, every second, or at
+    the end."""
+    from specfem3d_amd import sources as S
+    from specfem3d_amd.mesh.box import build_box, homogeneous
+    from specfem3d_amd.solver import GPUSolver
+    L = 500.0 * n
+    ext = (0.0, L, 0.0, L, -L, 0.0)
+    db = build_box(n, n, n, ext, material=homogeneous(2300.0, 2800.0, 1500.0), acoustic_top_layers=n - 1,
+                   acoustic_material=homogeneous(1020.0, 1500.0, 0.0), warp=smooth_warp(L) if warp else None,
+                   stacey_faces=(1, 2, 3, 4, 5))
+    db.finalize(0.004, stacey=True)
+    src = S.setup_cmt_sources(db, [S.CMTSource(0.43 * L, 0.57 * L, 0.3 * L / 1000.0, 0.0, 0.06, 3e13, 2e13, 3e13,
+                                               1e12, 0.0, 0.0)], 0.004)
+    assert db.ispec_is_acoustic[src.ispec].all()
+    wet = np.unique(db.ibool[np.asarray(db.ispec_is_acoustic, bool)].ravel()).astype(np.int64)
+    wet = wet - int(db.ibool.min())
+    rng = np.random.default_rng(n)
+    put = [np.zeros(db.nglob, np.float32) for _ in range(3)]
+    for x, s in zip(put, (1e2, 1e4, 1e6)):
+        x[wet] = rng.normal(size=wet.size).astype(np.float32) * np.float32(s)
+    for every in (1, 2, 12):
+        o = oracle_mod.OracleSolver(db, src, None, "f32")
+        o.stf_table = src.stf_table(40)
+        g = GPUSolver(db, src, None, nstep=40, exact=True, assembly=1)
+        print(f"[gpu] fluid gather n={n} warp={warp} every={every}", flush=True)
+        for k in range(12):
+            if k == 4:
+                nn = C.c_int(db.nglob)
+                g.L.transfer_fields_ac_to_device_(C.byref(nn), *[x.ctypes.data_as(C.c_void_p) for x in put], g.MP)
+                o.pot[:], o.potd[:], o.potdd[:] = put
+            g.step()
+            o.run(1)
+            if (k + 1) % every == 0:
+                for x, y in zip(g.potentials(), (o.pot, o.potd, o.potdd)):
+                    assert np.array_equal(x, y), (every, k)
+        g.close()
