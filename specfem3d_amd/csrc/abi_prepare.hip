@@ -1266,7 +1266,7 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
 // exact = 1: element kernels without fused multiply-add (the CPU reference's rounding);
 // assembly: the order in which a global point's element contributions are summed. 1 = element order
 // (the reference's serial order), 2 = the colour order of a greedy element colouring, 0 = any order
-// (element order; the face terms of the fluid and the coupling use float atomics). All of them store
+// (element order as well). All of them store
 // the local forces and sum them in the next update (k_gather_update).
 extern "C" void sf_set_options(long* Mesh_pointer, int exact, int assembly) {
   Mesh* m = from_handle(Mesh_pointer);

@@ -24,15 +24,6 @@ const std::vector<int>& host_ibool(Mesh* m);
 
 static inline int field_of(int foa) { return foa == 3 ? 1 : 0; }
 
-// face-point terms in one atomic launch when the element stiffness scatters with atomics (its
-// sums have no fixed order then), else one launch per round in the reference's face order. The
-// elastic Stacey term never uses atomics: one launch walks each point's occurrences in round order
-// (k_stacey_el_chain, the rounds' sums bit for bit). On the 96x96x48 workload its 0.63 M points take
-// 21.7 us so, against 37 us in three rounds and 65 us in one atomic launch; the fluid Stacey term
-// and both coupling directions were faster in one atomic launch (4.7 / 15.1 / 5.5 us against
-// 18.9 / 19.2 / 18.7 us in rounds).
-static inline bool face_atomics(const Mesh* m) { return m->assembly == 0; }
-
 static GatherArgs gather_args(Mesh* m, int f) {
   GatherArgs a;
   std::memset(&a, 0, sizeof(a));
@@ -493,8 +484,7 @@ extern "C" void FC_FUNC_(compute_stacey_viscoelastic_cuda, COMPUTE_STACEY_VISCOE
   if (foa == 0 || foa == 1) {
     flush_el(m, 0);
     const bool store = m->simulation_type == 1 && m->save_forward && b_absorb_field;
-    launch_stacey_elastic(m->stream, m->abs_el, m->el[0].veloc, m->el[0].accel, m->b_absorb_field, store ? 1 : 0,
-                          false);
+    launch_stacey_elastic(m->stream, m->abs_el, m->el[0].veloc, m->el[0].accel, m->b_absorb_field, store ? 1 : 0);
     if (store) {
       SF_CHECK(hipMemcpyAsync(b_absorb_field, m->b_absorb_field, sizeof(realw) * rec_len, hipMemcpyDeviceToHost,
                               m->stream));
@@ -522,7 +512,7 @@ extern "C" void FC_FUNC_(compute_stacey_viscoelastic_undoatt_cuda, COMPUTE_STACE
     if (foa == 3 && f == 0) continue;
     if (!m->el[f].displ) continue;
     flush_el(m, f);
-    launch_stacey_elastic(m->stream, m->abs_el, m->el[f].veloc, m->el[f].accel, nullptr, 0, false);
+    launch_stacey_elastic(m->stream, m->abs_el, m->el[f].veloc, m->el[f].accel, nullptr, 0);
   }
 }
 
@@ -537,8 +527,7 @@ extern "C" void FC_FUNC_(compute_stacey_acoustic_cuda, COMPUTE_STACEY_ACOUSTIC_C
   if (foa == 0 || foa == 1) {
     flush_ac_terms(m, 0);
     const bool store = m->simulation_type == 1 && m->save_forward && h_b_absorb_potential;
-    launch_stacey_acoustic(m->stream, m->abs_ac, m->ac[0].potd, m->ac[0].potdd, m->b_absorb_potential, store ? 1 : 0,
-                           face_atomics(m));
+    launch_stacey_acoustic(m->stream, m->abs_ac, m->ac[0].potd, m->ac[0].potdd, m->b_absorb_potential, store ? 1 : 0);
     if (store) {
       SF_CHECK(hipMemcpyAsync(h_b_absorb_potential, m->b_absorb_potential, sizeof(realw) * rec_len,
                               hipMemcpyDeviceToHost, m->stream));
@@ -564,7 +553,7 @@ extern "C" void FC_FUNC_(compute_stacey_acoustic_undoatt_cuda, COMPUTE_STACEY_AC
     if (foa == 3 && f == 0) continue;
     if (!m->ac[f].pot) continue;
     flush_ac_terms(m, f);
-    launch_stacey_acoustic(m->stream, m->abs_ac, m->ac[f].potd, m->ac[f].potdd, nullptr, 0, face_atomics(m));
+    launch_stacey_acoustic(m->stream, m->abs_ac, m->ac[f].potd, m->ac[f].potdd, nullptr, 0);
   }
 }
 
@@ -581,7 +570,7 @@ extern "C" void FC_FUNC_(compute_coupling_ac_el_cuda, COMPUTE_COUPLING_AC_EL_CUD
     if (!m->ac[f].pot || !m->el[f].displ) continue;
     flush_ac_terms(m, f);
     const int flip = (m->simulation_type != 1 && f == 0) ? 1 : 0;
-    launch_coupling_ac_el(m->stream, m->coupling, m->el[f].displ, m->ac[f].potdd, flip, face_atomics(m));
+    launch_coupling_ac_el(m->stream, m->coupling, m->el[f].displ, m->ac[f].potdd, flip);
   }
 }
 
@@ -599,7 +588,7 @@ extern "C" void FC_FUNC_(compute_coupling_el_ac_cuda, COMPUTE_COUPLING_EL_AC_CUD
     flush_ac(m, f);
     flush_el(m, f);
     const int flip = (m->simulation_type != 1 && f == 0) ? 1 : 0;
-    launch_coupling_el_ac(m->stream, m->coupling, m->ac[f].potdd, m->el[f].accel, flip, face_atomics(m));
+    launch_coupling_el_ac(m->stream, m->coupling, m->ac[f].potdd, m->el[f].accel, flip);
   }
 }
 

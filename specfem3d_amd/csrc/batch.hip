@@ -8,16 +8,16 @@
 //   * shots are placed in decreasing order of record length, so the live shots at any step are
 //     a prefix and a finished group costs no memory traffic;
 //   * a mesh with fluid elements also steps S potentials over its acoustic range of global points
-//     in the same layout: per step the potential predictor, free
-//     surface, acoustic stiffness, fluid Stacey and fluid side of the coupling, the corrector and
-//     the free surface again come first, then the solid side of the coupling with the elastic
-//     boundary terms (the single-shot call order of iterate_time.F90);
-//   * one step = sum of the local forces with the corrector and predictor (k_batch_gather), Stacey
-//     rounds, source rounds, stiffness (one launch that stores local forces), receivers, and a one-lane
+//     in the same layout: per step the potential predictor, fluid Stacey, fluid side of the coupling,
+//     acoustic stiffness, its sum with the corrector and the free surface come first, then the solid
+//     side of the coupling with the elastic boundary terms (the single-shot call order of
+//     iterate_time.F90);
+//   * one step = sum of the local forces with the corrector and predictor (k_batch_gather), Stacey,
+//     source rounds, stiffness (one launch that stores local forces), receivers, and a one-lane
 //     kernel that advances the device step counter. Every kernel reads the counter, so a group of
 //     steps is captured once into a hipGraph and replayed;
 //   * the per-point arithmetic and the order of every sum equal the single-shot path (same
-//     kernels' expressions, same colour order, same face rounds), so each shot of a batch is
+//     kernels' expressions, same colour order, same order of faces), so each shot of a batch is
 //     bit-identical to its single-shot run with the same options.
 // Shots-per-workgroup are chosen by an autotuner that times each candidate for a few steps from rest
 // and then resets the batch.
@@ -234,11 +234,13 @@ __global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs A) {
 }
 
 // the same for the potentials: chi'' -= local forces, then the corrector chi'' *= rmass, chi' += dt/2 chi''
-// (rows g - g0; the boundary terms are in chi'' already)
+// (rows g - g0; the boundary terms are in chi'' already). Points on the free surface (AF_EDGE) take no
+// forces and no terms: their potentials start at zero and stay there.
 template <typename T>
 __global__ void __launch_bounds__(256) k_batch_ac_gather(int64_t nrow, int64_t g0, const int* __restrict__ ptr,
                                                          const int* __restrict__ idx, const realw* __restrict__ local,
                                                          int64_t loc_group, int first_group,
+                                                         const uint16_t* __restrict__ info,
                                                          const int* __restrict__ nstep, const int* __restrict__ itp,
                                                          realw* __restrict__ potd, realw* __restrict__ potdd,
                                                          const realw* __restrict__ rm, realw dt2) {
@@ -252,8 +254,11 @@ __global__ void __launch_bounds__(256) k_batch_ac_gather(int64_t nrow, int64_t g
   float4 V = *reinterpret_cast<const float4*>(potd + o);
   const float4 a0 = *reinterpret_cast<const float4*>(potdd + o);
   const realw M = rm[row];
-  T a[4] = {a0.x, a0.y, a0.z, a0.w};
-  gather4<T>(a, ptr, idx, g0 + row, local + (int64_t)blockIdx.y * loc_group + 4 * (int)(t & 1), 8);
+  T a[4] = {0, 0, 0, 0};
+  if (!(info[g0 + row] & AF_EDGE)) {
+    a[0] = a0.x; a[1] = a0.y; a[2] = a0.z; a[3] = a0.w;
+    gather4<T>(a, ptr, idx, g0 + row, local + (int64_t)blockIdx.y * loc_group + 4 * (int)(t & 1), 8);
+  }
   float4 Ac = a0;
 #define SF_AG(c, r)                          \
   if (r == 0 || nstep[s + r] >= it) {        \
@@ -267,29 +272,51 @@ __global__ void __launch_bounds__(256) k_batch_ac_gather(int64_t nrow, int64_t g
   *reinterpret_cast<float4*>(potdd + o) = Ac;
 }
 
-// Stacey (k_stacey_el arithmetic) for every (face point of one round, live shot)
-__global__ void k_batch_stacey(int n, int S, int64_t nrow, const int* __restrict__ ig, const realw* __restrict__ nrm,
+// Face terms: a lane takes one global point (a face point of round 0) of one live shot and follows the
+// point's other face points (FacePoints::next), with the sums of k_boundary.hip. Eight consecutive lanes
+// are the shots of a group, blockIdx.y is the group. A launch takes about 5 us of a captured step at any
+// of these sizes: with one per term instead of one per round, and the free surface in the fluid's sum,
+// a step of 18x18x12 elements x 8 shots under a sea has 12 launches instead of 26 and takes 233 -> 203 us.
+struct FaceLane {
+  int t0, s;
+  bool live;
+};
+__device__ __forceinline__ FaceLane face_lane(int n0, const int* nstep, const int* itp) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  FaceLane f;
+  f.t0 = t >> 3;
+  f.s = 8 * (int)blockIdx.y + (t & 7);
+  f.live = f.t0 < n0 && nstep[f.s] >= load_it(itp);
+  return f;
+}
+
+// Stacey (k_stacey_el arithmetic)
+__global__ void k_batch_stacey(int n0, int64_t nrow, const int* __restrict__ ig, const realw* __restrict__ nrm,
                                const realw* __restrict__ jw, const realw* __restrict__ rvp,
-                               const realw* __restrict__ rvs, const int* __restrict__ nstep,
-                               const int* __restrict__ itp, const realw* __restrict__ veloc, realw* accel) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;  // n * S < 2^31 (checked by the caller)
-  const int q = t / S;
-  const int s = t - q * S;
-  if (q >= n) return;
-  if (nstep[s] < load_it(itp)) return;
-  const int64_t b = batch_idx(nrow, 3 * (int64_t)ig[q], s);
+                               const realw* __restrict__ rvs, const int* __restrict__ next,
+                               const int* __restrict__ nstep, const int* __restrict__ itp,
+                               const realw* __restrict__ veloc, realw* accel) {
+  const FaceLane f = face_lane(n0, nstep, itp);
+  if (!f.live) return;
+  const int64_t b = batch_idx(nrow, 3 * (int64_t)ig[f.t0], f.s);
   const realw vx = veloc[b], vy = veloc[b + 8], vz = veloc[b + 16];
-  const realw nx = nrm[3 * q], ny = nrm[3 * q + 1], nz = nrm[3 * q + 2];
-  const realw vn = vx * nx + vy * ny + vz * nz;
-  const realw p = rvp[q], sv = rvs[q];
-  const realw tx = p * vn * nx + sv * (vx - vn * nx);
-  const realw ty = p * vn * ny + sv * (vy - vn * ny);
-  const realw tz = p * vn * nz + sv * (vz - vn * nz);
-  const realw w = jw[q];
-  const realw fx = tx * w, fy = ty * w, fz = tz * w;
-  accel[b] = accel[b] - fx;
-  accel[b + 8] = accel[b + 8] - fy;
-  accel[b + 16] = accel[b + 16] - fz;
+  realw ax = accel[b], ay = accel[b + 8], az = accel[b + 16];
+  for (int q = f.t0; q >= 0; q = next[q]) {
+    const realw nx = nrm[3 * q], ny = nrm[3 * q + 1], nz = nrm[3 * q + 2];
+    const realw vn = vx * nx + vy * ny + vz * nz;
+    const realw p = rvp[q], sv = rvs[q];
+    const realw tx = p * vn * nx + sv * (vx - vn * nx);
+    const realw ty = p * vn * ny + sv * (vy - vn * ny);
+    const realw tz = p * vn * nz + sv * (vz - vn * nz);
+    const realw w = jw[q];
+    const realw fx = tx * w, fy = ty * w, fz = tz * w;
+    ax = ax - fx;
+    ay = ay - fy;
+    az = az - fz;
+  }
+  accel[b] = ax;
+  accel[b + 8] = ay;
+  accel[b + 16] = az;
 }
 
 // source entries of one round: accel += sourcearray * stf(it) (k_add_sources_el arithmetic)
@@ -375,71 +402,63 @@ __global__ void __launch_bounds__(256) k_batch_ac_predictor(int64_t nrow, const 
   *reinterpret_cast<float4*>(potdd + o) = A;
 }
 
-// free surface (k_free_surface): zero chi, chi', chi'' of every (free-surface point, live shot)
-__global__ void k_batch_free_surface(int n, int S, int64_t nrow, int64_t g0, const int* __restrict__ ig,
-                                     const int* __restrict__ nstep, const int* __restrict__ itp, realw* pot,
-                                     realw* potd, realw* potdd) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;  // n * S < 2^31 (checked by the caller)
-  const int q = t / S;
-  const int s = t - q * S;
-  if (q >= n) return;
-  if (nstep[s] < load_it(itp)) return;
-  const int64_t b = batch_idx(nrow, (int64_t)ig[q] - g0, s);
-  pot[b] = 0.f;
-  potd[b] = 0.f;
-  potdd[b] = 0.f;
-}
-
-// fluid Stacey (k_stacey_ac arithmetic) for every (face point of one round, live shot)
-__global__ void k_batch_stacey_ac(int n, int S, int64_t nrow, int64_t g0, const int* __restrict__ ig, const realw* __restrict__ jw,
-                                  const realw* __restrict__ rho, const realw* __restrict__ cp,
+// fluid Stacey (k_stacey_ac arithmetic)
+__global__ void k_batch_stacey_ac(int n0, int64_t nrow, int64_t g0, const int* __restrict__ ig,
+                                  const realw* __restrict__ jw, const realw* __restrict__ rho,
+                                  const realw* __restrict__ cp, const int* __restrict__ next,
                                   const int* __restrict__ nstep, const int* __restrict__ itp,
                                   const realw* __restrict__ potd, realw* potdd) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int q = t / S;
-  const int s = t - q * S;
-  if (q >= n) return;
-  if (nstep[s] < load_it(itp)) return;
-  const int64_t b = batch_idx(nrow, (int64_t)ig[q] - g0, s);
-  const realw absorbl = potd[b] * jw[q] / cp[q] / rho[q];
-  potdd[b] = potdd[b] - absorbl;
+  const FaceLane f = face_lane(n0, nstep, itp);
+  if (!f.live) return;
+  const int64_t b = batch_idx(nrow, (int64_t)ig[f.t0] - g0, f.s);
+  const realw v = potd[b];
+  realw a = potdd[b];
+  for (int q = f.t0; q >= 0; q = next[q]) {
+    const realw absorbl = v * jw[q] / cp[q] / rho[q];
+    a = a - absorbl;
+  }
+  potdd[b] = a;
 }
 
 // fluid side of the coupling (k_coupling_ac_el arithmetic, forward field): chi'' += w (u . n)
-__global__ void k_batch_coupling_ac_el(int n, int S, int64_t nrow, int64_t nrow_ac, int64_t g0, const int* __restrict__ ig,
+__global__ void k_batch_coupling_ac_el(int n0, int64_t nrow, int64_t nrow_ac, int64_t g0, const int* __restrict__ ig,
                                        const realw* __restrict__ nrm, const realw* __restrict__ jw,
-                                       const int* __restrict__ nstep, const int* __restrict__ itp,
-                                       const realw* __restrict__ u, realw* potdd) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int q = t / S;
-  const int s = t - q * S;
-  if (q >= n) return;
-  if (nstep[s] < load_it(itp)) return;
-  const int64_t g = ig[q];
-  const int64_t e = batch_idx(nrow, 3 * g, s);
+                                       const int* __restrict__ next, const int* __restrict__ nstep,
+                                       const int* __restrict__ itp, const realw* __restrict__ u, realw* potdd) {
+  const FaceLane f = face_lane(n0, nstep, itp);
+  if (!f.live) return;
+  const int64_t g = ig[f.t0];
+  const int64_t e = batch_idx(nrow, 3 * g, f.s);
   const realw ux = u[e], uy = u[e + 8], uz = u[e + 16];
-  const realw un = ux * nrm[3 * q] + uy * nrm[3 * q + 1] + uz * nrm[3 * q + 2];
-  const int64_t b = batch_idx(nrow_ac, g - g0, s);
-  potdd[b] = potdd[b] + jw[q] * un;
+  const int64_t b = batch_idx(nrow_ac, g - g0, f.s);
+  realw a = potdd[b];
+  for (int q = f.t0; q >= 0; q = next[q]) {
+    const realw un = ux * nrm[3 * q] + uy * nrm[3 * q + 1] + uz * nrm[3 * q + 2];
+    a = a + jw[q] * un;
+  }
+  potdd[b] = a;
 }
 
 // solid side of the coupling (k_coupling_el_ac arithmetic, forward field): a += w n (-chi'')
-__global__ void k_batch_coupling_el_ac(int n, int S, int64_t nrow, int64_t nrow_ac, int64_t g0, const int* __restrict__ ig,
+__global__ void k_batch_coupling_el_ac(int n0, int64_t nrow, int64_t nrow_ac, int64_t g0, const int* __restrict__ ig,
                                        const realw* __restrict__ nrm, const realw* __restrict__ jw,
-                                       const int* __restrict__ nstep, const int* __restrict__ itp,
-                                       const realw* __restrict__ potdd, realw* accel) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int q = t / S;
-  const int s = t - q * S;
-  if (q >= n) return;
-  if (nstep[s] < load_it(itp)) return;
-  const int64_t g = ig[q];
-  const realw pr = -potdd[batch_idx(nrow_ac, g - g0, s)];
-  const realw w = jw[q];
-  const int64_t e = batch_idx(nrow, 3 * g, s);
-  accel[e] = accel[e] + w * nrm[3 * q] * pr;
-  accel[e + 8] = accel[e + 8] + w * nrm[3 * q + 1] * pr;
-  accel[e + 16] = accel[e + 16] + w * nrm[3 * q + 2] * pr;
+                                       const int* __restrict__ next, const int* __restrict__ nstep,
+                                       const int* __restrict__ itp, const realw* __restrict__ potdd, realw* accel) {
+  const FaceLane f = face_lane(n0, nstep, itp);
+  if (!f.live) return;
+  const int64_t g = ig[f.t0];
+  const realw pr = -potdd[batch_idx(nrow_ac, g - g0, f.s)];
+  const int64_t e = batch_idx(nrow, 3 * g, f.s);
+  realw ax = accel[e], ay = accel[e + 8], az = accel[e + 16];
+  for (int q = f.t0; q >= 0; q = next[q]) {
+    const realw w = jw[q];
+    ax = ax + w * nrm[3 * q] * pr;
+    ay = ay + w * nrm[3 * q + 1] * pr;
+    az = az + w * nrm[3 * q + 2] * pr;
+  }
+  accel[e] = ax;
+  accel[e + 8] = ay;
+  accel[e + 16] = az;
 }
 
 __global__ void k_batch_tick(int* itp) {
@@ -567,6 +586,7 @@ static void build_gather(Batch* b) {
   if (m->stacey) launch_mark_points(m->stream, m->abs_el.n, m->abs_el.iglob, AF_TERM, b->info);
   if (b->ac) launch_mark_points(m->stream, m->coupling.n, m->coupling.iglob, AF_TERM, b->info);
   launch_mark_points(m->stream, b->src_n, b->src_ig, AF_TERM, b->info);
+  if (b->ac) launch_mark_points(m->stream, m->free_ac.n, m->free_ac.iglob, AF_EDGE, b->info);
 }
 
 static BatchGatherArgs gather_args(Batch* b) {
@@ -657,16 +677,13 @@ static void enqueue_seismo(Batch* b, hipStream_t st) {
   SF_LAUNCH_CHECK("k_batch_seismo");
 }
 
-// launches over (face point of one round, live shot) pairs
-static dim3 pair_grid(int cnt, int S, const char* what) {
-  if ((int64_t)cnt * S >= 0x7fffffff) fatal("sf_batch", what);
-  return sf_grid((int64_t)cnt * S, 256);
-}
+// launches over (global point of the faces, shot)
+static dim3 face_grid(const FacePoints& f, int S) { return dim3(sf_grid(8 * (int64_t)f.points(), 256).x, (unsigned)(S / 8)); }
 
 // the fluid part of a step (the acoustic calls of iterate_time.F90 before the elastic ones):
-// predictor, free surface, Stacey, coupling (fluid side), stiffness (all elements are inner at
-// NPROC = 1, so the stiffness runs in phase 2, after the boundary terms of phase 1), corrector,
-// free surface
+// predictor, Stacey, coupling (fluid side), stiffness (all elements are inner at NPROC = 1, so the
+// stiffness runs in phase 2, after the boundary terms of phase 1), corrector and free surface (the free
+// surface before the forces finds its points at zero)
 static void enqueue_fluid(Batch* b, hipStream_t st) {
   Mesh* m = b->m;
   const int S = b->S;
@@ -675,30 +692,18 @@ static void enqueue_fluid(Batch* b, hipStream_t st) {
   hipLaunchKernelGGL(k_batch_ac_predictor, rows, dim3(256), 0, st, na, b->d_nstep, b->d_it, b->pot, b->potd,
                      b->potdd, b->dt, b->dt2, b->dtsq2);
   SF_LAUNCH_CHECK("k_batch_ac_predictor");
-  const FacePoints& fs = m->free_ac;
-  if (fs.n > 0)
-    hipLaunchKernelGGL(k_batch_free_surface, pair_grid(fs.n, S, "too many free-surface points x shots"), dim3(256),
-                       0, st, fs.n, S, na, b->ac_g0, fs.iglob, b->d_nstep, b->d_it, b->pot, b->potd, b->potdd);
-  if (m->stacey) {
-    const FacePoints& f = m->abs_ac;
-    for (int r = 0; r < f.nrounds; r++) {
-      const int o = f.round_off[r], cnt = f.round_off[r + 1] - o;
-      if (cnt <= 0) continue;
-      hipLaunchKernelGGL(k_batch_stacey_ac, pair_grid(cnt, S, "too many fluid Stacey points x shots"), dim3(256), 0,
-                         st, cnt, S, na, b->ac_g0, f.iglob + o, f.jacw + o, f.imp_p + o, f.imp_s + o, b->d_nstep,
-                         b->d_it, b->potd, b->potdd);
-    }
+  const FacePoints& f = m->abs_ac;
+  if (m->stacey && f.points() > 0) {
+    hipLaunchKernelGGL(k_batch_stacey_ac, face_grid(f, S), dim3(256), 0, st, f.points(), na, b->ac_g0, f.iglob, f.jacw,
+                       f.imp_p, f.imp_s, f.next, b->d_nstep, b->d_it, b->potd, b->potdd);
     SF_LAUNCH_CHECK("k_batch_stacey_ac");
   }
   const FacePoints& cf = m->coupling;
-  for (int r = 0; r < cf.nrounds; r++) {
-    const int o = cf.round_off[r], cnt = cf.round_off[r + 1] - o;
-    if (cnt <= 0) continue;
-    hipLaunchKernelGGL(k_batch_coupling_ac_el, pair_grid(cnt, S, "too many coupling points x shots"), dim3(256), 0,
-                       st, cnt, S, nrow, na, b->ac_g0, cf.iglob + o, cf.normal + 3 * o, cf.jacw + o, b->d_nstep, b->d_it, b->u,
-                       b->potdd);
+  if (cf.points() > 0) {
+    hipLaunchKernelGGL(k_batch_coupling_ac_el, face_grid(cf, S), dim3(256), 0, st, cf.points(), nrow, na, b->ac_g0,
+                       cf.iglob, cf.normal, cf.jacw, cf.next, b->d_nstep, b->d_it, b->u, b->potdd);
+    SF_LAUNCH_CHECK("k_batch_coupling_ac_el");
   }
-  SF_LAUNCH_CHECK("k_batch_coupling_ac_el");
   BatchAcArgs A;
   std::memset(&A, 0, sizeof(A));
   A.elems = m->acoustic_elems;
@@ -724,14 +729,10 @@ static void enqueue_fluid(Batch* b, hipStream_t st) {
     launch_acoustic_batch(st, A, b->sc, m->exact != 0);
     auto* gather = m->exact ? &k_batch_ac_gather<float> : &k_batch_ac_gather<double>;
     hipLaunchKernelGGL(gather, dim3(rows.x, (unsigned)n), dim3(256), 0, st, na, b->ac_g0, b->ac_ptr, b->ac_idx,
-                       b->ac_local, A.loc_group, g, b->d_nstep, b->d_it, b->potd, b->potdd, m->rmass_ac + b->ac_g0,
+                       b->ac_local, A.loc_group, g, b->info, b->d_nstep, b->d_it, b->potd, b->potdd, m->rmass_ac + b->ac_g0,
                        b->dt2);
     SF_LAUNCH_CHECK("k_batch_ac_gather");
   }
-  if (fs.n > 0)
-    hipLaunchKernelGGL(k_batch_free_surface, pair_grid(fs.n, S, "too many free-surface points x shots"), dim3(256),
-                       0, st, fs.n, S, na, b->ac_g0, fs.iglob, b->d_nstep, b->d_it, b->pot, b->potd, b->potdd);
-  SF_LAUNCH_CHECK("k_batch_free_surface");
 }
 
 // one time step; `first`: the wavefields are zero
@@ -753,27 +754,16 @@ static void enqueue_step(Batch* b, hipStream_t st, bool first) {
     }
   }
   if (b->ac) enqueue_fluid(b, st);
-  if (m->stacey) {
-    const FacePoints& f = m->abs_el;
-    for (int r = 0; r < f.nrounds; r++) {
-      const int o = f.round_off[r], cnt = f.round_off[r + 1] - o;
-      if (cnt <= 0) continue;
-      if ((int64_t)cnt * b->S >= 0x7fffffff) fatal("sf_batch", "too many Stacey points x shots");
-      hipLaunchKernelGGL(k_batch_stacey, sf_grid((int64_t)cnt * b->S, 256), dim3(256), 0, st, cnt, b->S,
-                         3 * (int64_t)m->nglob, f.iglob + o, f.normal + 3 * o, f.jacw + o, f.imp_p + o, f.imp_s + o, b->d_nstep, b->d_it,
-                         b->v, b->a);
-    }
+  const FacePoints& f = m->abs_el;
+  if (m->stacey && f.points() > 0) {
+    hipLaunchKernelGGL(k_batch_stacey, face_grid(f, b->S), dim3(256), 0, st, f.points(), 3 * (int64_t)m->nglob, f.iglob,
+                       f.normal, f.jacw, f.imp_p, f.imp_s, f.next, b->d_nstep, b->d_it, b->v, b->a);
     SF_LAUNCH_CHECK("k_batch_stacey");
   }
-  if (b->ac) {
-    const FacePoints& cf = m->coupling;
-    for (int r = 0; r < cf.nrounds; r++) {
-      const int o = cf.round_off[r], cnt = cf.round_off[r + 1] - o;
-      if (cnt <= 0) continue;
-      hipLaunchKernelGGL(k_batch_coupling_el_ac, pair_grid(cnt, b->S, "too many coupling points x shots"), dim3(256),
-                         0, st, cnt, b->S, 3 * (int64_t)m->nglob, b->ac_n, b->ac_g0, cf.iglob + o, cf.normal + 3 * o, cf.jacw + o, b->d_nstep,
-                         b->d_it, b->potdd, b->a);
-    }
+  const FacePoints& cf = m->coupling;
+  if (b->ac && cf.points() > 0) {
+    hipLaunchKernelGGL(k_batch_coupling_el_ac, face_grid(cf, b->S), dim3(256), 0, st, cf.points(), 3 * (int64_t)m->nglob,
+                       b->ac_n, b->ac_g0, cf.iglob, cf.normal, cf.jacw, cf.next, b->d_nstep, b->d_it, b->potdd, b->a);
     SF_LAUNCH_CHECK("k_batch_coupling_el_ac");
   }
   for (int r = 0; r < b->src_nrounds; r++) {

@@ -1,65 +1,87 @@
 // k_sources.hip -- point sources, adjoint sources and receiver interpolation.
 //
 // Sources and adjoint sources are flattened to (owner, point) pairs sorted into rounds like
-// the face points (FacePoints.ispec holds the owner: source or adjoint-receiver index), so
-// points shared by two sources are summed in the reference's source order without atomics.
+// the face points (FacePoints.ispec holds the owner: source or adjoint-receiver index); a lane per
+// point of round 0 follows the point's other pairs (FacePoints::next), so points shared by several
+// sources are summed in the reference's source order by one launch without atomics.
 // Built with -ffp-contract=off (reference rounding).
 #include "kernels.h"
 
 namespace sf {
 
 // compute_add_sources_viscoelastic.F90:145-152: a(:,iglob) += sourcearray(isrc,:,i,j,k) * stf(isrc)
-__global__ void k_add_sources_el(int n, const int* __restrict__ ig, const int* __restrict__ owner,
-                                 const int* __restrict__ ploc, const realw* __restrict__ arr,
-                                 const realw* __restrict__ stf, realw* accel) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int64_t g = ig[t];
-  const int s = owner[t];
-  const realw* sa = arr + ((int64_t)s * 125 + ploc[t]) * 3;
-  const realw st = stf[s];
-  accel[3 * g] = accel[3 * g] + sa[0] * st;
-  accel[3 * g + 1] = accel[3 * g + 1] + sa[1] * st;
-  accel[3 * g + 2] = accel[3 * g + 2] + sa[2] * st;
+__global__ void k_add_sources_el(int n0, const int* __restrict__ ig, const int* __restrict__ owner,
+                                 const int* __restrict__ ploc, const int* __restrict__ next,
+                                 const realw* __restrict__ arr, const realw* __restrict__ stf, realw* accel) {
+  const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t0 >= n0) return;
+  const int64_t g = ig[t0];
+  realw ax = accel[3 * g], ay = accel[3 * g + 1], az = accel[3 * g + 2];
+  for (int t = t0; t >= 0; t = next[t]) {
+    const int s = owner[t];
+    const realw* sa = arr + ((int64_t)s * 125 + ploc[t]) * 3;
+    const realw st = stf[s];
+    ax = ax + sa[0] * st;
+    ay = ay + sa[1] * st;
+    az = az + sa[2] * st;
+  }
+  accel[3 * g] = ax;
+  accel[3 * g + 1] = ay;
+  accel[3 * g + 2] = az;
 }
 
 // compute_add_sources_acoustic.f90: chi'' -= sourcearray * stf / kappa (pressure source)
-__global__ void k_add_sources_ac(int n, const int* __restrict__ ig, const int* __restrict__ owner,
-                                 const int* __restrict__ ploc, const realw* __restrict__ arr,
-                                 const realw* __restrict__ kap, const realw* __restrict__ stf, realw* potdd) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int g = ig[t];
-  const int s = owner[t];
-  const realw sa = arr[((int64_t)s * 125 + ploc[t]) * 3];
-  potdd[g] = potdd[g] - sa * stf[s] / kap[(int64_t)s * 125 + ploc[t]];
+__global__ void k_add_sources_ac(int n0, const int* __restrict__ ig, const int* __restrict__ owner,
+                                 const int* __restrict__ ploc, const int* __restrict__ next,
+                                 const realw* __restrict__ arr, const realw* __restrict__ kap,
+                                 const realw* __restrict__ stf, realw* potdd) {
+  const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t0 >= n0) return;
+  const int g = ig[t0];
+  realw a = potdd[g];
+  for (int t = t0; t >= 0; t = next[t]) {
+    const int s = owner[t];
+    const int64_t q = (int64_t)s * 125 + ploc[t];
+    a = a - arr[3 * q] * stf[s] / kap[q];
+  }
+  potdd[g] = a;
 }
 
 // compute_add_sources_viscoelastic.F90:226-245: a += adj(:,irec) * hxi heta hgamma (CUSTOM_REAL)
-__global__ void k_adjoint_sources_el(int n, const int* __restrict__ ig, const int* __restrict__ owner,
-                                     const int* __restrict__ ploc, const realw* __restrict__ h,
-                                     const realw* __restrict__ adj, realw* accel) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int64_t g = ig[t];
-  const int r = owner[t];
-  const realw hl = h[(int64_t)r * 125 + ploc[t]];
-  accel[3 * g] = accel[3 * g] + adj[3 * r] * hl;
-  accel[3 * g + 1] = accel[3 * g + 1] + adj[3 * r + 1] * hl;
-  accel[3 * g + 2] = accel[3 * g + 2] + adj[3 * r + 2] * hl;
+__global__ void k_adjoint_sources_el(int n0, const int* __restrict__ ig, const int* __restrict__ owner,
+                                     const int* __restrict__ ploc, const int* __restrict__ next,
+                                     const realw* __restrict__ h, const realw* __restrict__ adj, realw* accel) {
+  const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t0 >= n0) return;
+  const int64_t g = ig[t0];
+  realw ax = accel[3 * g], ay = accel[3 * g + 1], az = accel[3 * g + 2];
+  for (int t = t0; t >= 0; t = next[t]) {
+    const int r = owner[t];
+    const realw hl = h[(int64_t)r * 125 + ploc[t]];
+    ax = ax + adj[3 * r] * hl;
+    ay = ay + adj[3 * r + 1] * hl;
+    az = az + adj[3 * r + 2] * hl;
+  }
+  accel[3 * g] = ax;
+  accel[3 * g + 1] = ay;
+  accel[3 * g + 2] = az;
 }
 
 // compute_add_sources_acoustic.f90:205-235 (adjoint sources in fluid elements):
 // chi'' += adj(1, irec) * hxi heta hgamma, the product of the CUSTOM_REAL interpolants, added as is
 // (no 1/kappa, positive sign)
-__global__ void k_adjoint_sources_ac(int n, const int* __restrict__ ig, const int* __restrict__ owner,
-                                     const int* __restrict__ ploc, const realw* __restrict__ h,
-                                     const realw* __restrict__ adj, realw* potdd) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int g = ig[t];
-  const int r = owner[t];
-  potdd[g] = potdd[g] + adj[3 * r] * h[(int64_t)r * 125 + ploc[t]];
+__global__ void k_adjoint_sources_ac(int n0, const int* __restrict__ ig, const int* __restrict__ owner,
+                                     const int* __restrict__ ploc, const int* __restrict__ next,
+                                     const realw* __restrict__ h, const realw* __restrict__ adj, realw* potdd) {
+  const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t0 >= n0) return;
+  const int g = ig[t0];
+  realw a = potdd[g];
+  for (int t = t0; t >= 0; t = next[t]) {
+    const int r = owner[t];
+    a = a + adj[3 * r] * h[(int64_t)r * 125 + ploc[t]];
+  }
+  potdd[g] = a;
 }
 
 // receiver interpolation (compute_interpolated_dva.f90:84-100): double-precision sum of
@@ -93,43 +115,35 @@ __global__ void __launch_bounds__(64) k_seismo_el(int n, const int* __restrict__
 }
 
 void launch_add_sources_el(hipStream_t s, const FacePoints& f, const realw* arr, const realw* stf, realw* accel) {
-  for (int r = 0; r < f.nrounds; r++) {
-    const int o = f.round_off[r], cnt = f.round_off[r + 1] - o;
-    if (cnt <= 0) continue;
-    hipLaunchKernelGGL(k_add_sources_el, sf_grid(cnt, 128), dim3(128), 0, s, cnt, f.iglob + o, f.ispec + o,
-                       f.ploc + o, arr, stf, accel);
-  }
+  const int n0 = f.points();
+  if (n0 <= 0) return;
+  hipLaunchKernelGGL(k_add_sources_el, sf_grid(n0, 128), dim3(128), 0, s, n0, f.iglob, f.ispec, f.ploc, f.next,
+                     arr, stf, accel);
   SF_LAUNCH_CHECK("k_add_sources_el");
 }
 
 void launch_add_sources_ac(hipStream_t s, const FacePoints& f, const realw* arr, const realw* kappa,
                            const realw* stf, realw* potdd) {
-  for (int r = 0; r < f.nrounds; r++) {
-    const int o = f.round_off[r], cnt = f.round_off[r + 1] - o;
-    if (cnt <= 0) continue;
-    hipLaunchKernelGGL(k_add_sources_ac, sf_grid(cnt, 128), dim3(128), 0, s, cnt, f.iglob + o, f.ispec + o,
-                       f.ploc + o, arr, kappa, stf, potdd);
-  }
+  const int n0 = f.points();
+  if (n0 <= 0) return;
+  hipLaunchKernelGGL(k_add_sources_ac, sf_grid(n0, 128), dim3(128), 0, s, n0, f.iglob, f.ispec, f.ploc, f.next,
+                     arr, kappa, stf, potdd);
   SF_LAUNCH_CHECK("k_add_sources_ac");
 }
 
 void launch_adjoint_sources_el(hipStream_t s, const FacePoints& f, const realw* h, const realw* adj, realw* accel) {
-  for (int r = 0; r < f.nrounds; r++) {
-    const int o = f.round_off[r], cnt = f.round_off[r + 1] - o;
-    if (cnt <= 0) continue;
-    hipLaunchKernelGGL(k_adjoint_sources_el, sf_grid(cnt, 128), dim3(128), 0, s, cnt, f.iglob + o, f.ispec + o,
-                       f.ploc + o, h, adj, accel);
-  }
+  const int n0 = f.points();
+  if (n0 <= 0) return;
+  hipLaunchKernelGGL(k_adjoint_sources_el, sf_grid(n0, 128), dim3(128), 0, s, n0, f.iglob, f.ispec, f.ploc, f.next,
+                     h, adj, accel);
   SF_LAUNCH_CHECK("k_adjoint_sources_el");
 }
 
 void launch_adjoint_sources_ac(hipStream_t s, const FacePoints& f, const realw* h, const realw* adj, realw* potdd) {
-  for (int r = 0; r < f.nrounds; r++) {
-    const int o = f.round_off[r], cnt = f.round_off[r + 1] - o;
-    if (cnt <= 0) continue;
-    hipLaunchKernelGGL(k_adjoint_sources_ac, sf_grid(cnt, 128), dim3(128), 0, s, cnt, f.iglob + o, f.ispec + o,
-                       f.ploc + o, h, adj, potdd);
-  }
+  const int n0 = f.points();
+  if (n0 <= 0) return;
+  hipLaunchKernelGGL(k_adjoint_sources_ac, sf_grid(n0, 128), dim3(128), 0, s, n0, f.iglob, f.ispec, f.ploc, f.next,
+                     h, adj, potdd);
   SF_LAUNCH_CHECK("k_adjoint_sources_ac");
 }
 

@@ -248,18 +248,14 @@ void launch_acoustic(hipStream_t s, const AcousticArgs& a, bool exact);
 
 
 // boundary terms (k_boundary.hip)
-// atomic: one launch with float atomics instead of one launch per round (used when the element
-// stiffness scatters with atomics, so the sums have no fixed order anyway)
 void launch_stacey_elastic(hipStream_t s, const FacePoints& f, const realw* veloc, realw* accel, realw* b_absorb,
-                           int mode, bool atomic);
+                           int mode);
 void launch_stacey_elastic_replay(hipStream_t s, const FacePoints& f, const realw* rec, realw* b_accel);
 void launch_stacey_acoustic(hipStream_t s, const FacePoints& f, const realw* potd, realw* potdd, realw* b_absorb,
-                            int mode, bool atomic);
+                            int mode);
 void launch_stacey_acoustic_replay(hipStream_t s, const FacePoints& f, const realw* rec, realw* b_potdd);
-void launch_coupling_ac_el(hipStream_t s, const FacePoints& f, const realw* displ, realw* potdd, int flip,
-                           bool atomic);
-void launch_coupling_el_ac(hipStream_t s, const FacePoints& f, const realw* potdd, realw* accel, int flip,
-                           bool atomic);
+void launch_coupling_ac_el(hipStream_t s, const FacePoints& f, const realw* displ, realw* potdd, int flip);
+void launch_coupling_el_ac(hipStream_t s, const FacePoints& f, const realw* potdd, realw* accel, int flip);
 void launch_free_surface(hipStream_t s, const FacePoints& f, realw* pot, realw* potd, realw* potdd);
 
 // sources / receivers (k_sources.hip); FacePoints.ispec holds the owning source / receiver

@@ -52,12 +52,13 @@ struct FacePoints {          // flattened boundary/coupling face points
   realw* imp_p = nullptr;    // rho*vp (elastic Stacey) or 1/(rho*c) factor (acoustic)
   realw* imp_s = nullptr;    // rho*vs (elastic Stacey)
   // Points are sorted into "rounds": round r holds the r-th occurrence of each global point in
-  // the host's face order, so one launch per round can update without atomics and the sum at
-  // shared edge/corner points keeps the reference's face order.
+  // the host's face order. A lane per point of round 0 that follows `next` updates without atomics, and
+  // the sum at shared edge/corner points keeps the reference's face order.
   int nrounds = 0;
   int round_off[17] = {0};
   int* slot = nullptr;       // original host slot (face*25 + igll) of each point, for records
   int* next = nullptr;       // index of the same global point's next occurrence (next round), -1 after the last
+  int points() const { return nrounds > 0 ? round_off[1] : 0; }  // distinct global points
 };
 
 struct Snapshot {            // one saved state of a wavefield (save_forward_arrays_undoatt)
