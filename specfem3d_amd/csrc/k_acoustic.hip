@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(128) k_acoustic(AcousticArgs A, GLLk G) {
 #pragma unroll
       for (int k = 0; k < 5; k++) sA[el * 125 + c + 25 * k] = chi[k];
     }
-    line_gradient(G.hp, chi, d3);
+    line_gradient(G, chi, d3);
   }
   lds_barrier();
   const int bx = el * 125 + 5 * c, by = el * 125 + i + 25 * j;  // first points of the lane's two rows
@@ -73,8 +73,8 @@ __global__ void __launch_bounds__(128) k_acoustic(AcousticArgs A, GLLk G) {
       r[l] = sA[bx + l];
       y[l] = sA[by + 5 * l];
     }
-    line_gradient(G.hp, r, x);
-    line_gradient(G.hp, y, r);
+    line_gradient(G, r, x);
+    line_gradient(G, y, r);
     if (lane) {
 #pragma unroll
       for (int l = 0; l < 5; l++) sB[by + 5 * l] = r[l];
@@ -119,17 +119,17 @@ __global__ void __launch_bounds__(128) k_acoustic(AcousticArgs A, GLLk G) {
       r[l] = sA[bx + l];
       y[l] = sB[by + 5 * l];
     }
-    line_divergence(G.hpw, r, o);
+    line_divergence(G, r, o);
     if (lane) {
 #pragma unroll
       for (int l = 0; l < 5; l++) sA[bx + l] = o[l];
     }
-    line_divergence(G.hpw, y, o);
+    line_divergence(G, y, o);
     if (lane) {
 #pragma unroll
       for (int l = 0; l < 5; l++) sB[by + 5 * l] = o[l];
     }
-    line_divergence(G.hpw, d3, o);
+    line_divergence(G, d3, o);
 #pragma unroll
     for (int k = 0; k < 5; k++) d3[k] = o[k];
   }

@@ -114,13 +114,13 @@ __global__ void __launch_bounds__(32 * SC) k_elastic_batch(BatchArgs B, GLLk G) 
         y[l] = sA[by + 5 * PS * l + SC * a];
         z[l] = sA[bp + 25 * PS * l + SC * a];
       }
-      line_gradient(G.hp, r, x[a]);
-      line_gradient(G.hp, y, r);
+      line_gradient(G, r, x[a]);
+      line_gradient(G, y, r);
       if (lane) {
 #pragma unroll
         for (int l = 0; l < 5; l++) sB[by + 5 * PS * l + SC * a] = r[l];
       }
-      line_gradient(G.hp, z, r);
+      line_gradient(G, z, r);
 #pragma unroll
       for (int k = 0; k < 5; k++) d3[k][a] = r[k];
     }
@@ -165,19 +165,19 @@ __global__ void __launch_bounds__(32 * SC) k_elastic_batch(BatchArgs B, GLLk G) 
       r[l] = sA[bx + PS * l + SC * a];
       y[l] = sB[by + 5 * PS * l + SC * a];
     }
-    line_divergence(G.hpw, r, o);
+    line_divergence(G, r, o);
     if (lane) {
 #pragma unroll
       for (int l = 0; l < 5; l++) sA[bx + PS * l + SC * a] = o[l];
     }
-    line_divergence(G.hpw, y, o);
+    line_divergence(G, y, o);
     if (lane) {
 #pragma unroll
       for (int l = 0; l < 5; l++) sB[by + 5 * PS * l + SC * a] = o[l];
     }
 #pragma unroll
     for (int k = 0; k < 5; k++) r[k] = d3[k][a];
-    line_divergence(G.hpw, r, o);
+    line_divergence(G, r, o);
 #pragma unroll
     for (int k = 0; k < 5; k++) d3[k][a] = o[k];
   }
@@ -498,13 +498,7 @@ void SFX(launch_elastic_batch)(hipStream_t st, const BatchArgs& a, int sc) {
   if (a.nelem <= 0 || a.ngroups <= 0) return;
   const bool reg = a.jac_plane == 0;
   GLLk G = g_gll_host;
-  if (reg && SF_FOLD) {
-    fold_gll(G, a.xix_regular, a.jacobian_regular);
-    for (int q = 0; q < 25; q++) {
-      G.hp[q] = G.hpr[q];
-      G.hpw[q] = G.hpwr[q];
-    }
-  }
+  if (reg && SF_FOLD) regular_gll(G, a.xix_regular, a.jacobian_regular);
   const int64_t nb = (int64_t)a.nelem * a.ngroups;
   if (nb > 0x7fffffff) fatal("launch_elastic_batch", "grid too large");
 #define SF_KB(SC, R) hipLaunchKernelGGL((k_elastic_batch<SC, R>), dim3((unsigned)nb), dim3(32 * SC), 0, st, a, G)

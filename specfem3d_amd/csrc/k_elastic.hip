@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk G) {
         for (int k = 0; k < 5; k++) sA[a][b + 25 * k] = u[a][k];
       }
       realw r[5];
-      line_gradient(G.hp, u[a], r);
+      line_gradient(G, u[a], r);
 #pragma unroll
       for (int k = 0; k < 5; k++) d3[k][a] = r[k];
     }
@@ -303,8 +303,8 @@ __global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk G) {
       r[l] = sA[a][bx + l];
       y[l] = sA[a][by + 5 * l];
     }
-    line_gradient(G.hp, r, x[a]);
-    line_gradient(G.hp, y, r);
+    line_gradient(G, r, x[a]);
+    line_gradient(G, y, r);
     if (lane) {
 #pragma unroll
       for (int l = 0; l < 5; l++) sB[a][by + 5 * l] = r[l];
@@ -363,19 +363,19 @@ __global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk G) {
       r[l] = sA[a][bx + l];
       y[l] = sB[a][by + 5 * l];
     }
-    line_divergence(G.hpw, r, o);
+    line_divergence(G, r, o);
     if (lane) {
 #pragma unroll
       for (int l = 0; l < 5; l++) sA[a][bx + l] = o[l];
     }
-    line_divergence(G.hpw, y, o);
+    line_divergence(G, y, o);
     if (lane) {
 #pragma unroll
       for (int l = 0; l < 5; l++) sB[a][by + 5 * l] = o[l];
     }
 #pragma unroll
     for (int k = 0; k < 5; k++) r[k] = d3[k][a];
-    line_divergence(G.hpw, r, o);
+    line_divergence(G, r, o);
 #pragma unroll
     for (int k = 0; k < 5; k++) d3[k][a] = o[k];
   }
@@ -477,7 +477,7 @@ using namespace SF_VNS;
 void SFX(launch_elastic)(hipStream_t s, const ElasticArgs& a, bool strain, bool att, int att_variant) {
   if (a.nelem <= 0) return;
   GLLk G = g_gll_host;
-  if (SF_FOLD) fold_gll(G, a.xix_regular, a.jacobian_regular);
+  if (att && SF_FOLD) fold_gll(G, a.xix_regular, a.jacobian_regular);
   dim3 grid(a.nelem), block(128);
 #define SF_K(V) hipLaunchKernelGGL((k_elastic_pt<V>), grid, block, 0, s, a, G)
   if (att) {
@@ -488,12 +488,7 @@ void SFX(launch_elastic)(hipStream_t s, const ElasticArgs& a, bool strain, bool 
     else SF_K(0);
   } else {
     const bool reg = a.jac_plane == 0;  // no irregular element in the mesh
-    if (reg && SF_FOLD) {
-      for (int q = 0; q < 25; q++) {
-        G.hp[q] = G.hpr[q];
-        G.hpw[q] = G.hpwr[q];
-      }
-    }
+    if (reg && SF_FOLD) regular_gll(G, a.xix_regular, a.jacobian_regular);
     const dim3 grid5((a.nelem + 4) / 5);
 #define SF_L(S, R) hipLaunchKernelGGL((k_elastic_line<S, R>), grid5, block, 0, s, a, G)
     if (strain) {

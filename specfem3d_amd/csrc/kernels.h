@@ -22,12 +22,35 @@ struct GLLk {
   // fold the regular mapping and the jacobian weight into the contractions (fold_gll)
   realw hpr[25];
   realw hpwr[25];
+  // FMA builds, line_gradient and line_divergence: sum over l of hp[m, l] and of hpw[l, m]
+  realw hs[5], hws[5];
 };
+// hs and hws from the tables and the factors folded into them
+inline void sum_gll(GLLk& G, double fg, double fd) {
+  for (int m = 0; m < 5; m++) {
+    double g = 0, d = 0;
+    for (int l = 0; l < 5; l++) {
+      g += G.hp[m * 5 + l];
+      d += G.hpw[l * 5 + m];
+    }
+    G.hs[m] = (realw)(fg * g);
+    G.hws[m] = (realw)(fd * d);
+  }
+}
 inline void fold_gll(GLLk& G, realw xix_regular, realw jacobian_regular) {
   const realw jx = jacobian_regular * xix_regular;
   for (int q = 0; q < 25; q++) {
     G.hpr[q] = G.hp[q] * xix_regular;
     G.hpwr[q] = G.hpw[q] * jx;
+  }
+}
+// the tables of a launch over regular elements alone: the folded ones in the place of the others
+inline void regular_gll(GLLk& G, realw xix_regular, realw jacobian_regular) {
+  fold_gll(G, xix_regular, jacobian_regular);
+  sum_gll(G, xix_regular, (double)jacobian_regular * xix_regular);
+  for (int q = 0; q < 25; q++) {
+    G.hp[q] = G.hpr[q];
+    G.hpw[q] = G.hpwr[q];
   }
 }
 extern GLLk g_gll_host;
