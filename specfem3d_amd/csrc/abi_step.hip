@@ -593,6 +593,21 @@ extern "C" void FC_FUNC_(compute_coupling_el_ac_cuda, COMPUTE_COUPLING_EL_AC_CUD
 }
 
 // ---------------------------------------------------------------- sources
+// the n values of a launch's sources (`prepared`: as many as its lists may name); more than fit its
+// arguments go to `buffer` on the device
+static SrcVals source_values(Mesh* m, const realw* vals, int n, int prepared, realw* (*buffer)(Mesh*, int)) {
+  SrcVals s;
+  s.p = nullptr;
+  if (std::max(n, prepared) <= SF_SRC_VALS) {
+    std::memcpy(s.v, vals, sizeof(realw) * (size_t)n);
+    std::fill(s.v + n, s.v + SF_SRC_VALS, 0.f);
+  } else {
+    s.p = stage_to_device(m, vals, n, buffer(m, n));
+  }
+  return s;
+}
+static realw* adj_device_buffer(Mesh* m, int) { return m->adj_src; }
+
 // compute_add_sources_viscoelastic_cuda.cu:39; stf_used = real(stf) per source (double on the host)
 static void add_sources_el(Mesh* m, int f, const double* h_stf, int nsrc) {
   if (m->src_pts.n == 0 || nsrc <= 0) return;
@@ -604,9 +619,8 @@ static void add_sources_el(Mesh* m, int f, const double* h_stf, int nsrc) {
   }
   if (!any) return;  // as the reference's GPU wrapper: nothing to add when all STFs are zero
   flush_el(m, f);
-  realw* d = stf_device_buffer(m, nsrc);
-  stage_to_device(m, s.data(), nsrc, d);
-  launch_add_sources_el(m->stream, m->src_pts, m->src_array, d, m->el[f].accel);
+  launch_add_sources_el(m->stream, m->src_pts, m->src_array, source_values(m, s.data(), nsrc, m->nsources, stf_device_buffer),
+                        m->el[f].accel);
 }
 
 extern "C" void FC_FUNC_(compute_add_sources_el_cuda, COMPUTE_ADD_SOURCES_EL_CUDA)(long* Mesh_pointer,
@@ -638,8 +652,8 @@ extern "C" void FC_FUNC_(add_sources_el_sim_type_2_or_3, ADD_SOURCES_EL_SIM_TYPE
   const int isample = nt - ((*it - 1) % nt);  // 1-based
   const realw* src = h_source_adjoint + (int64_t)3 * nadj * (isample - 1);
   flush_el(m, 0);
-  stage_to_device(m, src, 3 * nadj, m->adj_src);
-  launch_adjoint_sources_el(m->stream, m->adj_pts, m->adj_h, m->adj_src, m->el[0].accel);
+  launch_adjoint_sources_el(m->stream, m->adj_pts, m->adj_h, source_values(m, src, 3 * nadj, 3 * m->nadj_rec_local, adj_device_buffer),
+                            m->el[0].accel);
 }
 
 // compute_add_sources_acoustic_cuda.cu: sources in acoustic elements, chi'' -= sourcearray(1) stf / kappa
@@ -652,9 +666,8 @@ static void add_sources_ac(Mesh* m, int f, const double* h_stf, int nsrc, const 
   std::vector<realw> s(m->nsources);
   for (int i = 0; i < m->nsources; i++) s[i] = (realw)h_stf[i];
   flush_ac_terms(m, f);
-  realw* d = stf_device_buffer(m, m->nsources);
-  stage_to_device(m, s.data(), m->nsources, d);
-  launch_add_sources_ac(m->stream, m->src_ac_pts, m->src_array, m->src_kappa, d, m->ac[f].potdd);
+  launch_add_sources_ac(m->stream, m->src_ac_pts, m->src_array, m->src_kappa,
+                        source_values(m, s.data(), m->nsources, m->nsources, stf_device_buffer), m->ac[f].potdd);
 }
 
 extern "C" void FC_FUNC_(compute_add_sources_ac_cuda, COMPUTE_ADD_SOURCES_AC_CUDA)(long* Mesh_pointer,
@@ -690,8 +703,8 @@ extern "C" void FC_FUNC_(add_sources_ac_sim_2_or_3_cuda, ADD_SOURCES_AC_SIM_2_OR
   const int isample = nt - ((*it - 1) % nt);  // 1-based
   const realw* src = h_source_adjoint + (int64_t)3 * nadj * (isample - 1);
   flush_ac_terms(m, 0);
-  stage_to_device(m, src, 3 * nadj, m->adj_src);
-  launch_adjoint_sources_ac(m->stream, m->adj_ac_pts, m->adj_h, m->adj_src, m->ac[0].potdd);
+  launch_adjoint_sources_ac(m->stream, m->adj_ac_pts, m->adj_h, source_values(m, src, 3 * nadj, 3 * m->nadj_rec_local, adj_device_buffer),
+                            m->ac[0].potdd);
 }
 
 // ---------------------------------------------------------------- seismograms (write_seismograms_cuda.cu:34)

@@ -281,12 +281,18 @@ void launch_coupling_ac_el(hipStream_t s, const FacePoints& f, const realw* disp
 void launch_coupling_el_ac(hipStream_t s, const FacePoints& f, const realw* potdd, realw* accel, int flip);
 void launch_free_surface(hipStream_t s, const FacePoints& f, realw* pot, realw* potd, realw* potdd);
 
+// values of the sources in one step: as a launch argument where they fit, else in device memory
+constexpr int SF_SRC_VALS = 256;
+struct SrcVals {
+  realw v[SF_SRC_VALS];
+  const realw* p;
+};
 // sources / receivers (k_sources.hip); FacePoints.ispec holds the owning source / receiver
-void launch_add_sources_el(hipStream_t s, const FacePoints& f, const realw* arr, const realw* stf, realw* accel);
+void launch_add_sources_el(hipStream_t s, const FacePoints& f, const realw* arr, const SrcVals& stf, realw* accel);
 void launch_add_sources_ac(hipStream_t s, const FacePoints& f, const realw* arr, const realw* kappa,
-                           const realw* stf, realw* potdd);
-void launch_adjoint_sources_el(hipStream_t s, const FacePoints& f, const realw* h, const realw* adj, realw* accel);
-void launch_adjoint_sources_ac(hipStream_t s, const FacePoints& f, const realw* h, const realw* adj, realw* potdd);
+                           const SrcVals& stf, realw* potdd);
+void launch_adjoint_sources_el(hipStream_t s, const FacePoints& f, const realw* h, const SrcVals& adj, realw* accel);
+void launch_adjoint_sources_ac(hipStream_t s, const FacePoints& f, const realw* h, const SrcVals& adj, realw* potdd);
 // receivers: `list` holds the local receiver indices to record (n of them; null: receivers 0..n-1);
 // out[3 r + c] is written for each listed receiver r
 void launch_seismo_el(hipStream_t s, int n, const int* list, const int* iglob, const double* h, const double* nu,

@@ -110,3 +110,27 @@ def test_potentials_between_steps(oracle_mod, n, warp):
                 for x, y in zip(g.potentials(), (o.pot, o.potd, o.potdd)):
                     assert np.array_equal(x, y), (every, k)
         g.close()
+
+
+@pytest.mark.parametrize("nsrc", [1, 256, 257])
+def test_source_values(oracle_mod, nsrc):
+    """Source time functions as launch arguments (up to 256) and through device memory, sources of
+    neighbouring elements adding to shared points in the reference's order."""
+    from specfem3d_amd import sources as S
+    from specfem3d_amd.solver import GPUSolver
+    n, dt = 7, 0.004
+    db, _, rec = small_elastic_box(n=n, dt=dt)
+    L = 500.0 * n
+    cmt = []
+    for q in range(nsrc):
+        e = (q * 2) % 343
+        x, y, z = (0.5 + e % 7) * 500.0, (0.5 + (e // 7) % 7) * 500.0, (0.5 + e // 49) * 500.0
+        cmt.append(S.CMTSource(x, y, z / 1000.0, 0.0, 0.05 + 1e-4 * q, 1e13, 1e13 + q * 1e10, -1e13, 0.0, 1e12, 0.0))
+    src = S.setup_cmt_sources(db, cmt, dt)
+    assert src.n == nsrc and x < L
+    ref = oracle_mod.OracleSolver(db, src, rec, "f32").run(12)
+    g = GPUSolver(db, src, rec, nstep=12, exact=True, assembly=1)
+    print(f"[gpu] {nsrc} sources", flush=True)
+    out = g.run().copy()
+    g.close()
+    assert np.abs(ref).max() > 0 and np.array_equal(out, ref)
