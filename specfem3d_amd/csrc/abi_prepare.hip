@@ -779,6 +779,8 @@ void ensure_gather_assembly(Mesh* m, int f) {
   for (const FacePoints* fp : {&m->abs_el, &m->coupling, &m->src_pts, &m->adj_pts})
     launch_mark_points(m->stream, fp->n, fp->iglob, AF_TERM, m->asm_info);
   launch_mark_points(m->stream, m->pml_nbc, m->pml_bc_pts, AF_EDGE, m->asm_info);
+  if (!m->asm_rec) m->asm_rec = dmalloc<int>(125 * (int64_t)m->nrec_local);
+  launch_pick(m->stream, 125 * (int64_t)m->nrec_local, m->rec_iglob, ptr, m->asm_rec);
   dfree(ptr);
   m->asm_ready = 1;
 }
@@ -791,6 +793,7 @@ void release_gather_assembly(Mesh* m) {
   dfree(m->asm_idx);
   dfree(m->asm_info);
   dfree(m->asm_base);
+  dfree(m->asm_rec);
   dfree(m->rmass1);
   dfree(m->asm_buf[0]);
   dfree(m->asm_buf[1]);
@@ -798,6 +801,7 @@ void release_gather_assembly(Mesh* m) {
   dfree(m->asm_ac_idx);
   dfree(m->asm_ac_info);
   dfree(m->asm_ac_base);
+  dfree(m->asm_ac_rec);
   dfree(m->asm_ac_buf[0]);
   dfree(m->asm_ac_buf[1]);
   m->asm_ac_ready = 0;
@@ -823,6 +827,8 @@ void ensure_gather_acoustic(Mesh* m, int f) {
   for (const FacePoints* fp : {&m->abs_ac, &m->coupling, &m->src_ac_pts, &m->adj_ac_pts})
     launch_mark_points(m->stream, fp->n, fp->iglob, AF_TERM, m->asm_ac_info);
   launch_mark_points(m->stream, m->free_ac.n, m->free_ac.iglob, AF_EDGE, m->asm_ac_info);
+  if (!m->asm_ac_rec) m->asm_ac_rec = dmalloc<int>(125 * (int64_t)m->nrec_local);
+  launch_pick(m->stream, 125 * (int64_t)m->nrec_local, m->rec_iglob, ptr, m->asm_ac_rec);
   dfree(ptr);
   m->asm_ac_ready = 1;
 }
@@ -1242,11 +1248,11 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
   dfree(m->rec_ispec); dfree(m->rec_el_list); dfree(m->rec_ac_list);
   dfree(m->seismo_d); dfree(m->seismo_v); dfree(m->seismo_a); dfree(m->seismo_p);
   dfree(m->rho_kl); dfree(m->mu_kl); dfree(m->kappa_kl); dfree(m->rho_ac_kl); dfree(m->kappa_ac_kl);
-  dfree(m->asm_idx); dfree(m->asm_info); dfree(m->asm_base); dfree(m->rmass1); dfree(m->asm_buf[0]); dfree(m->asm_buf[1]);
+  dfree(m->asm_idx); dfree(m->asm_info); dfree(m->asm_base); dfree(m->asm_rec); dfree(m->rmass1); dfree(m->asm_buf[0]); dfree(m->asm_buf[1]);
   dfree(m->pml_elems); dfree(m->pml_cpml);
   dfree(m->pml_state); dfree(m->pml_coef); dfree(m->pml_masks); dfree(m->pml_off);
   dfree(m->pml_old); dfree(m->pml_pts); dfree(m->pml_bc_pts);
-  dfree(m->asm_ac_idx); dfree(m->asm_ac_info); dfree(m->asm_ac_base); dfree(m->asm_ac_buf[0]); dfree(m->asm_ac_buf[1]);
+  dfree(m->asm_ac_idx); dfree(m->asm_ac_info); dfree(m->asm_ac_base); dfree(m->asm_ac_rec); dfree(m->asm_ac_buf[0]); dfree(m->asm_ac_buf[1]);
   dfree(m->d_norm);
   if (m->h_norm) (void)hipHostFree(m->h_norm);
   if (m->timing_ev) {

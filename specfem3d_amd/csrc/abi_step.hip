@@ -725,19 +725,32 @@ extern "C" void FC_FUNC_(compute_seismograms_cuda, COMPUTE_SEISMOGRAMS_CUDA)(
   const int64_t off = (int64_t)(cur - 1) * m->nrec_local * 3;
   if (m->nrec_el > 0) {
     if (!m->el[f].displ) fatal("compute_seismograms_cuda", "elastic field not prepared");
-    if (m->save_v || m->save_a) flush_el(m, f);
     const Wavefield& w = m->el[f];
-    if (m->save_d) launch_seismo_el(m->stream, m->nrec_el, m->rec_el_list, m->rec_iglob, m->rec_h, m->rec_nu, w.displ, m->seismo_d + off);
-    if (m->save_v) launch_seismo_el(m->stream, m->nrec_el, m->rec_el_list, m->rec_iglob, m->rec_h, m->rec_nu, w.veloc, m->seismo_v + off);
-    if (m->save_a) launch_seismo_el(m->stream, m->nrec_el, m->rec_el_list, m->rec_iglob, m->rec_h, m->rec_nu, w.accel, m->seismo_a + off);
+    const bool wait = m->pending_gather_el[f] && m->pending_k3_el[f];  // records need no flush
+    if ((m->save_v || m->save_a) && !wait) flush_el(m, f);
+    auto record = [&](const realw* field, int what, realw* out) {
+      if (wait && what != WAIT_NONE)
+        launch_seismo_el_waiting(m->stream, m->nrec_el, m->rec_el_list, m->rec_iglob, m->rec_h, m->rec_nu,
+                                 gather_args(m, f), m->asm_rec, what, m->exact != 0, out);
+      else
+        launch_seismo_el(m->stream, m->nrec_el, m->rec_el_list, m->rec_iglob, m->rec_h, m->rec_nu, field, out);
+    };
+    if (m->save_d) record(w.displ, WAIT_NONE, m->seismo_d + off);
+    if (m->save_v) record(w.veloc, WAIT_VELOC, m->seismo_v + off);
+    if (m->save_a) record(w.accel, WAIT_ACCEL, m->seismo_a + off);
   }
   if (m->nrec_ac > 0) {
     // receivers in fluid elements (write_seismograms_cuda.cu: seismotype 1-3 from the gradient of the
     // potentials, 4 = pressure from the potential with the pressure trick, else its second derivative)
     const AcField& a = m->ac[fa];
     if (!a.pot) fatal("compute_seismograms_cuda", "acoustic field not prepared");
-    if (m->save_v || m->save_a || (m->save_p && !trick)) flush_ac(m, fa);
+    const bool wait = m->pending_gather_ac[fa] && m->pending_k3_ac[fa];
+    if ((m->save_v || m->save_a || (m->save_p && !trick)) && !wait) flush_ac(m, fa);
+    const int veloc = wait ? WAIT_VELOC : WAIT_NONE, accel = wait ? WAIT_ACCEL : WAIT_NONE;
     AcReceiverArgs ra;
+    ra.wait = gather_args_ac(m, fa);
+    ra.first = m->asm_ac_rec;
+    ra.exact = m->exact;
     ra.n = m->nrec_ac;
     ra.list = m->rec_ac_list;
     ra.rec_ispec = m->rec_ispec;
@@ -749,10 +762,11 @@ extern "C" void FC_FUNC_(compute_seismograms_cuda, COMPUTE_SEISMOGRAMS_CUDA)(
     ra.jac = m->jac;
     ra.jac_plane = (int64_t)m->nspec_irregular * 125;
     ra.rho = m->rho;
-    if (m->save_d) launch_seismo_ac(m->stream, ra, a.pot, 0, m->seismo_d + off);
-    if (m->save_v) launch_seismo_ac(m->stream, ra, a.potd, 0, m->seismo_v + off);
-    if (m->save_a) launch_seismo_ac(m->stream, ra, a.potdd, 0, m->seismo_a + off);
-    if (m->save_p) launch_seismo_ac(m->stream, ra, trick ? a.pot : a.potdd, 1, m->seismo_p + off);
+    if (m->save_d) launch_seismo_ac(m->stream, ra, a.pot, WAIT_NONE, 0, m->seismo_d + off);
+    if (m->save_v) launch_seismo_ac(m->stream, ra, a.potd, veloc, 0, m->seismo_v + off);
+    if (m->save_a) launch_seismo_ac(m->stream, ra, a.potdd, accel, 0, m->seismo_a + off);
+    if (m->save_p)
+      launch_seismo_ac(m->stream, ra, trick ? a.pot : a.potdd, trick ? WAIT_NONE : accel, 1, m->seismo_p + off);
   }
   if (cur == *nlength_seismogramf || *itf == *it_endf) {
     // host arrays seismograms_?(NDIM, nrec_local, nlength); pressure in component 1, the others zero

@@ -177,6 +177,11 @@ __global__ void k_gather_info(int64_t g0, int64_t n, const int* __restrict__ ptr
   if (t % 64 == 0) base[t / 64] = ptr[g];
 }
 
+__global__ void k_pick(int64_t n, const int* __restrict__ ig, const int* __restrict__ ptr, int* __restrict__ out) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) out[t] = ptr[ig[t]];
+}
+
 template <typename T>
 static T* alloc_dev(int64_t n) {
   void* p = nullptr;
@@ -230,6 +235,12 @@ void launch_mark_points(hipStream_t s, int n, const int* ig, uint16_t bit, uint1
   if (n <= 0) return;
   hipLaunchKernelGGL(k_mark_points, sf_grid(n, 256), dim3(256), 0, s, n, ig, bit, info);
   SF_LAUNCH_CHECK("k_mark_points");
+}
+
+void launch_pick(hipStream_t s, int64_t n, const int* ig, const int* ptr, int* out) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_pick, sf_grid(n, 256), dim3(256), 0, s, n, ig, ptr, out);
+  SF_LAUNCH_CHECK("k_pick");
 }
 
 void launch_gather_info(hipStream_t s, int64_t g0, int64_t n, const int* ptr, const realw* rm, uint16_t* info,

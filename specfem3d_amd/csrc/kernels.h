@@ -99,6 +99,28 @@ struct GatherArgs {
 // what follows the sum: nothing (accel is left assembled), the corrector, or the corrector and the
 // predictor of the next step (accel left zero)
 enum { GATHER_ONLY = 0, GATHER_CORRECT = 1, GATHER_STEP = 2 };
+// the acceleration or velocity that sum and corrector will give one point, from its slots at idx[first]
+// on: for the receivers, which record a few points while the whole field waits for the next update. The
+// operations are those of k_gather_update.
+enum { WAIT_NONE = 0, WAIT_ACCEL = 1, WAIT_VELOC = 2 };
+template <int NC, typename T>
+__device__ __forceinline__ void waiting_value(const GatherArgs& A, int what, int64_t g, int first, realw out[NC]) {
+  const int fl = A.info[g], cnt = fl >> AF_COUNT;
+  const bool zero = fl & A.skip, full = !A.clean || (fl & AF_TERM);
+  T a[NC];
+#pragma unroll
+  for (int c = 0; c < NC; c++) a[c] = full && !zero ? A.a[NC * g + c] : 0.f;
+  for (int s = 0; s < (zero ? 0 : cnt); s++) {
+    const realw* l = A.local + NC * (int64_t)A.idx[first + s];
+#pragma unroll
+    for (int c = 0; c < NC; c++) a[c] = a[c] + (-(T)l[c]);
+  }
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    a[c] = a[c] * (T)(NC == 3 && (fl & AF_MASS3) ? A.rm[NC * g + c] : A.rm1[g]);
+    out[c] = what == WAIT_ACCEL ? (realw)a[c] : (realw)((T)A.v[NC * g + c] + (T)A.dt2p * a[c]);
+  }
+}
 // exact: the reference's single-precision operations; else sums, corrector and predictor in double
 // precision, rounded once per stored value
 void launch_gather_update(hipStream_t s, const GatherArgs& a, int ncomp, int kind, bool exact);
@@ -111,6 +133,8 @@ int build_slot_lists(hipStream_t s, int nglob, int nspec, int nelem, const int* 
 void launch_mark_points(hipStream_t s, int n, const int* ig, uint16_t bit, uint16_t* info);
 // info (flags to be marked afterwards), base and rm1 of GatherArgs from the slot lists and the masses;
 // rm null: one mass per point, rm1 is not written
+// out[t] = ptr[ig[t]] (first slot entry of the receivers' points)
+void launch_pick(hipStream_t s, int64_t n, const int* ig, const int* ptr, int* out);
 void launch_gather_info(hipStream_t s, int64_t g0, int64_t n, const int* ptr, const realw* rm, uint16_t* info,
                         int* base, realw* rm1);
 
@@ -297,6 +321,10 @@ void launch_adjoint_sources_ac(hipStream_t s, const FacePoints& f, const realw* 
 // out[3 r + c] is written for each listed receiver r
 void launch_seismo_el(hipStream_t s, int n, const int* list, const int* iglob, const double* h, const double* nu,
                       const realw* field, realw* out);
+// ... of a field that waits to be summed (`what`: WAIT_*; first: slot entry of every receiver point)
+void launch_seismo_el_waiting(hipStream_t s, int n, const int* list, const int* iglob, const double* h,
+                              const double* nu, const GatherArgs& a, const int* first, int what, bool exact,
+                              realw* out);
 // receivers in acoustic elements: pressure = 1 records -sum h field into out[3 r] (out[3 r + 1..2] = 0),
 // pressure = 0 the vector (1/rho) grad(field) interpolated and rotated by nu
 struct AcReceiverArgs {
@@ -311,8 +339,11 @@ struct AcReceiverArgs {
   const realw* jac;
   int64_t jac_plane;
   const realw* rho;        // rhostore, nloc
+  GatherArgs wait;         // ... of a field that waits to be summed
+  const int* first;        // slot entry of every receiver point
+  int exact;
 };
-void launch_seismo_ac(hipStream_t s, const AcReceiverArgs& a, const realw* field, int pressure, realw* out);
+void launch_seismo_ac(hipStream_t s, const AcReceiverArgs& a, const realw* field, int what, int pressure, realw* out);
 
 // kernels / norms (k_kernels.hip)
 void launch_compute_kernels_el(hipStream_t s, int nelem, const int* elems, const int* ibool, const realw* accel,

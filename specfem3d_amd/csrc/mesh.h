@@ -221,6 +221,7 @@ struct Mesh {
   int* asm_base = nullptr;         // first slot entry of each 64 points of the elastic range
   realw* rmass1 = nullptr;         // inverse mass of the points whose three are equal (nglob)
   realw* asm_buf[2] = {nullptr, nullptr};      // local forces of each field, 3 per slot
+  int* asm_rec = nullptr;          // first slot entry of the receivers' points (125 per receiver)
   int asm_ready = 0;               // lists and flags match the element lists and terms
   // local forces of a field wait to be summed: by the next update together with the corrector, or
   // by whichever entry point reads or writes accel first
@@ -233,6 +234,7 @@ struct Mesh {
   uint16_t* asm_ac_info = nullptr;
   int* asm_ac_base = nullptr;
   realw* asm_ac_buf[2] = {nullptr, nullptr};
+  int* asm_ac_rec = nullptr;
   int asm_ac_ready = 0;
   int pending_gather_ac[2] = {0, 0};
   int gather_skip_ac[2] = {0, 0};
