@@ -19,6 +19,8 @@
 
 namespace sf {
 void flush_all(Mesh* m);
+void flush_field(Mesh* m, int f);
+void flush_ac(Mesh* m, int f);
 
 static inline int field_of_foa(int foa) { return foa == 3 ? 1 : 0; }
 
@@ -134,7 +136,7 @@ extern "C" void sf_history_store(long* Mesh_pointer, int FORWARD_OR_ADJOINT, int
   Mesh* m = from_handle(Mesh_pointer);
   if (frame < 0 || frame >= m->history_frames) fatal("sf_history_store", "frame outside the reserved history");
   const int f = field_of_foa(FORWARD_OR_ADJOINT);
-  flush_all(m);
+  flush_ac(m, f);  // displ and chi are not changed by a waiting sum or corrector
   const int64_t n = m->nglob;
   if (m->history_el && m->el[f].displ) ck_copy(m, m->history_el + (int64_t)frame * 3 * n, m->el[f].displ, 3 * n);
   if (m->history_ac && m->ac[f].pot) {
@@ -148,7 +150,7 @@ extern "C" void sf_history_load(long* Mesh_pointer, int FORWARD_OR_ADJOINT, int 
   Mesh* m = from_handle(Mesh_pointer);
   if (frame < 0 || frame >= m->history_frames) fatal("sf_history_load", "frame outside the reserved history");
   const int f = field_of_foa(FORWARD_OR_ADJOINT);
-  flush_all(m);
+  flush_field(m, f);
   const int64_t n = m->nglob;
   if (m->history_el && m->el[f].displ) ck_copy(m, m->el[f].displ, m->history_el + (int64_t)frame * 3 * n, 3 * n);
   if (m->history_ac && m->ac[f].pot) {

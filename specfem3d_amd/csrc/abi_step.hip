@@ -80,7 +80,7 @@ static GatherArgs gather_args_ac(Mesh* m, int f) {
   return a;
 }
 
-static void flush_ac(Mesh* m, int f) {
+void flush_ac(Mesh* m, int f) {
   int& fz = m->free_zero[f];
   if (m->pending_gather_ac[f]) {
     launch_gather_update(m->stream, gather_args_ac(m, f), 1, m->pending_k3_ac[f] ? GATHER_CORRECT : GATHER_ONLY,
@@ -104,11 +104,13 @@ static void flush_ac_terms(Mesh* m, int f) {
   flush_ac(m, f);
   m->free_zero[f] &= FREE_POT;
 }
+void flush_field(Mesh* m, int f) {
+  flush_el(m, f);
+  flush_ac(m, f);
+}
 void flush_all(Mesh* m) {
-  for (int f = 0; f < 2; f++) {
-    flush_el(m, f);
-    flush_ac(m, f);
-  }
+  flush_field(m, 0);
+  flush_field(m, 1);
 }
 
 static ElasticArgs elastic_args(Mesh* m, int f, realw deltat) {
@@ -335,7 +337,9 @@ extern "C" void FC_FUNC_(compute_forces_viscoelastic_cuda, COMPUTE_FORCES_VISCOE
     check_field(m, f, "compute_forces_viscoelastic_cuda");
     flush_el(m, f);
     if (strain && !m->att[f].eps) fatal("compute_forces_viscoelastic_cuda", "strain arrays not prepared");
-    elastic_forces(m, f, *deltat, strain, att && m->att[f].R != nullptr);
+    // the kernels recompute the strain of a reconstructed field; its memory variables need it stored
+    const bool keep = !(f == 1 && m->undo_attenuation && !m->attenuation);
+    elastic_forces(m, f, *deltat, strain && keep, att && m->att[f].R != nullptr);
   }
 }
 
@@ -791,7 +795,14 @@ extern "C" void FC_FUNC_(compute_kernels_elastic_cuda, COMPUTE_KERNELS_ELASTIC_C
   if (m->undo_attenuation) {
     // the reconstructed strain is recomputed from b_displ (compute_kernels_cuda.cu:57-100)
     ElasticArgs a = elastic_args(m, 1, 0.f);
-    launch_element_strain(m->stream, a, m->att[1].eps, m->eps_trace_over_3[1], m->attenuation != 0, m->exact != 0);
+    if (!m->attenuation) {
+      // nothing else reads it: it need not be stored
+      const KernelSums k = {m->el[0].accel, m->att[0].eps, m->eps_trace_over_3[0], *deltat_f,
+                            m->rho_kl, m->mu_kl, m->kappa_kl};
+      launch_kernels_line(m->stream, a, k, m->exact != 0);
+      return;
+    }
+    launch_element_strain(m->stream, a, m->att[1].eps, m->eps_trace_over_3[1], true, m->exact != 0);
   }
   launch_compute_kernels_el(m->stream, m->nspec_elastic, m->elastic_elems, m->ibool, m->el[0].accel, m->el[1].displ,
                             m->att[0].eps, m->eps_trace_over_3[0], m->att[1].eps, m->eps_trace_over_3[1], nl,

@@ -20,6 +20,8 @@ void launch_elastic_exact(hipStream_t, const ElasticArgs&, bool, bool, int);
 void launch_elastic_fast(hipStream_t, const ElasticArgs&, bool, bool, int);
 void launch_element_strain_exact(hipStream_t, const ElasticArgs&, realw*, realw*, bool);
 void launch_element_strain_fast(hipStream_t, const ElasticArgs&, realw*, realw*, bool);
+void launch_kernels_line_exact(hipStream_t, const ElasticArgs&, const KernelSums&);
+void launch_kernels_line_fast(hipStream_t, const ElasticArgs&, const KernelSums&);
 void launch_elastic_batch_exact(hipStream_t, const BatchArgs&, int);
 void launch_elastic_batch_fast(hipStream_t, const BatchArgs&, int);
 void launch_elastic_pml_exact(hipStream_t, const PmlArgs&);
@@ -74,6 +76,12 @@ void launch_acoustic_batch(hipStream_t s, const BatchAcArgs& a, int sc, bool exa
     launch_acoustic_batch_fast(s, a, sc);
 }
 
+void launch_kernels_line(hipStream_t s, const ElasticArgs& a, const KernelSums& k, bool exact) {
+  if (exact)
+    launch_kernels_line_exact(s, a, k);
+  else
+    launch_kernels_line_fast(s, a, k);
+}
 void launch_acoustic(hipStream_t s, const AcousticArgs& a, bool exact) {
   if (exact)
     launch_acoustic_exact(s, a);

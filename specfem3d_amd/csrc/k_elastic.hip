@@ -393,6 +393,101 @@ __global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk G) {
   }
 }
 
+// Elastic kernels of a run that recomputes the reconstructed field's strain from its displacement
+// (A.displ; compute_kernels.f90:151-186 with the strain of compute_element_strain.F90:28-130): the
+// gradient of k_elastic_line, then per point the sums of k_compute_kernels_el.
+// Bound by HBM: 78 B per local point (index, acceleration, displacement and strain of the adjoint
+// field, three sums read and written). The strain stored by one launch and read back by another
+// took 16.5 + 30 us on 24^3 elements, and 2 us more in every stiffness launch that stored it;
+// this launch takes 26.
+template <bool REG>
+__global__ void __launch_bounds__(128) k_kernels_line(ElasticArgs A, KernelSums S, GLLk G) {
+  constexpr bool FOLD = REG && SF_FOLD;
+  constexpr int PL = 626;
+  __shared__ realw sA[3][PL], sB[3][PL];
+  const int t = threadIdx.x;
+  const bool lane = t < 125;
+  const int el = lane ? t / 25 : 4, c = lane ? t - 25 * el : t - 125;
+  const int i = c % 5, j = c / 5;
+  const int ie = xcd_remap(blockIdx.x, gridDim.x) * 5 + el;
+  const bool active = lane && ie < A.nelem;
+  const int e = A.elems[ie < A.nelem ? ie : A.nelem - 1];
+  const int64_t ep = (int64_t)e * 125 + c;
+  const int irr = REG ? 0 : A.irregular[e];
+  const int64_t jp = REG ? 0 : (int64_t)(irr ? irr - 1 : 0) * 125 + c;
+  realw d3[5][3], dot[5];
+  {
+    realw u[3][5];
+    int g[5];
+#pragma unroll
+    for (int k = 0; k < 5; k++) g[k] = A.ibool[ep + 25 * k];
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+      const realw* d = A.displ + 3 * (int64_t)g[k];
+      const realw* a = S.accel + 3 * (int64_t)g[k];
+      u[0][k] = d[0]; u[1][k] = d[1]; u[2][k] = d[2];
+      dot[k] = a[0] * u[0][k] + a[1] * u[1][k] + a[2] * u[2][k];
+    }
+    const int b = el * 125 + c;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      if (lane) {
+#pragma unroll
+        for (int k = 0; k < 5; k++) sA[a][b + 25 * k] = u[a][k];
+      }
+      realw r[5];
+      line_gradient(G, u[a], r);
+#pragma unroll
+      for (int k = 0; k < 5; k++) d3[k][a] = r[k];
+    }
+  }
+  lds_barrier();
+  const int bx = el * 125 + 5 * c, by = el * 125 + i + 25 * j;
+  realw x[3][5];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    realw r[5], y[5];
+#pragma unroll
+    for (int l = 0; l < 5; l++) {
+      r[l] = sA[a][bx + l];
+      y[l] = sA[a][by + 5 * l];
+    }
+    line_gradient(G, r, x[a]);
+    line_gradient(G, y, r);
+    if (lane) {
+#pragma unroll
+      for (int l = 0; l < 5; l++) sB[a][by + 5 * l] = r[l];
+    }
+  }
+  lds_barrier();                                   // every row of u has been read
+  if (lane) {
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+      for (int l = 0; l < 5; l++) sA[a][bx + l] = x[a][l];
+  }
+  lds_barrier();
+  if (!active) return;
+  const realw ONE_THIRD = (realw)1 / (realw)3;
+#pragma unroll
+  for (int k = 0; k < 5; k++) {
+    const int b = el * 125 + c + 25 * k, p = c + 25 * k;
+    const int64_t q = ep + 25 * k;
+    const Grad9 tg = {sA[0][b], sA[1][b], sA[2][b], sB[0][b], sB[1][b], sB[2][b], d3[k][0], d3[k][1], d3[k][2]};
+    JacPt J = {};
+    if (!REG && irr) J = load_jac(A.jac, A.jac_plane, jp + 25 * k);
+    const Du9 du = map_gradient<FOLD>(tg, irr != 0, J, A.xix_regular);
+    const realw templ = ONE_THIRD * (du.xx + du.yy + du.zz);
+    const realw b1 = du.xx - templ, b2 = du.yy - templ, b3 = (realw)0.5 * (du.xy + du.yx),
+                b4 = (realw)0.5 * (du.zx + du.xz), b5 = (realw)0.5 * (du.zy + du.yz);
+    const realw e1 = S.eps[eps_idx(e, 0, p)], e2 = S.eps[eps_idx(e, 1, p)], e3 = S.eps[eps_idx(e, 2, p)],
+                e4 = S.eps[eps_idx(e, 3, p)], e5 = S.eps[eps_idx(e, 4, p)];
+    S.rho_kl[q] = S.rho_kl[q] + S.deltat * dot[k];
+    S.mu_kl[q] = S.mu_kl[q] + S.deltat * (e1 * b1 + e2 * b2 + (e1 + e2) * (b1 + b2) + (realw)2 * (e3 * b3 + e4 * b4 + e5 * b5));
+    S.kappa_kl[q] = S.kappa_kl[q] + S.deltat * ((realw)9 * S.eps_tr3[q] * templ);
+  }
+}
+
 // element strain of a displacement field (compute_element_strain.F90:28-130); one lane per point
 __global__ void __launch_bounds__(128) k_element_strain(ElasticArgs A, GLLk G, realw* eps, realw* eps_tr3,
                                                         int with_trace) {
@@ -502,6 +597,19 @@ void SFX(launch_elastic)(hipStream_t s, const ElasticArgs& a, bool strain, bool 
   }
 #undef SF_K
   SF_LAUNCH_CHECK("k_elastic_pt");
+}
+
+void SFX(launch_kernels_line)(hipStream_t s, const ElasticArgs& a, const KernelSums& k) {
+  if (a.nelem <= 0) return;
+  GLLk G = g_gll_host;
+  const dim3 grid((a.nelem + 4) / 5), block(128);
+  if (a.jac_plane == 0) {
+    if (SF_FOLD) regular_gll(G, a.xix_regular, a.jacobian_regular);
+    hipLaunchKernelGGL(k_kernels_line<true>, grid, block, 0, s, a, k, G);
+  } else {
+    hipLaunchKernelGGL(k_kernels_line<false>, grid, block, 0, s, a, k, G);
+  }
+  SF_LAUNCH_CHECK("k_kernels_line");
 }
 
 void SFX(launch_element_strain)(hipStream_t s, const ElasticArgs& a, realw* eps, realw* eps_tr3, bool with_trace) {

@@ -171,6 +171,14 @@ void launch_elastic(hipStream_t s, const ElasticArgs& a, bool strain, bool att, 
 void launch_element_strain(hipStream_t s, const ElasticArgs& a, realw* eps, realw* eps_tr3, bool with_trace,
                            bool exact);
 
+// elastic kernel sums with the strain of the reconstructed displacement ElasticArgs::displ formed on the way
+struct KernelSums {
+  const realw *accel, *eps, *eps_tr3;  // adjoint field
+  realw deltat;
+  realw *rho_kl, *mu_kl, *kappa_kl;
+};
+void launch_kernels_line(hipStream_t s, const ElasticArgs& a, const KernelSums& k, bool exact);
+
 // C-PML elements (k_pml.hip): stiffness with the convolution memory variables of
 // compute_forces_viscoelastic_PML; per C-PML element blocks of 125-point planes
 constexpr int SF_PML_NSTATE = 48;
