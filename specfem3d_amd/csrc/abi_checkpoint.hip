@@ -99,7 +99,7 @@ extern "C" void sf_snapshot_load(long* Mesh_pointer, int FORWARD_OR_ADJOINT, int
     ck_copy(m, m->el[f].displ, s.el, 3 * n);
     ck_copy(m, m->el[f].veloc, s.el + 3 * n, 3 * n);
     ck_copy(m, m->el[f].accel, s.el + 6 * n, 3 * n);
-    m->accel_clean[f] = 0;
+    m->accel_clean[f] = m->low_set[f] = 0;
   }
   if (m->ac[f].pot) {
     if (!s.ac) fatal("sf_snapshot_load", "snapshot holds no acoustic field");
@@ -152,7 +152,10 @@ extern "C" void sf_history_load(long* Mesh_pointer, int FORWARD_OR_ADJOINT, int 
   const int f = field_of_foa(FORWARD_OR_ADJOINT);
   flush_field(m, f);
   const int64_t n = m->nglob;
-  if (m->history_el && m->el[f].displ) ck_copy(m, m->el[f].displ, m->history_el + (int64_t)frame * 3 * n, 3 * n);
+  if (m->history_el && m->el[f].displ) {
+    ck_copy(m, m->el[f].displ, m->history_el + (int64_t)frame * 3 * n, 3 * n);
+    m->low_set[f] = 0;
+  }
   if (m->history_ac && m->ac[f].pot) {
     ck_copy(m, m->ac[f].pot, m->history_ac + (int64_t)frame * 2 * n, n);
     ck_copy(m, m->ac[f].potdd, m->history_ac + (int64_t)frame * 2 * n + n, n);

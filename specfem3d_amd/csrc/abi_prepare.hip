@@ -754,6 +754,10 @@ void ensure_gather_assembly(Mesh* m, int f) {
   const int eb = 20;  // elements per block of slots: a multiple of the five of a k_elastic_line workgroup
   const int first_pml = (m->nspec_elastic + eb - 1) / eb * eb;
   if (!m->asm_buf[f]) m->asm_buf[f] = dmalloc<realw>(3 * 125 * ((int64_t)m->nspec + 2 * eb));  // both lists, rounded up
+  if (m->simulation_type == 3 && !m->low[f]) {
+    m->low[f] = dmalloc<uint16_t>(3 * (int64_t)m->nglob);
+    m->low_set[f] = 0;
+  }
   if (m->asm_ready) return;
   flush_all(m);       // local forces in the old slots
   if (m->assembly == 2) ensure_element_colors(m);
@@ -797,6 +801,8 @@ void release_gather_assembly(Mesh* m) {
   dfree(m->rmass1);
   dfree(m->asm_buf[0]);
   dfree(m->asm_buf[1]);
+  dfree(m->low[0]);
+  dfree(m->low[1]);
   m->asm_ready = 0;
   dfree(m->asm_ac_idx);
   dfree(m->asm_ac_info);
@@ -1249,6 +1255,7 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
   dfree(m->seismo_d); dfree(m->seismo_v); dfree(m->seismo_a); dfree(m->seismo_p);
   dfree(m->rho_kl); dfree(m->mu_kl); dfree(m->kappa_kl); dfree(m->rho_ac_kl); dfree(m->kappa_ac_kl);
   dfree(m->asm_idx); dfree(m->asm_info); dfree(m->asm_base); dfree(m->asm_rec); dfree(m->rmass1); dfree(m->asm_buf[0]); dfree(m->asm_buf[1]);
+  dfree(m->low[0]); dfree(m->low[1]);
   dfree(m->pml_elems); dfree(m->pml_cpml);
   dfree(m->pml_state); dfree(m->pml_coef); dfree(m->pml_masks); dfree(m->pml_off);
   dfree(m->pml_old); dfree(m->pml_pts); dfree(m->pml_bc_pts);

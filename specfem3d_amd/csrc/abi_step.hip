@@ -41,6 +41,8 @@ static GatherArgs gather_args(Mesh* m, int f) {
   a.rm = m->rmass;
   a.rm1 = m->rmass1;
   a.dt2p = m->pending_dt2_el[f];
+  a.lo = m->exact ? nullptr : m->low[f];
+  a.lo_set = m->low_set[f];
   return a;
 }
 
@@ -49,6 +51,7 @@ static void flush_el(Mesh* m, int f) {
   if (m->pending_gather_el[f]) {
     launch_gather_update(m->stream, gather_args(m, f), 3, m->pending_k3_el[f] ? GATHER_CORRECT : GATHER_ONLY,
                          m->exact != 0);
+    if (m->pending_k3_el[f]) m->low_set[f] = m->low[f] && !m->exact;
     m->pending_gather_el[f] = 0;
     m->gather_skip_el[f] = 0;
     m->accel_clean[f] = 0;
@@ -57,6 +60,7 @@ static void flush_el(Mesh* m, int f) {
     launch_corrector(m->stream, 3 * m->el_n, m->el[f].veloc + o, m->el[f].accel + o, m->rmass + o,
                      m->pending_dt2_el[f]);
     m->accel_clean[f] = 0;
+    m->low_set[f] = 0;
   }
   m->pending_k3_el[f] = 0;
 }
@@ -232,10 +236,16 @@ extern "C" void FC_FUNC_(update_displacement_cuda, UPDATE_DISPLACMENT_CUDA)(long
     a.t1 = m->pml_t1;
     a.t2 = m->pml_t2;
     launch_gather_update(m->stream, a, 3, GATHER_STEP, m->exact != 0);
+    m->low_set[f] = a.lo != nullptr;
   } else if (m->pending_k3_el[f]) {
+    m->low_set[f] = 0;
     launch_corrector_predictor(m->stream, n, w.displ + o, w.veloc + o, w.accel + o, m->rmass + o,
                                m->pending_dt2_el[f], *deltat_F, *deltatover2_F, *deltatsqover2_F,
                                pml ? m->pml_old + o : nullptr, m->pml_t1, m->pml_t2);
+  } else if (m->low[f] && !m->exact) {
+    launch_predictor_low(m->stream, n, w.displ + o, w.veloc + o, w.accel + o, *deltat_F, *deltatover2_F,
+                         *deltatsqover2_F, m->low[f] + o, m->low_set[f]);
+    m->low_set[f] = 1;
   } else {
     launch_predictor(m->stream, n, w.displ + o, w.veloc + o, w.accel + o, *deltat_F, *deltatover2_F,
                      *deltatsqover2_F);
@@ -875,7 +885,7 @@ static void d2h(Mesh* m, realw* h, const realw* d, int64_t n) {
     DIR(m, m->el[F].displ, displ, *size);                                                                     \
     DIR(m, m->el[F].veloc, veloc, *size);                                                                     \
     DIR(m, m->el[F].accel, accel, *size);                                                                     \
-    m->accel_clean[F] = 0;                                                                                    \
+    m->accel_clean[F] = m->low_set[F] = 0;                                                                    \
   }
 #define SF_XFER1(NAME, F, MEMBER, DIR)                                                   \
   extern "C" void FC_FUNC_(NAME, X)(int* size, realw* arr, long* Mesh_pointer) {        \
@@ -883,7 +893,7 @@ static void d2h(Mesh* m, realw* h, const realw* d, int64_t n) {
     check_field(m, F, #NAME);                                                            \
     flush_el(m, F);                                                                      \
     DIR(m, m->el[F].MEMBER, arr, *size);                                                 \
-    m->accel_clean[F] = 0;                                                               \
+    m->accel_clean[F] = m->low_set[F] = 0;                                               \
   }
 #define H2D(m, d, h, n) h2d(m, d, h, n)
 #define D2H(m, d, h, n) d2h(m, h, d, n)

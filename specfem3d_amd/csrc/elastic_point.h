@@ -219,25 +219,19 @@ __device__ __forceinline__ const realw* gll_hpw(const realw* sG, bool irr) {
 // One line of five GLL points against the derivative tables, held by one lane: the coefficients have
 // constant indices and come from scalar registers, and each point of the line is read once instead
 // of once per output. Sums left to right, as tile_gradient and tile_divergence.
-// FMA builds apply the tables to what the line's points differ from its middle point by, and the tables'
-// sums (GLLk) to the middle point: neighbouring points are alike, so the products round relative to
-// their differences instead of to the field itself, and a field without differences gives what the
-// tables' own rounding gives, also after a factor was folded into them. Against the same loop in 64 bits, the records of 32x32x16
-// elements and 16 shots are off by 0.61 times what single-precision sums everywhere gave, 0.79 without
-// this (geometric means over 96 records); the launch times are the same (103 us on 64x64x32 elements).
+// The divergence of FMA builds applies the table to what the line's values differ from its middle value
+// by, and the table's sums (GLLk::hws) to the middle value: away from the ends of a line the sums are
+// zero, so a stress that hardly varies along it cancels before it is rounded, and the tables keep
+// their sums when a factor is folded into them. Against the same loop in 64 bits, the records of
+// 32x32x16 elements and 16 shots are off by 0.59 times what single-precision sums everywhere gave, 0.80
+// without this (geometric means over 160 records); the launch times are the same. The same for the
+// gradient: 0.59 still, and kernels under a sea 0.68 instead of 0.56.
 __device__ __forceinline__ void line_gradient(const GLLk& G, const realw in[5], realw out[5]) {
 #pragma unroll
   for (int m = 0; m < 5; m++) {
-#if SF_EXACT
     realw r = G.hp[m * 5] * in[0];
 #pragma unroll
     for (int l = 1; l < 5; l++) r = r + G.hp[m * 5 + l] * in[l];
-#else
-    realw r = G.hs[m] * in[2];
-#pragma unroll
-    for (int l = 0; l < 5; l++)
-      if (l != 2) r = r + G.hp[m * 5 + l] * (in[l] - in[2]);
-#endif
     out[m] = r;
   }
 }

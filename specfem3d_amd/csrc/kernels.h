@@ -22,19 +22,15 @@ struct GLLk {
   // fold the regular mapping and the jacobian weight into the contractions (fold_gll)
   realw hpr[25];
   realw hpwr[25];
-  // FMA builds, line_gradient and line_divergence: sum over l of hp[m, l] and of hpw[l, m]
-  realw hs[5], hws[5];
+  // FMA builds, line_divergence: sum over l of hpw[l, m]
+  realw hws[5];
 };
-// hs and hws from the tables and the factors folded into them
-inline void sum_gll(GLLk& G, double fg, double fd) {
+// hws from the table and a factor folded into it
+inline void sum_gll(GLLk& G, double factor) {
   for (int m = 0; m < 5; m++) {
-    double g = 0, d = 0;
-    for (int l = 0; l < 5; l++) {
-      g += G.hp[m * 5 + l];
-      d += G.hpw[l * 5 + m];
-    }
-    G.hs[m] = (realw)(fg * g);
-    G.hws[m] = (realw)(fd * d);
+    double d = 0;
+    for (int l = 0; l < 5; l++) d += G.hpw[l * 5 + m];
+    G.hws[m] = (realw)(factor * d);
   }
 }
 inline void fold_gll(GLLk& G, realw xix_regular, realw jacobian_regular) {
@@ -47,7 +43,7 @@ inline void fold_gll(GLLk& G, realw xix_regular, realw jacobian_regular) {
 // the tables of a launch over regular elements alone: the folded ones in the place of the others
 inline void regular_gll(GLLk& G, realw xix_regular, realw jacobian_regular) {
   fold_gll(G, xix_regular, jacobian_regular);
-  sum_gll(G, xix_regular, (double)jacobian_regular * xix_regular);
+  sum_gll(G, (double)jacobian_regular * xix_regular);
   for (int q = 0; q < 25; q++) {
     G.hp[q] = G.hpr[q];
     G.hpw[q] = G.hpwr[q];
@@ -59,6 +55,9 @@ void set_gll_constants(const realw* hprime, const realw* hprimewgll, const realw
 // Newmark pieces (k_update.hip)
 void launch_predictor(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, realw dt, realw dt2, realw dtsq2);
 void launch_corrector(hipStream_t s, int64_t n, realw* v, realw* a, const realw* rmass, realw dt2);
+// ... in double precision with the low parts of u and v (`set`: they are set, else zero)
+void launch_predictor_low(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, realw dt, realw dt2, realw dtsq2,
+                          uint16_t* lo, int set);
 // with `old`, also PML_displ_old = u + t1 v + t2 a of the corrected field (before the predictor)
 void launch_corrector_predictor(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, const realw* rmass,
                                 realw dt2_prev, realw dt, realw dt2, realw dtsq2, realw* old = nullptr,
@@ -95,7 +94,25 @@ struct GatherArgs {
   realw dt, dt2, dtsq2;        // predictor
   realw* old;                  // PML_displ_old = u + t1 v + t2 a of the corrected field, or null
   realw t1, t2;
+  uint16_t* lo;                // low parts of v and u (LowParts), 3 per point, or null
+  int lo_set;                  // they are set (else zero)
 };
+// Low parts of u and v: what the stored single-precision values miss, in 1/256 of their last place, one
+// byte each (u in the low one). Kernel runs of FMA builds keep them (see k_gather_update). Values
+// below 2^-95, infinities and NaN have none.
+__device__ __forceinline__ double with_low(realw x, int low) {
+  const int e = __float_as_uint(x) >> 23 & 255;
+  const realw unit = e >= 32 && e < 255 ? __uint_as_float((uint32_t)(e - 31) << 23) : 0.f;
+  return (double)x + (double)((realw)(int8_t)low * unit);
+}
+// rounds x to `hi`, returns the byte of the rest
+__device__ __forceinline__ int split_low(double x, realw& hi) {
+  hi = (realw)x;
+  const int e = __float_as_uint(hi) >> 23 & 255;
+  if (e < 32 || e == 255) return 0;
+  const realw q = rintf((realw)(x - (double)hi) * __uint_as_float((uint32_t)(285 - e) << 23));
+  return (int)fminf(fmaxf(q, -127.f), 127.f) & 0xff;
+}
 // what follows the sum: nothing (accel is left assembled), the corrector, or the corrector and the
 // predictor of the next step (accel left zero)
 enum { GATHER_ONLY = 0, GATHER_CORRECT = 1, GATHER_STEP = 2 };

@@ -228,6 +228,8 @@ struct Mesh {
   int pending_gather_el[2] = {0, 0};
   int gather_skip_el[2] = {0, 0};  // AF_* of the points that the pending sum leaves out
   int accel_clean[2] = {0, 0};     // accel is zero at every point without AF_TERM
+  uint16_t* low[2] = {nullptr, nullptr};  // low parts of u and v (GatherArgs::lo): kernel runs
+  int low_set[2] = {0, 0};         // they belong to the stored u and v
   // the same for the fluid (1 component; the inverse mass is rmass_ac)
   int* asm_ac_idx = nullptr;
   int asm_ac_eb = 1;

@@ -134,3 +134,29 @@ def test_source_values(oracle_mod, nsrc):
     out = g.run().copy()
     g.close()
     assert np.abs(ref).max() > 0 and np.array_equal(out, ref)
+
+
+@pytest.mark.parametrize("n,warp,nt_dump", [(2, False, 7), (3, True, 40), (5, False, 16)])
+def test_kernel_run_low_parts(oracle_mod, n, warp, nt_dump):
+    """FMA kernel runs carry u and v with low parts through fused and separate updates, snapshots, history
+    frames and fields put to zero. Tolerance: the moduli, masses and tables in single precision (about
+    eight factors of 2^-24 on the way from displacement to displacement) and the rounding of the forces
+    in each of 40 steps, 2^-24 (8 + sqrt(40)) = 8.5e-7, times 6 for the fields of a product."""
+    from specfem3d_amd.adjoint import KernelSolver
+    nstep, tol = 40, 5e-6
+    db, src, rec = small_elastic_box(n=n, warp=smooth_warp(500.0 * n) if warp else None, dt=0.008)
+    t = np.arange(nstep)[:, None, None] / nstep
+    r, c = np.arange(rec.n)[None, :, None], np.arange(3)[None, None, :]
+    adj = (np.sin(2 * np.pi * (2 * t + 0.17 * r + 0.3 * c)) * np.sin(np.pi * t)).astype(np.float32)
+    ref = oracle_mod.kernel_run(db, src, rec, nstep, adj.astype(np.float64), nt_dump, "f64")
+    print(f"[gpu] low parts n={n} warp={warp} nt_dump={nt_dump}", flush=True)
+    ks = KernelSolver(db, src, rec, nstep, nt_dump=nt_dump, exact=False, assembly=-1)
+    seis = ks.forward()
+    k = ks.adjoint(adj)
+    seis2, k2 = ks.seis_d[: nstep].copy(), ks.adjoint(adj)      # the same run again gives the same bits
+    ks.close()
+    assert all(np.array_equal(a, b) for a, b in zip(k, k2)) and np.array_equal(seis, seis2[: len(seis)])
+    for name, a, b in zip(("seis", "rho", "mu", "kappa"), (seis,) + tuple(k), ref):
+        e = np.linalg.norm(a.ravel().astype(np.float64) - b.ravel()) / np.linalg.norm(b)
+        print(f"[gpu]   {name} {e:.2e}", flush=True)
+        assert np.abs(b).max() > 0 and e < tol, (name, e)
