@@ -20,9 +20,15 @@ namespace sf {
 void free_checkpoints(Mesh* m);
 void flush_all(Mesh* m);
 
-Mesh* from_handle(long* p) {
+Mesh* from_handle_waiting(long* p) {
   if (!p || !*p) fatal("Mesh_pointer", "null handle (prepare_constants_device not called?)");
   return reinterpret_cast<Mesh*>(*p);
+}
+void flush_terms(Mesh* m);
+Mesh* from_handle(long* p) {
+  Mesh* m = from_handle_waiting(p);
+  flush_terms(m);
+  return m;
 }
 
 // Set-up progress on stderr when SF_VERBOSE_PREPARE=1 (large meshes take minutes to prepare).
@@ -747,6 +753,31 @@ static void build_colors(Mesh* m, const std::vector<int>& elems, int*& d_list, i
   d_list = lst.empty() ? nullptr : dupload(lst.data(), (int64_t)lst.size());
 }
 
+// points that the terms of one domain touch, with the heads of each term's chain (TermArgs)
+static void build_term_points(Mesh* m, int fluid) {
+  const FacePoints* lists[4] = {fluid ? &m->abs_ac : &m->abs_el, &m->coupling, fluid ? &m->src_ac_pts : &m->src_pts,
+                                fluid ? &m->adj_ac_pts : &m->adj_pts};
+  std::vector<int> at((size_t)m->nglob, -1), ig, head;
+  for (int k = 0; k < 4; k++) {
+    std::vector<int> g(lists[k]->points());
+    if (g.empty()) continue;
+    SF_CHECK(hipMemcpy(g.data(), lists[k]->iglob, sizeof(int) * g.size(), hipMemcpyDeviceToHost));
+    for (size_t q = 0; q < g.size(); q++) {
+      if (at[g[q]] < 0) {
+        at[g[q]] = (int)ig.size();
+        ig.push_back(g[q]);
+        head.insert(head.end(), {-1, -1, -1, -1});
+      }
+      head[4 * (size_t)at[g[q]] + k] = (int)q;
+    }
+  }
+  dfree(m->term_iglob[fluid]);
+  dfree(m->term_head[fluid]);
+  m->term_n[fluid] = (int)ig.size();
+  m->term_iglob[fluid] = dupload(ig.data(), (int64_t)ig.size());
+  m->term_head[fluid] = dupload(head.data(), (int64_t)head.size());
+}
+
 // Lists and buffers of the gather assembly for one field: the slots of each point in the processing
 // order, or in the colour order under assembly = 2 (the sums a coloured scatter makes, bit for bit),
 // those of the C-PML elements last (compute_forces_viscoelastic, then compute_forces_viscoelastic_PML).
@@ -786,6 +817,7 @@ void ensure_gather_assembly(Mesh* m, int f) {
   if (!m->asm_rec) m->asm_rec = dmalloc<int>(125 * (int64_t)m->nrec_local);
   launch_pick(m->stream, 125 * (int64_t)m->nrec_local, m->rec_iglob, ptr, m->asm_rec);
   dfree(ptr);
+  build_term_points(m, 0);
   m->asm_ready = 1;
 }
 
@@ -836,6 +868,7 @@ void ensure_gather_acoustic(Mesh* m, int f) {
   if (!m->asm_ac_rec) m->asm_ac_rec = dmalloc<int>(125 * (int64_t)m->nrec_local);
   launch_pick(m->stream, 125 * (int64_t)m->nrec_local, m->rec_iglob, ptr, m->asm_ac_rec);
   dfree(ptr);
+  build_term_points(m, 1);
   m->asm_ac_ready = 1;
 }
 
@@ -1260,6 +1293,12 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
   dfree(m->pml_state); dfree(m->pml_coef); dfree(m->pml_masks); dfree(m->pml_off);
   dfree(m->pml_old); dfree(m->pml_pts); dfree(m->pml_bc_pts);
   dfree(m->asm_ac_idx); dfree(m->asm_ac_info); dfree(m->asm_ac_base); dfree(m->asm_ac_rec); dfree(m->asm_ac_buf[0]); dfree(m->asm_ac_buf[1]);
+  for (int d = 0; d < 2; d++) {
+    dfree(m->term_iglob[d]);
+    dfree(m->term_head[d]);
+    delete m->terms[d][0];
+    delete m->terms[d][1];
+  }
   dfree(m->d_norm);
   if (m->h_norm) (void)hipHostFree(m->h_norm);
   if (m->timing_ev) {

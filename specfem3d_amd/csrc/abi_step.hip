@@ -22,6 +22,8 @@ void ensure_gather_assembly(Mesh* m, int f);
 void ensure_gather_acoustic(Mesh* m, int f);
 const std::vector<int>& host_ibool(Mesh* m);
 
+Mesh* from_handle_waiting(long* p);  // the waiting terms stay so
+
 static inline int field_of(int foa) { return foa == 3 ? 1 : 0; }
 
 static GatherArgs gather_args(Mesh* m, int f) {
@@ -46,8 +48,20 @@ static GatherArgs gather_args(Mesh* m, int f) {
   return a;
 }
 
+// launch the terms that wait for one field
+static void flush_terms(Mesh* m, int fluid, int f) {
+  TermArgs* t = m->terms[fluid][f];
+  if (!t || !t->terms) return;
+  launch_terms(m->stream, *t, fluid);
+  t->terms = 0;
+}
+void flush_terms(Mesh* m) {
+  for (int d = 0; d < 2; d++)
+    for (int f = 0; f < 2; f++) flush_terms(m, d, f);
+}
+
 // sum the waiting local forces and run the pending corrector
-static void flush_el(Mesh* m, int f) {
+static void sum_el(Mesh* m, int f) {
   if (m->pending_gather_el[f]) {
     launch_gather_update(m->stream, gather_args(m, f), 3, m->pending_k3_el[f] ? GATHER_CORRECT : GATHER_ONLY,
                          m->exact != 0);
@@ -63,6 +77,11 @@ static void flush_el(Mesh* m, int f) {
     m->low_set[f] = 0;
   }
   m->pending_k3_el[f] = 0;
+}
+
+static void flush_el(Mesh* m, int f) {
+  flush_terms(m, 0, f);
+  sum_el(m, f);
 }
 
 static GatherArgs gather_args_ac(Mesh* m, int f) {
@@ -84,7 +103,7 @@ static GatherArgs gather_args_ac(Mesh* m, int f) {
   return a;
 }
 
-void flush_ac(Mesh* m, int f) {
+static void sum_ac(Mesh* m, int f) {
   int& fz = m->free_zero[f];
   if (m->pending_gather_ac[f]) {
     launch_gather_update(m->stream, gather_args_ac(m, f), 1, m->pending_k3_ac[f] ? GATHER_CORRECT : GATHER_ONLY,
@@ -103,11 +122,46 @@ void flush_ac(Mesh* m, int f) {
   }
   m->pending_k3_ac[f] = 0;
 }
-// before boundary, coupling or source terms are added to chi''
-static void flush_ac_terms(Mesh* m, int f) {
-  flush_ac(m, f);
-  m->free_zero[f] &= FREE_POT;
+void flush_ac(Mesh* m, int f) {
+  flush_terms(m, 1, f);
+  sum_ac(m, f);
 }
+
+// One term more for a field's next launch of terms: those that wait come before it in the reference's
+// order, or are launched first.
+static TermArgs& add_term(Mesh* m, int fluid, int f, int term) {
+  if (fluid) {
+    flush_terms(m, 0, f);  // the coupling of the solid reads chi''
+    sum_ac(m, f);
+    ensure_gather_acoustic(m, f);
+    m->free_zero[f] &= FREE_POT;
+  } else {
+    sum_el(m, f);
+    ensure_gather_assembly(m, f);
+  }
+  TermArgs*& t = m->terms[fluid][f];
+  if (!t) {
+    t = new TermArgs;
+    t->terms = 0;
+  }
+  if (t->terms >= term) flush_terms(m, fluid, f);
+  t->n = m->term_n[fluid];
+  t->iglob = m->term_iglob[fluid];
+  t->head = m->term_head[fluid];
+  t->stacey = fluid ? m->abs_ac : m->abs_el;
+  t->coupling = m->coupling;
+  t->source = fluid ? m->src_ac_pts : m->src_pts;
+  t->adjoint = fluid ? m->adj_ac_pts : m->adj_pts;
+  t->in = fluid ? m->ac[f].potd : m->el[f].veloc;
+  t->other = fluid ? m->el[f].displ : m->ac[f].potdd;
+  t->out = fluid ? m->ac[f].potdd : m->el[f].accel;
+  t->src_array = m->src_array;
+  t->src_kappa = m->src_kappa;
+  t->adj_h = m->adj_h;
+  t->terms |= term;
+  return *t;
+}
+
 void flush_field(Mesh* m, int f) {
   flush_el(m, f);
   flush_ac(m, f);
@@ -331,7 +385,7 @@ extern "C" void FC_FUNC_(kernel_3_acoustic_cuda, KERNEL_3_ACOUSTIC_CUDA)(long* M
 extern "C" void FC_FUNC_(compute_forces_viscoelastic_cuda, COMPUTE_FORCES_VISCOELASTIC_CUDA)(
     long* Mesh_pointer, int* iphase, realw* deltat, int* nspec_outer_elastic, int* nspec_inner_elastic,
     int* COMPUTE_AND_STORE_STRAIN, int* ATTENUATION, int* FORWARD_OR_ADJOINT_f) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   // NPROC=1: every element is "inner"; all elements are computed in phase 2
   (void)nspec_outer_elastic; (void)nspec_inner_elastic;
   if (*iphase != 2) return;
@@ -358,7 +412,7 @@ extern "C" void FC_FUNC_(compute_forces_acoustic_cuda, COMPUTE_FORCES_ACOUSTIC_C
                                                                                    int* nspec_outer_acoustic,
                                                                                    int* nspec_inner_acoustic,
                                                                                    int* FORWARD_OR_ADJOINT_f) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   (void)nspec_outer_acoustic; (void)nspec_inner_acoustic;
   if (*iphase != 2) return;
   const int foa = *FORWARD_OR_ADJOINT_f;
@@ -366,8 +420,9 @@ extern "C" void FC_FUNC_(compute_forces_acoustic_cuda, COMPUTE_FORCES_ACOUSTIC_C
     if (foa == 1 && f == 1) continue;
     if (foa == 3 && f == 0) continue;
     if (!m->ac[f].pot) continue;
-    if (m->nspec_acoustic <= 0) continue;
+    flush_terms(m, 0, f);  // the coupling of the solid reads chi''
     flush_ac(m, f);
+    if (m->nspec_acoustic <= 0) continue;
     ensure_gather_acoustic(m, f);
     AcousticArgs a;
     a.nelem = m->nspec_acoustic;
@@ -491,15 +546,17 @@ extern "C" void FC_FUNC_(transfer_pml_displ_to_device, TRANSFER_PML_DISPL_TO_DEV
 // run: subtract the record the host read into b_absorb_field.
 extern "C" void FC_FUNC_(compute_stacey_viscoelastic_cuda, COMPUTE_STACEY_VISCOELASTIC_CUDA)(
     long* Mesh_pointer, int* iphasef, realw* b_absorb_field, int* FORWARD_OR_ADJOINT_f) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   if (*iphasef != 1 || !m->stacey || m->abs_el.n == 0) return;
   const int foa = *FORWARD_OR_ADJOINT_f;
   const int64_t rec_len = 3 * 25 * (int64_t)m->num_abs_boundary_faces;
   if (foa == 0 || foa == 1) {
-    flush_el(m, 0);
     const bool store = m->simulation_type == 1 && m->save_forward && b_absorb_field;
-    launch_stacey_elastic(m->stream, m->abs_el, m->el[0].veloc, m->el[0].accel, m->b_absorb_field, store ? 1 : 0);
-    if (store) {
+    if (!store) {
+      add_term(m, 0, 0, TERM_STACEY);
+    } else {
+      flush_el(m, 0);
+      launch_stacey_elastic(m->stream, m->abs_el, m->el[0].veloc, m->el[0].accel, m->b_absorb_field);
       SF_CHECK(hipMemcpyAsync(b_absorb_field, m->b_absorb_field, sizeof(realw) * rec_len, hipMemcpyDeviceToHost,
                               m->stream));
       SF_CHECK(hipStreamSynchronize(m->stream));
@@ -518,15 +575,14 @@ extern "C" void FC_FUNC_(compute_stacey_viscoelastic_cuda, COMPUTE_STACEY_VISCOE
 // reconstructed field forward in time, so Stacey is applied to it directly.
 extern "C" void FC_FUNC_(compute_stacey_viscoelastic_undoatt_cuda, COMPUTE_STACEY_VISCOELASTIC_UNDOATT_CUDA)(
     long* Mesh_pointer, int* iphasef, int* FORWARD_OR_ADJOINT_f) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   if (*iphasef != 1 || !m->stacey || m->abs_el.n == 0) return;
   const int foa = *FORWARD_OR_ADJOINT_f;
   for (int f = 0; f < 2; f++) {
     if (foa == 1 && f == 1) continue;
     if (foa == 3 && f == 0) continue;
     if (!m->el[f].displ) continue;
-    flush_el(m, f);
-    launch_stacey_elastic(m->stream, m->abs_el, m->el[f].veloc, m->el[f].accel, nullptr, 0);
+    add_term(m, 0, f, TERM_STACEY);
   }
 }
 
@@ -534,22 +590,28 @@ extern "C" void FC_FUNC_(compute_stacey_acoustic_cuda, COMPUTE_STACEY_ACOUSTIC_C
                                                                                    int* iphasef,
                                                                                    realw* h_b_absorb_potential,
                                                                                    int* FORWARD_OR_ADJOINT_f) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   if (*iphasef != 1 || !m->stacey || m->abs_ac.n == 0) return;
   const int foa = *FORWARD_OR_ADJOINT_f;
   const int64_t rec_len = 25 * (int64_t)m->num_abs_boundary_faces;
   if (foa == 0 || foa == 1) {
-    flush_ac_terms(m, 0);
     const bool store = m->simulation_type == 1 && m->save_forward && h_b_absorb_potential;
-    launch_stacey_acoustic(m->stream, m->abs_ac, m->ac[0].potd, m->ac[0].potdd, m->b_absorb_potential, store ? 1 : 0);
-    if (store) {
+    if (!store) {
+      add_term(m, 1, 0, TERM_STACEY);
+    } else {
+      flush_terms(m, 0, 0);
+      flush_ac(m, 0);
+      m->free_zero[0] &= FREE_POT;
+      launch_stacey_acoustic(m->stream, m->abs_ac, m->ac[0].potd, m->ac[0].potdd, m->b_absorb_potential);
       SF_CHECK(hipMemcpyAsync(h_b_absorb_potential, m->b_absorb_potential, sizeof(realw) * rec_len,
                               hipMemcpyDeviceToHost, m->stream));
       SF_CHECK(hipStreamSynchronize(m->stream));
     }
   }
   if ((foa == 0 || foa == 3) && m->simulation_type == 3 && m->ac[1].pot) {
-    flush_ac_terms(m, 1);
+    flush_terms(m, 0, 1);
+    flush_ac(m, 1);
+    m->free_zero[1] &= FREE_POT;
     SF_CHECK(hipMemcpyAsync(m->b_absorb_potential, h_b_absorb_potential, sizeof(realw) * rec_len,
                             hipMemcpyHostToDevice, m->stream));
     launch_stacey_acoustic_replay(m->stream, m->abs_ac, m->b_absorb_potential, m->ac[1].potdd);
@@ -559,15 +621,14 @@ extern "C" void FC_FUNC_(compute_stacey_acoustic_cuda, COMPUTE_STACEY_ACOUSTIC_C
 
 extern "C" void FC_FUNC_(compute_stacey_acoustic_undoatt_cuda, COMPUTE_STACEY_ACOUSTIC_UNDOATT_CUDA)(
     long* Mesh_pointer, int* iphasef, int* FORWARD_OR_ADJOINT_f) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   if (*iphasef != 1 || !m->stacey || m->abs_ac.n == 0) return;
   const int foa = *FORWARD_OR_ADJOINT_f;
   for (int f = 0; f < 2; f++) {
     if (foa == 1 && f == 1) continue;
     if (foa == 3 && f == 0) continue;
     if (!m->ac[f].pot) continue;
-    flush_ac_terms(m, f);
-    launch_stacey_acoustic(m->stream, m->abs_ac, m->ac[f].potd, m->ac[f].potdd, nullptr, 0);
+    add_term(m, 1, f, TERM_STACEY);
   }
 }
 
@@ -575,16 +636,14 @@ extern "C" void FC_FUNC_(compute_stacey_acoustic_undoatt_cuda, COMPUTE_STACEY_AC
 extern "C" void FC_FUNC_(compute_coupling_ac_el_cuda, COMPUTE_COUPLING_AC_EL_CUDA)(long* Mesh_pointer, int* iphasef,
                                                                                  int* num_coupling_ac_el_facesf,
                                                                                  int* FORWARD_OR_ADJOINT) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   if (*iphasef != 1 || *num_coupling_ac_el_facesf == 0 || m->coupling.n == 0) return;
   const int foa = *FORWARD_OR_ADJOINT;
   for (int f = 0; f < 2; f++) {
     if (foa == 1 && f == 1) continue;
     if (foa == 3 && f == 0) continue;
     if (!m->ac[f].pot || !m->el[f].displ) continue;
-    flush_ac_terms(m, f);
-    const int flip = (m->simulation_type != 1 && f == 0) ? 1 : 0;
-    launch_coupling_ac_el(m->stream, m->coupling, m->el[f].displ, m->ac[f].potdd, flip);
+    add_term(m, 1, f, TERM_COUPLING).flip = (m->simulation_type != 1 && f == 0) ? 1 : 0;
   }
 }
 
@@ -592,33 +651,31 @@ extern "C" void FC_FUNC_(compute_coupling_ac_el_cuda, COMPUTE_COUPLING_AC_EL_CUD
 extern "C" void FC_FUNC_(compute_coupling_el_ac_cuda, COMPUTE_COUPLING_EL_AC_CUDA)(long* Mesh_pointer, int* iphasef,
                                                                                  int* num_coupling_ac_el_facesf,
                                                                                  int* FORWARD_OR_ADJOINT) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   if (*iphasef != 1 || *num_coupling_ac_el_facesf == 0 || m->coupling.n == 0) return;
   const int foa = *FORWARD_OR_ADJOINT;
   for (int f = 0; f < 2; f++) {
     if (foa == 1 && f == 1) continue;
     if (foa == 3 && f == 0) continue;
     if (!m->ac[f].pot || !m->el[f].displ) continue;
-    flush_ac(m, f);
-    flush_el(m, f);
-    const int flip = (m->simulation_type != 1 && f == 0) ? 1 : 0;
-    launch_coupling_el_ac(m->stream, m->coupling, m->ac[f].potdd, m->el[f].accel, flip);
+    flush_ac(m, f);  // reads chi''
+    add_term(m, 0, f, TERM_COUPLING).flip = (m->simulation_type != 1 && f == 0) ? 1 : 0;
   }
 }
 
 // ---------------------------------------------------------------- sources
-// the n values of a launch's sources (`prepared`: as many as its lists may name); more than fit its
-// arguments go to `buffer` on the device
-static SrcVals source_values(Mesh* m, const realw* vals, int n, int prepared, realw* (*buffer)(Mesh*, int)) {
-  SrcVals s;
+// the n values of a field's waiting sources (`prepared`: as many as its lists may name); more than fit the
+// launch's arguments go to `buffer` on the device, and the launch follows at once
+static void source_values(Mesh* m, int fluid, int f, SrcVals& s, const realw* vals, int n, int prepared,
+                          realw* (*buffer)(Mesh*, int)) {
   s.p = nullptr;
   if (std::max(n, prepared) <= SF_SRC_VALS) {
     std::memcpy(s.v, vals, sizeof(realw) * (size_t)n);
     std::fill(s.v + n, s.v + SF_SRC_VALS, 0.f);
   } else {
     s.p = stage_to_device(m, vals, n, buffer(m, n));
+    flush_terms(m, fluid, f);
   }
-  return s;
 }
 static realw* adj_device_buffer(Mesh* m, int) { return m->adj_src; }
 
@@ -632,22 +689,20 @@ static void add_sources_el(Mesh* m, int f, const double* h_stf, int nsrc) {
     any = any || h_stf[i] != 0.0;
   }
   if (!any) return;  // as the reference's GPU wrapper: nothing to add when all STFs are zero
-  flush_el(m, f);
-  launch_add_sources_el(m->stream, m->src_pts, m->src_array, source_values(m, s.data(), nsrc, m->nsources, stf_device_buffer),
-                        m->el[f].accel);
+  source_values(m, 0, f, add_term(m, 0, f, TERM_SOURCE).src, s.data(), nsrc, m->nsources, stf_device_buffer);
 }
 
 extern "C" void FC_FUNC_(compute_add_sources_el_cuda, COMPUTE_ADD_SOURCES_EL_CUDA)(long* Mesh_pointer,
                                                                                  double* h_stf_pre_compute,
                                                                                  int* h_NSOURCES) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   add_sources_el(m, 0, h_stf_pre_compute, *h_NSOURCES);
 }
 
 extern "C" void FC_FUNC_(compute_add_sources_el_s3_cuda, COMPUTE_ADD_SOURCES_EL_S3_CUDA)(long* Mesh_pointer,
                                                                                        double* h_stf_pre_compute,
                                                                                        int* h_NSOURCES) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   check_field(m, 1, "compute_add_sources_el_s3_cuda");
   add_sources_el(m, 1, h_stf_pre_compute, *h_NSOURCES);
 }
@@ -658,16 +713,15 @@ extern "C" void FC_FUNC_(compute_add_sources_el_s3_cuda, COMPUTE_ADD_SOURCES_EL_
 extern "C" void FC_FUNC_(add_sources_el_sim_type_2_or_3, ADD_SOURCES_EL_SIM_TYPE_2_OR_3)(
     long* Mesh_pointer, realw* h_source_adjoint, int* nrec, int* nadj_rec_local, int* NTSTEP_BETWEEN_READ_ADJSRC,
     int* it) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   (void)nrec;
   const int nadj = *nadj_rec_local;
   if (nadj <= 0 || m->adj_pts.n == 0) return;
   const int nt = *NTSTEP_BETWEEN_READ_ADJSRC;
   const int isample = nt - ((*it - 1) % nt);  // 1-based
   const realw* src = h_source_adjoint + (int64_t)3 * nadj * (isample - 1);
-  flush_el(m, 0);
-  launch_adjoint_sources_el(m->stream, m->adj_pts, m->adj_h, source_values(m, src, 3 * nadj, 3 * m->nadj_rec_local, adj_device_buffer),
-                            m->el[0].accel);
+  source_values(m, 0, 0, add_term(m, 0, 0, TERM_ADJOINT).adj, src, 3 * nadj, 3 * m->nadj_rec_local,
+                adj_device_buffer);
 }
 
 // compute_add_sources_acoustic_cuda.cu: sources in acoustic elements, chi'' -= sourcearray(1) stf / kappa
@@ -679,16 +733,14 @@ static void add_sources_ac(Mesh* m, int f, const double* h_stf, int nsrc, const 
   if (nsrc < m->nsources) fatal(where, "NSOURCES smaller than the number of prepared sources");
   std::vector<realw> s(m->nsources);
   for (int i = 0; i < m->nsources; i++) s[i] = (realw)h_stf[i];
-  flush_ac_terms(m, f);
-  launch_add_sources_ac(m->stream, m->src_ac_pts, m->src_array, m->src_kappa,
-                        source_values(m, s.data(), m->nsources, m->nsources, stf_device_buffer), m->ac[f].potdd);
+  source_values(m, 1, f, add_term(m, 1, f, TERM_SOURCE).src, s.data(), m->nsources, m->nsources, stf_device_buffer);
 }
 
 extern "C" void FC_FUNC_(compute_add_sources_ac_cuda, COMPUTE_ADD_SOURCES_AC_CUDA)(long* Mesh_pointer,
                                                                                  int* NSOURCESf,
                                                                                  double* h_stf_pre_compute,
                                                                                  int* run_number_of_the_source) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   (void)run_number_of_the_source;  // NB_RUNS_ACOUSTIC_GPU = 1 (prepare_constants_device refuses others)
   add_sources_ac(m, 0, h_stf_pre_compute, *NSOURCESf, "compute_add_sources_ac_cuda");
 }
@@ -697,7 +749,7 @@ extern "C" void FC_FUNC_(compute_add_sources_ac_s3_cuda, COMPUTE_ADD_SOURCES_AC_
                                                                                        int* NSOURCESf,
                                                                                        double* h_stf_pre_compute,
                                                                                        int* run_number_of_the_source) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   (void)run_number_of_the_source;
   add_sources_ac(m, 1, h_stf_pre_compute, *NSOURCESf, "compute_add_sources_ac_s3_cuda");
 }
@@ -708,7 +760,7 @@ extern "C" void FC_FUNC_(compute_add_sources_ac_s3_cuda, COMPUTE_ADD_SOURCES_AC_
 extern "C" void FC_FUNC_(add_sources_ac_sim_2_or_3_cuda, ADD_SOURCES_AC_SIM_2_OR_3_CUDA)(
     long* Mesh_pointer, realw* h_source_adjoint, int* nrec, int* nadj_rec_local, int* NTSTEP_BETWEEN_READ_ADJSRC,
     int* it) {
-  Mesh* m = from_handle(Mesh_pointer);
+  Mesh* m = from_handle_waiting(Mesh_pointer);
   (void)nrec;
   const int nadj = *nadj_rec_local;
   if (nadj <= 0 || m->adj_ac_pts.n == 0) return;
@@ -716,9 +768,8 @@ extern "C" void FC_FUNC_(add_sources_ac_sim_2_or_3_cuda, ADD_SOURCES_AC_SIM_2_OR
   const int nt = *NTSTEP_BETWEEN_READ_ADJSRC;
   const int isample = nt - ((*it - 1) % nt);  // 1-based
   const realw* src = h_source_adjoint + (int64_t)3 * nadj * (isample - 1);
-  flush_ac_terms(m, 0);
-  launch_adjoint_sources_ac(m->stream, m->adj_ac_pts, m->adj_h, source_values(m, src, 3 * nadj, 3 * m->nadj_rec_local, adj_device_buffer),
-                            m->ac[0].potdd);
+  source_values(m, 1, 0, add_term(m, 1, 0, TERM_ADJOINT).adj, src, 3 * nadj, 3 * m->nadj_rec_local,
+                adj_device_buffer);
 }
 
 // ---------------------------------------------------------------- seismograms (write_seismograms_cuda.cu:34)

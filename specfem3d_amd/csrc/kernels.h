@@ -320,30 +320,35 @@ void launch_acoustic(hipStream_t s, const AcousticArgs& a, bool exact);
 
 
 // boundary terms (k_boundary.hip)
-void launch_stacey_elastic(hipStream_t s, const FacePoints& f, const realw* veloc, realw* accel, realw* b_absorb,
-                           int mode);
-void launch_stacey_elastic_replay(hipStream_t s, const FacePoints& f, const realw* rec, realw* b_accel);
-void launch_stacey_acoustic(hipStream_t s, const FacePoints& f, const realw* potd, realw* potdd, realw* b_absorb,
-                            int mode);
-void launch_stacey_acoustic_replay(hipStream_t s, const FacePoints& f, const realw* rec, realw* b_potdd);
-void launch_coupling_ac_el(hipStream_t s, const FacePoints& f, const realw* displ, realw* potdd, int flip);
-void launch_coupling_el_ac(hipStream_t s, const FacePoints& f, const realw* potdd, realw* accel, int flip);
-void launch_free_surface(hipStream_t s, const FacePoints& f, realw* pot, realw* potd, realw* potdd);
-
-// values of the sources in one step: as a launch argument where they fit, else in device memory
+// values of the sources in one step: as a launch argument where they fit (a copy from pinned memory to
+// the device before the launch took 4 us of a 38 us step on 20x20x20 elements), else in device memory
 constexpr int SF_SRC_VALS = 256;
 struct SrcVals {
   realw v[SF_SRC_VALS];
   const realw* p;
 };
-// sources / receivers (k_sources.hip); FacePoints.ispec holds the owning source / receiver
-void launch_add_sources_el(hipStream_t s, const FacePoints& f, const realw* arr, const SrcVals& stf, realw* accel);
-void launch_add_sources_ac(hipStream_t s, const FacePoints& f, const realw* arr, const realw* kappa,
-                           const SrcVals& stf, realw* potdd);
-void launch_adjoint_sources_el(hipStream_t s, const FacePoints& f, const realw* h, const SrcVals& adj, realw* accel);
-void launch_adjoint_sources_ac(hipStream_t s, const FacePoints& f, const realw* h, const SrcVals& adj, realw* potdd);
-// receivers: `list` holds the local receiver indices to record (n of them; null: receivers 0..n-1);
-// out[3 r + c] is written for each listed receiver r
+enum { TERM_STACEY = 1, TERM_COUPLING = 2, TERM_SOURCE = 4, TERM_ADJOINT = 8 };
+struct TermArgs {
+  int n;                       // points that any term may touch
+  const int* iglob;
+  const int* head;             // 4 per point: its first face point, coupling point, source and adjoint pair, or -1
+  int terms, flip;             // TERM_*; sign of the coupling
+  FacePoints stacey, coupling, source, adjoint;  // of sources, ispec holds the owner
+  const realw* in;             // veloc or chi'
+  const realw* other;          // chi'' or displ of the coupling
+  realw* out;                  // accel or chi''
+  const realw *src_array, *src_kappa, *adj_h;
+  SrcVals src, adj;
+};
+void launch_terms(hipStream_t s, const TermArgs& a, bool fluid);
+// Stacey alone, also writing the boundary record
+void launch_stacey_elastic(hipStream_t s, const FacePoints& f, const realw* veloc, realw* accel, realw* b_absorb);
+void launch_stacey_elastic_replay(hipStream_t s, const FacePoints& f, const realw* rec, realw* b_accel);
+void launch_stacey_acoustic(hipStream_t s, const FacePoints& f, const realw* potd, realw* potdd, realw* b_absorb);
+void launch_stacey_acoustic_replay(hipStream_t s, const FacePoints& f, const realw* rec, realw* b_potdd);
+void launch_free_surface(hipStream_t s, const FacePoints& f, realw* pot, realw* potd, realw* potdd);
+
+// receivers (k_sources.hip)
 void launch_seismo_el(hipStream_t s, int n, const int* list, const int* iglob, const double* h, const double* nu,
                       const realw* field, realw* out);
 // ... of a field that waits to be summed (`what`: WAIT_*; first: slot entry of every receiver point)

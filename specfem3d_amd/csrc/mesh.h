@@ -67,6 +67,8 @@ struct Snapshot {            // one saved state of a wavefield (save_forward_arr
   realw* R = nullptr;        // 18 memory-variable planes (attenuation)
 };
 
+struct TermArgs;
+
 struct Mesh {
   int nspec = 0, nglob = 0, nspec_irregular = 0;
   int simulation_type = 1;
@@ -212,6 +214,12 @@ struct Mesh {
   realw pending_dt2_el[2] = {0.f, 0.f};
   int pending_k3_ac[2] = {0, 0};
   realw pending_dt2_ac[2] = {0.f, 0.f};
+  // terms of a step that wait to be launched together (TermArgs, k_boundary.hip), per domain (0 solid, 1
+  // fluid) and field: every entry point but those that add terms or start the stiffness launches them
+  TermArgs* terms[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
+  int term_n[2] = {0, 0};          // points that any term of the domain may touch
+  int* term_iglob[2] = {nullptr, nullptr};
+  int* term_head[2] = {nullptr, nullptr};
   // gather assembly of the solid: slots of each global point in list order (the processing order, or
   // the colour order under assembly = 2), the C-PML elements last
   int* asm_idx = nullptr;
