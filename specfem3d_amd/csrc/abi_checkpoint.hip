@@ -106,7 +106,7 @@ extern "C" void sf_snapshot_load(long* Mesh_pointer, int FORWARD_OR_ADJOINT, int
     ck_copy(m, m->ac[f].pot, s.ac, n);
     ck_copy(m, m->ac[f].potd, s.ac + n, n);
     ck_copy(m, m->ac[f].potdd, s.ac + 2 * n, n);
-    m->potdd_clean[f] = m->free_zero[f] = 0;
+    m->potdd_clean[f] = m->free_zero[f] = m->low_ac_set[f] = 0;
   }
   if (m->attenuation && m->att[f].R) {
     if (!s.R) fatal("sf_snapshot_load", "snapshot holds no memory variables");
@@ -159,7 +159,7 @@ extern "C" void sf_history_load(long* Mesh_pointer, int FORWARD_OR_ADJOINT, int 
   if (m->history_ac && m->ac[f].pot) {
     ck_copy(m, m->ac[f].pot, m->history_ac + (int64_t)frame * 2 * n, n);
     ck_copy(m, m->ac[f].potdd, m->history_ac + (int64_t)frame * 2 * n + n, n);
-    m->potdd_clean[f] = m->free_zero[f] = 0;
+    m->potdd_clean[f] = m->free_zero[f] = m->low_ac_set[f] = 0;
   }
 }
 

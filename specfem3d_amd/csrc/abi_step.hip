@@ -100,6 +100,8 @@ static GatherArgs gather_args_ac(Mesh* m, int f) {
   a.a = m->ac[f].potdd;
   a.rm1 = m->rmass_ac;
   a.dt2p = m->pending_dt2_ac[f];
+  a.lo = m->exact ? nullptr : m->low_ac[f];
+  a.lo_set = m->low_ac_set[f];
   return a;
 }
 
@@ -108,6 +110,7 @@ static void sum_ac(Mesh* m, int f) {
   if (m->pending_gather_ac[f]) {
     launch_gather_update(m->stream, gather_args_ac(m, f), 1, m->pending_k3_ac[f] ? GATHER_CORRECT : GATHER_ONLY,
                          m->exact != 0);
+    if (m->pending_k3_ac[f]) m->low_ac_set[f] = m->low_ac[f] && !m->exact;
     if (m->gather_skip_ac[f]) fz |= FREE_DD;
     else fz = m->pending_k3_ac[f] ? 0 : fz & FREE_POT;
     m->pending_gather_ac[f] = 0;
@@ -119,6 +122,7 @@ static void sum_ac(Mesh* m, int f) {
                      m->pending_dt2_ac[f]);
     if (!(fz & FREE_DD)) fz = 0;
     m->potdd_clean[f] = 0;
+    m->low_ac_set[f] = 0;
   }
   m->pending_k3_ac[f] = 0;
 }
@@ -329,9 +333,15 @@ extern "C" void FC_FUNC_(update_displacement_ac_cuda, UPDATE_DISPLACEMENT_AC_CUD
     ga.dtsq2 = *deltatsqover2_F;
     launch_gather_update(m->stream, ga, 1, GATHER_STEP, m->exact != 0);
     dd = m->gather_skip_ac[f] != 0;
+    m->low_ac_set[f] = ga.lo != nullptr;
   } else if (m->pending_k3_ac[f]) {
+    m->low_ac_set[f] = 0;
     launch_corrector_predictor(m->stream, m->ac_n, a.pot + g0, a.potd + g0, a.potdd + g0, m->rmass_ac + g0,
                                m->pending_dt2_ac[f], *deltat_F, *deltatover2_F, *deltatsqover2_F);
+  } else if (m->low_ac[f] && !m->exact) {
+    launch_predictor_low(m->stream, m->ac_n, a.pot + g0, a.potd + g0, a.potdd + g0, *deltat_F, *deltatover2_F,
+                         *deltatsqover2_F, m->low_ac[f] + g0, m->low_ac_set[f]);
+    m->low_ac_set[f] = 1;
   } else {
     launch_predictor(m->stream, m->ac_n, a.pot + g0, a.potd + g0, a.potdd + g0, *deltat_F, *deltatover2_F,
                      *deltatsqover2_F);
@@ -457,7 +467,7 @@ extern "C" void FC_FUNC_(acoustic_enforce_free_surf_cuda, ACOUSTIC_ENFORCE_FREE_
     if (!m->ac[f].pot) continue;
     const int known = m->pending_gather_ac[f] ? FREE_POT : FREE_POT | FREE_DD;
     if ((m->free_zero[f] & known) != known)
-      launch_free_surface(m->stream, m->free_ac, m->ac[f].pot, m->ac[f].potd, m->ac[f].potdd);
+      launch_free_surface(m->stream, m->free_ac, m->ac[f].pot, m->ac[f].potd, m->ac[f].potdd);  // low parts of 0 are 0
     if (m->pending_gather_ac[f]) m->gather_skip_ac[f] |= AF_EDGE;
     m->free_zero[f] |= known;
   }
@@ -974,7 +984,7 @@ SF_XFER1(transfer_b_accel_from_device, 1, accel, D2H)
     DIR(m, m->ac[F].pot, p, *size);                                                                            \
     DIR(m, m->ac[F].potd, pd, *size);                                                                          \
     DIR(m, m->ac[F].potdd, pdd, *size);                                                                        \
-    m->potdd_clean[F] = m->free_zero[F] = 0;                                                                   \
+    m->potdd_clean[F] = m->free_zero[F] = m->low_ac_set[F] = 0;                                                \
   }
 #define SF_XFERAC1(NAME, F, MEMBER, DIR)                                          \
   extern "C" void FC_FUNC_(NAME, X)(int* size, realw* arr, long* Mesh_pointer) { \
@@ -982,7 +992,7 @@ SF_XFER1(transfer_b_accel_from_device, 1, accel, D2H)
     if (!m->ac[F].pot) fatal(#NAME, "acoustic field not prepared");               \
     flush_ac(m, F);                                                               \
     DIR(m, m->ac[F].MEMBER, arr, *size);                                          \
-    m->potdd_clean[F] = m->free_zero[F] = 0;                                      \
+    m->potdd_clean[F] = m->free_zero[F] = m->low_ac_set[F] = 0;                   \
   }
 SF_XFERAC3(transfer_fields_ac_to_device, 0, H2D)
 SF_XFERAC3(transfer_fields_ac_from_device, 0, D2H)

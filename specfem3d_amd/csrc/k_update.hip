@@ -216,7 +216,9 @@ __device__ __forceinline__ int wave_prefix(int x) {
 // Against 64 bits, the kernels of 19x17x16 elements under a sea are off by 0.53 instead of 0.84 times, of
 // 24^3 elements by 0.44 instead of 0.69 times what single-precision sums gave (geometric means over 48
 // and 24 outputs). Each pass takes 2 us more on 24^3 elements (15.7 -> 17.4, k_predictor 10.5 -> 12.7),
-// 3 % of a run.
+// 3 % of a run. Runs of a fluid alone keep them too: chi'' is made of differences of chi, so the
+// rounding of chi reaches the pressure 10 times larger than that of u the displacement: pressure
+// records of 40x40x30 elements are off by 4.4e-7 instead of 2e-6, for 20.2 -> 22.7 us per pass.
 template <int NC, int KIND, bool OLD, typename T, bool LOW>
 __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
   const int nb = (int)gridDim.x, b = (int)blockIdx.x;
@@ -314,8 +316,8 @@ template <int NC, int KIND, bool OLD>
 static void launch_gather(hipStream_t s, const GatherArgs& a, bool exact) {
   const dim3 grid = sf_grid(a.n, 256), block(256);
   if (exact) hipLaunchKernelGGL((k_gather_update<NC, KIND, OLD, float, false>), grid, block, 0, s, a);
-  else if (NC == 3 && !OLD && KIND != GATHER_ONLY && a.lo)
-    hipLaunchKernelGGL((k_gather_update<3, KIND, false, double, (KIND != GATHER_ONLY)>), grid, block, 0, s, a);
+  else if (!OLD && KIND != GATHER_ONLY && a.lo)
+    hipLaunchKernelGGL((k_gather_update<NC, KIND, false, double, (KIND != GATHER_ONLY)>), grid, block, 0, s, a);
   else hipLaunchKernelGGL((k_gather_update<NC, KIND, OLD, double, false>), grid, block, 0, s, a);
 }
 

@@ -98,7 +98,7 @@ struct GatherArgs {
   int lo_set;                  // they are set (else zero)
 };
 // Low parts of u and v: what the stored single-precision values miss, in 1/256 of their last place, one
-// byte each (u in the low one). Kernel runs of FMA builds keep them (see k_gather_update). Values
+// byte each (u in the low one). FMA builds keep them in kernel runs and in runs of a fluid alone (see k_gather_update). Values
 // below 2^-95, infinities and NaN have none.
 __device__ __forceinline__ double with_low(realw x, int low) {
   const int e = __float_as_uint(x) >> 23 & 255;
@@ -135,7 +135,9 @@ __device__ __forceinline__ void waiting_value(const GatherArgs& A, int what, int
 #pragma unroll
   for (int c = 0; c < NC; c++) {
     a[c] = a[c] * (T)(NC == 3 && (fl & AF_MASS3) ? A.rm[NC * g + c] : A.rm1[g]);
-    out[c] = what == WAIT_ACCEL ? (realw)a[c] : (realw)((T)A.v[NC * g + c] + (T)A.dt2p * a[c]);
+    T v = A.v[NC * g + c];
+    if (sizeof(T) == 8 && A.lo && A.lo_set) v = (T)with_low(A.v[NC * g + c], A.lo[NC * g + c] >> 8);
+    out[c] = what == WAIT_ACCEL ? (realw)a[c] : (realw)(v + (T)A.dt2p * a[c]);
   }
 }
 // exact: the reference's single-precision operations; else sums, corrector and predictor in double
