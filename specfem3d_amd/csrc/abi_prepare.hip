@@ -786,7 +786,7 @@ void ensure_gather_assembly(Mesh* m, int f) {
   const int first_pml = (m->nspec_elastic + eb - 1) / eb * eb;
   if (!m->asm_buf[f]) m->asm_buf[f] = dmalloc<realw>(3 * 125 * ((int64_t)m->nspec + 2 * eb));  // both lists, rounded up
   if (m->simulation_type == 3 && !m->low[f]) {
-    m->low[f] = dmalloc<uint16_t>(3 * (int64_t)m->nglob);
+    m->low[f] = dmalloc<uint8_t>(3 * (int64_t)m->nglob);
     m->low_set[f] = 0;
   }
   if (m->asm_ready) return;
@@ -852,7 +852,7 @@ void ensure_gather_acoustic(Mesh* m, int f) {
   const int eb = 20;
   if (!m->asm_ac_buf[f]) m->asm_ac_buf[f] = dmalloc<realw>(125 * ((int64_t)m->nspec_acoustic + eb));
   if (m->nspec_elastic == 0 && m->pml_n == 0 && !m->low_ac[f]) {
-    m->low_ac[f] = dmalloc<uint16_t>(m->nglob);
+    m->low_ac[f] = dmalloc<uint8_t>(m->nglob);
     m->low_ac_set[f] = 0;
   }
   if (m->asm_ac_ready) return;

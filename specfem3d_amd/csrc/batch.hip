@@ -56,6 +56,7 @@ struct Batch {
   // of `loc_groups` groups of eight shots (all of them unless the card has no room)
   int *asm_ptr = nullptr, *asm_idx = nullptr, *ac_ptr = nullptr, *ac_idx = nullptr;
   uint16_t* info = nullptr;
+  uint8_t* low = nullptr;        // low parts of u and v (BatchGatherArgs::low)
   realw *local = nullptr, *ac_local = nullptr;
   int loc_groups = 0, ac_loc_groups = 0;
   int max_groups = 1 << 20;      // "local_groups"
@@ -145,6 +146,12 @@ __global__ void __launch_bounds__(256) k_batch_update(int64_t nrow, const int* _
 // LDS 1.6) and this one by HBM (3.96 ms, 19.3 GB, 4.9 TB/s). Steps before and after: 32x32x16 x 16
 // shots 598 -> 500 us, 64x64x32 x 32 8.53 -> 7.56 ms, viscoelastic 18x18x12 x 8 319 -> 233 us and
 // 40x40x20 x 16 4.02 -> 3.41 ms.
+// LOW (FMA builds that sum all groups here): u and v are carried with their low parts. Records of shots
+// from rest are often the first arrival of a front that grows by decades, and what the rounding of u in
+// every step left behind it is most of their error: against 64 bits those
+// of 32x32x16 x 16 are off by 0.40 instead of 0.59 times what single-precision sums gave (geometric mean
+// over 96), and none of 140 by more than 1.5 times, where 5 of 21 were; 235 -> 259 us per pass there, 28 ->
+// 33 on 18x18x12 x 8.
 struct BatchGatherArgs {
   int64_t g0, n, nrow;           // global points [g0, g0 + n), rows of a group
   const int *ptr, *idx;
@@ -156,6 +163,7 @@ struct BatchGatherArgs {
   realw *u, *v, *a;
   const realw* rm;
   realw dt2p, dt, dt2, dtsq2;
+  uint8_t* low;                  // low parts of u and v (with_low) in the layout of u, or null
 };
 
 // a -= the local forces of slots ptr[g] .. ptr[g + 1], `unit` floats per slot, four slots in flight
@@ -190,7 +198,7 @@ __device__ __forceinline__ int64_t xcd_block() {
 }
 
 // T: float follows the reference's operations (exact builds), double rounds once per stored value
-template <bool STEP, typename T>
+template <bool STEP, typename T, bool LOW>
 __global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs A) {
   const int64_t t = xcd_block() * 256 + threadIdx.x;
   const int64_t pt = t / 6;
@@ -210,6 +218,8 @@ __global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs A) {
     V = *reinterpret_cast<const float4*>(A.v + o);
     M = A.rm[3 * g + c];
   }
+  uchar4 L = make_uchar4(0, 0, 0, 0);
+  if (LOW) L = *reinterpret_cast<const uchar4*>(A.low + o);
   if (term) {
     const float4 a0 = *reinterpret_cast<const float4*>(A.a + o);
     a[0] = a0.x; a[1] = a0.y; a[2] = a0.z; a[3] = a0.w;
@@ -222,14 +232,22 @@ __global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs A) {
 #define SF_BG(c, r)                                             \
   if (r == 0 || A.nstep[s + r] >= it) {                         \
     const T ac = a[r] * (T)M;                                   \
-    T vc = (T)V.c + (T)A.dt2p * ac;                             \
-    U.c = (realw)((T)U.c + (T)A.dt * vc + (T)A.dtsq2 * ac);     \
-    V.c = (realw)(vc + (T)A.dt2 * ac);                          \
+    T vc = (LOW ? (T)with_low(V.c, L.c >> 4) : (T)V.c) + (T)A.dt2p * ac;                                    \
+    const T un = (LOW ? (T)with_low(U.c, L.c) : (T)U.c) + (T)A.dt * vc + (T)A.dtsq2 * ac;                   \
+    vc = vc + (T)A.dt2 * ac;                                    \
+    if (LOW) {                                                  \
+      const int lu = split_low(un, U.c);                        \
+      L.c = (uint8_t)(lu | split_low(vc, V.c) << 4);            \
+    } else {                                                    \
+      U.c = (realw)un;                                          \
+      V.c = (realw)vc;                                          \
+    }                                                           \
   }
   SF_BG(x, 0) SF_BG(y, 1) SF_BG(z, 2) SF_BG(w, 3)
 #undef SF_BG
   *reinterpret_cast<float4*>(A.u + o) = U;
   *reinterpret_cast<float4*>(A.v + o) = V;
+  if (LOW) *reinterpret_cast<uchar4*>(A.low + o) = L;
   if (term) *reinterpret_cast<float4*>(A.a + o) = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
@@ -505,6 +523,8 @@ static void zero_state(Batch* b) {
   const int64_t n = 3 * (int64_t)m->nglob * b->S;
   for (realw* p : {b->u, b->v, b->a})
     hipLaunchKernelGGL(k_batch_fill, sf_grid(n, 256), dim3(256), 0, m->stream, n, p);
+  if (b->low)  // a byte each; S is a multiple of eight
+    hipLaunchKernelGGL(k_batch_fill, sf_grid(n / 4, 256), dim3(256), 0, m->stream, n / 4, reinterpret_cast<realw*>(b->low));
   if (b->ac) {
     const int64_t na = b->ac_n * b->S;
     for (realw* p : {b->pot, b->potd, b->potdd})
@@ -581,6 +601,17 @@ static void build_gather(Batch* b) {
                            m->nspec_acoustic, 0, 1, 1, m->ibool, b->ac_ptr, b->ac_idx);
   if (b->ac && !b->ac_local)
     b->ac_local = local_room((int64_t)m->nspec_acoustic * 1000, std::min(b->S / 8, b->max_groups), &b->ac_loc_groups);
+  if (!b->low && !m->exact && b->loc_groups == b->S / 8) {
+    // less precise without, where the card has no room for it
+    const size_t bytes = 3 * (size_t)m->nglob * b->S;
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) {
+      b->low = reinterpret_cast<uint8_t*>(p);
+      SF_CHECK(hipMemsetAsync(b->low, 0, bytes, m->stream));
+    } else {
+      (void)hipGetLastError();
+    }
+  }
   if (!b->info) b->info = balloc<uint16_t>(m->nglob);
   SF_CHECK(hipMemsetAsync(b->info, 0, sizeof(uint16_t) * (size_t)m->nglob, m->stream));
   if (m->stacey) launch_mark_points(m->stream, m->abs_el.n, m->abs_el.iglob, AF_TERM, b->info);
@@ -592,6 +623,7 @@ static void build_gather(Batch* b) {
 static BatchGatherArgs gather_args(Batch* b) {
   Mesh* m = b->m;
   BatchGatherArgs A;
+  A.low = b->loc_groups == b->S / 8 ? b->low : nullptr;
   A.g0 = m->el_g0;
   A.n = m->el_n;
   A.nrow = 3 * (int64_t)m->nglob;
@@ -663,8 +695,8 @@ static void enqueue_stiffness(Batch* b, hipStream_t st) {
       BatchGatherArgs ga = gather_args(b);
       ga.first_group = g;
       const dim3 grid(sf_grid(6 * ga.n, 256).x, (unsigned)n);
-      if (m->exact) hipLaunchKernelGGL((k_batch_gather<false, float>), grid, dim3(256), 0, st, ga);
-      else hipLaunchKernelGGL((k_batch_gather<false, double>), grid, dim3(256), 0, st, ga);
+      if (m->exact) hipLaunchKernelGGL((k_batch_gather<false, float, false>), grid, dim3(256), 0, st, ga);
+      else hipLaunchKernelGGL((k_batch_gather<false, double, false>), grid, dim3(256), 0, st, ga);
       SF_LAUNCH_CHECK("k_batch_gather");
     }
   }
@@ -743,8 +775,9 @@ static void enqueue_step(Batch* b, hipStream_t st, bool first) {
     if (b->loc_groups == b->S / 8) {
       const BatchGatherArgs ga = gather_args(b);
       const dim3 grid(sf_grid(6 * ga.n, 256).x, (unsigned)(b->S / 8));
-      if (m->exact) hipLaunchKernelGGL((k_batch_gather<true, float>), grid, dim3(256), 0, st, ga);
-      else hipLaunchKernelGGL((k_batch_gather<true, double>), grid, dim3(256), 0, st, ga);
+      if (m->exact) hipLaunchKernelGGL((k_batch_gather<true, float, false>), grid, dim3(256), 0, st, ga);
+      else if (ga.low) hipLaunchKernelGGL((k_batch_gather<true, double, true>), grid, dim3(256), 0, st, ga);
+      else hipLaunchKernelGGL((k_batch_gather<true, double, false>), grid, dim3(256), 0, st, ga);
       SF_LAUNCH_CHECK("k_batch_gather");
     } else {
       const int64_t nrow = 3 * (int64_t)m->nglob;
@@ -1181,7 +1214,7 @@ extern "C" void sf_batch_destroy(long h) {
   drop_graph(b);
   bfree(b->d_nstep); bfree(b->d_it); bfree(b->u); bfree(b->v); bfree(b->a); bfree(b->R); bfree(b->eps);
   bfree(b->pot); bfree(b->potd); bfree(b->potdd);
-  bfree(b->asm_ptr); bfree(b->asm_idx); bfree(b->ac_ptr); bfree(b->ac_idx); bfree(b->info);
+  bfree(b->asm_ptr); bfree(b->asm_idx); bfree(b->ac_ptr); bfree(b->ac_idx); bfree(b->info); bfree(b->low);
   bfree(b->local); bfree(b->ac_local);
   bfree(b->src_ig); bfree(b->src_slot); bfree(b->src_id); bfree(b->src_ploc); bfree(b->src_arr); bfree(b->src_stf);
   bfree(b->rec_slot); bfree(b->rec_ig); bfree(b->rec_h); bfree(b->rec_nu); bfree(b->seis);

@@ -38,22 +38,22 @@ __global__ void k_predictor(int64_t n4, int64_t n, realw* __restrict__ u, realw*
 }
 
 // the predictor with the low parts of u and v
-__device__ __forceinline__ void predict_low(realw& u, realw& v, realw a, realw dt, realw dt2, realw dtsq2, uint16_t& lo,
+__device__ __forceinline__ void predict_low(realw& u, realw& v, realw a, realw dt, realw dt2, realw dtsq2, uint8_t& lo,
                                             int set) {
   const int low = set ? lo : 0;
-  const double vc = with_low(v, low >> 8), uc = with_low(u, low), ac = a;
+  const double vc = with_low(v, low >> 4), uc = with_low(u, low), ac = a;
   const int lu = split_low(uc + (double)dt * vc + (double)dtsq2 * ac, u);
-  lo = (uint16_t)(lu | split_low(vc + (double)dt2 * ac, v) << 8);
+  lo = (uint8_t)(lu | split_low(vc + (double)dt2 * ac, v) << 4);
 }
 __global__ void k_predictor_low(int64_t n4, int64_t n, realw* __restrict__ u, realw* __restrict__ v,
-                                realw* __restrict__ a, realw dt, realw dt2, realw dtsq2, uint16_t* __restrict__ lo,
+                                realw* __restrict__ a, realw dt, realw dt2, realw dtsq2, uint8_t* __restrict__ lo,
                                 int set) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n4) {
     float4 U = reinterpret_cast<float4*>(u)[t];
     float4 V = reinterpret_cast<float4*>(v)[t];
     const float4 A = reinterpret_cast<float4*>(a)[t];
-    ushort4 L = reinterpret_cast<ushort4*>(lo)[t];
+    uchar4 L = reinterpret_cast<uchar4*>(lo)[t];
     predict_low(U.x, V.x, A.x, dt, dt2, dtsq2, L.x, set);
     predict_low(U.y, V.y, A.y, dt, dt2, dtsq2, L.y, set);
     predict_low(U.z, V.z, A.z, dt, dt2, dtsq2, L.z, set);
@@ -61,7 +61,7 @@ __global__ void k_predictor_low(int64_t n4, int64_t n, realw* __restrict__ u, re
     reinterpret_cast<float4*>(u)[t] = U;
     reinterpret_cast<float4*>(v)[t] = V;
     reinterpret_cast<float4*>(a)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-    reinterpret_cast<ushort4*>(lo)[t] = L;
+    reinterpret_cast<uchar4*>(lo)[t] = L;
   }
   const int64_t r = 4 * n4 + t;
   if (t < 4 && r < n) {
@@ -210,15 +210,16 @@ __device__ __forceinline__ int wave_prefix(int x) {
 }
 
 //
-// LOW: with the low parts of u and v, so that the values carried from step to step have 8 more bits
+// LOW: with the low parts of u and v, so that the values carried from step to step have 4 more bits
 // (other kernels read u and v as stored). Kernel runs keep them: their outputs are products of two
 // fields, some of them a few points large, where the rounding of u in every step is most of the error.
-// Against 64 bits, the kernels of 19x17x16 elements under a sea are off by 0.53 instead of 0.84 times, of
-// 24^3 elements by 0.44 instead of 0.69 times what single-precision sums gave (geometric means over 48
-// and 24 outputs). Each pass takes 2 us more on 24^3 elements (15.7 -> 17.4, k_predictor 10.5 -> 12.7),
-// 3 % of a run. Runs of a fluid alone keep them too: chi'' is made of differences of chi, so the
-// rounding of chi reaches the pressure 10 times larger than that of u the displacement: pressure
-// records of 40x40x30 elements are off by 4.4e-7 instead of 2e-6, for 20.2 -> 22.7 us per pass.
+// Against 64 bits, the kernels of 19x17x16 elements under a sea are off by 0.48 instead of 0.84 times, of
+// 24^3 elements by 0.52 instead of 0.69 times what single-precision sums gave (geometric means over 36
+// and 16 outputs; 8 more bits instead of 4: 0.53 and 0.44 over 48 and 24). Each pass takes 1.5 us more
+// on 24^3 elements (15.7 -> 17.2, k_predictor 10.5 -> 12.0). Runs of a fluid alone keep them too: chi''
+// is made of differences of chi, so the rounding of chi reaches the pressure 10 times larger than that of u
+// the displacement: pressure records of 40x40x30 elements are off by 4.9e-7 instead of 2e-6, for 20.2 ->
+// 22.2 us per pass.
 template <int NC, int KIND, bool OLD, typename T, bool LOW>
 __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
   const int nb = (int)gridDim.x, b = (int)blockIdx.x;
@@ -289,13 +290,13 @@ __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
 #pragma unroll
   for (int c = 0; c < NC; c++) {
     a[c] = a[c] * (T)m[c];
-    T vc = (LOW ? (T)with_low(v[c], low[c] >> 8) : (T)v[c]) + (T)A.dt2p * a[c];
+    T vc = (LOW ? (T)with_low(v[c], low[c] >> 4) : (T)v[c]) + (T)A.dt2p * a[c];
     if (KIND == GATHER_STEP) {
       T uc = LOW ? (T)with_low(u[c], low[c]) : (T)u[c];
       if (OLD) A.old[NC * g + c] = (realw)(uc + (T)A.t1 * vc + (T)A.t2 * a[c]);
       uc = uc + (T)A.dt * vc + (T)A.dtsq2 * a[c];
       vc = vc + (T)A.dt2 * a[c];
-      if (LOW) low[c] = (low[c] & 0xff00) | split_low(uc, u[c]);
+      if (LOW) low[c] = (low[c] & 0xf0) | split_low(uc, u[c]);
       else u[c] = (realw)uc;
       A.u[NC * g + c] = u[c];
       if (full) A.a[NC * g + c] = 0.f;
@@ -303,8 +304,8 @@ __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
       A.a[NC * g + c] = (realw)a[c];
     }
     if (LOW) {
-      low[c] = (low[c] & 0xff) | split_low(vc, v[c]) << 8;
-      A.lo[NC * g + c] = (uint16_t)low[c];
+      low[c] = (low[c] & 15) | split_low(vc, v[c]) << 4;
+      A.lo[NC * g + c] = (uint8_t)low[c];
     } else {
       v[c] = (realw)vc;
     }
@@ -350,7 +351,7 @@ void launch_predictor(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, re
 }
 
 void launch_predictor_low(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, realw dt, realw dt2, realw dtsq2,
-                          uint16_t* lo, int set) {
+                          uint8_t* lo, int set) {
   if (n <= 0) return;
   const int64_t n4 = n / 4;
   hipLaunchKernelGGL(k_predictor_low, grid_for(n4, 256), dim3(256), 0, s, n4, n, u, v, a, dt, dt2, dtsq2, lo, set);

@@ -57,7 +57,7 @@ void launch_predictor(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, re
 void launch_corrector(hipStream_t s, int64_t n, realw* v, realw* a, const realw* rmass, realw dt2);
 // ... in double precision with the low parts of u and v (`set`: they are set, else zero)
 void launch_predictor_low(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, realw dt, realw dt2, realw dtsq2,
-                          uint16_t* lo, int set);
+                          uint8_t* lo, int set);
 // with `old`, also PML_displ_old = u + t1 v + t2 a of the corrected field (before the predictor)
 void launch_corrector_predictor(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, const realw* rmass,
                                 realw dt2_prev, realw dt, realw dt2, realw dtsq2, realw* old = nullptr,
@@ -94,24 +94,24 @@ struct GatherArgs {
   realw dt, dt2, dtsq2;        // predictor
   realw* old;                  // PML_displ_old = u + t1 v + t2 a of the corrected field, or null
   realw t1, t2;
-  uint16_t* lo;                // low parts of v and u (LowParts), 3 per point, or null
+  uint8_t* lo;                 // low parts of u and v (with_low), 3 per point, or null
   int lo_set;                  // they are set (else zero)
 };
-// Low parts of u and v: what the stored single-precision values miss, in 1/256 of their last place, one
-// byte each (u in the low one). FMA builds keep them in kernel runs and in runs of a fluid alone (see k_gather_update). Values
-// below 2^-95, infinities and NaN have none.
+// Low parts of u and v: what the stored single-precision values miss, in 1/16 of their last place, four
+// bits each (u in the low ones). FMA builds keep them in batches, in kernel runs and in runs of a fluid
+// alone (see k_gather_update). Values below 2^-95, infinities and NaN have none.
 __device__ __forceinline__ double with_low(realw x, int low) {
   const int e = __float_as_uint(x) >> 23 & 255;
-  const realw unit = e >= 32 && e < 255 ? __uint_as_float((uint32_t)(e - 31) << 23) : 0.f;
-  return (double)x + (double)((realw)(int8_t)low * unit);
+  const realw unit = e >= 32 && e < 255 ? __uint_as_float((uint32_t)(e - 27) << 23) : 0.f;
+  return (double)x + (double)((realw)((int)((uint32_t)low << 28) >> 28) * unit);
 }
-// rounds x to `hi`, returns the byte of the rest
+// rounds x to `hi`, returns the four bits of the rest
 __device__ __forceinline__ int split_low(double x, realw& hi) {
   hi = (realw)x;
   const int e = __float_as_uint(hi) >> 23 & 255;
   if (e < 32 || e == 255) return 0;
-  const realw q = rintf((realw)(x - (double)hi) * __uint_as_float((uint32_t)(285 - e) << 23));
-  return (int)fminf(fmaxf(q, -127.f), 127.f) & 0xff;
+  const realw q = rintf((realw)(x - (double)hi) * __uint_as_float((uint32_t)(281 - e) << 23));
+  return (int)fminf(fmaxf(q, -8.f), 7.f) & 15;
 }
 // what follows the sum: nothing (accel is left assembled), the corrector, or the corrector and the
 // predictor of the next step (accel left zero)
@@ -136,7 +136,7 @@ __device__ __forceinline__ void waiting_value(const GatherArgs& A, int what, int
   for (int c = 0; c < NC; c++) {
     a[c] = a[c] * (T)(NC == 3 && (fl & AF_MASS3) ? A.rm[NC * g + c] : A.rm1[g]);
     T v = A.v[NC * g + c];
-    if (sizeof(T) == 8 && A.lo && A.lo_set) v = (T)with_low(A.v[NC * g + c], A.lo[NC * g + c] >> 8);
+    if (sizeof(T) == 8 && A.lo && A.lo_set) v = (T)with_low(A.v[NC * g + c], A.lo[NC * g + c] >> 4);
     out[c] = what == WAIT_ACCEL ? (realw)a[c] : (realw)(v + (T)A.dt2p * a[c]);
   }
 }

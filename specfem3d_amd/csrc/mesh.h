@@ -236,9 +236,9 @@ struct Mesh {
   int pending_gather_el[2] = {0, 0};
   int gather_skip_el[2] = {0, 0};  // AF_* of the points that the pending sum leaves out
   int accel_clean[2] = {0, 0};     // accel is zero at every point without AF_TERM
-  uint16_t* low[2] = {nullptr, nullptr};  // low parts of u and v (GatherArgs::lo): kernel runs
+  uint8_t* low[2] = {nullptr, nullptr};  // low parts of u and v (GatherArgs::lo): kernel runs
   int low_set[2] = {0, 0};         // they belong to the stored u and v
-  uint16_t* low_ac[2] = {nullptr, nullptr};  // the same of chi and chi': runs of a fluid alone
+  uint8_t* low_ac[2] = {nullptr, nullptr};  // the same of chi and chi': runs of a fluid alone
   int low_ac_set[2] = {0, 0};
   // the same for the fluid (1 component; the inverse mass is rmass_ac)
   int* asm_ac_idx = nullptr;
