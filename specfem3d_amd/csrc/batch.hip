@@ -13,12 +13,12 @@
 //     side of the coupling with the elastic boundary terms (the single-shot call order of
 //     iterate_time.F90);
 //   * one step = sum of the local forces with the corrector and predictor (k_batch_gather), Stacey,
-//     source rounds, stiffness (one launch that stores local forces), receivers, and a one-lane
-//     kernel that advances the device step counter. Every kernel reads the counter, so a group of
-//     steps is captured once into a hipGraph and replayed;
+//     with the receivers, source rounds, stiffness (one launch that stores local forces), and a kernel
+//     that advances the device step counter after a step or a captured group. Every kernel reads the
+//     counter, so a group of steps is captured once into a hipGraph and replayed;
 //   * the per-point arithmetic and the order of every sum equal the single-shot path (same
-//     kernels' expressions, same colour order, same order of faces), so each shot of a batch is
-//     bit-identical to its single-shot run with the same options.
+//     kernels' expressions, same colour order, same order of faces), so without FMA contraction each shot
+//     of a batch is bit-identical to its single-shot run; FMA builds also carry low parts of u and v.
 // Shots-per-workgroup are chosen by an autotuner that times each candidate for a few steps from rest
 // and then resets the batch.
 #include <algorithm>
@@ -44,7 +44,8 @@ struct Batch {
   std::vector<int> nstep_user;   // per user shot
   std::vector<int> slot_of;      // user shot -> slot
   int* d_nstep = nullptr;        // per slot (S entries, decreasing, padding 0)
-  int* d_it = nullptr;
+  int* d_it = nullptr;           // step counter, plus 0, 1 .. IT_AHEAD - 1
+  int at = 0;                    // entry that the launches of a step read
   int h_it = 1;                  // host mirror of the step counter
   realw *u = nullptr, *v = nullptr, *a = nullptr;
   bool att = false;              // 3-SLS attenuation: per-shot memory variables and strain
@@ -91,6 +92,10 @@ static Batch* batch_of(long h) {
 }
 
 // ------------------------------------------------------------------------------ kernels
+// The step counter is kept with the next steps' values beside it: the steps of a captured group read one
+// each, and one launch advances them all (a launch per step took 4.5 us of it).
+constexpr int IT_AHEAD = 32;
+
 static __device__ __forceinline__ int load_it(const int* it) {
   return __hip_atomic_load(it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -308,35 +313,6 @@ __device__ __forceinline__ FaceLane face_lane(int n0, const int* nstep, const in
   return f;
 }
 
-// Stacey (k_stacey_el arithmetic)
-__global__ void k_batch_stacey(int n0, int64_t nrow, const int* __restrict__ ig, const realw* __restrict__ nrm,
-                               const realw* __restrict__ jw, const realw* __restrict__ rvp,
-                               const realw* __restrict__ rvs, const int* __restrict__ next,
-                               const int* __restrict__ nstep, const int* __restrict__ itp,
-                               const realw* __restrict__ veloc, realw* accel) {
-  const FaceLane f = face_lane(n0, nstep, itp);
-  if (!f.live) return;
-  const int64_t b = batch_idx(nrow, 3 * (int64_t)ig[f.t0], f.s);
-  const realw vx = veloc[b], vy = veloc[b + 8], vz = veloc[b + 16];
-  realw ax = accel[b], ay = accel[b + 8], az = accel[b + 16];
-  for (int q = f.t0; q >= 0; q = next[q]) {
-    const realw nx = nrm[3 * q], ny = nrm[3 * q + 1], nz = nrm[3 * q + 2];
-    const realw vn = vx * nx + vy * ny + vz * nz;
-    const realw p = rvp[q], sv = rvs[q];
-    const realw tx = p * vn * nx + sv * (vx - vn * nx);
-    const realw ty = p * vn * ny + sv * (vy - vn * ny);
-    const realw tz = p * vn * nz + sv * (vz - vn * nz);
-    const realw w = jw[q];
-    const realw fx = tx * w, fy = ty * w, fz = tz * w;
-    ax = ax - fx;
-    ay = ay - fy;
-    az = az - fz;
-  }
-  accel[b] = ax;
-  accel[b + 8] = ay;
-  accel[b + 16] = az;
-}
-
 // source entries of one round: accel += sourcearray * stf(it) (k_add_sources_el arithmetic)
 __global__ void k_batch_sources(int n, int64_t nrow, int max_nstep, const int* __restrict__ ig, const int* __restrict__ slot,
                                 const int* __restrict__ sid, const int* __restrict__ ploc,
@@ -356,17 +332,16 @@ __global__ void k_batch_sources(int n, int64_t nrow, int max_nstep, const int* _
 }
 
 // receivers (k_seismo_el arithmetic): one wave64 per receiver, FP64 sums, rotation by nu
-__global__ void __launch_bounds__(64) k_batch_seismo(int nrec, int64_t nrow, const int* __restrict__ slot,
-                                                     const int* __restrict__ ig, const double* __restrict__ h,
-                                                     const double* __restrict__ nu, const int* __restrict__ nstep,
-                                                     const int* __restrict__ itp, const realw* __restrict__ u,
-                                                     realw* __restrict__ seis) {
-  const int r = blockIdx.x;
+__device__ __forceinline__ void record(int r, int nrec, int64_t nrow, const int* __restrict__ slot,
+                                       const int* __restrict__ ig, const double* __restrict__ h,
+                                       const double* __restrict__ nu, const int* __restrict__ nstep,
+                                       const int* __restrict__ itp, const realw* __restrict__ u,
+                                       realw* __restrict__ seis) {
   if (r >= nrec) return;
   const int s = slot[r];
   const int it = load_it(itp);
   if (nstep[s] < it) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   double sx = 0.0, sy = 0.0, sz = 0.0;
   for (int p = lane; p < 125; p += 64) {
     const int64_t b = batch_idx(nrow, 3 * (int64_t)ig[(int64_t)r * 125 + p], s);
@@ -388,6 +363,45 @@ __global__ void __launch_bounds__(64) k_batch_seismo(int nrec, int64_t nrow, con
     o[1] = (realw)(n[3] * sx + n[4] * sy + n[5] * sz);
     o[2] = (realw)(n[6] * sx + n[7] * sy + n[8] * sz);
   }
+}
+
+// Stacey (k_stacey_el arithmetic)
+// and, in the blocks behind the first `fb`, the receivers: both need only the updated u and v, and a
+// launch of its own for the receivers took 5 us of a captured step
+__global__ void __launch_bounds__(256) k_batch_stacey_seismo(
+    int fb, int n0, int64_t nrow, const int* __restrict__ ig, const realw* __restrict__ nrm,
+    const realw* __restrict__ jw, const realw* __restrict__ rvp, const realw* __restrict__ rvs,
+    const int* __restrict__ next, const int* __restrict__ nstep, const int* __restrict__ itp,
+    const realw* __restrict__ veloc, realw* accel, int nrec, const int* __restrict__ slot,
+    const int* __restrict__ rec_ig, const double* __restrict__ h, const double* __restrict__ nu,
+    const realw* __restrict__ u, realw* __restrict__ seis) {
+  if ((int)blockIdx.x >= fb) {
+    // a wave per receiver
+    record(((((int)blockIdx.x - fb) * (int)gridDim.y + (int)blockIdx.y) << 2) + (int)(threadIdx.x >> 6), nrec, nrow, slot,
+           rec_ig, h, nu, nstep, itp, u, seis);
+    return;
+  }
+  const FaceLane f = face_lane(n0, nstep, itp);
+  if (!f.live) return;
+  const int64_t b = batch_idx(nrow, 3 * (int64_t)ig[f.t0], f.s);
+  const realw vx = veloc[b], vy = veloc[b + 8], vz = veloc[b + 16];
+  realw ax = accel[b], ay = accel[b + 8], az = accel[b + 16];
+  for (int q = f.t0; q >= 0; q = next[q]) {
+    const realw nx = nrm[3 * q], ny = nrm[3 * q + 1], nz = nrm[3 * q + 2];
+    const realw vn = vx * nx + vy * ny + vz * nz;
+    const realw p = rvp[q], sv = rvs[q];
+    const realw tx = p * vn * nx + sv * (vx - vn * nx);
+    const realw ty = p * vn * ny + sv * (vy - vn * ny);
+    const realw tz = p * vn * nz + sv * (vz - vn * nz);
+    const realw w = jw[q];
+    const realw fx = tx * w, fy = ty * w, fz = tz * w;
+    ax = ax - fx;
+    ay = ay - fy;
+    az = az - fz;
+  }
+  accel[b] = ax;
+  accel[b + 8] = ay;
+  accel[b + 16] = az;
 }
 
 // ---- fluid domain: potentials over the acoustic range, rows g - g0
@@ -479,9 +493,7 @@ __global__ void k_batch_coupling_el_ac(int n0, int64_t nrow, int64_t nrow_ac, in
   accel[e + 16] = az;
 }
 
-__global__ void k_batch_tick(int* itp) {
-  if (threadIdx.x == 0) itp[0] = itp[0] + 1;
-}
+__global__ void k_batch_tick(int* itp, int n) { itp[threadIdx.x] = itp[threadIdx.x] + n; }
 
 __global__ void k_batch_fill(int64_t n, realw* p) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -541,7 +553,9 @@ static void zero_state(Batch* b) {
   }
   SF_LAUNCH_CHECK("k_batch_fill");
   b->h_it = 1;
-  SF_CHECK(hipMemcpyAsync(b->d_it, &b->h_it, sizeof(int), hipMemcpyHostToDevice, m->stream));
+  int it[IT_AHEAD];
+  for (int k = 0; k < IT_AHEAD; k++) it[k] = b->h_it + k;
+  SF_CHECK(hipMemcpyAsync(b->d_it, it, sizeof(it), hipMemcpyHostToDevice, m->stream));
   SF_CHECK(hipStreamSynchronize(m->stream));
 }
 
@@ -634,7 +648,7 @@ static BatchGatherArgs gather_args(Batch* b) {
   A.first_group = 0;
   A.info = b->info;
   A.nstep = b->d_nstep;
-  A.it = b->d_it;
+  A.it = b->d_it + b->at;
   A.u = b->u;
   A.v = b->v;
   A.a = b->a;
@@ -666,7 +680,7 @@ static void enqueue_stiffness(Batch* b, hipStream_t st) {
   A.dt = b->dt;
   A.loc_group = (int64_t)m->nspec_elastic * 3000;
   A.nstep = b->d_nstep;
-  A.it = b->d_it;
+  A.it = b->d_it + b->at;
   if (b->att) {
     A.R = b->R;
     A.eps = b->eps;
@@ -702,13 +716,6 @@ static void enqueue_stiffness(Batch* b, hipStream_t st) {
   }
 }
 
-static void enqueue_seismo(Batch* b, hipStream_t st) {
-  if (b->nrec <= 0) return;
-  hipLaunchKernelGGL(k_batch_seismo, dim3(b->nrec), dim3(64), 0, st, b->nrec, 3 * (int64_t)b->m->nglob, b->rec_slot, b->rec_ig,
-                     b->rec_h, b->rec_nu, b->d_nstep, b->d_it, b->u, b->seis);
-  SF_LAUNCH_CHECK("k_batch_seismo");
-}
-
 // launches over (global point of the faces, shot)
 static dim3 face_grid(const FacePoints& f, int S) { return dim3(sf_grid(8 * (int64_t)f.points(), 256).x, (unsigned)(S / 8)); }
 
@@ -721,19 +728,19 @@ static void enqueue_fluid(Batch* b, hipStream_t st) {
   const int S = b->S;
   const int64_t na = b->ac_n, nrow = 3 * (int64_t)m->nglob;
   const dim3 rows(sf_grid(2 * na, 256).x, (unsigned)(S / 8));
-  hipLaunchKernelGGL(k_batch_ac_predictor, rows, dim3(256), 0, st, na, b->d_nstep, b->d_it, b->pot, b->potd,
+  hipLaunchKernelGGL(k_batch_ac_predictor, rows, dim3(256), 0, st, na, b->d_nstep, b->d_it + b->at, b->pot, b->potd,
                      b->potdd, b->dt, b->dt2, b->dtsq2);
   SF_LAUNCH_CHECK("k_batch_ac_predictor");
   const FacePoints& f = m->abs_ac;
   if (m->stacey && f.points() > 0) {
     hipLaunchKernelGGL(k_batch_stacey_ac, face_grid(f, S), dim3(256), 0, st, f.points(), na, b->ac_g0, f.iglob, f.jacw,
-                       f.imp_p, f.imp_s, f.next, b->d_nstep, b->d_it, b->potd, b->potdd);
+                       f.imp_p, f.imp_s, f.next, b->d_nstep, b->d_it + b->at, b->potd, b->potdd);
     SF_LAUNCH_CHECK("k_batch_stacey_ac");
   }
   const FacePoints& cf = m->coupling;
   if (cf.points() > 0) {
     hipLaunchKernelGGL(k_batch_coupling_ac_el, face_grid(cf, S), dim3(256), 0, st, cf.points(), nrow, na, b->ac_g0,
-                       cf.iglob, cf.normal, cf.jacw, cf.next, b->d_nstep, b->d_it, b->u, b->potdd);
+                       cf.iglob, cf.normal, cf.jacw, cf.next, b->d_nstep, b->d_it + b->at, b->u, b->potdd);
     SF_LAUNCH_CHECK("k_batch_coupling_ac_el");
   }
   BatchAcArgs A;
@@ -752,7 +759,7 @@ static void enqueue_fluid(Batch* b, hipStream_t st) {
   A.pot = b->pot;
   A.loc_group = (int64_t)m->nspec_acoustic * 1000;
   A.nstep = b->d_nstep;
-  A.it = b->d_it;
+  A.it = b->d_it + b->at;
   for (int g = 0; g < S / 8; g += b->ac_loc_groups) {
     const int n = std::min(b->ac_loc_groups, S / 8 - g);
     A.s_first = 8 * g;
@@ -761,7 +768,7 @@ static void enqueue_fluid(Batch* b, hipStream_t st) {
     launch_acoustic_batch(st, A, b->sc, m->exact != 0);
     auto* gather = m->exact ? &k_batch_ac_gather<float> : &k_batch_ac_gather<double>;
     hipLaunchKernelGGL(gather, dim3(rows.x, (unsigned)n), dim3(256), 0, st, na, b->ac_g0, b->ac_ptr, b->ac_idx,
-                       b->ac_local, A.loc_group, g, b->info, b->d_nstep, b->d_it, b->potd, b->potdd, m->rmass_ac + b->ac_g0,
+                       b->ac_local, A.loc_group, g, b->info, b->d_nstep, b->d_it + b->at, b->potd, b->potdd, m->rmass_ac + b->ac_g0,
                        b->dt2);
     SF_LAUNCH_CHECK("k_batch_ac_gather");
   }
@@ -782,28 +789,31 @@ static void enqueue_step(Batch* b, hipStream_t st, bool first) {
     } else {
       const int64_t nrow = 3 * (int64_t)m->nglob;
       hipLaunchKernelGGL(k_batch_update, dim3(sf_grid(2 * nrow, 256).x, (unsigned)(b->S / 8)), dim3(256), 0, st, nrow,
-                         b->d_nstep, b->d_it, b->u, b->v, b->a, m->rmass, b->dt2, b->dt, b->dt2, b->dtsq2);
+                         b->d_nstep, b->d_it + b->at, b->u, b->v, b->a, m->rmass, b->dt2, b->dt, b->dt2, b->dtsq2);
       SF_LAUNCH_CHECK("k_batch_update");
     }
   }
   if (b->ac) enqueue_fluid(b, st);
   const FacePoints& f = m->abs_el;
-  if (m->stacey && f.points() > 0) {
-    hipLaunchKernelGGL(k_batch_stacey, face_grid(f, b->S), dim3(256), 0, st, f.points(), 3 * (int64_t)m->nglob, f.iglob,
-                       f.normal, f.jacw, f.imp_p, f.imp_s, f.next, b->d_nstep, b->d_it, b->v, b->a);
-    SF_LAUNCH_CHECK("k_batch_stacey");
+  const int groups = b->S / 8, n0 = m->stacey ? f.points() : 0;
+  const int fb = n0 > 0 ? (int)sf_grid(8 * (int64_t)n0, 256).x : 0, rb = (b->nrec + 4 * groups - 1) / (4 * groups);
+  if (fb + rb > 0) {
+    hipLaunchKernelGGL(k_batch_stacey_seismo, dim3((unsigned)(fb + rb), (unsigned)groups), dim3(256), 0, st, fb, n0,
+                       3 * (int64_t)m->nglob, f.iglob, f.normal, f.jacw, f.imp_p, f.imp_s, f.next, b->d_nstep,
+                       b->d_it + b->at, b->v, b->a, b->nrec, b->rec_slot, b->rec_ig, b->rec_h, b->rec_nu, b->u, b->seis);
+    SF_LAUNCH_CHECK("k_batch_stacey_seismo");
   }
   const FacePoints& cf = m->coupling;
   if (b->ac && cf.points() > 0) {
     hipLaunchKernelGGL(k_batch_coupling_el_ac, face_grid(cf, b->S), dim3(256), 0, st, cf.points(), 3 * (int64_t)m->nglob,
-                       b->ac_n, b->ac_g0, cf.iglob, cf.normal, cf.jacw, cf.next, b->d_nstep, b->d_it, b->potdd, b->a);
+                       b->ac_n, b->ac_g0, cf.iglob, cf.normal, cf.jacw, cf.next, b->d_nstep, b->d_it + b->at, b->potdd, b->a);
     SF_LAUNCH_CHECK("k_batch_coupling_el_ac");
   }
   for (int r = 0; r < b->src_nrounds; r++) {
     const int o = b->src_round_off[r], cnt = b->src_round_off[r + 1] - o;
     if (cnt <= 0) continue;
     hipLaunchKernelGGL(k_batch_sources, sf_grid(cnt, 128), dim3(128), 0, st, cnt, 3 * (int64_t)m->nglob, b->max_nstep, b->src_ig + o,
-                       b->src_slot + o, b->src_id + o, b->src_ploc + o, b->src_arr, b->src_stf, b->d_nstep, b->d_it,
+                       b->src_slot + o, b->src_id + o, b->src_ploc + o, b->src_arr, b->src_stf, b->d_nstep, b->d_it + b->at,
                        b->a);
     SF_LAUNCH_CHECK("k_batch_sources");
   }
@@ -814,8 +824,11 @@ static void enqueue_step(Batch* b, hipStream_t st, bool first) {
     SF_CHECK(hipEventRecord(b->ev[b->ev_used + 1], st));
     b->ev_used += 2;
   }
-  enqueue_seismo(b, st);
-  hipLaunchKernelGGL(k_batch_tick, dim3(1), dim3(64), 0, st, b->d_it);
+}
+
+// after n steps
+static void enqueue_tick(Batch* b, hipStream_t st, int n) {
+  hipLaunchKernelGGL(k_batch_tick, dim3(1), dim3(IT_AHEAD), 0, st, b->d_it, n);
   SF_LAUNCH_CHECK("k_batch_tick");
 }
 
@@ -826,6 +839,7 @@ static void run_steps(Batch* b, int n, int graph_steps) {
   while (n > 0) {
     if (b->h_it == 1 || graph_steps <= 1 || n < graph_steps) {
       enqueue_step(b, m->stream, b->h_it == 1);
+      enqueue_tick(b, m->stream, 1);
       b->h_it++;
       n--;
       continue;
@@ -834,7 +848,12 @@ static void run_steps(Batch* b, int n, int graph_steps) {
       drop_graph(b);
       hipGraph_t g;
       SF_CHECK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-      for (int k = 0; k < graph_steps; k++) enqueue_step(b, m->stream, false);
+      for (int k = 0; k < graph_steps; k++) {
+        b->at = k % IT_AHEAD;
+        enqueue_step(b, m->stream, false);
+        if (b->at == IT_AHEAD - 1 || k == graph_steps - 1) enqueue_tick(b, m->stream, b->at + 1);
+      }
+      b->at = 0;
       SF_CHECK(hipStreamEndCapture(m->stream, &g));
       SF_CHECK(hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0));
       SF_CHECK(hipGraphDestroy(g));
@@ -895,7 +914,7 @@ extern "C" long sf_batch_create(long* Mesh_pointer, int nshots, const int* nstep
     ns[k] = nstep[order[k]];
   }
   b->d_nstep = bupload(ns.data(), b->S);
-  b->d_it = balloc<int>(1);
+  b->d_it = balloc<int>(IT_AHEAD);
   const int64_t n = 3 * (int64_t)m->nglob * b->S;
   b->u = balloc<realw>(n);
   b->v = balloc<realw>(n);
