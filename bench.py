@@ -171,8 +171,7 @@ def batched_measurement(args) -> dict:
     src, rec, n = w.shots[0]
     ps = min(args.plain_steps, n)
     pw = min(10, ps // 2)
-    # the fastest single-shot configuration on this elastic mesh: coloured assembly (plain
-    # read-modify-write per colour) runs the stiffness ~3x faster than float atomics here
+    # the single-shot path with the batch's order of sums
     g = GPUSolver(db, src, rec, nstep=ps, exact=False, assembly=2)
     for _ in range(pw):
         g.step()
@@ -255,7 +254,7 @@ def batched_visco_measurement(args) -> dict:
 
 def homogeneous_box_measurement(args) -> dict:
     """The 20^3 homogeneous elastic box (531,441 points, 2000 steps, the CPU-runnable case) through the
-    ABI call sequence with the library's defaults (FMA kernels, coloured assembly without attenuation),
+    ABI call sequence with the library's defaults (FMA kernels, element-order sums),
     the FP32 oracle on one host core over a sample of its steps, and the reference's own Fortran
     solver figure for the same case (measured on another host)."""
     import numpy as np
@@ -290,7 +289,7 @@ def homogeneous_box_measurement(args) -> dict:
     log(f"[bench] 20^3 homogeneous box: {value:.3e} GLL-pt updates/s ({wall / (n - 20) * 1e3:.3f} ms/step), "
         f"finite={finite}")
     return {"workload": w.name, "nglob": db.nglob, "value": value, "unit": "GLL-point updates/s",
-            "ms_per_step": wall / (n - 20) * 1e3, "steps": n - 20, "assembly": "library default (coloured)",
+            "ms_per_step": wall / (n - 20) * 1e3, "steps": n - 20, "assembly": "library default (element order)",
             "seismograms_finite": finite, "cpu_baseline": cpu,
             "reference_fortran_cpu": {"value": 7.16e6, "unit": "GLL-point updates/s", "cores": 1,
                                       "kind": "reference",

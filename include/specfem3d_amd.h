@@ -341,9 +341,9 @@ void transfer_swf_data_tohost_(long* p1, int* p2, int* p3, realw* p4, realw* p5,
 
 /* ---- library extensions (no counterpart in the reference interface) ---------------------- */
 /* exact = 1: element kernels without fused multiply-add (the CPU solver's rounding);
-   assembly = 0: float atomic scatter-add; 1: element contributions summed per point in element
-   order (deterministic, the CPU solver's order); 2: one launch per colour of a greedy element
-   colouring with a plain read-modify-write scatter (deterministic, no atomics). */
+   assembly: order of a point's sums of element contributions, which the stiffness stores and the next
+   update adds up. 1: element order (the CPU solver's); 2: the colour order of a greedy element
+   colouring; 0: any (element order). All are deterministic. */
 void sf_set_options(long* Mesh_pointer, int exact, int assembly);
 /* tuning switch by name: "att_variant" 0..4 = scheduling of the attenuation state in the point
    stiffness kernel (same results; 4, the default, loads it straight into LDS);
@@ -413,8 +413,8 @@ void sf_batch_destroy(long batch);
    point */
 int sf_batch_point_flags(int nglob, int nelem, const int* ibool0, const int* elems, const int* color,
                          const unsigned char* forced, unsigned char* flags);
-/* launch order (0-based elastic elements, each once) of the atomic and coloured stiffness launches,
-   e.g. a locality (Morton) order from the host; the ordered assembly keeps the processing list */
+/* launch order (0-based elastic elements, each once) of the stiffness: where its local forces lie, not the
+   order of the sums, except that the colours of assembly = 2 follow it */
 void sf_set_element_order(long* Mesh_pointer, int n, const int* order);
 /* greedy first-fit element colouring of assembly = 2 (host only): color[q] for elems[q], elements
    sharing a global point differ; returns the number of colours or -1 (more than 32) */

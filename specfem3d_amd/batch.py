@@ -22,11 +22,9 @@ from .solver import GPUSolver
 class BatchSolver:
     def __init__(self, db, shots, exact: bool = False, device: int = 0, shots_per_group: int | None = None,
                  assembly: int | None = None, attenuation=None):
-        """``shots``: list of (SourceSet, ReceiverSet, nstep), one per shot. ``assembly``: 0 atomic
-        scatter, 2 one launch per element colour, 3 coloured with the Newmark update fused into the
-        colour launches (same bits as 2); None keeps the library default until ``autotune``.
-        ``attenuation``: 3-SLS set-up of the mesh (each shot then carries its own memory variables;
-        coloured assembly only)."""
+        """``shots``: list of (SourceSet, ReceiverSet, nstep), one per shot. ``assembly``
+        (0, 2, 3) is stored and has no effect: every shot's sums run in the colour order of the mesh.
+        ``attenuation``: 3-SLS set-up of the mesh (each shot then carries its own memory variables)."""
         if not shots:
             raise ValueError("no shots")
         self.db = db

@@ -692,8 +692,7 @@ extern "C" void FC_FUNC_(prepare_fields_elastic_device, PREPARE_FIELDS_ELASTIC_D
 }
 
 namespace sf {
-// elastic element colours for coloured launches that are not the mesh's own assembly mode
-// (the batched engine)
+// elastic element colours: the order of the sums of the batched engine and of assembly = 2
 void ensure_element_colors(Mesh* m) {
   if (m->el_color_elems || m->nspec_elastic <= 0 || !m->elastic_elems) return;
   std::vector<int> lst(m->nspec_elastic);
@@ -702,8 +701,7 @@ void ensure_element_colors(Mesh* m) {
   build_colors(m, lst, m->el_color_elems, m->el_color_off, m->el_ncolor);
 }
 
-// acoustic element colours for the batched engine (the same colours a coloured single-shot run
-// builds: greedy first-fit over the acoustic element list in its processing order)
+// the same for the acoustic elements (greedy first-fit over their list in its processing order)
 void ensure_acoustic_colors(Mesh* m) {
   if (m->ac_color_elems || m->nspec_acoustic <= 0 || !m->acoustic_elems) return;
   std::vector<int> lst(m->nspec_acoustic);
@@ -718,9 +716,8 @@ bool element_is_elastic(Mesh* m, int e) {
 }
 
 // Greedy first-fit colouring of an element list (in list order): an element takes the lowest
-// colour not yet used by any element sharing one of its global points. Each colour is then one
-// launch whose element-to-global scatter needs no atomics. Elements keep their list order
-// inside a colour. At most 32 colours (a bit mask per global point); a structured hexahedral
+// colour not yet used by any element sharing one of its global points. The colours give an order of
+// a point's sums that does not depend on the launch. Elements keep their list order inside a colour. At most 32 colours (a bit mask per global point); a structured hexahedral
 // mesh needs 8.
 static int color_elements(int nglob, int nelem, const int* ibool0, const int* elems, int* col) {
   std::vector<uint32_t> used((size_t)nglob, 0u);
@@ -1358,10 +1355,10 @@ extern "C" void sf_set_tuning(long* Mesh_pointer, const char* name, int value) {
   }
 }
 
-// Launch order of the elastic elements for the atomic and coloured stiffness launches (results do
-// not depend on it except for float-atomic rounding): `order` lists the 0-based elastic elements,
-// each once. Hosts pass a locality order (e.g. Morton order of element centres) so that elements
-// sharing points run close together and their shared rows meet in L2. Re-colours when coloured.
+// Launch order of the elastic elements: `order` lists the 0-based elastic elements, each once. Hosts pass a
+// locality order (e.g. Morton order of element centres) so that elements sharing points run close together
+// and their shared rows meet in L2. It moves the slots of the local forces, not the order of the sums,
+// except that the colours are built in it.
 extern "C" void sf_set_element_order(long* Mesh_pointer, int n, const int* order) {
   Mesh* m = from_handle(Mesh_pointer);
   HostSide* H = host_of(m);

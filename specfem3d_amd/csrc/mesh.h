@@ -87,8 +87,8 @@ struct Mesh {
   // domains
   int nspec_elastic = 0, nspec_acoustic = 0;
   int* elastic_elems = nullptr;    // element lists in processing order
-  int* elastic_launch = nullptr;   // optional locality order of the elastic elements for the atomic
-                                   // and coloured launches (sf_set_element_order); null: elastic_elems
+  int* elastic_launch = nullptr;   // optional locality order of the stiffness launches
+                                   // (sf_set_element_order); null: elastic_elems
   int* acoustic_elems = nullptr;
   unsigned char* h_is_elastic = nullptr;
   unsigned char* h_is_acoustic = nullptr;
@@ -201,9 +201,8 @@ struct Mesh {
 
   // execution
   hipStream_t stream = nullptr;
-  // Defaults for a host that never calls sf_set_options (the Fortran drop-in): the FMA build and,
-  // once prepare_fields_elastic_device knows whether attenuation is on, element-order sums (fluid
-  // atomics with it).
+  // Defaults for a host that never calls sf_set_options (the Fortran drop-in): the FMA build and
+  // element-order sums.
   int exact = 0;                   // 1: kernels built without fused multiply-add (oracle order)
   int assembly = -1;               // order of the element sums: 1 element order (oracle order), 2 colour
                                    // order, 0 any (sf_set_options), -1 automatic
@@ -254,7 +253,7 @@ struct Mesh {
   // points of the fluid's free surface: FREE_POT = chi and chi' are zero there, FREE_DD = chi'' is (as
   // stored: a waiting sum and a deferred corrector not counted)
   int free_zero[2] = {0, 0};
-  // coloured assembly (assembly = 2): element lists regrouped by colour; elements of one
+  // colour order (assembly = 2, batches): element lists regrouped by colour; elements of one
   // colour share no global point, colour c is elems[off[c] .. off[c+1])
   int el_ncolor = 0, ac_ncolor = 0;
   int el_color_off[33] = {0}, ac_color_off[33] = {0};
