@@ -51,15 +51,15 @@ def copy_peak_gbs() -> float:
     return 2 * 4 * n / (ms / 1e3) / 1e9
 
 
-def measured_traffic(assembly: int, exact: int):
-    """HBM bytes per stiffness launch from the committed rocprofv3 PMC summary of this mode.
+def measured_traffic(exact: int):
+    """HBM bytes per stiffness launch from the committed rocprofv3 PMC summary.
 
     The summary holds FETCH_SIZE and WRITE_SIZE of the kernel, each scaled by what the same
     counter reads for a plain 1 GiB device copy; returns (bytes, summary path) or (None, None).
     """
     if exact:
         return None, None
-    name = os.path.join("profiles", f"k_elastic_pt_sea_over_visco_96x96x48_{['atomic', 'ordered', 'coloured'][assembly]}.md")
+    name = os.path.join("profiles", "k_elastic_pt_sea_over_visco_96x96x48.md")
     try:
         txt = open(os.path.join(HERE, name)).read()
     except OSError:
@@ -185,7 +185,7 @@ def batched_measurement(args) -> dict:
     log(f"[bench] batched {value:.3e} GLL-pt updates/s in {wall:.2f}s (stiffness {kms:.3f} ms/step, step {sms:.3f} ms "
         f"with all shots live), plain single shot {plain:.3e}, ratio {value / plain:.2f}, finite={finite}")
     return {"workload": w.name, "value": value, "unit": "GLL-point updates/s", "wall_s": round(wall, 3),
-            "shot_steps": int(sum(nsteps)), "plain_single_shot": plain, "plain_assembly": "coloured",
+            "shot_steps": int(sum(nsteps)), "plain_single_shot": plain, "plain_assembly": "colour order",
             "ratio_vs_plain": value / plain,
             "all_live_value": db.nglob * len(w.shots) / (sms / 1e3),
             "all_live_ratio_vs_plain": db.nglob * len(w.shots) / (sms / 1e3) / plain,
@@ -505,7 +505,7 @@ def adjoint_measurement(args) -> dict:
     finite = bool(np.isfinite(mk).all() and np.abs(mk).max() > 0)
     log(f"[bench] kernel run {wall:.2f}s (forward with snapshots {tf:.2f}s), misfit {chi:.4e}, kernels finite={finite}")
     return {"workload": w.name, "wall_s": round(wall, 3), "forward_s": round(tf, 3), "steps": n, "nt_dump": 64,
-            "assembly": ["atomic", "ordered", "coloured"][args.adjoint_assembly],
+            "assembly": ["any order", "element order", "colour order"][args.adjoint_assembly],
             "nglob": db.nglob, "misfit": chi, "kernels_finite": finite,
             "unit": "s (forward with checkpoints + adjoint with recompute)"}
 
@@ -577,7 +577,7 @@ def main():
     ap.add_argument("--scale", type=float, default=1.0, help="shrink the mesh (tests only)")
     ap.add_argument("--exact", type=int, default=0, help="1: kernels without FMA (CPU rounding)")
     ap.add_argument("--assembly", type=int, default=0,
-                    help="0 atomic scatter, 1 ordered (CPU element order), 2 coloured (no atomics)")
+                    help="order of the element sums: 0 any, 1 CPU element order, 2 colour order")
     ap.add_argument("--element-order", default="none",
                     choices=["morton", "none", "brick1x2", "brick2x1", "brick2x2", "brick1x4", "brick4x4", "brick2x4"],
                     help="launch order of the elastic elements of the single-shot run")
@@ -717,7 +717,7 @@ def main():
     kbytes = stiffness_bytes_per_launch(db, w.attenuation)
     kavg_s = tot.value / max(cnt.value, 1) / 1e3
     achieved = kbytes / kavg_s / 1e9
-    traffic, tsrc = measured_traffic(args.assembly, args.exact) if args.scale == 1.0 else (None, None)
+    traffic, tsrc = measured_traffic(args.exact) if args.scale == 1.0 else (None, None)
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                 "kernel": "k_elastic_pt (viscoelastic 3-SLS stiffness)", "bytes_per_launch": kbytes,
@@ -777,7 +777,7 @@ def main():
                    "attenuation": (f"{len(w.attenuation.tau_sigma)} SLS, Q_mu={w.meta.get('qmu'):g}"
                                    if w.attenuation is not None else "none"),
                    "receivers": w.receivers.n, "exact": args.exact,
-                   "assembly": ["atomic", "ordered", "coloured"][args.assembly],
+                   "assembly": ["any order", "element order", "colour order"][args.assembly],
                    "element_order": args.element_order,
                    "att_variant": "default" if args.att_variant < 0 else args.att_variant},
         "roofline": roofline,

@@ -307,6 +307,7 @@ extern "C" void FC_FUNC_(update_displacement_cuda, UPDATE_DISPLACMENT_CUDA)(long
   } else {
     launch_predictor(m->stream, n, w.displ + o, w.veloc + o, w.accel + o, *deltat_F, *deltatover2_F,
                      *deltatsqover2_F);
+    m->low_set[f] = 0;
   }
   m->pending_gather_el[f] = 0;
   m->gather_skip_el[f] = 0;
@@ -345,6 +346,7 @@ extern "C" void FC_FUNC_(update_displacement_ac_cuda, UPDATE_DISPLACEMENT_AC_CUD
   } else {
     launch_predictor(m->stream, m->ac_n, a.pot + g0, a.potd + g0, a.potdd + g0, *deltat_F, *deltatover2_F,
                      *deltatsqover2_F);
+    m->low_ac_set[f] = 0;
   }
   m->free_zero[f] = FREE_DD | (dd ? m->free_zero[f] & FREE_POT : 0);
   m->pending_gather_ac[f] = 0;
