@@ -300,7 +300,7 @@ def homogeneous_box_measurement(args) -> dict:
 def cpml_example_measurement(args) -> dict:
     """The reference example CPML_examples/homogeneous_halfspace_HEX8_elastic_absorbing_CPML_5sides
     (36 x 36 x 16 irregular elements, 1,366,625 points, 9036 C-PML elements, 2400 steps) with the
-    library defaults (FMA kernels, coloured assembly), and its seismograms against the example's
+    library defaults (FMA kernels, element-order sums), and its seismograms against the example's
     REF_SEIS."""
     import ctypes as C
     import numpy as np
@@ -598,14 +598,14 @@ def main():
     ap.add_argument("--adjoint-steps", type=int, default=4000,
                     help="steps of the checkpointed kernel run on the 48^3 adjoint workload (0: skip)")
     ap.add_argument("--adjoint-assembly", type=int, default=2,
-                    help="assembly of the kernel run: 0 atomic, 1 ordered, 2 coloured (default: the fastest here)")
+                    help="order of the sums of the kernel run: 0 any, 1 element order, 2 colour order")
     ap.add_argument("--adjoint-scale", type=float, default=1.0, help="shrink the adjoint mesh (tests only)")
     ap.add_argument("--homogeneous-box", type=int, default=1,
                     help="1: also run the 20^3 homogeneous box single-shot figures")
     ap.add_argument("--cpml-example", type=int, default=1,
                     help="1: also run the reference's C-PML example (2400 steps) and compare with its REF_SEIS")
     ap.add_argument("--cpml-assembly", type=int, default=-1,
-                    help="assembly of the C-PML example run (-1: library default, coloured without attenuation)")
+                    help="order of the sums of the C-PML example run (-1: library default)")
     ap.add_argument("--coupled-shots", type=int, default=8,
                     help="shots of the batched fluid-over-viscoelastic workload (0: skip)")
     ap.add_argument("--coupled-steps", type=int, default=300, help="steps of each batched coupled shot")
@@ -627,7 +627,7 @@ def main():
 
     if args.kernel_probe:
         # short fixed sequence for PMC counter runs: 4 batched steps of the 32-shot workload with
-        # each batched kernel variant, then 6 single-shot steps with coloured assembly
+        # each batched kernel variant, then 6 single-shot steps with colour-order sums
         from specfem3d_amd import workloads as W
         from specfem3d_amd.batch import BatchSolver
         from specfem3d_amd.solver import GPUSolver
@@ -644,7 +644,7 @@ def main():
         g = GPUSolver(w.db, src, rec, nstep=6, exact=False, assembly=2)
         g.run()
         g.close()
-        log("[bench] kernel probe: 6 single-shot steps, coloured assembly")
+        log("[bench] kernel probe: 6 single-shot steps, colour-order sums")
         return
 
     if args.copy_probe:
