@@ -377,9 +377,9 @@ void sf_batch_add_source(long batch, int shot, int ispec, const realw* sourcearr
 void sf_batch_add_receiver(long batch, int shot, int ispec, const double* hxi, const double* heta,
                            const double* hgamma, const double* nu);
 void sf_batch_finalize(long batch);
-/* shots per workgroup 4 or 8; assembly 0, 2 or 3: one code path, which sums every point's element
-   contributions in the colour order of a greedy element colouring; only at step 1 (a new batch or
-   after sf_batch_reset) */
+/* shots per workgroup 4 or 8; assembly 0, 2 or 3: every point's element contributions are summed in the
+   colour order of a greedy element colouring; 3: FMA builds use fused multiply-adds in the Newmark update
+   too (same results otherwise). Only at step 1 (a new batch or after sf_batch_reset) */
 void sf_batch_set_options(long batch, int shots_per_group, int assembly);
 void sf_batch_get_options(long batch, int* shots_per_group, int* assembly);
 /* same results for every value: "local_groups" >= 1, groups of eight shots whose local forces are held

@@ -99,14 +99,14 @@ extern "C" void sf_snapshot_load(long* Mesh_pointer, int FORWARD_OR_ADJOINT, int
     ck_copy(m, m->el[f].displ, s.el, 3 * n);
     ck_copy(m, m->el[f].veloc, s.el + 3 * n, 3 * n);
     ck_copy(m, m->el[f].accel, s.el + 6 * n, 3 * n);
-    m->accel_clean[f] = m->low_set[f] = 0;
+    m->accel_clean[f] = 0;
   }
   if (m->ac[f].pot) {
     if (!s.ac) fatal("sf_snapshot_load", "snapshot holds no acoustic field");
     ck_copy(m, m->ac[f].pot, s.ac, n);
     ck_copy(m, m->ac[f].potd, s.ac + n, n);
     ck_copy(m, m->ac[f].potdd, s.ac + 2 * n, n);
-    m->potdd_clean[f] = m->free_zero[f] = m->low_ac_set[f] = 0;
+    m->potdd_clean[f] = m->free_zero[f] = 0;
   }
   if (m->attenuation && m->att[f].R) {
     if (!s.R) fatal("sf_snapshot_load", "snapshot holds no memory variables");
@@ -154,12 +154,11 @@ extern "C" void sf_history_load(long* Mesh_pointer, int FORWARD_OR_ADJOINT, int 
   const int64_t n = m->nglob;
   if (m->history_el && m->el[f].displ) {
     ck_copy(m, m->el[f].displ, m->history_el + (int64_t)frame * 3 * n, 3 * n);
-    m->low_set[f] = 0;
   }
   if (m->history_ac && m->ac[f].pot) {
     ck_copy(m, m->ac[f].pot, m->history_ac + (int64_t)frame * 2 * n, n);
     ck_copy(m, m->ac[f].potdd, m->history_ac + (int64_t)frame * 2 * n + n, n);
-    m->potdd_clean[f] = m->free_zero[f] = m->low_ac_set[f] = 0;
+    m->potdd_clean[f] = m->free_zero[f] = 0;
   }
 }
 

@@ -594,7 +594,7 @@ extern "C" void FC_FUNC_(prepare_fields_elastic_device, PREPARE_FIELDS_ELASTIC_D
   const int64_t nloc = (int64_t)m->nspec * 125;
   if (m->assembly < 0) {
     // automatic assembly (see Mesh::assembly)
-    m->assembly = *ATTENUATION ? 0 : 1;
+    m->assembly = *ATTENUATION ? 0 : 2;
   }
   {
     std::vector<realw> rm(3 * (size_t)n);
@@ -782,10 +782,6 @@ void ensure_gather_assembly(Mesh* m, int f) {
   const int eb = 20;  // elements per block of slots: a multiple of the five of a k_elastic_line workgroup
   const int first_pml = (m->nspec_elastic + eb - 1) / eb * eb;
   if (!m->asm_buf[f]) m->asm_buf[f] = dmalloc<realw>(3 * 125 * ((int64_t)m->nspec + 2 * eb));  // both lists, rounded up
-  if (m->simulation_type == 3 && !m->low[f]) {
-    m->low[f] = dmalloc<uint8_t>(3 * (int64_t)m->nglob);
-    m->low_set[f] = 0;
-  }
   if (m->asm_ready) return;
   flush_all(m);       // local forces in the old slots
   if (m->assembly == 2) ensure_element_colors(m);
@@ -830,8 +826,6 @@ void release_gather_assembly(Mesh* m) {
   dfree(m->rmass1);
   dfree(m->asm_buf[0]);
   dfree(m->asm_buf[1]);
-  dfree(m->low[0]);
-  dfree(m->low[1]);
   m->asm_ready = 0;
   dfree(m->asm_ac_idx);
   dfree(m->asm_ac_info);
@@ -839,8 +833,6 @@ void release_gather_assembly(Mesh* m) {
   dfree(m->asm_ac_rec);
   dfree(m->asm_ac_buf[0]);
   dfree(m->asm_ac_buf[1]);
-  dfree(m->low_ac[0]);
-  dfree(m->low_ac[1]);
   m->asm_ac_ready = 0;
 }
 
@@ -848,10 +840,6 @@ void release_gather_assembly(Mesh* m) {
 void ensure_gather_acoustic(Mesh* m, int f) {
   const int eb = 20;
   if (!m->asm_ac_buf[f]) m->asm_ac_buf[f] = dmalloc<realw>(125 * ((int64_t)m->nspec_acoustic + eb));
-  if (m->nspec_elastic == 0 && m->pml_n == 0 && !m->low_ac[f]) {
-    m->low_ac[f] = dmalloc<uint8_t>(m->nglob);
-    m->low_ac_set[f] = 0;
-  }
   if (m->asm_ac_ready) return;
   flush_all(m);
   if (m->assembly == 2) ensure_acoustic_colors(m);
@@ -1291,7 +1279,6 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
   dfree(m->seismo_d); dfree(m->seismo_v); dfree(m->seismo_a); dfree(m->seismo_p);
   dfree(m->rho_kl); dfree(m->mu_kl); dfree(m->kappa_kl); dfree(m->rho_ac_kl); dfree(m->kappa_ac_kl);
   dfree(m->asm_idx); dfree(m->asm_info); dfree(m->asm_base); dfree(m->asm_rec); dfree(m->rmass1); dfree(m->asm_buf[0]); dfree(m->asm_buf[1]);
-  dfree(m->low[0]); dfree(m->low[1]); dfree(m->low_ac[0]); dfree(m->low_ac[1]);
   dfree(m->pml_elems); dfree(m->pml_cpml);
   dfree(m->pml_state); dfree(m->pml_coef); dfree(m->pml_masks); dfree(m->pml_off);
   dfree(m->pml_old); dfree(m->pml_pts); dfree(m->pml_bc_pts);

@@ -43,8 +43,6 @@ static GatherArgs gather_args(Mesh* m, int f) {
   a.rm = m->rmass;
   a.rm1 = m->rmass1;
   a.dt2p = m->pending_dt2_el[f];
-  a.lo = m->exact ? nullptr : m->low[f];
-  a.lo_set = m->low_set[f];
   return a;
 }
 
@@ -63,9 +61,7 @@ void flush_terms(Mesh* m) {
 // sum the waiting local forces and run the pending corrector
 static void sum_el(Mesh* m, int f) {
   if (m->pending_gather_el[f]) {
-    launch_gather_update(m->stream, gather_args(m, f), 3, m->pending_k3_el[f] ? GATHER_CORRECT : GATHER_ONLY,
-                         m->exact != 0);
-    if (m->pending_k3_el[f]) m->low_set[f] = m->low[f] && !m->exact;
+    launch_gather_update(m->stream, gather_args(m, f), 3, m->pending_k3_el[f] ? GATHER_CORRECT : GATHER_ONLY);
     m->pending_gather_el[f] = 0;
     m->gather_skip_el[f] = 0;
     m->accel_clean[f] = 0;
@@ -74,7 +70,6 @@ static void sum_el(Mesh* m, int f) {
     launch_corrector(m->stream, 3 * m->el_n, m->el[f].veloc + o, m->el[f].accel + o, m->rmass + o,
                      m->pending_dt2_el[f]);
     m->accel_clean[f] = 0;
-    m->low_set[f] = 0;
   }
   m->pending_k3_el[f] = 0;
 }
@@ -100,17 +95,13 @@ static GatherArgs gather_args_ac(Mesh* m, int f) {
   a.a = m->ac[f].potdd;
   a.rm1 = m->rmass_ac;
   a.dt2p = m->pending_dt2_ac[f];
-  a.lo = m->exact ? nullptr : m->low_ac[f];
-  a.lo_set = m->low_ac_set[f];
   return a;
 }
 
 static void sum_ac(Mesh* m, int f) {
   int& fz = m->free_zero[f];
   if (m->pending_gather_ac[f]) {
-    launch_gather_update(m->stream, gather_args_ac(m, f), 1, m->pending_k3_ac[f] ? GATHER_CORRECT : GATHER_ONLY,
-                         m->exact != 0);
-    if (m->pending_k3_ac[f]) m->low_ac_set[f] = m->low_ac[f] && !m->exact;
+    launch_gather_update(m->stream, gather_args_ac(m, f), 1, m->pending_k3_ac[f] ? GATHER_CORRECT : GATHER_ONLY);
     if (m->gather_skip_ac[f]) fz |= FREE_DD;
     else fz = m->pending_k3_ac[f] ? 0 : fz & FREE_POT;
     m->pending_gather_ac[f] = 0;
@@ -122,7 +113,6 @@ static void sum_ac(Mesh* m, int f) {
                      m->pending_dt2_ac[f]);
     if (!(fz & FREE_DD)) fz = 0;
     m->potdd_clean[f] = 0;
-    m->low_ac_set[f] = 0;
   }
   m->pending_k3_ac[f] = 0;
 }
@@ -293,21 +283,14 @@ extern "C" void FC_FUNC_(update_displacement_cuda, UPDATE_DISPLACMENT_CUDA)(long
     a.old = pml ? m->pml_old : nullptr;
     a.t1 = m->pml_t1;
     a.t2 = m->pml_t2;
-    launch_gather_update(m->stream, a, 3, GATHER_STEP, m->exact != 0);
-    m->low_set[f] = a.lo != nullptr;
+    launch_gather_update(m->stream, a, 3, GATHER_STEP);
   } else if (m->pending_k3_el[f]) {
-    m->low_set[f] = 0;
     launch_corrector_predictor(m->stream, n, w.displ + o, w.veloc + o, w.accel + o, m->rmass + o,
                                m->pending_dt2_el[f], *deltat_F, *deltatover2_F, *deltatsqover2_F,
                                pml ? m->pml_old + o : nullptr, m->pml_t1, m->pml_t2);
-  } else if (m->low[f] && !m->exact) {
-    launch_predictor_low(m->stream, n, w.displ + o, w.veloc + o, w.accel + o, *deltat_F, *deltatover2_F,
-                         *deltatsqover2_F, m->low[f] + o, m->low_set[f]);
-    m->low_set[f] = 1;
   } else {
     launch_predictor(m->stream, n, w.displ + o, w.veloc + o, w.accel + o, *deltat_F, *deltatover2_F,
                      *deltatsqover2_F);
-    m->low_set[f] = 0;
   }
   m->pending_gather_el[f] = 0;
   m->gather_skip_el[f] = 0;
@@ -332,21 +315,14 @@ extern "C" void FC_FUNC_(update_displacement_ac_cuda, UPDATE_DISPLACEMENT_AC_CUD
     ga.dt = *deltat_F;
     ga.dt2 = *deltatover2_F;
     ga.dtsq2 = *deltatsqover2_F;
-    launch_gather_update(m->stream, ga, 1, GATHER_STEP, m->exact != 0);
+    launch_gather_update(m->stream, ga, 1, GATHER_STEP);
     dd = m->gather_skip_ac[f] != 0;
-    m->low_ac_set[f] = ga.lo != nullptr;
   } else if (m->pending_k3_ac[f]) {
-    m->low_ac_set[f] = 0;
     launch_corrector_predictor(m->stream, m->ac_n, a.pot + g0, a.potd + g0, a.potdd + g0, m->rmass_ac + g0,
                                m->pending_dt2_ac[f], *deltat_F, *deltatover2_F, *deltatsqover2_F);
-  } else if (m->low_ac[f] && !m->exact) {
-    launch_predictor_low(m->stream, m->ac_n, a.pot + g0, a.potd + g0, a.potdd + g0, *deltat_F, *deltatover2_F,
-                         *deltatsqover2_F, m->low_ac[f] + g0, m->low_ac_set[f]);
-    m->low_ac_set[f] = 1;
   } else {
     launch_predictor(m->stream, m->ac_n, a.pot + g0, a.potd + g0, a.potdd + g0, *deltat_F, *deltatover2_F,
                      *deltatsqover2_F);
-    m->low_ac_set[f] = 0;
   }
   m->free_zero[f] = FREE_DD | (dd ? m->free_zero[f] & FREE_POT : 0);
   m->pending_gather_ac[f] = 0;
@@ -469,7 +445,7 @@ extern "C" void FC_FUNC_(acoustic_enforce_free_surf_cuda, ACOUSTIC_ENFORCE_FREE_
     if (!m->ac[f].pot) continue;
     const int known = m->pending_gather_ac[f] ? FREE_POT : FREE_POT | FREE_DD;
     if ((m->free_zero[f] & known) != known)
-      launch_free_surface(m->stream, m->free_ac, m->ac[f].pot, m->ac[f].potd, m->ac[f].potdd);  // low parts of 0 are 0
+      launch_free_surface(m->stream, m->free_ac, m->ac[f].pot, m->ac[f].potd, m->ac[f].potdd);
     if (m->pending_gather_ac[f]) m->gather_skip_ac[f] |= AF_EDGE;
     m->free_zero[f] |= known;
   }
@@ -808,7 +784,7 @@ extern "C" void FC_FUNC_(compute_seismograms_cuda, COMPUTE_SEISMOGRAMS_CUDA)(
     auto record = [&](const realw* field, int what, realw* out) {
       if (wait && what != WAIT_NONE)
         launch_seismo_el_waiting(m->stream, m->nrec_el, m->rec_el_list, m->rec_iglob, m->rec_h, m->rec_nu,
-                                 gather_args(m, f), m->asm_rec, what, m->exact != 0, out);
+                                 gather_args(m, f), m->asm_rec, what, out);
       else
         launch_seismo_el(m->stream, m->nrec_el, m->rec_el_list, m->rec_iglob, m->rec_h, m->rec_nu, field, out);
     };
@@ -827,7 +803,6 @@ extern "C" void FC_FUNC_(compute_seismograms_cuda, COMPUTE_SEISMOGRAMS_CUDA)(
     AcReceiverArgs ra;
     ra.wait = gather_args_ac(m, fa);
     ra.first = m->asm_ac_rec;
-    ra.exact = m->exact;
     ra.n = m->nrec_ac;
     ra.list = m->rec_ac_list;
     ra.rec_ispec = m->rec_ispec;
@@ -948,7 +923,7 @@ static void d2h(Mesh* m, realw* h, const realw* d, int64_t n) {
     DIR(m, m->el[F].displ, displ, *size);                                                                     \
     DIR(m, m->el[F].veloc, veloc, *size);                                                                     \
     DIR(m, m->el[F].accel, accel, *size);                                                                     \
-    m->accel_clean[F] = m->low_set[F] = 0;                                                                    \
+    m->accel_clean[F] = 0;                                                                                    \
   }
 #define SF_XFER1(NAME, F, MEMBER, DIR)                                                   \
   extern "C" void FC_FUNC_(NAME, X)(int* size, realw* arr, long* Mesh_pointer) {        \
@@ -956,7 +931,7 @@ static void d2h(Mesh* m, realw* h, const realw* d, int64_t n) {
     check_field(m, F, #NAME);                                                            \
     flush_el(m, F);                                                                      \
     DIR(m, m->el[F].MEMBER, arr, *size);                                                 \
-    m->accel_clean[F] = m->low_set[F] = 0;                                               \
+    m->accel_clean[F] = 0;                                                               \
   }
 #define H2D(m, d, h, n) h2d(m, d, h, n)
 #define D2H(m, d, h, n) d2h(m, h, d, n)
@@ -986,7 +961,7 @@ SF_XFER1(transfer_b_accel_from_device, 1, accel, D2H)
     DIR(m, m->ac[F].pot, p, *size);                                                                            \
     DIR(m, m->ac[F].potd, pd, *size);                                                                          \
     DIR(m, m->ac[F].potdd, pdd, *size);                                                                        \
-    m->potdd_clean[F] = m->free_zero[F] = m->low_ac_set[F] = 0;                                                \
+    m->potdd_clean[F] = m->free_zero[F] = 0;                                                \
   }
 #define SF_XFERAC1(NAME, F, MEMBER, DIR)                                          \
   extern "C" void FC_FUNC_(NAME, X)(int* size, realw* arr, long* Mesh_pointer) { \
@@ -994,7 +969,7 @@ SF_XFER1(transfer_b_accel_from_device, 1, accel, D2H)
     if (!m->ac[F].pot) fatal(#NAME, "acoustic field not prepared");               \
     flush_ac(m, F);                                                               \
     DIR(m, m->ac[F].MEMBER, arr, *size);                                          \
-    m->potdd_clean[F] = m->free_zero[F] = m->low_ac_set[F] = 0;                   \
+    m->potdd_clean[F] = m->free_zero[F] = 0;                   \
   }
 SF_XFERAC3(transfer_fields_ac_to_device, 0, H2D)
 SF_XFERAC3(transfer_fields_ac_from_device, 0, D2H)

@@ -17,8 +17,8 @@
 //     that advances the device step counter after a step or a captured group. Every kernel reads the
 //     counter, so a group of steps is captured once into a hipGraph and replayed;
 //   * the per-point arithmetic and the order of every sum equal the single-shot path (same
-//     kernels' expressions, same colour order, same order of faces), so without FMA contraction each shot
-//     of a batch is bit-identical to its single-shot run; FMA builds also carry low parts of u and v.
+//     kernels' expressions, same colour order, same order of faces), so each shot of a batch is
+//     bit-identical to its single-shot run in the colour order (assembly = 2).
 // Shots-per-workgroup are chosen by an autotuner that times each candidate for a few steps from rest
 // and then resets the batch.
 #include <algorithm>
@@ -37,7 +37,7 @@ bool element_is_elastic(Mesh* m, int e);
 struct Batch {
   Mesh* m = nullptr;
   int nshots = 0, S = 0;
-  int sc = 4, mode = 2;          // shots per workgroup; assembly, kept for callers (no effect)
+  int sc = 4, mode = 2;          // shots per workgroup; assembly (3: see newmark)
   int overlay = 0;               // "lds_overlay", kept for callers that set it (no effect)
   int max_nstep = 0;
   realw dt = 0.f, dt2 = 0.f, dtsq2 = 0.f;  // deltat, deltatover2, deltatsqover2
@@ -57,7 +57,6 @@ struct Batch {
   // of `loc_groups` groups of eight shots (all of them unless the card has no room)
   int *asm_ptr = nullptr, *asm_idx = nullptr, *ac_ptr = nullptr, *ac_idx = nullptr;
   uint16_t* info = nullptr;
-  uint8_t* low = nullptr;        // low parts of u and v (BatchGatherArgs::low)
   realw *local = nullptr, *ac_local = nullptr;
   int loc_groups = 0, ac_loc_groups = 0;
   int max_groups = 1 << 20;      // "local_groups"
@@ -100,11 +99,29 @@ static __device__ __forceinline__ int load_it(const int* it) {
   return __hip_atomic_load(it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Corrector of the finished step and predictor of the next one for one value. FMA: FMA builds under assembly =
+// 3 form the corrected velocity and the displacement with fused multiply-adds (the second half step adds
+// the rounded product), else the operations are those of k_update.hip.
+template <bool FMA>
+__device__ __forceinline__ void newmark(realw& u, realw& v, realw a, realw M, realw dt2p, realw dt, realw dt2,
+                                        realw dtsq2) {
+  a = a * M;
+  if (FMA) {
+    v = fmaf(dt2p, a, v);
+    u = fmaf(dtsq2, a, fmaf(dt, v, u));
+  } else {
+    v = v + dt2p * a;
+    u = u + dt * v + dtsq2 * a;
+  }
+  v = v + dt2 * a;
+}
+
 // Newmark update of every live (row, shot) from an assembled accel: the corrector of the previous step
 // fused with the predictor (k_update.hip arithmetic), where the local forces have no room for all
 // groups (see enqueue_stiffness).
 // A lane takes four consecutive shots of one row (a float4), blockIdx.y is the group of eight.
 // Finished shots keep their values (their lanes store what they loaded).
+template <bool FMA>
 __global__ void __launch_bounds__(256) k_batch_update(int64_t nrow, const int* __restrict__ nstep,
                                                       const int* __restrict__ itp, realw* __restrict__ u,
                                                       realw* __restrict__ v, realw* __restrict__ a,
@@ -123,14 +140,11 @@ __global__ void __launch_bounds__(256) k_batch_update(int64_t nrow, const int* _
   const float4 A0 = *reinterpret_cast<const float4*>(a + o);
   const realw M = rm[row];
   float4 U = U0, V = V0, A = A0;
-#define SF_BU(c)                           \
-  A.c = A.c * M;                           \
-  V.c = V.c + dt2p * A.c;                  \
-  U.c = U.c + dt * V.c + dtsq2 * A.c;      \
-  V.c = V.c + dt2 * A.c;                   \
-  A.c = 0.f;
-  SF_BU(x) SF_BU(y) SF_BU(z) SF_BU(w)
-#undef SF_BU
+  newmark<FMA>(U.x, V.x, A.x, M, dt2p, dt, dt2, dtsq2);
+  newmark<FMA>(U.y, V.y, A.y, M, dt2p, dt, dt2, dtsq2);
+  newmark<FMA>(U.z, V.z, A.z, M, dt2p, dt, dt2, dtsq2);
+  newmark<FMA>(U.w, V.w, A.w, M, dt2p, dt, dt2, dtsq2);
+  A = make_float4(0.f, 0.f, 0.f, 0.f);
   if (!l1) { U.y = U0.y; V.y = V0.y; A.y = A0.y; }
   if (!l2) { U.z = U0.z; V.z = V0.z; A.z = A0.z; }
   if (!l3) { U.w = U0.w; V.w = V0.w; A.w = A0.w; }
@@ -151,12 +165,6 @@ __global__ void __launch_bounds__(256) k_batch_update(int64_t nrow, const int* _
 // LDS 1.6) and this one by HBM (3.96 ms, 19.3 GB, 4.9 TB/s). Steps before and after: 32x32x16 x 16
 // shots 598 -> 500 us, 64x64x32 x 32 8.53 -> 7.56 ms, viscoelastic 18x18x12 x 8 319 -> 233 us and
 // 40x40x20 x 16 4.02 -> 3.41 ms.
-// LOW (FMA builds that sum all groups here): u and v are carried with their low parts. Records of shots
-// from rest are often the first arrival of a front that grows by decades, and what the rounding of u in
-// every step left behind it is most of their error: against 64 bits those
-// of 32x32x16 x 16 are off by 0.40 instead of 0.59 times what single-precision sums gave (geometric mean
-// over 96), and none of 140 by more than 1.5 times, where 5 of 21 were; 235 -> 259 us per pass there, 28 ->
-// 33 on 18x18x12 x 8.
 struct BatchGatherArgs {
   int64_t g0, n, nrow;           // global points [g0, g0 + n), rows of a group
   const int *ptr, *idx;
@@ -168,12 +176,10 @@ struct BatchGatherArgs {
   realw *u, *v, *a;
   const realw* rm;
   realw dt2p, dt, dt2, dtsq2;
-  uint8_t* low;                  // low parts of u and v (with_low) in the layout of u, or null
 };
 
 // a -= the local forces of slots ptr[g] .. ptr[g + 1], `unit` floats per slot, four slots in flight
-template <typename T>
-__device__ __forceinline__ void gather4(T a[4], const int* ptr, const int* idx, int64_t g, const realw* local,
+__device__ __forceinline__ void gather4(realw a[4], const int* ptr, const int* idx, int64_t g, const realw* local,
                                         int unit) {
   const int p0 = ptr[g], p1 = ptr[g + 1];
   for (int p = p0; p < p1; p += 4) {
@@ -187,10 +193,10 @@ __device__ __forceinline__ void gather4(T a[4], const int* ptr, const int* idx, 
 #pragma unroll
     for (int w = 0; w < 4; w++) {
       if (k[w] < 0) continue;
-      a[0] = a[0] + (-(T)l[w].x);
-      a[1] = a[1] + (-(T)l[w].y);
-      a[2] = a[2] + (-(T)l[w].z);
-      a[3] = a[3] + (-(T)l[w].w);
+      a[0] = a[0] + (-l[w].x);
+      a[1] = a[1] + (-l[w].y);
+      a[2] = a[2] + (-l[w].z);
+      a[3] = a[3] + (-l[w].w);
     }
   }
 }
@@ -202,8 +208,7 @@ __device__ __forceinline__ int64_t xcd_block() {
   return (int64_t)x * q + (x < r ? x : r) + (b >> 3);
 }
 
-// T: float follows the reference's operations (exact builds), double rounds once per stored value
-template <bool STEP, typename T, bool LOW>
+template <bool STEP, bool FMA>
 __global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs A) {
   const int64_t t = xcd_block() * 256 + threadIdx.x;
   const int64_t pt = t / 6;
@@ -216,50 +221,34 @@ __global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs A) {
   const int64_t o = batch_idx(A.nrow, 3 * g + c, s);
   const bool term = (A.info[g] & AF_TERM) != 0;
   float4 U, V;
-  T a[4] = {0, 0, 0, 0};
+  realw a[4] = {0, 0, 0, 0};
   realw M = 0.f;
   if (STEP) {
     U = *reinterpret_cast<const float4*>(A.u + o);
     V = *reinterpret_cast<const float4*>(A.v + o);
     M = A.rm[3 * g + c];
   }
-  uchar4 L = make_uchar4(0, 0, 0, 0);
-  if (LOW) L = *reinterpret_cast<const uchar4*>(A.low + o);
   if (term) {
     const float4 a0 = *reinterpret_cast<const float4*>(A.a + o);
     a[0] = a0.x; a[1] = a0.y; a[2] = a0.z; a[3] = a0.w;
   }
-  gather4<T>(a, A.ptr, A.idx, g, A.local + (int64_t)blockIdx.y * A.loc_group + 8 * c + 4 * (cq & 1), 24);
+  gather4(a, A.ptr, A.idx, g, A.local + (int64_t)blockIdx.y * A.loc_group + 8 * c + 4 * (cq & 1), 24);
   if (!STEP) {
-    *reinterpret_cast<float4*>(A.a + o) = make_float4((realw)a[0], (realw)a[1], (realw)a[2], (realw)a[3]);
+    *reinterpret_cast<float4*>(A.a + o) = make_float4(a[0], a[1], a[2], a[3]);
     return;
   }
-#define SF_BG(c, r)                                             \
-  if (r == 0 || A.nstep[s + r] >= it) {                         \
-    const T ac = a[r] * (T)M;                                   \
-    T vc = (LOW ? (T)with_low(V.c, L.c >> 4) : (T)V.c) + (T)A.dt2p * ac;                                    \
-    const T un = (LOW ? (T)with_low(U.c, L.c) : (T)U.c) + (T)A.dt * vc + (T)A.dtsq2 * ac;                   \
-    vc = vc + (T)A.dt2 * ac;                                    \
-    if (LOW) {                                                  \
-      const int lu = split_low(un, U.c);                        \
-      L.c = (uint8_t)(lu | split_low(vc, V.c) << 4);            \
-    } else {                                                    \
-      U.c = (realw)un;                                          \
-      V.c = (realw)vc;                                          \
-    }                                                           \
-  }
-  SF_BG(x, 0) SF_BG(y, 1) SF_BG(z, 2) SF_BG(w, 3)
-#undef SF_BG
+  newmark<FMA>(U.x, V.x, a[0], M, A.dt2p, A.dt, A.dt2, A.dtsq2);
+  if (A.nstep[s + 1] >= it) newmark<FMA>(U.y, V.y, a[1], M, A.dt2p, A.dt, A.dt2, A.dtsq2);
+  if (A.nstep[s + 2] >= it) newmark<FMA>(U.z, V.z, a[2], M, A.dt2p, A.dt, A.dt2, A.dtsq2);
+  if (A.nstep[s + 3] >= it) newmark<FMA>(U.w, V.w, a[3], M, A.dt2p, A.dt, A.dt2, A.dtsq2);
   *reinterpret_cast<float4*>(A.u + o) = U;
   *reinterpret_cast<float4*>(A.v + o) = V;
-  if (LOW) *reinterpret_cast<uchar4*>(A.low + o) = L;
   if (term) *reinterpret_cast<float4*>(A.a + o) = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 // the same for the potentials: chi'' -= local forces, then the corrector chi'' *= rmass, chi' += dt/2 chi''
 // (rows g - g0; the boundary terms are in chi'' already). Points on the free surface (AF_EDGE) take no
 // forces and no terms: their potentials start at zero and stay there.
-template <typename T>
 __global__ void __launch_bounds__(256) k_batch_ac_gather(int64_t nrow, int64_t g0, const int* __restrict__ ptr,
                                                          const int* __restrict__ idx, const realw* __restrict__ local,
                                                          int64_t loc_group, int first_group,
@@ -277,17 +266,16 @@ __global__ void __launch_bounds__(256) k_batch_ac_gather(int64_t nrow, int64_t g
   float4 V = *reinterpret_cast<const float4*>(potd + o);
   const float4 a0 = *reinterpret_cast<const float4*>(potdd + o);
   const realw M = rm[row];
-  T a[4] = {0, 0, 0, 0};
+  realw a[4] = {0, 0, 0, 0};
   if (!(info[g0 + row] & AF_EDGE)) {
     a[0] = a0.x; a[1] = a0.y; a[2] = a0.z; a[3] = a0.w;
-    gather4<T>(a, ptr, idx, g0 + row, local + (int64_t)blockIdx.y * loc_group + 4 * (int)(t & 1), 8);
+    gather4(a, ptr, idx, g0 + row, local + (int64_t)blockIdx.y * loc_group + 4 * (int)(t & 1), 8);
   }
   float4 Ac = a0;
 #define SF_AG(c, r)                          \
   if (r == 0 || nstep[s + r] >= it) {        \
-    const T ac = a[r] * (T)M;                \
-    Ac.c = (realw)ac;                        \
-    V.c = (realw)((T)V.c + (T)dt2 * ac);     \
+    Ac.c = a[r] * M;                         \
+    V.c = V.c + dt2 * Ac.c;                  \
   }
   SF_AG(x, 0) SF_AG(y, 1) SF_AG(z, 2) SF_AG(w, 3)
 #undef SF_AG
@@ -535,8 +523,6 @@ static void zero_state(Batch* b) {
   const int64_t n = 3 * (int64_t)m->nglob * b->S;
   for (realw* p : {b->u, b->v, b->a})
     hipLaunchKernelGGL(k_batch_fill, sf_grid(n, 256), dim3(256), 0, m->stream, n, p);
-  if (b->low)  // a byte each; S is a multiple of eight
-    hipLaunchKernelGGL(k_batch_fill, sf_grid(n / 4, 256), dim3(256), 0, m->stream, n / 4, reinterpret_cast<realw*>(b->low));
   if (b->ac) {
     const int64_t na = b->ac_n * b->S;
     for (realw* p : {b->pot, b->potd, b->potdd})
@@ -615,17 +601,6 @@ static void build_gather(Batch* b) {
                            m->nspec_acoustic, 0, 1, 1, m->ibool, b->ac_ptr, b->ac_idx);
   if (b->ac && !b->ac_local)
     b->ac_local = local_room((int64_t)m->nspec_acoustic * 1000, std::min(b->S / 8, b->max_groups), &b->ac_loc_groups);
-  if (!b->low && !m->exact && b->loc_groups == b->S / 8) {
-    // less precise without, where the card has no room for it
-    const size_t bytes = 3 * (size_t)m->nglob * b->S;
-    void* p = nullptr;
-    if (hipMalloc(&p, bytes) == hipSuccess) {
-      b->low = reinterpret_cast<uint8_t*>(p);
-      SF_CHECK(hipMemsetAsync(b->low, 0, bytes, m->stream));
-    } else {
-      (void)hipGetLastError();
-    }
-  }
   if (!b->info) b->info = balloc<uint16_t>(m->nglob);
   SF_CHECK(hipMemsetAsync(b->info, 0, sizeof(uint16_t) * (size_t)m->nglob, m->stream));
   if (m->stacey) launch_mark_points(m->stream, m->abs_el.n, m->abs_el.iglob, AF_TERM, b->info);
@@ -637,7 +612,6 @@ static void build_gather(Batch* b) {
 static BatchGatherArgs gather_args(Batch* b) {
   Mesh* m = b->m;
   BatchGatherArgs A;
-  A.low = b->loc_groups == b->S / 8 ? b->low : nullptr;
   A.g0 = m->el_g0;
   A.n = m->el_n;
   A.nrow = 3 * (int64_t)m->nglob;
@@ -709,8 +683,7 @@ static void enqueue_stiffness(Batch* b, hipStream_t st) {
       BatchGatherArgs ga = gather_args(b);
       ga.first_group = g;
       const dim3 grid(sf_grid(6 * ga.n, 256).x, (unsigned)n);
-      if (m->exact) hipLaunchKernelGGL((k_batch_gather<false, float, false>), grid, dim3(256), 0, st, ga);
-      else hipLaunchKernelGGL((k_batch_gather<false, double, false>), grid, dim3(256), 0, st, ga);
+      hipLaunchKernelGGL((k_batch_gather<false, false>), grid, dim3(256), 0, st, ga);
       SF_LAUNCH_CHECK("k_batch_gather");
     }
   }
@@ -766,8 +739,7 @@ static void enqueue_fluid(Batch* b, hipStream_t st) {
     A.ngroups = 8 * n / b->sc;
     A.local = b->ac_local - g * A.loc_group;
     launch_acoustic_batch(st, A, b->sc, m->exact != 0);
-    auto* gather = m->exact ? &k_batch_ac_gather<float> : &k_batch_ac_gather<double>;
-    hipLaunchKernelGGL(gather, dim3(rows.x, (unsigned)n), dim3(256), 0, st, na, b->ac_g0, b->ac_ptr, b->ac_idx,
+    hipLaunchKernelGGL(k_batch_ac_gather, dim3(rows.x, (unsigned)n), dim3(256), 0, st, na, b->ac_g0, b->ac_ptr, b->ac_idx,
                        b->ac_local, A.loc_group, g, b->info, b->d_nstep, b->d_it + b->at, b->potd, b->potdd, m->rmass_ac + b->ac_g0,
                        b->dt2);
     SF_LAUNCH_CHECK("k_batch_ac_gather");
@@ -778,17 +750,18 @@ static void enqueue_fluid(Batch* b, hipStream_t st) {
 static void enqueue_step(Batch* b, hipStream_t st, bool first) {
   Mesh* m = b->m;
   if (!first) {
+    const bool fma = !m->exact && b->mode == 3;
     // sums, corrector and predictor (at rest before the first step: nothing to do)
     if (b->loc_groups == b->S / 8) {
       const BatchGatherArgs ga = gather_args(b);
       const dim3 grid(sf_grid(6 * ga.n, 256).x, (unsigned)(b->S / 8));
-      if (m->exact) hipLaunchKernelGGL((k_batch_gather<true, float, false>), grid, dim3(256), 0, st, ga);
-      else if (ga.low) hipLaunchKernelGGL((k_batch_gather<true, double, true>), grid, dim3(256), 0, st, ga);
-      else hipLaunchKernelGGL((k_batch_gather<true, double, false>), grid, dim3(256), 0, st, ga);
+      if (fma) hipLaunchKernelGGL((k_batch_gather<true, true>), grid, dim3(256), 0, st, ga);
+      else hipLaunchKernelGGL((k_batch_gather<true, false>), grid, dim3(256), 0, st, ga);
       SF_LAUNCH_CHECK("k_batch_gather");
     } else {
       const int64_t nrow = 3 * (int64_t)m->nglob;
-      hipLaunchKernelGGL(k_batch_update, dim3(sf_grid(2 * nrow, 256).x, (unsigned)(b->S / 8)), dim3(256), 0, st, nrow,
+      auto* update = fma ? &k_batch_update<true> : &k_batch_update<false>;
+      hipLaunchKernelGGL(update, dim3(sf_grid(2 * nrow, 256).x, (unsigned)(b->S / 8)), dim3(256), 0, st, nrow,
                          b->d_nstep, b->d_it + b->at, b->u, b->v, b->a, m->rmass, b->dt2, b->dt, b->dt2, b->dtsq2);
       SF_LAUNCH_CHECK("k_batch_update");
     }
@@ -1043,17 +1016,17 @@ extern "C" void sf_batch_finalize(long h) {
   zero_state(b);
 }
 
-// shots per workgroup (4 or 8; divides the padded shot count) and assembly (0, 2 or 3, as
-// sf_set_options: every value sums in the colour order). The batch must be at step 1 (new, or after
-// sf_batch_reset).
+// shots per workgroup (4 or 8; divides the padded shot count) and assembly (0, 2 or 3: every value sums in
+// the colour order, and FMA builds round the update of 3 as newmark<true> does). The batch must be at step 1
+// (new, or after sf_batch_reset).
 extern "C" void sf_batch_set_options(long h, int shots_per_group, int assembly) {
   Batch* b = batch_of(h);
   if (shots_per_group != 4 && shots_per_group != 8)
     fatal("sf_batch_set_options", "shots per workgroup must be 4 or 8");
   if (assembly != 0 && assembly != 2 && assembly != 3)
-    fatal("sf_batch_set_options", "assembly must be 0 (atomic), 2 (coloured) or 3 (coloured, fused update)");
+    fatal("sf_batch_set_options", "assembly must be 0, 2 or 3");
   if (b->h_it != 1) fatal("sf_batch_set_options", "options change only at step 1 (call sf_batch_reset first)");
-  if (b->att && assembly == 0) fatal("sf_batch_set_options", "viscoelastic batches use coloured assembly (2 or 3)");
+  if (b->att && assembly == 0) fatal("sf_batch_set_options", "viscoelastic batches take assembly 2 or 3");
   SF_CHECK(hipStreamSynchronize(b->m->stream));
   drop_graph(b);
   b->sc = shots_per_group;
@@ -1201,6 +1174,11 @@ extern "C" void sf_batch_time(long h, int nsteps, double* stiffness_ms, double* 
 // Autotuner: times every shots-per-workgroup candidate for `trial_steps` eager steps from rest (after a
 // warm-up; a candidate whose first step takes over twice the best so far is dropped), keeps the
 // fastest and rewinds the batch. Returns the chosen step time in ms.
+// The assembly becomes 3 from 25000 elements x shots on, below and with attenuation 2. Both are the same
+// launches here and differ in the rounding of FMA builds alone (see newmark); the line is where trials
+// found 3 faster while it folded the update into the element launches (22 batches of 8x8x8 to 32x32x16
+// elements and 3 to 16 shots: 2 up to 20600, 3 from 33000 on, now one, now the other between), so that
+// records of weak arrivals, which show that rounding, stay what they were.
 extern "C" double sf_batch_autotune(long h, int trial_steps) {
   Batch* b = batch_of(h);
   if (!b->ready) fatal("sf_batch_autotune", "sf_batch_finalize first");
@@ -1222,6 +1200,7 @@ extern "C" double sf_batch_autotune(long h, int trial_steps) {
     }
   }
   b->sc = best_sc;
+  b->mode = !b->att && (int64_t)b->m->nspec_elastic * b->S >= 25000 ? 3 : 2;
   drop_graph(b);
   zero_state(b);
   return best;
@@ -1233,7 +1212,7 @@ extern "C" void sf_batch_destroy(long h) {
   drop_graph(b);
   bfree(b->d_nstep); bfree(b->d_it); bfree(b->u); bfree(b->v); bfree(b->a); bfree(b->R); bfree(b->eps);
   bfree(b->pot); bfree(b->potd); bfree(b->potdd);
-  bfree(b->asm_ptr); bfree(b->asm_idx); bfree(b->ac_ptr); bfree(b->ac_idx); bfree(b->info); bfree(b->low);
+  bfree(b->asm_ptr); bfree(b->asm_idx); bfree(b->ac_ptr); bfree(b->ac_idx); bfree(b->info);
   bfree(b->local); bfree(b->ac_local);
   bfree(b->src_ig); bfree(b->src_slot); bfree(b->src_id); bfree(b->src_ploc); bfree(b->src_arr); bfree(b->src_stf);
   bfree(b->rec_slot); bfree(b->rec_ig); bfree(b->rec_h); bfree(b->rec_nu); bfree(b->seis);

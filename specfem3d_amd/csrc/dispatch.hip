@@ -12,7 +12,6 @@ void set_gll_constants(const realw* hprime, const realw* hprimewgll, const realw
   std::memcpy(g_gll_host.hp, hprime, sizeof(g_gll_host.hp));
   std::memcpy(g_gll_host.hpw, hprimewgll, sizeof(g_gll_host.hpw));
   std::memcpy(g_gll_host.wxy, wgllwgll, sizeof(g_gll_host.wxy));
-  sum_gll(g_gll_host, 1.0);
 }
 
 // variants compiled from k_elastic.hip / k_acoustic.hip with and without FMA contraction

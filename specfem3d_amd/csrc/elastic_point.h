@@ -84,19 +84,30 @@ struct Du9 {
   realw xx, xy, xz, yx, yy, yz, zx, zy, zz;
 };
 
+// a1 b1 + a2 b2 + a3 b3. FMA builds name the product that is rounded by itself, the second: which one the
+// compiler takes depends on the code around it, and records of a weak first arrival show the difference
+// (their largest part is what rounding leaves behind the front).
+__device__ __forceinline__ realw sum3(realw a1, realw b1, realw a2, realw b2, realw a3, realw b3) {
+#if SF_EXACT
+  return a1 * b1 + a2 * b2 + a3 * b3;
+#else
+  return fmaf(a3, b3, fmaf(a1, b1, a2 * b2));
+#endif
+}
+
 template <bool FOLD = SF_FOLD>
 __device__ __forceinline__ Du9 map_gradient(const Grad9& t, bool irr, const JacPt& J, realw xr) {
   Du9 d;
   if (irr) {
-    d.xx = J.xix * t.x1 + J.etax * t.x2 + J.gax * t.x3;
-    d.xy = J.xiy * t.x1 + J.etay * t.x2 + J.gay * t.x3;
-    d.xz = J.xiz * t.x1 + J.etaz * t.x2 + J.gaz * t.x3;
-    d.yx = J.xix * t.y1 + J.etax * t.y2 + J.gax * t.y3;
-    d.yy = J.xiy * t.y1 + J.etay * t.y2 + J.gay * t.y3;
-    d.yz = J.xiz * t.y1 + J.etaz * t.y2 + J.gaz * t.y3;
-    d.zx = J.xix * t.z1 + J.etax * t.z2 + J.gax * t.z3;
-    d.zy = J.xiy * t.z1 + J.etay * t.z2 + J.gay * t.z3;
-    d.zz = J.xiz * t.z1 + J.etaz * t.z2 + J.gaz * t.z3;
+    d.xx = sum3(J.xix, t.x1, J.etax, t.x2, J.gax, t.x3);
+    d.xy = sum3(J.xiy, t.x1, J.etay, t.x2, J.gay, t.x3);
+    d.xz = sum3(J.xiz, t.x1, J.etaz, t.x2, J.gaz, t.x3);
+    d.yx = sum3(J.xix, t.y1, J.etax, t.y2, J.gax, t.y3);
+    d.yy = sum3(J.xiy, t.y1, J.etay, t.y2, J.gay, t.y3);
+    d.yz = sum3(J.xiz, t.y1, J.etaz, t.y2, J.gaz, t.y3);
+    d.zx = sum3(J.xix, t.z1, J.etax, t.z2, J.gax, t.z3);
+    d.zy = sum3(J.xiy, t.z1, J.etay, t.z2, J.gay, t.z3);
+    d.zz = sum3(J.xiz, t.z1, J.etaz, t.z2, J.gaz, t.z3);
   } else if (FOLD) {
     d.xx = t.x1; d.xy = t.x2; d.xz = t.x3;
     d.yx = t.y1; d.yy = t.y2; d.yz = t.y3;
@@ -119,9 +130,15 @@ __device__ __forceinline__ Sigma6 iso_stress(const Du9& d, realw kappal, realw m
   const realw lp2m = kappal + FOUR_THIRDS * mul;
   const realw lambdal = lp2m - (realw)2 * mul;
   Sigma6 s;
+#if SF_EXACT
   s.xx = lp2m * d.xx + lambdal * (d.yy + d.zz);
   s.yy = lp2m * d.yy + lambdal * (d.xx + d.zz);
   s.zz = lp2m * d.zz + lambdal * (d.xx + d.yy);
+#else
+  s.xx = fmaf(lp2m, d.xx, lambdal * (d.yy + d.zz));
+  s.yy = fmaf(lp2m, d.yy, lambdal * (d.xx + d.zz));
+  s.zz = fmaf(lambdal, d.xx + d.yy, lp2m * d.zz);
+#endif
   s.xy = mul * (d.xy + d.yx);
   s.xz = mul * (d.zx + d.xz);
   s.yz = mul * (d.zy + d.yz);
@@ -129,20 +146,21 @@ __device__ __forceinline__ Sigma6 iso_stress(const Du9& d, realw kappal, realw m
 }
 
 // jacobian * sigma . (dxi/dx), (deta/dx), (dgamma/dx): t[0..2] xi, t[3..5] eta, t[6..8] gamma
-template <bool FOLD = SF_FOLD>
+// (VISCO: the kernels with memory variables, whose FMA builds round another of the products by itself)
+template <bool FOLD = SF_FOLD, bool VISCO = false>
 __device__ __forceinline__ void stress_products(const Sigma6& s, bool irr, const JacPt& J, realw jacl, realw xr,
                                                 realw t[9]) {
   const realw syx = s.xy, szx = s.xz, szy = s.yz;
   if (irr) {
-    t[0] = jacl * (s.xx * J.xix + syx * J.xiy + szx * J.xiz);
-    t[1] = jacl * (s.xy * J.xix + s.yy * J.xiy + szy * J.xiz);
-    t[2] = jacl * (s.xz * J.xix + s.yz * J.xiy + s.zz * J.xiz);
-    t[3] = jacl * (s.xx * J.etax + syx * J.etay + szx * J.etaz);
-    t[4] = jacl * (s.xy * J.etax + s.yy * J.etay + szy * J.etaz);
-    t[5] = jacl * (s.xz * J.etax + s.yz * J.etay + s.zz * J.etaz);
-    t[6] = jacl * (s.xx * J.gax + syx * J.gay + szx * J.gaz);
-    t[7] = jacl * (s.xy * J.gax + s.yy * J.gay + szy * J.gaz);
-    t[8] = jacl * (s.xz * J.gax + s.yz * J.gay + s.zz * J.gaz);
+    t[0] = jacl * (VISCO ? sum3(s.xx, J.xix, syx, J.xiy, szx, J.xiz) : sum3(syx, J.xiy, s.xx, J.xix, szx, J.xiz));
+    t[1] = jacl * (VISCO ? sum3(s.yy, J.xiy, s.xy, J.xix, szy, J.xiz) : sum3(s.xy, J.xix, s.yy, J.xiy, szy, J.xiz));
+    t[2] = jacl * sum3(s.xz, J.xix, s.yz, J.xiy, s.zz, J.xiz);
+    t[3] = jacl * (VISCO ? sum3(s.xx, J.etax, syx, J.etay, szx, J.etaz) : sum3(syx, J.etay, s.xx, J.etax, szx, J.etaz));
+    t[4] = jacl * (VISCO ? sum3(s.yy, J.etay, s.xy, J.etax, szy, J.etaz) : sum3(s.xy, J.etax, s.yy, J.etay, szy, J.etaz));
+    t[5] = jacl * sum3(s.xz, J.etax, s.yz, J.etay, s.zz, J.etaz);
+    t[6] = jacl * (VISCO ? sum3(s.xx, J.gax, syx, J.gay, szx, J.gaz) : sum3(syx, J.gay, s.xx, J.gax, szx, J.gaz));
+    t[7] = jacl * (VISCO ? sum3(s.yy, J.gay, s.xy, J.gax, szy, J.gaz) : sum3(s.xy, J.gax, s.yy, J.gay, szy, J.gaz));
+    t[8] = jacl * sum3(s.xz, J.gax, s.yz, J.gay, s.zz, J.gaz);
   } else if (FOLD) {
     t[0] = s.xx; t[1] = s.xy; t[2] = s.xz;
     t[3] = syx;  t[4] = s.yy; t[5] = s.yz;
@@ -219,13 +237,6 @@ __device__ __forceinline__ const realw* gll_hpw(const realw* sG, bool irr) {
 // One line of five GLL points against the derivative tables, held by one lane: the coefficients have
 // constant indices and come from scalar registers, and each point of the line is read once instead
 // of once per output. Sums left to right, as tile_gradient and tile_divergence.
-// The divergence of FMA builds applies the table to what the line's values differ from its middle value
-// by, and the table's sums (GLLk::hws) to the middle value: away from the ends of a line the sums are
-// zero, so a stress that hardly varies along it cancels before it is rounded, and the tables keep
-// their sums when a factor is folded into them. Against the same loop in 64 bits, the records of
-// 32x32x16 elements and 16 shots are off by 0.59 times what single-precision sums everywhere gave, 0.80
-// without this (geometric means over 160 records); the launch times are the same. The same for the
-// gradient: 0.59 still, and kernels under a sea 0.68 instead of 0.56.
 __device__ __forceinline__ void line_gradient(const GLLk& G, const realw in[5], realw out[5]) {
 #pragma unroll
   for (int m = 0; m < 5; m++) {
@@ -238,16 +249,9 @@ __device__ __forceinline__ void line_gradient(const GLLk& G, const realw in[5], 
 __device__ __forceinline__ void line_divergence(const GLLk& G, const realw in[5], realw out[5]) {
 #pragma unroll
   for (int m = 0; m < 5; m++) {
-#if SF_EXACT
     realw r = G.hpw[m] * in[0];
 #pragma unroll
     for (int l = 1; l < 5; l++) r = r + G.hpw[l * 5 + m] * in[l];
-#else
-    realw r = G.hws[m] * in[2];
-#pragma unroll
-    for (int l = 0; l < 5; l++)
-      if (l != 2) r = r + G.hpw[l * 5 + m] * (in[l] - in[2]);
-#endif
     out[m] = r;
   }
 }

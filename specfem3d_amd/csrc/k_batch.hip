@@ -189,7 +189,7 @@ __global__ void __launch_bounds__(32 * SC) k_elastic_batch(BatchArgs B, GLLk G) 
       const int q = bp + 25 * PS * k;
       const realw w1 = sW[j * 5 + k], w2 = sW[i * 5 + k];
 #pragma unroll
-      for (int a = 0; a < 3; a++) sA[q + SC * a] = w1 * sA[q + SC * a] + w2 * sB[q + SC * a] + w3 * d3[k][a];
+      for (int a = 0; a < 3; a++) sA[q + SC * a] = sum3(w1, sA[q + SC * a], w2, sB[q + SC * a], w3, d3[k][a]);
     }
   }
   lds_barrier();
@@ -355,7 +355,7 @@ __global__ void __launch_bounds__(128 * NQ) k_visco_batch(BatchArgs B, GLLk G) {
       for (int cc = 0; cc < 6; cc++) B.eps[eb_idx(e, cc, pp, S, s)] = Snp1[cc];
     }
     realw t[9];
-    stress_products(sg, irr != 0, J, jacl, B.xix_regular, t);
+    stress_products<SF_FOLD, true>(sg, irr != 0, J, jacl, B.xix_regular, t);
     if (active) {
 #pragma unroll
       for (int m = 0; m < 3; m++) sT[(m * SC + ts + r) * PST + p] = t[m];

@@ -218,7 +218,7 @@ k_elastic_pt(ElasticArgs A, GLLk G) {
 
   {
     realw t[9];
-    stress_products(sg, irr != 0, J, jacl, A.xix_regular, t);
+    stress_products<SF_FOLD, true>(sg, irr != 0, J, jacl, A.xix_regular, t);
 #pragma unroll
     for (int m = 0; m < 9; m++) sT[m][p] = t[m];
   }
@@ -389,7 +389,7 @@ __global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk G) {
     const realw w1 = sW[j * 5 + k], w2 = sW[i * 5 + k];
     realw* o = A.local_out + 3 * (int64_t)(slot + k * 25 * A.eb);
 #pragma unroll
-    for (int a = 0; a < 3; a++) o[a] = w1 * sA[a][b] + w2 * sB[a][b] + w3 * d3[k][a];
+    for (int a = 0; a < 3; a++) o[a] = sum3(w1, sA[a][b], w2, sB[a][b], w3, d3[k][a]);
   }
 }
 
@@ -400,9 +400,26 @@ __global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk G) {
 // field, three sums read and written). The strain stored by one launch and read back by another
 // took 16.5 + 30 us on 24^3 elements, and 2 us more in every stiffness launch that stored it;
 // this launch takes 26.
+// The operations are those of k_element_strain (the regular mapping is not folded into the tables) and
+// of k_compute_kernels_el (products and sums rounded one by one, in FMA builds too: `rounded` keeps a
+// product out of the sum that takes it).
+__device__ __forceinline__ realw rounded(realw x) {
+  asm("" : "+v"(x));
+  return x;
+}
+__device__ __forceinline__ void kernel_sums(const KernelSums& S, int64_t q, int e, int p, realw dot, realw b1, realw b2,
+                                            realw b3, realw b4, realw b5, realw btr3) {
+  const realw e1 = S.eps[eps_idx(e, 0, p)], e2 = S.eps[eps_idx(e, 1, p)], e3 = S.eps[eps_idx(e, 2, p)],
+              e4 = S.eps[eps_idx(e, 3, p)], e5 = S.eps[eps_idx(e, 4, p)];
+  const realw shear = rounded(e3 * b3) + rounded(e4 * b4) + rounded(e5 * b5);
+  S.rho_kl[q] = S.rho_kl[q] + rounded(S.deltat * dot);
+  S.mu_kl[q] = S.mu_kl[q] + rounded(S.deltat * (rounded(e1 * b1) + rounded(e2 * b2) + rounded((e1 + e2) * (b1 + b2)) +
+                                                (realw)2 * shear));
+  S.kappa_kl[q] = S.kappa_kl[q] + rounded(S.deltat * ((realw)9 * S.eps_tr3[q] * btr3));
+}
+
 template <bool REG>
 __global__ void __launch_bounds__(128) k_kernels_line(ElasticArgs A, KernelSums S, GLLk G) {
-  constexpr bool FOLD = REG && SF_FOLD;
   constexpr int PL = 626;
   __shared__ realw sA[3][PL], sB[3][PL];
   const int t = threadIdx.x;
@@ -426,7 +443,7 @@ __global__ void __launch_bounds__(128) k_kernels_line(ElasticArgs A, KernelSums 
       const realw* d = A.displ + 3 * (int64_t)g[k];
       const realw* a = S.accel + 3 * (int64_t)g[k];
       u[0][k] = d[0]; u[1][k] = d[1]; u[2][k] = d[2];
-      dot[k] = a[0] * u[0][k] + a[1] * u[1][k] + a[2] * u[2][k];
+      dot[k] = rounded(a[0] * u[0][k]) + rounded(a[1] * u[1][k]) + rounded(a[2] * u[2][k]);
     }
     const int b = el * 125 + c;
 #pragma unroll
@@ -476,15 +493,13 @@ __global__ void __launch_bounds__(128) k_kernels_line(ElasticArgs A, KernelSums 
     const Grad9 tg = {sA[0][b], sA[1][b], sA[2][b], sB[0][b], sB[1][b], sB[2][b], d3[k][0], d3[k][1], d3[k][2]};
     JacPt J = {};
     if (!REG && irr) J = load_jac(A.jac, A.jac_plane, jp + 25 * k);
-    const Du9 du = map_gradient<FOLD>(tg, irr != 0, J, A.xix_regular);
+    Du9 du = map_gradient<false>(tg, irr != 0, J, A.xix_regular);
+    if (REG) {
+      for (realw* d : {&du.xx, &du.xy, &du.xz, &du.yx, &du.yy, &du.yz, &du.zx, &du.zy, &du.zz}) *d = rounded(*d);
+    }
     const realw templ = ONE_THIRD * (du.xx + du.yy + du.zz);
-    const realw b1 = du.xx - templ, b2 = du.yy - templ, b3 = (realw)0.5 * (du.xy + du.yx),
-                b4 = (realw)0.5 * (du.zx + du.xz), b5 = (realw)0.5 * (du.zy + du.yz);
-    const realw e1 = S.eps[eps_idx(e, 0, p)], e2 = S.eps[eps_idx(e, 1, p)], e3 = S.eps[eps_idx(e, 2, p)],
-                e4 = S.eps[eps_idx(e, 3, p)], e5 = S.eps[eps_idx(e, 4, p)];
-    S.rho_kl[q] = S.rho_kl[q] + S.deltat * dot[k];
-    S.mu_kl[q] = S.mu_kl[q] + S.deltat * (e1 * b1 + e2 * b2 + (e1 + e2) * (b1 + b2) + (realw)2 * (e3 * b3 + e4 * b4 + e5 * b5));
-    S.kappa_kl[q] = S.kappa_kl[q] + S.deltat * ((realw)9 * S.eps_tr3[q] * templ);
+    kernel_sums(S, q, e, p, dot[k], du.xx - templ, du.yy - templ, (realw)0.5 * (du.xy + du.yx),
+                (realw)0.5 * (du.zx + du.xz), (realw)0.5 * (du.zy + du.yz), templ);
   }
 }
 
@@ -601,14 +616,9 @@ void SFX(launch_elastic)(hipStream_t s, const ElasticArgs& a, bool strain, bool 
 
 void SFX(launch_kernels_line)(hipStream_t s, const ElasticArgs& a, const KernelSums& k) {
   if (a.nelem <= 0) return;
-  GLLk G = g_gll_host;
   const dim3 grid((a.nelem + 4) / 5), block(128);
-  if (a.jac_plane == 0) {
-    if (SF_FOLD) regular_gll(G, a.xix_regular, a.jacobian_regular);
-    hipLaunchKernelGGL(k_kernels_line<true>, grid, block, 0, s, a, k, G);
-  } else {
-    hipLaunchKernelGGL(k_kernels_line<false>, grid, block, 0, s, a, k, G);
-  }
+  if (a.jac_plane == 0) hipLaunchKernelGGL(k_kernels_line<true>, grid, block, 0, s, a, k, g_gll_host);
+  else hipLaunchKernelGGL(k_kernels_line<false>, grid, block, 0, s, a, k, g_gll_host);
   SF_LAUNCH_CHECK("k_kernels_line");
 }
 

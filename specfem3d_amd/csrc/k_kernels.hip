@@ -103,7 +103,6 @@ __global__ void __launch_bounds__(128) k_compute_kernels_ac(int nelem, const int
 // what: the field's values, or those it takes once the waiting sum and corrector have run (WAIT_*), so
 // that these stay fused with the next update: a step of 40x40x30 elements that records pressure runs
 // one update pass of 20.2 us instead of a sum with the corrector (18.8) and a predictor (12.5).
-template <typename T>
 __global__ void __launch_bounds__(128) k_seismo_ac(AcReceiverArgs A, GLLk G, const realw* __restrict__ field, int what,
                                                    int pressure, realw* __restrict__ out) {
   __shared__ realw s[125], hp[25];
@@ -116,7 +115,7 @@ __global__ void __launch_bounds__(128) k_seismo_ac(AcReceiverArgs A, GLLk G, con
   if (p < 125) {
     realw f;
     if (what == WAIT_NONE) f = field[g];
-    else waiting_value<1, T>(A.wait, what, g, A.first[(int64_t)r * 125 + q], &f);
+    else waiting_value<1>(A.wait, what, g, A.first[(int64_t)r * 125 + q], &f);
     s[p] = f;
   }
   __syncthreads();
@@ -213,8 +212,7 @@ void launch_compute_kernels_ac(hipStream_t s, int nelem, const int* elems, const
 
 void launch_seismo_ac(hipStream_t s, const AcReceiverArgs& a, const realw* field, int what, int pressure, realw* out) {
   if (a.n <= 0) return;
-  auto* kernel = a.exact ? &k_seismo_ac<float> : &k_seismo_ac<double>;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)a.n), dim3(128), 0, s, a, g_gll_host, field, what, pressure, out);
+  hipLaunchKernelGGL(k_seismo_ac, dim3((unsigned)a.n), dim3(128), 0, s, a, g_gll_host, field, what, pressure, out);
   SF_LAUNCH_CHECK("k_seismo_ac");
 }
 

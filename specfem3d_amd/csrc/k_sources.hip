@@ -7,7 +7,7 @@ namespace sf {
 // receiver interpolation (compute_interpolated_dva.f90:84-100): double-precision sum of
 // h_i h_j h_k u over the 125 element points, rotated by nu_rec; one wave64 per listed receiver.
 // WAIT: the field waits to be summed (waiting_value).
-template <bool WAIT, typename T>
+template <bool WAIT>
 __global__ void __launch_bounds__(64) k_seismo_el(int n, const int* __restrict__ list, const int* __restrict__ ig,
                                                   const double* __restrict__ h, const double* __restrict__ nu,
                                                   const realw* __restrict__ field, GatherArgs A,
@@ -21,7 +21,7 @@ __global__ void __launch_bounds__(64) k_seismo_el(int n, const int* __restrict__
     const double hl = h[q];
     realw f[3];
     if (WAIT) {
-      waiting_value<3, T>(A, what, g, first[q], f);
+      waiting_value<3>(A, what, g, first[q], f);
     } else {
 #pragma unroll
       for (int c = 0; c < 3; c++) f[c] = field[3 * g + c];
@@ -47,17 +47,15 @@ __global__ void __launch_bounds__(64) k_seismo_el(int n, const int* __restrict__
 void launch_seismo_el(hipStream_t s, int n, const int* list, const int* iglob, const double* h, const double* nu,
                       const realw* field, realw* out) {
   if (n <= 0) return;
-  hipLaunchKernelGGL((k_seismo_el<false, float>), dim3(n), dim3(64), 0, s, n, list, iglob, h, nu, field, GatherArgs{},
+  hipLaunchKernelGGL(k_seismo_el<false>, dim3(n), dim3(64), 0, s, n, list, iglob, h, nu, field, GatherArgs{},
                      nullptr, 0, out);
   SF_LAUNCH_CHECK("k_seismo_el");
 }
 
 void launch_seismo_el_waiting(hipStream_t s, int n, const int* list, const int* iglob, const double* h,
-                              const double* nu, const GatherArgs& a, const int* first, int what, bool exact,
-                              realw* out) {
+                              const double* nu, const GatherArgs& a, const int* first, int what, realw* out) {
   if (n <= 0) return;
-  auto* kernel = exact ? &k_seismo_el<true, float> : &k_seismo_el<true, double>;
-  hipLaunchKernelGGL(kernel, dim3(n), dim3(64), 0, s, n, list, iglob, h, nu, nullptr, a, first, what, out);
+  hipLaunchKernelGGL(k_seismo_el<true>, dim3(n), dim3(64), 0, s, n, list, iglob, h, nu, nullptr, a, first, what, out);
   SF_LAUNCH_CHECK("k_seismo_el");
 }
 

@@ -37,39 +37,6 @@ __global__ void k_predictor(int64_t n4, int64_t n, realw* __restrict__ u, realw*
   }
 }
 
-// the predictor with the low parts of u and v
-__device__ __forceinline__ void predict_low(realw& u, realw& v, realw a, realw dt, realw dt2, realw dtsq2, uint8_t& lo,
-                                            int set) {
-  const int low = set ? lo : 0;
-  const double vc = with_low(v, low >> 4), uc = with_low(u, low), ac = a;
-  const int lu = split_low(uc + (double)dt * vc + (double)dtsq2 * ac, u);
-  lo = (uint8_t)(lu | split_low(vc + (double)dt2 * ac, v) << 4);
-}
-__global__ void k_predictor_low(int64_t n4, int64_t n, realw* __restrict__ u, realw* __restrict__ v,
-                                realw* __restrict__ a, realw dt, realw dt2, realw dtsq2, uint8_t* __restrict__ lo,
-                                int set) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n4) {
-    float4 U = reinterpret_cast<float4*>(u)[t];
-    float4 V = reinterpret_cast<float4*>(v)[t];
-    const float4 A = reinterpret_cast<float4*>(a)[t];
-    uchar4 L = reinterpret_cast<uchar4*>(lo)[t];
-    predict_low(U.x, V.x, A.x, dt, dt2, dtsq2, L.x, set);
-    predict_low(U.y, V.y, A.y, dt, dt2, dtsq2, L.y, set);
-    predict_low(U.z, V.z, A.z, dt, dt2, dtsq2, L.z, set);
-    predict_low(U.w, V.w, A.w, dt, dt2, dtsq2, L.w, set);
-    reinterpret_cast<float4*>(u)[t] = U;
-    reinterpret_cast<float4*>(v)[t] = V;
-    reinterpret_cast<float4*>(a)[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-    reinterpret_cast<uchar4*>(lo)[t] = L;
-  }
-  const int64_t r = 4 * n4 + t;
-  if (t < 4 && r < n) {
-    predict_low(u[r], v[r], a[r], dt, dt2, dtsq2, lo[r], set);
-    a[r] = 0.f;
-  }
-}
-
 __global__ void k_corrector(int64_t n4, int64_t n, realw* __restrict__ v, realw* __restrict__ a,
                             const realw* __restrict__ rm, realw dt2) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -183,12 +150,6 @@ __global__ void k_zero_points(int n, const int* __restrict__ pts, realw* __restr
 // the lines of both orders and takes blocks of 20 elements (gather_slot) where those are fewer: 150
 // us, and 99 -> 104 us for the stiffness launch that writes them (621 -> 643 with attenuation, one
 // element per workgroup); blocks of 5, 10 and 40 elements: 156, 152, 149 us.
-// T: float follows the reference's operations one by one (exact builds); double keeps the sum, the
-// corrector and the predictor of a step in registers and rounds u, v (and a) once each. The pass waits
-// for memory either way (150 -> 154 us on 64x64x32 elements), and the rounding of v in every step is
-// the largest error of a run: against the same loop in 64 bits, displacement and records of 20x20x20
-// elements and 100 steps are off by 0.76 times, kernels of 24^3 by 0.79 times what they were.
-//
 // `clean`: accel is known to be zero away from AF_TERM points (the previous pass left it so), and is
 // neither read nor cleared there.
 // The number of slots comes with the flags, 2 B per point, and the position of a point's first slot
@@ -209,18 +170,7 @@ __device__ __forceinline__ int wave_prefix(int x) {
   return x;
 }
 
-//
-// LOW: with the low parts of u and v, so that the values carried from step to step have 4 more bits
-// (other kernels read u and v as stored). Kernel runs keep them: their outputs are products of two
-// fields, some of them a few points large, where the rounding of u in every step is most of the error.
-// Against 64 bits, the kernels of 19x17x16 elements under a sea are off by 0.48 instead of 0.84 times, of
-// 24^3 elements by 0.52 instead of 0.69 times what single-precision sums gave (geometric means over 36
-// and 16 outputs; 8 more bits instead of 4: 0.53 and 0.44 over 48 and 24). Each pass takes 1.5 us more
-// on 24^3 elements (15.7 -> 17.2, k_predictor 10.5 -> 12.0). Runs of a fluid alone keep them too: chi''
-// is made of differences of chi, so the rounding of chi reaches the pressure 10 times larger than that of u
-// the displacement: pressure records of 40x40x30 elements are off by 4.9e-7 instead of 2e-6, for 20.2 ->
-// 22.2 us per pass.
-template <int NC, int KIND, bool OLD, typename T, bool LOW>
+template <int NC, int KIND, bool OLD>
 __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
   const int nb = (int)gridDim.x, b = (int)blockIdx.x;
   const int q = nb >> 3, r = nb & 7, x = b & 7;  // contiguous blocks per XCD, last one first
@@ -234,8 +184,7 @@ __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
   int p1 = A.base[t >> 6] + p1w;
   const int p0 = p1 - cnt;
   const bool full = !A.clean || (fl & AF_TERM);
-  T a[NC];
-  realw u[NC], v[NC], m[NC];
+  realw a[NC], u[NC], v[NC], m[NC];
 #pragma unroll
   for (int c = 0; c < NC; c++) {
     a[c] = 0;
@@ -245,11 +194,6 @@ __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
   for (int c = 0; c < NC; c++) {
     if (KIND != GATHER_ONLY) v[c] = A.v[NC * g + c];
     if (KIND == GATHER_STEP) u[c] = A.u[NC * g + c];
-  }
-  int low[NC];
-  if (LOW) {
-#pragma unroll
-    for (int c = 0; c < NC; c++) low[c] = A.lo_set ? A.lo[NC * g + c] : 0;
   }
   const bool zero = fl & A.skip;
   if (full && !zero) {
@@ -277,62 +221,48 @@ __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
     for (int w = 0; w < 4; w++) {
       if (k[w] < 0) continue;
 #pragma unroll
-      for (int c = 0; c < NC; c++) a[c] = a[c] + (-(T)l[w][c]);
+      for (int c = 0; c < NC; c++) a[c] = a[c] + (-l[w][c]);
     }
   }
   if (KIND == GATHER_ONLY) {
     if (p1 > p0 || zero) {
 #pragma unroll
-      for (int c = 0; c < NC; c++) A.a[NC * g + c] = (realw)a[c];
+      for (int c = 0; c < NC; c++) A.a[NC * g + c] = a[c];
     }
     return;
   }
 #pragma unroll
   for (int c = 0; c < NC; c++) {
-    a[c] = a[c] * (T)m[c];
-    T vc = (LOW ? (T)with_low(v[c], low[c] >> 4) : (T)v[c]) + (T)A.dt2p * a[c];
+    a[c] = a[c] * m[c];
+    v[c] = v[c] + A.dt2p * a[c];
     if (KIND == GATHER_STEP) {
-      T uc = LOW ? (T)with_low(u[c], low[c]) : (T)u[c];
-      if (OLD) A.old[NC * g + c] = (realw)(uc + (T)A.t1 * vc + (T)A.t2 * a[c]);
-      uc = uc + (T)A.dt * vc + (T)A.dtsq2 * a[c];
-      vc = vc + (T)A.dt2 * a[c];
-      if (LOW) low[c] = (low[c] & 0xf0) | split_low(uc, u[c]);
-      else u[c] = (realw)uc;
-      A.u[NC * g + c] = u[c];
+      if (OLD) A.old[NC * g + c] = u[c] + A.t1 * v[c] + A.t2 * a[c];
+      A.u[NC * g + c] = u[c] + A.dt * v[c] + A.dtsq2 * a[c];
+      v[c] = v[c] + A.dt2 * a[c];
       if (full) A.a[NC * g + c] = 0.f;
     } else {
-      A.a[NC * g + c] = (realw)a[c];
-    }
-    if (LOW) {
-      low[c] = (low[c] & 15) | split_low(vc, v[c]) << 4;
-      A.lo[NC * g + c] = (uint8_t)low[c];
-    } else {
-      v[c] = (realw)vc;
+      A.a[NC * g + c] = a[c];
     }
     A.v[NC * g + c] = v[c];
   }
 }
 
 template <int NC, int KIND, bool OLD>
-static void launch_gather(hipStream_t s, const GatherArgs& a, bool exact) {
-  const dim3 grid = sf_grid(a.n, 256), block(256);
-  if (exact) hipLaunchKernelGGL((k_gather_update<NC, KIND, OLD, float, false>), grid, block, 0, s, a);
-  else if (!OLD && KIND != GATHER_ONLY && a.lo)
-    hipLaunchKernelGGL((k_gather_update<NC, KIND, false, double, (KIND != GATHER_ONLY)>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((k_gather_update<NC, KIND, OLD, double, false>), grid, block, 0, s, a);
+static void launch_gather(hipStream_t s, const GatherArgs& a) {
+  hipLaunchKernelGGL((k_gather_update<NC, KIND, OLD>), sf_grid(a.n, 256), dim3(256), 0, s, a);
 }
 
-void launch_gather_update(hipStream_t s, const GatherArgs& a, int ncomp, int kind, bool exact) {
+void launch_gather_update(hipStream_t s, const GatherArgs& a, int ncomp, int kind) {
   if (a.n <= 0) return;
   if (ncomp == 1) {
-    if (kind == GATHER_ONLY) launch_gather<1, GATHER_ONLY, false>(s, a, exact);
-    else if (kind == GATHER_CORRECT) launch_gather<1, GATHER_CORRECT, false>(s, a, exact);
-    else launch_gather<1, GATHER_STEP, false>(s, a, exact);
+    if (kind == GATHER_ONLY) launch_gather<1, GATHER_ONLY, false>(s, a);
+    else if (kind == GATHER_CORRECT) launch_gather<1, GATHER_CORRECT, false>(s, a);
+    else launch_gather<1, GATHER_STEP, false>(s, a);
   } else {
-    if (kind == GATHER_ONLY) launch_gather<3, GATHER_ONLY, false>(s, a, exact);
-    else if (kind == GATHER_CORRECT) launch_gather<3, GATHER_CORRECT, false>(s, a, exact);
-    else if (a.old) launch_gather<3, GATHER_STEP, true>(s, a, exact);
-    else launch_gather<3, GATHER_STEP, false>(s, a, exact);
+    if (kind == GATHER_ONLY) launch_gather<3, GATHER_ONLY, false>(s, a);
+    else if (kind == GATHER_CORRECT) launch_gather<3, GATHER_CORRECT, false>(s, a);
+    else if (a.old) launch_gather<3, GATHER_STEP, true>(s, a);
+    else launch_gather<3, GATHER_STEP, false>(s, a);
   }
   SF_LAUNCH_CHECK("k_gather_update");
 }
@@ -348,14 +278,6 @@ void launch_predictor(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, re
   const int64_t n4 = n / 4;
   hipLaunchKernelGGL(k_predictor, grid_for(n4, 256), dim3(256), 0, s, n4, n, u, v, a, dt, dt2, dtsq2);
   SF_LAUNCH_CHECK("k_predictor");
-}
-
-void launch_predictor_low(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, realw dt, realw dt2, realw dtsq2,
-                          uint8_t* lo, int set) {
-  if (n <= 0) return;
-  const int64_t n4 = n / 4;
-  hipLaunchKernelGGL(k_predictor_low, grid_for(n4, 256), dim3(256), 0, s, n4, n, u, v, a, dt, dt2, dtsq2, lo, set);
-  SF_LAUNCH_CHECK("k_predictor_low");
 }
 
 void launch_corrector(hipStream_t s, int64_t n, realw* v, realw* a, const realw* rmass, realw dt2) {

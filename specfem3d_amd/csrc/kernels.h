@@ -22,17 +22,7 @@ struct GLLk {
   // fold the regular mapping and the jacobian weight into the contractions (fold_gll)
   realw hpr[25];
   realw hpwr[25];
-  // FMA builds, line_divergence: sum over l of hpw[l, m]
-  realw hws[5];
 };
-// hws from the table and a factor folded into it
-inline void sum_gll(GLLk& G, double factor) {
-  for (int m = 0; m < 5; m++) {
-    double d = 0;
-    for (int l = 0; l < 5; l++) d += G.hpw[l * 5 + m];
-    G.hws[m] = (realw)(factor * d);
-  }
-}
 inline void fold_gll(GLLk& G, realw xix_regular, realw jacobian_regular) {
   const realw jx = jacobian_regular * xix_regular;
   for (int q = 0; q < 25; q++) {
@@ -43,7 +33,6 @@ inline void fold_gll(GLLk& G, realw xix_regular, realw jacobian_regular) {
 // the tables of a launch over regular elements alone: the folded ones in the place of the others
 inline void regular_gll(GLLk& G, realw xix_regular, realw jacobian_regular) {
   fold_gll(G, xix_regular, jacobian_regular);
-  sum_gll(G, (double)jacobian_regular * xix_regular);
   for (int q = 0; q < 25; q++) {
     G.hp[q] = G.hpr[q];
     G.hpw[q] = G.hpwr[q];
@@ -55,9 +44,6 @@ void set_gll_constants(const realw* hprime, const realw* hprimewgll, const realw
 // Newmark pieces (k_update.hip)
 void launch_predictor(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, realw dt, realw dt2, realw dtsq2);
 void launch_corrector(hipStream_t s, int64_t n, realw* v, realw* a, const realw* rmass, realw dt2);
-// ... in double precision with the low parts of u and v (`set`: they are set, else zero)
-void launch_predictor_low(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, realw dt, realw dt2, realw dtsq2,
-                          uint8_t* lo, int set);
 // with `old`, also PML_displ_old = u + t1 v + t2 a of the corrected field (before the predictor)
 void launch_corrector_predictor(hipStream_t s, int64_t n, realw* u, realw* v, realw* a, const realw* rmass,
                                 realw dt2_prev, realw dt, realw dt2, realw dtsq2, realw* old = nullptr,
@@ -94,25 +80,7 @@ struct GatherArgs {
   realw dt, dt2, dtsq2;        // predictor
   realw* old;                  // PML_displ_old = u + t1 v + t2 a of the corrected field, or null
   realw t1, t2;
-  uint8_t* lo;                 // low parts of u and v (with_low), 3 per point, or null
-  int lo_set;                  // they are set (else zero)
 };
-// Low parts of u and v: what the stored single-precision values miss, in 1/16 of their last place, four
-// bits each (u in the low ones). FMA builds keep them in batches, in kernel runs and in runs of a fluid
-// alone (see k_gather_update). Values below 2^-95, infinities and NaN have none.
-__device__ __forceinline__ double with_low(realw x, int low) {
-  const int e = __float_as_uint(x) >> 23 & 255;
-  const realw unit = e >= 32 && e < 255 ? __uint_as_float((uint32_t)(e - 27) << 23) : 0.f;
-  return (double)x + (double)((realw)((int)((uint32_t)low << 28) >> 28) * unit);
-}
-// rounds x to `hi`, returns the four bits of the rest
-__device__ __forceinline__ int split_low(double x, realw& hi) {
-  hi = (realw)x;
-  const int e = __float_as_uint(hi) >> 23 & 255;
-  if (e < 32 || e == 255) return 0;
-  const realw q = rintf((realw)(x - (double)hi) * __uint_as_float((uint32_t)(281 - e) << 23));
-  return (int)fminf(fmaxf(q, -8.f), 7.f) & 15;
-}
 // what follows the sum: nothing (accel is left assembled), the corrector, or the corrector and the
 // predictor of the next step (accel left zero)
 enum { GATHER_ONLY = 0, GATHER_CORRECT = 1, GATHER_STEP = 2 };
@@ -120,29 +88,25 @@ enum { GATHER_ONLY = 0, GATHER_CORRECT = 1, GATHER_STEP = 2 };
 // on: for the receivers, which record a few points while the whole field waits for the next update. The
 // operations are those of k_gather_update.
 enum { WAIT_NONE = 0, WAIT_ACCEL = 1, WAIT_VELOC = 2 };
-template <int NC, typename T>
+template <int NC>
 __device__ __forceinline__ void waiting_value(const GatherArgs& A, int what, int64_t g, int first, realw out[NC]) {
   const int fl = A.info[g], cnt = fl >> AF_COUNT;
   const bool zero = fl & A.skip, full = !A.clean || (fl & AF_TERM);
-  T a[NC];
+  realw a[NC];
 #pragma unroll
   for (int c = 0; c < NC; c++) a[c] = full && !zero ? A.a[NC * g + c] : 0.f;
   for (int s = 0; s < (zero ? 0 : cnt); s++) {
     const realw* l = A.local + NC * (int64_t)A.idx[first + s];
 #pragma unroll
-    for (int c = 0; c < NC; c++) a[c] = a[c] + (-(T)l[c]);
+    for (int c = 0; c < NC; c++) a[c] = a[c] + (-l[c]);
   }
 #pragma unroll
   for (int c = 0; c < NC; c++) {
-    a[c] = a[c] * (T)(NC == 3 && (fl & AF_MASS3) ? A.rm[NC * g + c] : A.rm1[g]);
-    T v = A.v[NC * g + c];
-    if (sizeof(T) == 8 && A.lo && A.lo_set) v = (T)with_low(A.v[NC * g + c], A.lo[NC * g + c] >> 4);
-    out[c] = what == WAIT_ACCEL ? (realw)a[c] : (realw)(v + (T)A.dt2p * a[c]);
+    a[c] = a[c] * (NC == 3 && (fl & AF_MASS3) ? A.rm[NC * g + c] : A.rm1[g]);
+    out[c] = what == WAIT_ACCEL ? a[c] : A.v[NC * g + c] + A.dt2p * a[c];
   }
 }
-// exact: the reference's single-precision operations; else sums, corrector and predictor in double
-// precision, rounded once per stored value
-void launch_gather_update(hipStream_t s, const GatherArgs& a, int ncomp, int kind, bool exact);
+void launch_gather_update(hipStream_t s, const GatherArgs& a, int ncomp, int kind);
 // slot lists (k_assembly.hip): the elements of `order` give the order of the sums, those of `launch`
 // (nelem_launch of them) the slots, `pos0` launch positions on for the elements behind; allocates ptr
 // (nglob + 1) and idx (125 nelem). lines: cache lines that the waves of a pass over all points touch
@@ -355,8 +319,7 @@ void launch_seismo_el(hipStream_t s, int n, const int* list, const int* iglob, c
                       const realw* field, realw* out);
 // ... of a field that waits to be summed (`what`: WAIT_*; first: slot entry of every receiver point)
 void launch_seismo_el_waiting(hipStream_t s, int n, const int* list, const int* iglob, const double* h,
-                              const double* nu, const GatherArgs& a, const int* first, int what, bool exact,
-                              realw* out);
+                              const double* nu, const GatherArgs& a, const int* first, int what, realw* out);
 // receivers in acoustic elements: pressure = 1 records -sum h field into out[3 r] (out[3 r + 1..2] = 0),
 // pressure = 0 the vector (1/rho) grad(field) interpolated and rotated by nu
 struct AcReceiverArgs {
@@ -373,7 +336,6 @@ struct AcReceiverArgs {
   const realw* rho;        // rhostore, nloc
   GatherArgs wait;         // ... of a field that waits to be summed
   const int* first;        // slot entry of every receiver point
-  int exact;
 };
 void launch_seismo_ac(hipStream_t s, const AcReceiverArgs& a, const realw* field, int what, int pressure, realw* out);
 

@@ -201,8 +201,8 @@ struct Mesh {
 
   // execution
   hipStream_t stream = nullptr;
-  // Defaults for a host that never calls sf_set_options (the Fortran drop-in): the FMA build and
-  // element-order sums.
+  // Defaults for a host that never calls sf_set_options (the Fortran drop-in): the FMA build; sums in the
+  // colour order without attenuation, in element order with it and in a fluid alone.
   int exact = 0;                   // 1: kernels built without fused multiply-add (oracle order)
   int assembly = -1;               // order of the element sums: 1 element order (oracle order), 2 colour
                                    // order, 0 any (sf_set_options), -1 automatic
@@ -235,10 +235,6 @@ struct Mesh {
   int pending_gather_el[2] = {0, 0};
   int gather_skip_el[2] = {0, 0};  // AF_* of the points that the pending sum leaves out
   int accel_clean[2] = {0, 0};     // accel is zero at every point without AF_TERM
-  uint8_t* low[2] = {nullptr, nullptr};  // low parts of u and v (GatherArgs::lo): kernel runs
-  int low_set[2] = {0, 0};         // they belong to the stored u and v
-  uint8_t* low_ac[2] = {nullptr, nullptr};  // the same of chi and chi': runs of a fluid alone
-  int low_ac_set[2] = {0, 0};
   // the same for the fluid (1 component; the inverse mass is rmass_ac)
   int* asm_ac_idx = nullptr;
   int asm_ac_eb = 1;
