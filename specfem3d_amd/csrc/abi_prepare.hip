@@ -775,6 +775,18 @@ static void build_term_points(Mesh* m, int fluid) {
   m->term_head[fluid] = dupload(head.data(), (int64_t)head.size());
 }
 
+// `list` with its regular elements first, so that launches over them alone can fold their one mapping into
+// the tables (k_elastic_line): a device list of the caller's, or null where only one kind is listed.
+int* regular_first(Mesh* m, const int* list, int n, int* nreg) {
+  *nreg = m->nspec_irregular ? 0 : n;
+  if (!m->nspec_irregular || n <= 0) return nullptr;
+  std::vector<int> in(n), irr(m->nspec);
+  SF_CHECK(hipMemcpy(in.data(), list, sizeof(int) * in.size(), hipMemcpyDeviceToHost));
+  SF_CHECK(hipMemcpy(irr.data(), m->irregular, sizeof(int) * irr.size(), hipMemcpyDeviceToHost));
+  *nreg = (int)(std::stable_partition(in.begin(), in.end(), [&](int e) { return irr[e] == 0; }) - in.begin());
+  return *nreg == 0 || *nreg == n ? nullptr : dupload(in.data(), n);
+}
+
 // Lists and buffers of the gather assembly for one field: the slots of each point in the processing
 // order, or in the colour order under assembly = 2 (the sums a coloured scatter makes, bit for bit),
 // those of the C-PML elements last (compute_forces_viscoelastic, then compute_forces_viscoelastic_PML).
@@ -792,11 +804,13 @@ void ensure_gather_assembly(Mesh* m, int f) {
     SF_CHECK(hipMemcpyAsync(lst + m->nspec_elastic, m->pml_elems, sizeof(int) * m->pml_n, hipMemcpyDeviceToDevice,
                             m->stream));
   dfree(m->asm_idx);
+  dfree(m->asm_elems);
+  const int* launch = m->elastic_launch ? m->elastic_launch : m->elastic_elems;
+  m->asm_elems = regular_first(m, launch, m->nspec_elastic, &m->asm_nreg);
   int* ptr = nullptr;
   m->asm_pos0 = first_pml;
   m->asm_eb = build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_elastic + m->pml_n, lst,
-                               m->elastic_launch ? m->elastic_launch : m->elastic_elems, m->nspec_elastic, first_pml,
-                               3, eb, m->ibool, ptr, m->asm_idx);
+                               m->asm_elems ? m->asm_elems : launch, m->nspec_elastic, first_pml, 3, eb, m->ibool, ptr, m->asm_idx);
   dfree(lst);
   if (!m->asm_info) {
     m->asm_info = dmalloc<uint16_t>(m->nglob);
@@ -820,6 +834,7 @@ void release_gather_assembly(Mesh* m) {
   flush_all(m);
   SF_CHECK(hipStreamSynchronize(m->stream));
   dfree(m->asm_idx);
+  dfree(m->asm_elems);
   dfree(m->asm_info);
   dfree(m->asm_base);
   dfree(m->asm_rec);
@@ -1278,7 +1293,7 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
   dfree(m->rec_ispec); dfree(m->rec_el_list); dfree(m->rec_ac_list);
   dfree(m->seismo_d); dfree(m->seismo_v); dfree(m->seismo_a); dfree(m->seismo_p);
   dfree(m->rho_kl); dfree(m->mu_kl); dfree(m->kappa_kl); dfree(m->rho_ac_kl); dfree(m->kappa_ac_kl);
-  dfree(m->asm_idx); dfree(m->asm_info); dfree(m->asm_base); dfree(m->asm_rec); dfree(m->rmass1); dfree(m->asm_buf[0]); dfree(m->asm_buf[1]);
+  dfree(m->asm_idx); dfree(m->asm_elems); dfree(m->asm_info); dfree(m->asm_base); dfree(m->asm_rec); dfree(m->rmass1); dfree(m->asm_buf[0]); dfree(m->asm_buf[1]);
   dfree(m->pml_elems); dfree(m->pml_cpml);
   dfree(m->pml_state); dfree(m->pml_coef); dfree(m->pml_masks); dfree(m->pml_off);
   dfree(m->pml_old); dfree(m->pml_pts); dfree(m->pml_bc_pts);

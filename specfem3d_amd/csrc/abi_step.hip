@@ -170,7 +170,8 @@ static ElasticArgs elastic_args(Mesh* m, int f, realw deltat) {
   std::memset(&a, 0, sizeof(a));
   a.nelem = m->nspec_elastic;
   // the launch may walk the elements in the host's locality order: the gather has its own
-  a.elems = m->elastic_launch ? m->elastic_launch : m->elastic_elems;
+  a.elems = m->asm_elems ? m->asm_elems : m->elastic_launch ? m->elastic_launch : m->elastic_elems;
+  a.nreg = m->asm_nreg;
   a.ibool = m->ibool;
   a.irregular = m->irregular;
   a.xix_regular = m->xix_regular;

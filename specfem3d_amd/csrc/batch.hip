@@ -31,6 +31,7 @@
 namespace sf {
 void ensure_element_colors(Mesh* m);
 void release_gather_assembly(Mesh* m);
+int* regular_first(Mesh* m, const int* list, int n, int* nreg);
 void ensure_acoustic_colors(Mesh* m);
 bool element_is_elastic(Mesh* m, int e);
 
@@ -56,6 +57,8 @@ struct Batch {
   // gather assembly: slots of each global point in colour order, AF_TERM per global point, local forces
   // of `loc_groups` groups of eight shots (all of them unless the card has no room)
   int *asm_ptr = nullptr, *asm_idx = nullptr, *ac_ptr = nullptr, *ac_idx = nullptr;
+  int* elems = nullptr;          // launch order where the solid has regular and irregular elements (regular_first)
+  int nreg = 0;
   uint16_t* info = nullptr;
   realw *local = nullptr, *ac_local = nullptr;
   int loc_groups = 0, ac_loc_groups = 0;
@@ -592,8 +595,9 @@ static realw* local_room(int64_t per_group, int groups, int* got) {
 // buffers of the local forces
 static void build_gather(Batch* b) {
   Mesh* m = b->m;
+  if (!b->asm_ptr) b->elems = regular_first(m, m->elastic_elems, m->nspec_elastic, &b->nreg);
   if (!b->asm_ptr)
-    (void)build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_elastic, m->el_color_elems, m->elastic_elems,
+    (void)build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_elastic, m->el_color_elems, b->elems ? b->elems : m->elastic_elems,
                            m->nspec_elastic, 0, 3, 1, m->ibool, b->asm_ptr, b->asm_idx);
   if (!b->local) b->local = local_room((int64_t)m->nspec_elastic * 3000, std::min(b->S / 8, b->max_groups), &b->loc_groups);
   if (b->ac && !b->ac_ptr)
@@ -638,8 +642,9 @@ static void enqueue_stiffness(Batch* b, hipStream_t st) {
   Mesh* m = b->m;
   BatchArgs A;
   std::memset(&A, 0, sizeof(A));
-  A.elems = m->elastic_elems;
+  A.elems = b->elems ? b->elems : m->elastic_elems;
   A.nelem = m->nspec_elastic;
+  A.nreg = b->nreg;
   A.S = b->S;
   A.nrow = 3 * (int64_t)m->nglob;
   A.ibool = m->ibool;
@@ -1213,7 +1218,7 @@ extern "C" void sf_batch_destroy(long h) {
   bfree(b->d_nstep); bfree(b->d_it); bfree(b->u); bfree(b->v); bfree(b->a); bfree(b->R); bfree(b->eps);
   bfree(b->pot); bfree(b->potd); bfree(b->potdd);
   bfree(b->asm_ptr); bfree(b->asm_idx); bfree(b->ac_ptr); bfree(b->ac_idx); bfree(b->info);
-  bfree(b->local); bfree(b->ac_local);
+  bfree(b->local); bfree(b->ac_local); bfree(b->elems);
   bfree(b->src_ig); bfree(b->src_slot); bfree(b->src_id); bfree(b->src_ploc); bfree(b->src_arr); bfree(b->src_stf);
   bfree(b->rec_slot); bfree(b->rec_ig); bfree(b->rec_h); bfree(b->rec_nu); bfree(b->seis);
   delete b;

@@ -40,6 +40,27 @@ struct JacPt {  // inverse-Jacobian terms and determinant at one point (irregula
   realw xix, xiy, xiz, etax, etay, etaz, gax, gay, gaz, jac;
 };
 
+// Sums of products, left to right. FMA builds name the one product that is rounded by itself, the second: which
+// one the compiler takes depends on the code around it, and records of a weak first arrival show the
+// difference (their largest part is what rounding leaves behind the front).
+__device__ __forceinline__ realw add_product(realw sum, realw a, realw b) {
+#if SF_EXACT
+  return sum + a * b;
+#else
+  return fmaf(a, b, sum);
+#endif
+}
+__device__ __forceinline__ realw sum2(realw a1, realw b1, realw a2, realw b2) {
+#if SF_EXACT
+  return a1 * b1 + a2 * b2;
+#else
+  return fmaf(a1, b1, a2 * b2);
+#endif
+}
+__device__ __forceinline__ realw sum3(realw a1, realw b1, realw a2, realw b2, realw a3, realw b3) {
+  return add_product(sum2(a1, b1, a2, b2), a3, b3);
+}
+
 // tempx1 = sum_l hprime(i,l) u(l,j,k), tempx2 = sum_l hprime(j,l) u(i,l,k),
 // tempx3 = sum_l hprime(k,l) u(i,j,l), summed left to right.
 template <int PS>
@@ -47,17 +68,21 @@ __device__ __forceinline__ Grad9 tile_gradient(const realw* sx, const realw* sy,
                                                int i, int j, int k) {
   const int b1 = 5 * j + 25 * k, b2 = i + 25 * k, b3 = i + 5 * j;
   Grad9 t;
-  const realw h1 = hp[i * 5], h2 = hp[j * 5], h3 = hp[k * 5];
-  t.x1 = h1 * sx[b1 * PS]; t.y1 = h1 * sy[b1 * PS]; t.z1 = h1 * sz[b1 * PS];
-  t.x2 = h2 * sx[b2 * PS]; t.y2 = h2 * sy[b2 * PS]; t.z2 = h2 * sz[b2 * PS];
-  t.x3 = h3 * sx[b3 * PS]; t.y3 = h3 * sy[b3 * PS]; t.z3 = h3 * sz[b3 * PS];
+  {
+    const realw h1 = hp[i * 5], h2 = hp[j * 5], h3 = hp[k * 5];
+    const realw a1 = hp[i * 5 + 1], a2 = hp[j * 5 + 1], a3 = hp[k * 5 + 1];
+    const int p1 = b1 * PS, p2 = b2 * PS, p3 = b3 * PS, q1 = (b1 + 1) * PS, q2 = (b2 + 5) * PS, q3 = (b3 + 25) * PS;
+    t.x1 = sum2(h1, sx[p1], a1, sx[q1]); t.y1 = sum2(h1, sy[p1], a1, sy[q1]); t.z1 = sum2(h1, sz[p1], a1, sz[q1]);
+    t.x2 = sum2(h2, sx[p2], a2, sx[q2]); t.y2 = sum2(h2, sy[p2], a2, sy[q2]); t.z2 = sum2(h2, sz[p2], a2, sz[q2]);
+    t.x3 = sum2(h3, sx[p3], a3, sx[q3]); t.y3 = sum2(h3, sy[p3], a3, sy[q3]); t.z3 = sum2(h3, sz[p3], a3, sz[q3]);
+  }
 #pragma unroll
-  for (int l = 1; l < 5; l++) {
+  for (int l = 2; l < 5; l++) {
     const realw a1 = hp[i * 5 + l], a2 = hp[j * 5 + l], a3 = hp[k * 5 + l];
     const int q1 = (b1 + l) * PS, q2 = (b2 + 5 * l) * PS, q3 = (b3 + 25 * l) * PS;
-    t.x1 = t.x1 + a1 * sx[q1]; t.y1 = t.y1 + a1 * sy[q1]; t.z1 = t.z1 + a1 * sz[q1];
-    t.x2 = t.x2 + a2 * sx[q2]; t.y2 = t.y2 + a2 * sy[q2]; t.z2 = t.z2 + a2 * sz[q2];
-    t.x3 = t.x3 + a3 * sx[q3]; t.y3 = t.y3 + a3 * sy[q3]; t.z3 = t.z3 + a3 * sz[q3];
+    t.x1 = add_product(t.x1, a1, sx[q1]); t.y1 = add_product(t.y1, a1, sy[q1]); t.z1 = add_product(t.z1, a1, sz[q1]);
+    t.x2 = add_product(t.x2, a2, sx[q2]); t.y2 = add_product(t.y2, a2, sy[q2]); t.z2 = add_product(t.z2, a2, sz[q2]);
+    t.x3 = add_product(t.x3, a3, sx[q3]); t.y3 = add_product(t.y3, a3, sy[q3]); t.z3 = add_product(t.z3, a3, sz[q3]);
   }
   return t;
 }
@@ -72,9 +97,9 @@ __device__ __forceinline__ Grad9 tile_gradient_continue(Grad9 t, const realw* wx
   for (int l = 0; l < 5; l++) {
     const realw h1 = hp[i * 5 + l], h2 = hp[j * 5 + l], h3 = hp[k * 5 + l];
     const int q1 = (b1 + l) * PS, q2 = (b2 + 5 * l) * PS, q3 = (b3 + 25 * l) * PS;
-    t.x1 = t.x1 + wx[q1] * h1; t.y1 = t.y1 + wy[q1] * h1; t.z1 = t.z1 + wz[q1] * h1;
-    t.x2 = t.x2 + wx[q2] * h2; t.y2 = t.y2 + wy[q2] * h2; t.z2 = t.z2 + wz[q2] * h2;
-    t.x3 = t.x3 + wx[q3] * h3; t.y3 = t.y3 + wy[q3] * h3; t.z3 = t.z3 + wz[q3] * h3;
+    t.x1 = add_product(t.x1, wx[q1], h1); t.y1 = add_product(t.y1, wy[q1], h1); t.z1 = add_product(t.z1, wz[q1], h1);
+    t.x2 = add_product(t.x2, wx[q2], h2); t.y2 = add_product(t.y2, wy[q2], h2); t.z2 = add_product(t.z2, wz[q2], h2);
+    t.x3 = add_product(t.x3, wx[q3], h3); t.y3 = add_product(t.y3, wy[q3], h3); t.z3 = add_product(t.z3, wz[q3], h3);
   }
   return t;
 }
@@ -83,17 +108,6 @@ __device__ __forceinline__ Grad9 tile_gradient_continue(Grad9 t, const realw* wx
 struct Du9 {
   realw xx, xy, xz, yx, yy, yz, zx, zy, zz;
 };
-
-// a1 b1 + a2 b2 + a3 b3. FMA builds name the product that is rounded by itself, the second: which one the
-// compiler takes depends on the code around it, and records of a weak first arrival show the difference
-// (their largest part is what rounding leaves behind the front).
-__device__ __forceinline__ realw sum3(realw a1, realw b1, realw a2, realw b2, realw a3, realw b3) {
-#if SF_EXACT
-  return a1 * b1 + a2 * b2 + a3 * b3;
-#else
-  return fmaf(a3, b3, fmaf(a1, b1, a2 * b2));
-#endif
-}
 
 template <bool FOLD = SF_FOLD>
 __device__ __forceinline__ Du9 map_gradient(const Grad9& t, bool irr, const JacPt& J, realw xr) {
@@ -137,7 +151,7 @@ __device__ __forceinline__ Sigma6 iso_stress(const Du9& d, realw kappal, realw m
 #else
   s.xx = fmaf(lp2m, d.xx, lambdal * (d.yy + d.zz));
   s.yy = fmaf(lp2m, d.yy, lambdal * (d.xx + d.zz));
-  s.zz = fmaf(lambdal, d.xx + d.yy, lp2m * d.zz);
+  s.zz = fmaf(lambdal, d.xx + d.yy, lp2m * d.zz);  // the other product here: as it has always been rounded
 #endif
   s.xy = mul * (d.xy + d.yx);
   s.xz = mul * (d.zx + d.xz);
@@ -181,41 +195,26 @@ __device__ __forceinline__ void stress_products(const Sigma6& s, bool irr, const
 // f_c = wgllwgll_yz(j,k) sum_l hprimewgll(l,i) t1_c(l,j,k) + wgllwgll_xz(i,k) sum_l hprimewgll(l,j) t2_c(i,l,k)
 //     + wgllwgll_xy(i,j) sum_l hprimewgll(l,k) t3_c(i,j,l); plane m of the tile at sT + m * plane.
 template <int PS>
-__device__ __forceinline__ void tile_divergence(const realw* sT, int plane, const realw* hpw, const realw* wxy, int i,
-                                                int j, int k, realw f[3]) {
-  const int b1 = 5 * j + 25 * k, b2 = i + 25 * k, b3 = i + 5 * j;
-#pragma unroll
-  for (int cc = 0; cc < 3; cc++) {
-    const realw *s1 = sT + cc * plane, *s2 = sT + (3 + cc) * plane, *s3 = sT + (6 + cc) * plane;
-    realw n1 = hpw[i] * s1[b1 * PS];
-    realw n2 = hpw[j] * s2[b2 * PS];
-    realw n3 = hpw[k] * s3[b3 * PS];
-#pragma unroll
-    for (int l = 1; l < 5; l++) {
-      n1 = n1 + hpw[l * 5 + i] * s1[(b1 + l) * PS];
-      n2 = n2 + hpw[l * 5 + j] * s2[(b2 + 5 * l) * PS];
-      n3 = n3 + hpw[l * 5 + k] * s3[(b3 + 25 * l) * PS];
-    }
-    f[cc] = wxy[j * 5 + k] * n1 + wxy[i * 5 + k] * n2 + wxy[i * 5 + j] * n3;
-  }
-}
-
-// one component cc of tile_divergence (same expressions)
-template <int PS>
 __device__ __forceinline__ realw tile_divergence_c(const realw* sT, int plane, const realw* hpw, const realw* wxy,
                                                    int i, int j, int k, int cc) {
   const int b1 = 5 * j + 25 * k, b2 = i + 25 * k, b3 = i + 5 * j;
   const realw *s1 = sT + cc * plane, *s2 = sT + (3 + cc) * plane, *s3 = sT + (6 + cc) * plane;
-  realw n1 = hpw[i] * s1[b1 * PS];
-  realw n2 = hpw[j] * s2[b2 * PS];
-  realw n3 = hpw[k] * s3[b3 * PS];
+  realw n1 = sum2(hpw[i], s1[b1 * PS], hpw[5 + i], s1[(b1 + 1) * PS]);
+  realw n2 = sum2(hpw[j], s2[b2 * PS], hpw[5 + j], s2[(b2 + 5) * PS]);
+  realw n3 = sum2(hpw[k], s3[b3 * PS], hpw[5 + k], s3[(b3 + 25) * PS]);
 #pragma unroll
-  for (int l = 1; l < 5; l++) {
-    n1 = n1 + hpw[l * 5 + i] * s1[(b1 + l) * PS];
-    n2 = n2 + hpw[l * 5 + j] * s2[(b2 + 5 * l) * PS];
-    n3 = n3 + hpw[l * 5 + k] * s3[(b3 + 25 * l) * PS];
+  for (int l = 2; l < 5; l++) {
+    n1 = add_product(n1, hpw[l * 5 + i], s1[(b1 + l) * PS]);
+    n2 = add_product(n2, hpw[l * 5 + j], s2[(b2 + 5 * l) * PS]);
+    n3 = add_product(n3, hpw[l * 5 + k], s3[(b3 + 25 * l) * PS]);
   }
-  return wxy[j * 5 + k] * n1 + wxy[i * 5 + k] * n2 + wxy[i * 5 + j] * n3;
+  return sum3(wxy[j * 5 + k], n1, wxy[i * 5 + k], n2, wxy[i * 5 + j], n3);
+}
+template <int PS>
+__device__ __forceinline__ void tile_divergence(const realw* sT, int plane, const realw* hpw, const realw* wxy, int i,
+                                                int j, int k, realw f[3]) {
+#pragma unroll
+  for (int cc = 0; cc < 3; cc++) f[cc] = tile_divergence_c<PS>(sT, plane, hpw, wxy, i, j, k, cc);
 }
 
 // stage the GLL coefficients of G in LDS (lanes 0..124 of the workgroup; needs a barrier before
@@ -240,18 +239,18 @@ __device__ __forceinline__ const realw* gll_hpw(const realw* sG, bool irr) {
 __device__ __forceinline__ void line_gradient(const GLLk& G, const realw in[5], realw out[5]) {
 #pragma unroll
   for (int m = 0; m < 5; m++) {
-    realw r = G.hp[m * 5] * in[0];
+    realw r = sum2(G.hp[m * 5], in[0], G.hp[m * 5 + 1], in[1]);
 #pragma unroll
-    for (int l = 1; l < 5; l++) r = r + G.hp[m * 5 + l] * in[l];
+    for (int l = 2; l < 5; l++) r = add_product(r, G.hp[m * 5 + l], in[l]);
     out[m] = r;
   }
 }
 __device__ __forceinline__ void line_divergence(const GLLk& G, const realw in[5], realw out[5]) {
 #pragma unroll
   for (int m = 0; m < 5; m++) {
-    realw r = G.hpw[m] * in[0];
+    realw r = sum2(G.hpw[m], in[0], G.hpw[5 + m], in[1]);
 #pragma unroll
-    for (int l = 1; l < 5; l++) r = r + G.hpw[l * 5 + m] * in[l];
+    for (int l = 2; l < 5; l++) r = add_product(r, G.hpw[l * 5 + m], in[l]);
     out[m] = r;
   }
 }

@@ -94,12 +94,12 @@ __global__ void __launch_bounds__(128) k_acoustic(AcousticArgs A, GLLk G) {
     realw t1, t2;
     if (irr) {
       const JacPt J = load_jac(A.jac, A.jac_plane, jp + 25 * k);
-      const realw dpdx = J.xix * a1 + J.etax * a2 + J.gax * a3;
-      const realw dpdy = J.xiy * a1 + J.etay * a2 + J.gay * a3;
-      const realw dpdz = J.xiz * a1 + J.etaz * a2 + J.gaz * a3;
-      t1 = rho_invl * J.jac * (J.xix * dpdx + J.xiy * dpdy + J.xiz * dpdz);
-      t2 = rho_invl * J.jac * (J.etax * dpdx + J.etay * dpdy + J.etaz * dpdz);
-      d3[k] = rho_invl * J.jac * (J.gax * dpdx + J.gay * dpdy + J.gaz * dpdz);
+      const realw dpdx = sum3(J.xix, a1, J.etax, a2, J.gax, a3);
+      const realw dpdy = sum3(J.xiy, a1, J.etay, a2, J.gay, a3);
+      const realw dpdz = sum3(J.xiz, a1, J.etaz, a2, J.gaz, a3);
+      t1 = rho_invl * J.jac * sum3(J.xix, dpdx, J.xiy, dpdy, J.xiz, dpdz);
+      t2 = rho_invl * J.jac * sum3(J.etax, dpdx, J.etay, dpdy, J.etaz, dpdz);
+      d3[k] = rho_invl * J.jac * sum3(J.gax, dpdx, J.gay, dpdy, J.gaz, dpdz);
     } else {
       const realw jl = A.jacobian_regular, xr = A.xix_regular;
       t1 = rho_invl * jl * xr * xr * a1;
@@ -140,7 +140,7 @@ __global__ void __launch_bounds__(128) k_acoustic(AcousticArgs A, GLLk G) {
 #pragma unroll
   for (int k = 0; k < 5; k++) {
     const int b = el * 125 + c + 25 * k;
-    A.local_out[slot + k * 25 * A.eb] = sW[j * 5 + k] * sA[b] + sW[i * 5 + k] * sB[b] + w3 * d3[k];
+    A.local_out[slot + k * 25 * A.eb] = sum3(sW[j * 5 + k], sA[b], sW[i * 5 + k], sB[b], w3, d3[k]);
   }
 }
 

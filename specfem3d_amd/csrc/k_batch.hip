@@ -52,21 +52,21 @@ __device__ __forceinline__ int xcd_remap_b(int b, int nb) {
 // workgroups per CU. Two or three elements per workgroup fill the lanes better (25 SC of 32 SC work
 // here) and are slower all the same (572 and 700 us against 523 for the whole step of 16 shots on
 // 32x32x16 elements, same source otherwise): seven or ten waves wait for each other at each barrier.
-// REG: no irregular element in the mesh (FMA build: the mapping is folded into the tables).
+// REG: the regular elements of a mesh (FMA build: the mapping is folded into the tables); workgroups take
+// one kind each, as in k_elastic_line.
 template <int SC, bool REG>
-__global__ void __launch_bounds__(32 * SC) k_elastic_batch(BatchArgs B, GLLk G) {
+__device__ __forceinline__ void elastic_batch(const BatchArgs& B, const GLLk& G, const int* elems, int pos0, int block,
+                                              int blocks, realw (&sA)[375 * SC], realw (&sB)[375 * SC], realw (&sW)[25]) {
   constexpr bool FOLD = REG && SF_FOLD;
   constexpr int NQ = SC / 4, NU = 375 * NQ, NT = 32 * SC, PS = 3 * SC;
-  __shared__ __attribute__((aligned(16))) realw sA[375 * SC], sB[375 * SC];  // (p, a, s) at p PS + a SC + s
-  __shared__ realw sW[25];
   const int t = threadIdx.x;
   const int it = __hip_atomic_load(B.it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const int b = xcd_remap_b(blockIdx.x, gridDim.x);
+  const int b = xcd_remap_b(block, blocks);
   const int ie = b / B.ngroups;
   const int s0 = B.s_first + (b - ie * B.ngroups) * SC;
   if (B.nstep[s0] < it) return;                   // every shot of this group has finished
   if (t < 25) sW[t] = G.wxy[t];
-  const int e = B.elems[ie];
+  const int e = elems[ie];
   const int irr = REG ? 0 : B.irregular[e];
   // memory role: units t, t + NT, t + 2 NT of 375 NQ
   const int q4 = t % NQ, sq = s0 + 4 * q4;        // NT is a multiple of NQ: one quad for all three
@@ -194,12 +194,23 @@ __global__ void __launch_bounds__(32 * SC) k_elastic_batch(BatchArgs B, GLLk G) 
   }
   lds_barrier();
   // finished shots of a live quad store what their last displacement gives; nothing reads it
-  realw* o = B.local + (int64_t)(sq >> 3) * B.loc_group + (int64_t)ie * 3000 + (sq & 7);
+  realw* o = B.local + (int64_t)(sq >> 3) * B.loc_group + (int64_t)(pos0 + ie) * 3000 + (sq & 7);
 #pragma unroll
   for (int m = 0; m < 3; m++) {
     const int n = t + m * NT;
     if (mine[m]) *reinterpret_cast<float4*>(o + 8 * (n / NQ)) = *reinterpret_cast<const float4*>(&sA[4 * n]);
   }
+}
+
+// R: tables of the regular elements, the first nreg; G: of the others
+template <int SC, int KIND>
+__global__ void __launch_bounds__(32 * SC) k_elastic_batch(BatchArgs B, GLLk R, GLLk G) {
+  __shared__ __attribute__((aligned(16))) realw sA[375 * SC], sB[375 * SC];  // (p, a, s) at (3 p + a) SC + s
+  __shared__ realw sW[25];
+  const int nb = KIND == LINE_REG ? (int)gridDim.x : KIND == LINE_IRR ? 0 : B.nreg * B.ngroups, b = (int)blockIdx.x;
+  if (KIND != LINE_IRR && b < nb) elastic_batch<SC, true>(B, R, B.elems, 0, b, nb, sA, sB, sW);
+  if (KIND != LINE_REG && b >= nb)
+    elastic_batch<SC, false>(B, G, B.elems + B.nreg, B.nreg, b - nb, (int)gridDim.x - nb, sA, sB, sW);
 }
 
 // Viscoelastic (3-SLS) variant: each shot also carries its memory variables and stored strain
@@ -437,23 +448,23 @@ __global__ void __launch_bounds__(128 * NQ) k_acoustic_batch(BatchAcArgs B, GLLk
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const realw* s = sBuf + (ts + r) * PST;
-    realw a1 = hp[i * 5] * s[b1];
-    realw a2 = hp[j * 5] * s[b2];
-    realw a3 = hp[k * 5] * s[b3];
+    realw a1 = sum2(hp[i * 5], s[b1], hp[i * 5 + 1], s[b1 + 1]);
+    realw a2 = sum2(hp[j * 5], s[b2], hp[j * 5 + 1], s[b2 + 5]);
+    realw a3 = sum2(hp[k * 5], s[b3], hp[k * 5 + 1], s[b3 + 25]);
 #pragma unroll
-    for (int l = 1; l < 5; l++) {
-      a1 = a1 + hp[i * 5 + l] * s[b1 + l];
-      a2 = a2 + hp[j * 5 + l] * s[b2 + 5 * l];
-      a3 = a3 + hp[k * 5 + l] * s[b3 + 25 * l];
+    for (int l = 2; l < 5; l++) {
+      a1 = add_product(a1, hp[i * 5 + l], s[b1 + l]);
+      a2 = add_product(a2, hp[j * 5 + l], s[b2 + 5 * l]);
+      a3 = add_product(a3, hp[k * 5 + l], s[b3 + 25 * l]);
     }
     realw t1, t2, t3;
     if (irr) {
-      const realw dpdx = J.xix * a1 + J.etax * a2 + J.gax * a3;
-      const realw dpdy = J.xiy * a1 + J.etay * a2 + J.gay * a3;
-      const realw dpdz = J.xiz * a1 + J.etaz * a2 + J.gaz * a3;
-      t1 = rho_invl * J.jac * (J.xix * dpdx + J.xiy * dpdy + J.xiz * dpdz);
-      t2 = rho_invl * J.jac * (J.etax * dpdx + J.etay * dpdy + J.etaz * dpdz);
-      t3 = rho_invl * J.jac * (J.gax * dpdx + J.gay * dpdy + J.gaz * dpdz);
+      const realw dpdx = sum3(J.xix, a1, J.etax, a2, J.gax, a3);
+      const realw dpdy = sum3(J.xiy, a1, J.etay, a2, J.gay, a3);
+      const realw dpdz = sum3(J.xiz, a1, J.etaz, a2, J.gaz, a3);
+      t1 = rho_invl * J.jac * sum3(J.xix, dpdx, J.xiy, dpdy, J.xiz, dpdz);
+      t2 = rho_invl * J.jac * sum3(J.etax, dpdx, J.etay, dpdy, J.etaz, dpdz);
+      t3 = rho_invl * J.jac * sum3(J.gax, dpdx, J.gay, dpdy, J.gaz, dpdz);
     } else {
       const realw jl = B.jacobian_regular, xr = B.xix_regular;
       t1 = rho_invl * jl * xr * xr * a1;
@@ -476,16 +487,16 @@ __global__ void __launch_bounds__(128 * NQ) k_acoustic_batch(BatchAcArgs B, GLLk
     const realw* s1 = sBuf + (1 * SC + ts + r) * PST;
     const realw* s2 = sBuf + (2 * SC + ts + r) * PST;
     const realw* s3 = sBuf + (3 * SC + ts + r) * PST;
-    realw n1 = hpw[i] * s1[b1];
-    realw n2 = hpw[j] * s2[b2];
-    realw n3 = hpw[k] * s3[b3];
+    realw n1 = sum2(hpw[i], s1[b1], hpw[5 + i], s1[b1 + 1]);
+    realw n2 = sum2(hpw[j], s2[b2], hpw[5 + j], s2[b2 + 5]);
+    realw n3 = sum2(hpw[k], s3[b3], hpw[5 + k], s3[b3 + 25]);
 #pragma unroll
-    for (int l = 1; l < 5; l++) {
-      n1 = n1 + hpw[l * 5 + i] * s1[b1 + l];
-      n2 = n2 + hpw[l * 5 + j] * s2[b2 + 5 * l];
-      n3 = n3 + hpw[l * 5 + k] * s3[b3 + 25 * l];
+    for (int l = 2; l < 5; l++) {
+      n1 = add_product(n1, hpw[l * 5 + i], s1[b1 + l]);
+      n2 = add_product(n2, hpw[l * 5 + j], s2[b2 + 5 * l]);
+      n3 = add_product(n3, hpw[l * 5 + k], s3[b3 + 25 * l]);
     }
-    f[r] = wxy[j * 5 + k] * n1 + wxy[i * 5 + k] * n2 + wxy[i * 5 + j] * n3;
+    f[r] = sum3(wxy[j * 5 + k], n1, wxy[i * 5 + k], n2, wxy[i * 5 + j], n3);
   }
   realw* o = B.local + (int64_t)(sq >> 3) * B.loc_group + ((int64_t)ie * 125 + p) * 8 + (sq & 7);
   *reinterpret_cast<float4*>(o) = make_float4(f[0], f[1], f[2], f[3]);
@@ -496,20 +507,21 @@ using namespace SF_VNS;
 
 void SFX(launch_elastic_batch)(hipStream_t st, const BatchArgs& a, int sc) {
   if (a.nelem <= 0 || a.ngroups <= 0) return;
-  const bool reg = a.jac_plane == 0;
-  GLLk G = g_gll_host;
-  if (reg && SF_FOLD) regular_gll(G, a.xix_regular, a.jacobian_regular);
-  const int64_t nb = (int64_t)a.nelem * a.ngroups;
-  if (nb > 0x7fffffff) fatal("launch_elastic_batch", "grid too large");
-#define SF_KB(SC, R) hipLaunchKernelGGL((k_elastic_batch<SC, R>), dim3((unsigned)nb), dim3(32 * SC), 0, st, a, G)
-  if (sc == 4) {
-    if (reg) SF_KB(4, true);
-    else SF_KB(4, false);
-  } else if (sc == 8) {
-    if (reg) SF_KB(8, true);
-    else SF_KB(8, false);
+  if ((int64_t)a.nelem * a.ngroups > 0x7fffffff) fatal("launch_elastic_batch", "grid too large");
+  if (sc != 4 && sc != 8) fatal("launch_elastic_batch", "shots per workgroup must be 4 or 8");
+  GLLk G = g_gll_host, R = G;
+  if (SF_FOLD) regular_gll(R, a.xix_regular, a.jacobian_regular);
+  const unsigned nb = (unsigned)(a.nelem * a.ngroups);
+#define SF_KB(SC, K) hipLaunchKernelGGL((k_elastic_batch<SC, K>), dim3(nb), dim3(32 * SC), 0, st, a, R, G)
+  if (a.nreg == a.nelem) {
+    if (sc == 4) SF_KB(4, LINE_REG);
+    else SF_KB(8, LINE_REG);
+  } else if (a.nreg == 0) {
+    if (sc == 4) SF_KB(4, LINE_IRR);
+    else SF_KB(8, LINE_IRR);
   } else {
-    fatal("launch_elastic_batch", "shots per workgroup must be 4 or 8");
+    if (sc == 4) SF_KB(4, LINE_BOTH);
+    else SF_KB(8, LINE_BOTH);
   }
 #undef SF_KB
   SF_LAUNCH_CHECK("k_elastic_batch");

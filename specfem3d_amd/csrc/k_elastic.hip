@@ -247,20 +247,24 @@ k_elastic_pt(ElasticArgs A, GLLk G) {
 // k_elastic_pt storing the same forces: 64x64x32 elements 187 -> 100 us (0.50 GB: the rate of a large
 // copy), 20x20x20 14.3 -> 12.5, 24^3 with strain 22.2 -> 19.5, irregular 43x37x29 89 -> 87 (its 40 B of
 // Jacobian terms per point were already the limit).
-// REG: no irregular element in the mesh (FMA build: the mapping is folded into the tables).
+// REG: the regular elements of a mesh (FMA build: the mapping is folded into the tables, so that a regular
+// element rounds the same whatever the mesh around it). A mesh with both kinds lists them before the
+// irregular ones and its workgroups take one kind each. A step of 48x48x48 elements, half of them
+// irregular: 294 us, with the choice per lane 325; 16x16x16: 22.1 and 21.5 (with a launch per kind 298 and
+// 28.7).
+constexpr int LINE_PL = 626;
 template <bool STRAIN, bool REG>
-__global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk G) {
+__device__ __forceinline__ void elastic_line(const ElasticArgs& A, const GLLk& G, int n, const int* elems, int pos0,
+                                             int block, int blocks, realw (&sA)[3][LINE_PL], realw (&sB)[3][LINE_PL],
+                                             realw (&sW)[25]) {
   constexpr bool FOLD = REG && SF_FOLD;
-  constexpr int PL = 626;
-  __shared__ realw sA[3][PL], sB[3][PL];
-  __shared__ realw sW[25];
   const int t = threadIdx.x;
   const bool lane = t < 125;                       // lanes 125..127 shadow the last element's first points
   const int el = lane ? t / 25 : 4, c = lane ? t - 25 * el : t - 125;
   const int i = c % 5, j = c / 5;
-  const int ie = xcd_remap(blockIdx.x, gridDim.x) * 5 + el;
-  const bool active = lane && ie < A.nelem;
-  const int e = A.elems[ie < A.nelem ? ie : A.nelem - 1];
+  const int ie = xcd_remap(block, blocks) * 5 + el;
+  const bool active = lane && ie < n;
+  const int e = elems[ie < n ? ie : n - 1];
   const int64_t ep = (int64_t)e * 125 + c;         // local point of k = 0
   const int irr = REG ? 0 : A.irregular[e];
   const int64_t jp = REG ? 0 : (int64_t)(irr ? irr - 1 : 0) * 125 + c;
@@ -382,7 +386,7 @@ __global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk G) {
   lds_barrier();
   if (!active) return;
   const realw w3 = sW[i * 5 + j];
-  const int slot = gather_slot(ie, j, i, A.eb);    // of k = 0
+  const int slot = gather_slot(pos0 + ie, j, i, A.eb);  // of k = 0
 #pragma unroll
   for (int k = 0; k < 5; k++) {
     const int b = el * 125 + c + 25 * k;
@@ -391,6 +395,17 @@ __global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk G) {
 #pragma unroll
     for (int a = 0; a < 3; a++) o[a] = sum3(w1, sA[a][b], w2, sB[a][b], w3, d3[k][a]);
   }
+}
+
+// R: tables of the regular elements, the first nreg; G: of the others
+template <bool STRAIN, int KIND>
+__global__ void __launch_bounds__(128) k_elastic_line(ElasticArgs A, GLLk R, GLLk G) {
+  __shared__ realw sA[3][LINE_PL], sB[3][LINE_PL];
+  __shared__ realw sW[25];
+  const int nb = KIND == LINE_REG ? (int)gridDim.x : KIND == LINE_IRR ? 0 : (A.nreg + 4) / 5, b = (int)blockIdx.x;
+  if (KIND != LINE_IRR && b < nb) elastic_line<STRAIN, true>(A, R, A.nreg, A.elems, 0, b, nb, sA, sB, sW);
+  if (KIND != LINE_REG && b >= nb)
+    elastic_line<STRAIN, false>(A, G, A.nelem - A.nreg, A.elems + A.nreg, A.nreg, b - nb, (int)gridDim.x - nb, sA, sB, sW);
 }
 
 // Elastic kernels of a run that recomputes the reconstructed field's strain from its displacement
@@ -597,16 +612,19 @@ void SFX(launch_elastic)(hipStream_t s, const ElasticArgs& a, bool strain, bool 
     else if (att_variant == 4) SF_K(4);
     else SF_K(0);
   } else {
-    const bool reg = a.jac_plane == 0;  // no irregular element in the mesh
-    if (reg && SF_FOLD) regular_gll(G, a.xix_regular, a.jacobian_regular);
-    const dim3 grid5((a.nelem + 4) / 5);
-#define SF_L(S, R) hipLaunchKernelGGL((k_elastic_line<S, R>), grid5, block, 0, s, a, G)
-    if (strain) {
-      if (reg) SF_L(true, true);
-      else SF_L(true, false);
+    GLLk R = G;
+    if (SF_FOLD) regular_gll(R, a.xix_regular, a.jacobian_regular);
+    const int nb = (a.nreg + 4) / 5 + (a.nelem - a.nreg + 4) / 5;
+#define SF_L(S, K) hipLaunchKernelGGL((k_elastic_line<S, K>), dim3(nb), block, 0, s, a, R, G)
+    if (a.nreg == a.nelem) {
+      if (strain) SF_L(true, LINE_REG);
+      else SF_L(false, LINE_REG);
+    } else if (a.nreg == 0) {
+      if (strain) SF_L(true, LINE_IRR);
+      else SF_L(false, LINE_IRR);
     } else {
-      if (reg) SF_L(false, true);
-      else SF_L(false, false);
+      if (strain) SF_L(true, LINE_BOTH);
+      else SF_L(false, LINE_BOTH);
     }
 #undef SF_L
   }

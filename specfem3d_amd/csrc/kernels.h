@@ -122,6 +122,8 @@ void launch_gather_info(hipStream_t s, int64_t g0, int64_t n, const int* ptr, co
                         int* base, realw* rm1);
 
 // element stiffness (k_elastic.hip / k_acoustic.hip)
+// kinds of elements in a launch: regular ones, irregular ones, or the one before the other
+enum { LINE_REG = 0, LINE_IRR = 1, LINE_BOTH = 2 };
 struct ElasticArgs {
   int nelem;
   const int* elems;
@@ -146,6 +148,7 @@ struct ElasticArgs {
   realw alpha[3], beta[3], gamma[3];
   realw* local_out;        // local forces, 3 per slot (gather_slot)
   int eb;
+  int nreg;                // listed regular elements, before the irregular ones
 };
 // att_variant: scheduling of the attenuation state in the point kernel (k_elastic_pt's AV)
 void launch_elastic(hipStream_t s, const ElasticArgs& a, bool strain, bool att, bool exact,
@@ -224,6 +227,7 @@ struct BatchArgs {
   // floats per group of eight
   realw* local;
   int64_t loc_group;
+  int nreg;                // listed regular elements, before the irregular ones
   const int* nstep;        // per shot slot, decreasing (padding slots 0)
   const int* it;           // device step counter, 1-based current step
   // 3-SLS attenuation (k_visco_batch): per-shot memory variables and strain, one block per

@@ -223,6 +223,8 @@ struct Mesh {
   // the colour order under assembly = 2), the C-PML elements last
   int* asm_idx = nullptr;
   int asm_eb = 1;                  // elements per block of slots (gather_slot)
+  int asm_nreg = 0;                // launch positions of regular elements, before those of irregular ones
+  int* asm_elems = nullptr;        // the launch order where it has both kinds (regular_first)
   int asm_pos0 = 0;                // launch position of the first C-PML element
   uint16_t* asm_info = nullptr;    // AF_* and the number of slots, per global point
   int* asm_base = nullptr;         // first slot entry of each 64 points of the elastic range

@@ -20,12 +20,22 @@ pytestmark = pytest.mark.gpu
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "fma_rounding.npz")
 DT = 0.008
-# (elements a side, fluid layers, warped, viscoelastic, steps)
+# (elements a side, fluid layers, warped: 0 no, 1 every element, 2 the upper half, viscoelastic, steps)
 FORWARD = {"elastic": (5, 0, False, False, 45), "elastic_warped": (6, 0, True, False, 45), "sea": (5, 1, False, False, 45),
-           "sea_visco": (5, 1, True, True, 45), "fluid": (4, 4, False, False, 40), "fluid_warped": (4, 4, True, False, 40)}
-KERNELS = {"kernels": (5, 0, False, 48), "kernels_warped": (6, 0, True, 48), "kernels_sea": (6, 2, False, 48)}
-BATCH = {"batch_2": (2, False), "batch_3": (3, False), "batch_visco": (2, True)}
+           "sea_visco": (5, 1, True, True, 45), "fluid": (4, 4, False, False, 40), "fluid_warped": (4, 4, True, False, 40),
+           "elastic_mixed": (6, 0, 2, False, 45), "sea_visco_mixed": (6, 1, 2, True, 45)}
+KERNELS = {"kernels": (5, 0, False, 48), "kernels_warped": (6, 0, True, 48), "kernels_sea": (6, 2, False, 48),
+           "kernels_mixed": (6, 0, 2, 48)}
+BATCH = {"batch_2": (2, False, 0), "batch_3": (3, False, 0), "batch_visco": (2, True, 0), "batch_mixed": (2, False, 2), "batch_sea": (2, False, 1)}
 CASES = [*FORWARD, *KERNELS, *BATCH]
+
+
+def upper_half(L):
+    """Elements below the middle stay cubes."""
+    def w(x, y, z):
+        d = 0.05 * L * np.sin(np.pi * x / L) * np.sin(np.pi * y / L) * np.sin(2 * np.pi * np.maximum(0.0, 0.5 + z / L))
+        return x + 0.5 * d, y - 0.3 * d, z + 0.4 * d
+    return w
 
 
 def corner_to_corner(n, fluid, warped, hdurs=(4.0,)):
@@ -36,9 +46,10 @@ def corner_to_corner(n, fluid, warped, hdurs=(4.0,)):
     L = 500.0 * n
     ext = (0.0, L, 0.0, L, -L, 0.0)
     db = build_box(n, n, n, ext, material=gradient_grf_model(ext, seed=0, corr_len=700.0), acoustic_top_layers=fluid,
-                   acoustic_material=homogeneous(1020.0, 1500.0, 0.0), warp=smooth_warp(L) if warped else None,
+                   acoustic_material=homogeneous(1020.0, 1500.0, 0.0), warp=[None, smooth_warp(L), upper_half(L)][warped],
                    stacey_faces=(1, 2, 3, 4, 5))
     db.finalize(DT, stacey=True)
+    assert warped != 2 or 0 < db.nspec_irregular < db.nspec
     shots = [S.setup_cmt_sources(db, [S.CMTSource(300.0 + 50.0 * k, 400.0, 0.9 * L / 1000.0, 0.0, h, 1e13, -2e13, 0.7e13,
                                                   0.3e13, -0.5e13, 0.2e13)], DT, ricker=True) for k, h in enumerate(hdurs)]
     rec = S.setup_receivers(db, [S.Station(f"R{i}", "T", 0.9 * L, (0.1 + 0.4 * i) * L, 0.0, 0.6 * L) for i in range(3)])
@@ -64,8 +75,8 @@ def kernel_solver(case, nt_dump=16):
 
 def batch_solver(case):
     from specfem3d_amd.batch import BatchSolver
-    assembly, visco = BATCH[case]
-    db, shots, rec = corner_to_corner(8, 1 if visco else 0, False, (4.0, 5.0, 6.0))
+    assembly, visco, warped = BATCH[case]
+    db, shots, rec = corner_to_corner(8, 2 if case == "batch_sea" else 1 if visco else 0, warped, (4.0, 5.0, 6.0))
     return BatchSolver(db, [(s, rec, n) for s, n in zip(shots, (48, 45, 36))], exact=False, shots_per_group=8,
                        assembly=assembly, attenuation=attenuation(db) if visco else None)
 
