@@ -970,6 +970,7 @@ extern "C" void FC_FUNC_(prepare_fields_acoustic_device, PREPARE_FIELDS_ACOUSTIC
     if (m->save_forward || m->simulation_type == 3)
       m->b_absorb_potential = dmalloc<realw>(25 * (int64_t)std::max(1, m->num_abs_boundary_faces));
   }
+  m->asm_ready = m->asm_ac_ready = 0;  // the coupling points take terms
 }
 
 // prepare_mesh_constants_cuda.cu:1176 -- C-PML elements of the elastic domain. The convolution
