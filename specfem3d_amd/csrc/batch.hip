@@ -1179,11 +1179,12 @@ extern "C" void sf_batch_time(long h, int nsteps, double* stiffness_ms, double* 
 // Autotuner: times every shots-per-workgroup candidate for `trial_steps` eager steps from rest (after a
 // warm-up; a candidate whose first step takes over twice the best so far is dropped), keeps the
 // fastest and rewinds the batch. Returns the chosen step time in ms.
-// The assembly becomes 3 from 25000 elements x shots on, below and with attenuation 2. Both are the same
-// launches here and differ in the rounding of FMA builds alone (see newmark); the line is where trials
-// found 3 faster while it folded the update into the element launches (22 batches of 8x8x8 to 32x32x16
-// elements and 3 to 16 shots: 2 up to 20600, 3 from 33000 on, now one, now the other between), so that
-// records of weak arrivals, which show that rounding, stay what they were.
+// The assembly becomes 3 from 25000 elements x shots on, with attenuation from 160000, and 2 below. Both are
+// the same launches here and differ in the rounding of FMA builds alone (see newmark); the lines are
+// where trials found 3 faster while it folded the update into the element launches, so that records of weak
+// arrivals, which show that rounding, stay what they were. 14 batches without attenuation of 7900 to 262000
+// elements x shots: 2 up to 20600, 3 from 33000 on (three took now one, now the other); 19 with attenuation of
+// 8400 to 1.05 million: 2 up to 138000, 3 from 197000 on, between them either.
 extern "C" double sf_batch_autotune(long h, int trial_steps) {
   Batch* b = batch_of(h);
   if (!b->ready) fatal("sf_batch_autotune", "sf_batch_finalize first");
@@ -1205,7 +1206,7 @@ extern "C" double sf_batch_autotune(long h, int trial_steps) {
     }
   }
   b->sc = best_sc;
-  b->mode = !b->att && (int64_t)b->m->nspec_elastic * b->S >= 25000 ? 3 : 2;
+  b->mode = (int64_t)b->m->nspec_elastic * b->S >= (b->att ? 160000 : 25000) ? 3 : 2;
   drop_graph(b);
   zero_state(b);
   return best;

@@ -180,3 +180,23 @@ def test_groups_held_at_a_time_change_no_bit(assembly, visco):
         b.close()
     assert max(np.abs(x).max() for x in out[0]) > 0
     assert all(np.array_equal(x, y) for x, y in zip(*out))
+
+
+@pytest.mark.parametrize("nx,nz,nshots,visco,assembly", [(5, 5, 9, False, 2), (12, 10, 9, False, 2), (14, 10, 9, False, 3),
+                                                         (14, 10, 3, True, 2), (32, 20, 3, True, 3)])
+def test_assembly_after_a_trial(nx, nz, nshots, visco, assembly):
+    """The line between the two roundings of the update, in elements x shots (a multiple of eight): 25000, with
+    attenuation 160000."""
+    from specfem3d_amd import sources as S
+    from specfem3d_amd.batch import BatchSolver
+    from specfem3d_amd.mesh.box import build_box, homogeneous
+    assert (nx * nx * nz * (-(-nshots // 8) * 8) >= (160000 if visco else 25000)) == (assembly == 3)
+    L = 500.0 * nx
+    db = build_box(nx, nx, nz, (0.0, L, 0.0, L, -500.0 * nz, 0.0), material=homogeneous(2300.0, 2800.0, 1500.0))
+    db.finalize(DT)
+    src = S.setup_cmt_sources(db, [S.CMTSource(0.4 * L, 0.4 * L, 0.6, 0.0, 4.0, 1e13, 1e13, 1e13, 0.0, 0.0, 0.0)], DT, ricker=True)
+    rec = S.setup_receivers(db, [S.Station("R", "T", 0.6 * L, 0.6 * L, 0.0, 0.0)])
+    b = BatchSolver(db, [(src, rec, 12)] * nshots, exact=False, attenuation=attenuation(db) if visco else None)
+    print(f"[gpu] trial of {nx}x{nx}x{nz} elements x {nshots} shots, attenuation {visco}", flush=True)
+    assert b.autotune(2)["assembly"] == assembly
+    b.close()
