@@ -60,8 +60,8 @@ struct Batch {
   int* elems = nullptr;          // launch order where the solid has regular and irregular elements (regular_first)
   int nreg = 0;
   uint16_t* info = nullptr;
-  realw *local = nullptr, *ac_local = nullptr;
-  int loc_groups = 0, ac_loc_groups = 0;
+  realw *local = nullptr, *ac_local = nullptr;  // ac_local: behind the solid's, in the same allocation
+  int loc_groups = 0;
   int max_groups = 1 << 20;      // "local_groups"
   // sources: (source, point) entries sorted into rounds (the k-th source of each shot)
   struct Src { int shot, ispec; std::vector<realw> arr, stf; };
@@ -599,13 +599,16 @@ static void build_gather(Batch* b) {
   if (!b->asm_ptr)
     (void)build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_elastic, m->el_color_elems, b->elems ? b->elems : m->elastic_elems,
                            m->nspec_elastic, 0, 3, 1, m->ibool, b->asm_ptr, b->asm_idx);
-  if (!b->local) b->local = local_room((int64_t)m->nspec_elastic * 3000, std::min(b->S / 8, b->max_groups), &b->loc_groups);
   if (b->ac && !b->ac_ptr)
     (void)build_slot_lists(m->stream, m->nglob, m->nspec, m->nspec_acoustic, m->ac_color_elems, m->acoustic_elems,
                            m->nspec_acoustic, 0, 1, 1, m->ibool, b->ac_ptr, b->ac_idx);
-  if (b->ac && !b->ac_local)
-    b->ac_local = local_room((int64_t)m->nspec_acoustic * 1000, std::min(b->S / 8, b->max_groups), &b->ac_loc_groups);
   if (!b->info) b->info = balloc<uint16_t>(m->nglob);
+  if (!b->local) {
+    // last, and the solid's and the fluid's together: the one must not take the room of the other
+    const int64_t el = (int64_t)m->nspec_elastic * 3000, ac = b->ac ? (int64_t)m->nspec_acoustic * 1000 : 0;
+    b->local = local_room(el + ac, std::min(b->S / 8, b->max_groups), &b->loc_groups);
+    b->ac_local = b->local + el * b->loc_groups;
+  }
   SF_CHECK(hipMemsetAsync(b->info, 0, sizeof(uint16_t) * (size_t)m->nglob, m->stream));
   if (m->stacey) launch_mark_points(m->stream, m->abs_el.n, m->abs_el.iglob, AF_TERM, b->info);
   if (b->ac) launch_mark_points(m->stream, m->coupling.n, m->coupling.iglob, AF_TERM, b->info);
@@ -738,8 +741,8 @@ static void enqueue_fluid(Batch* b, hipStream_t st) {
   A.loc_group = (int64_t)m->nspec_acoustic * 1000;
   A.nstep = b->d_nstep;
   A.it = b->d_it + b->at;
-  for (int g = 0; g < S / 8; g += b->ac_loc_groups) {
-    const int n = std::min(b->ac_loc_groups, S / 8 - g);
+  for (int g = 0; g < S / 8; g += b->loc_groups) {
+    const int n = std::min(b->loc_groups, S / 8 - g);
     A.s_first = 8 * g;
     A.ngroups = 8 * n / b->sc;
     A.local = b->ac_local - g * A.loc_group;
@@ -1055,7 +1058,6 @@ extern "C" void sf_batch_set_tuning(long h, const char* name, int value) {
     SF_CHECK(hipStreamSynchronize(b->m->stream));
     drop_graph(b);
     bfree(b->local);
-    bfree(b->ac_local);
     b->max_groups = value;
     if (b->ready) build_gather(b);
   } else {
@@ -1219,7 +1221,7 @@ extern "C" void sf_batch_destroy(long h) {
   bfree(b->d_nstep); bfree(b->d_it); bfree(b->u); bfree(b->v); bfree(b->a); bfree(b->R); bfree(b->eps);
   bfree(b->pot); bfree(b->potd); bfree(b->potdd);
   bfree(b->asm_ptr); bfree(b->asm_idx); bfree(b->ac_ptr); bfree(b->ac_idx); bfree(b->info);
-  bfree(b->local); bfree(b->ac_local); bfree(b->elems);
+  bfree(b->local); bfree(b->elems);
   bfree(b->src_ig); bfree(b->src_slot); bfree(b->src_id); bfree(b->src_ploc); bfree(b->src_arr); bfree(b->src_stf);
   bfree(b->rec_slot); bfree(b->rec_ig); bfree(b->rec_h); bfree(b->rec_nu); bfree(b->seis);
   delete b;
