@@ -916,6 +916,9 @@ static void d2h(Mesh* m, realw* h, const realw* d, int64_t n) {
   SF_CHECK(hipStreamSynchronize(m->stream));
 }
 
+// what a write to the device ends: a read changes no value, and what is known of the fields stays known
+#define WRITTEN_H2D(x) x
+#define WRITTEN_D2H(x)
 #define SF_XFER3(NAME, F, DIR)                                                                                  \
   extern "C" void FC_FUNC_(NAME, X)(int* size, realw* displ, realw* veloc, realw* accel, long* Mesh_pointer) { \
     Mesh* m = from_handle(Mesh_pointer);                                                                      \
@@ -924,7 +927,7 @@ static void d2h(Mesh* m, realw* h, const realw* d, int64_t n) {
     DIR(m, m->el[F].displ, displ, *size);                                                                     \
     DIR(m, m->el[F].veloc, veloc, *size);                                                                     \
     DIR(m, m->el[F].accel, accel, *size);                                                                     \
-    m->accel_clean[F] = 0;                                                                                    \
+    WRITTEN_##DIR(m->accel_clean[F] = 0);                                                                     \
   }
 #define SF_XFER1(NAME, F, MEMBER, DIR)                                                   \
   extern "C" void FC_FUNC_(NAME, X)(int* size, realw* arr, long* Mesh_pointer) {        \
@@ -932,7 +935,7 @@ static void d2h(Mesh* m, realw* h, const realw* d, int64_t n) {
     check_field(m, F, #NAME);                                                            \
     flush_el(m, F);                                                                      \
     DIR(m, m->el[F].MEMBER, arr, *size);                                                 \
-    m->accel_clean[F] = 0;                                                               \
+    WRITTEN_##DIR(m->accel_clean[F] = 0);                                                \
   }
 #define H2D(m, d, h, n) h2d(m, d, h, n)
 #define D2H(m, d, h, n) d2h(m, h, d, n)
@@ -962,7 +965,7 @@ SF_XFER1(transfer_b_accel_from_device, 1, accel, D2H)
     DIR(m, m->ac[F].pot, p, *size);                                                                            \
     DIR(m, m->ac[F].potd, pd, *size);                                                                          \
     DIR(m, m->ac[F].potdd, pdd, *size);                                                                        \
-    m->potdd_clean[F] = m->free_zero[F] = 0;                                                \
+    WRITTEN_##DIR(m->potdd_clean[F] = m->free_zero[F] = 0);                                                    \
   }
 #define SF_XFERAC1(NAME, F, MEMBER, DIR)                                          \
   extern "C" void FC_FUNC_(NAME, X)(int* size, realw* arr, long* Mesh_pointer) { \
@@ -970,7 +973,7 @@ SF_XFER1(transfer_b_accel_from_device, 1, accel, D2H)
     if (!m->ac[F].pot) fatal(#NAME, "acoustic field not prepared");               \
     flush_ac(m, F);                                                               \
     DIR(m, m->ac[F].MEMBER, arr, *size);                                          \
-    m->potdd_clean[F] = m->free_zero[F] = 0;                   \
+    WRITTEN_##DIR(m->potdd_clean[F] = m->free_zero[F] = 0);                       \
   }
 SF_XFERAC3(transfer_fields_ac_to_device, 0, H2D)
 SF_XFERAC3(transfer_fields_ac_from_device, 0, D2H)
