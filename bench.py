@@ -96,31 +96,28 @@ def stiffness_bytes_per_launch(db, attenuation=None) -> float:
     return float(per_glob * nglob_el + per_loc * nloc_el + 40 * nirr_el)
 
 
-def batch_stiffness_bytes(db, nshots: int, fused: bool = False, attenuation=None) -> float:
+def batch_stiffness_bytes(db, nshots: int, attenuation=None) -> float:
     """Algorithmic HBM bytes of one batched stiffness pass with every shot live: per shot and global
     point u read (12 B) and accel read + write (24 B); per local point, shared by the shots, ibool +
-    kappa + mu (12 B) and 40 B of Jacobian terms in irregular elements. With the Newmark update fused
-    into the pass (assembly 3) the pass is the whole step: u, v, accel each read and written
-    (72 B per shot and point) plus the inverse mass (12 B per point). With attenuation each shot also
-    reads and writes its 18 memory variables and 6 stored strains per local point (192 B), and the
-    SLS factors are shared (a 2-byte row index, or 24 B of planes beyond 65535 distinct rows); a
-    separate (unfused) pass also reads v (12 B per shot and point)."""
+    kappa + mu (12 B) and 40 B of Jacobian terms in irregular elements. With attenuation each shot also
+    reads v (12 B per point), reads and writes its 18 memory variables and 6 stored strains per local
+    point (192 B), and the SLS factors are shared (a 2-byte row index, or 24 B of planes beyond 65535
+    distinct rows)."""
     import numpy as np
     el = db.ispec_is_elastic
     nloc = int(el.sum()) * 125
     nglob_el = int(np.unique(db.ibool[el]).size)
     nirr = int((db.irregular_element_number[el] > 0).sum()) * 125
-    per_shot = 72 if fused else 36
+    per_shot = 36
     per_shot_loc = 0
     shared_loc = 12
     if attenuation is not None:
-        per_shot += 0 if fused else 12
+        per_shot += 12
         per_shot_loc = 192
         rows = np.unique(np.concatenate([attenuation.factor_common.reshape(-1, 3),
                                          attenuation.factor_common_kappa.reshape(-1, 3)], 1), axis=0).shape[0]
         shared_loc += 2 if rows <= 65535 else 24
-    return float(per_shot * nglob_el * nshots + per_shot_loc * nloc * nshots + shared_loc * nloc + 40 * nirr
-                 + (12 * nglob_el if fused else 0))
+    return float(per_shot * nglob_el * nshots + per_shot_loc * nloc * nshots + shared_loc * nloc + 40 * nirr)
 
 
 def batch_step_bytes(db, shot_steps: int, nsteps: int) -> float:
@@ -164,7 +161,7 @@ def batched_measurement(args) -> dict:
     finite = all(bool(np.isfinite(b.seismograms(i)).all()) for i in range(len(w.shots)))
     b.close()
     value = db.nglob * float(sum(nsteps)) / wall
-    kbytes = batch_stiffness_bytes(db, len(w.shots), fused=False)
+    kbytes = batch_stiffness_bytes(db, len(w.shots))
     ach = kbytes / (kms / 1e3) / 1e9
     run_gbs = batch_step_bytes(db, sum(nsteps), max(nsteps)) / wall / 1e9
     # plain single-shot path on the same mesh (first shot), timed the same way
@@ -227,7 +224,7 @@ def batched_visco_measurement(args) -> dict:
     finite = all(bool(np.isfinite(b.seismograms(i)).all()) for i in range(len(shots)))
     b.close()
     value = db.nglob * float(n * len(shots)) / wall
-    kbytes = batch_stiffness_bytes(db, len(shots), fused=False, attenuation=att)
+    kbytes = batch_stiffness_bytes(db, len(shots), attenuation=att)
     ach = kbytes / (kms / 1e3) / 1e9
     src, rec, _ = shots[0]
     ps = min(args.plain_steps, n)
@@ -247,14 +244,14 @@ def batched_visco_measurement(args) -> dict:
     return {"workload": f"{w.name.split(',')[0]} viscoelastic Q_mu=100, {len(shots)} shots x {n} steps",
             "value": value, "unit": "GLL-point updates/s", "wall_s": round(wall, 3), "plain_single_shot": plain,
             "ratio_vs_plain": value / plain, "autotuned": choice, "seismograms_finite": finite,
-            "roofline": {"bound": "hbm", "kernel": "k_visco_batch (all shots live" + ")", "achieved": round(ach, 1),
+            "roofline": {"bound": "hbm", "kernel": "k_visco_batch (all shots live)", "achieved": round(ach, 1),
                          "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                          "bytes_per_launch": kbytes, "avg_pass_ms": round(kms, 4), "step_ms": round(sms, 4)}}
 
 
 def homogeneous_box_measurement(args) -> dict:
     """The 20^3 homogeneous elastic box (531,441 points, 2000 steps, the CPU-runnable case) through the
-    ABI call sequence with the library's defaults (FMA kernels, element-order sums),
+    ABI call sequence with the library's defaults (FMA kernels, colour-order sums),
     the FP32 oracle on one host core over a sample of its steps, and the reference's own Fortran
     solver figure for the same case (measured on another host)."""
     import numpy as np
@@ -289,7 +286,7 @@ def homogeneous_box_measurement(args) -> dict:
     log(f"[bench] 20^3 homogeneous box: {value:.3e} GLL-pt updates/s ({wall / (n - 20) * 1e3:.3f} ms/step), "
         f"finite={finite}")
     return {"workload": w.name, "nglob": db.nglob, "value": value, "unit": "GLL-point updates/s",
-            "ms_per_step": wall / (n - 20) * 1e3, "steps": n - 20, "assembly": "library default (element order)",
+            "ms_per_step": wall / (n - 20) * 1e3, "steps": n - 20, "assembly": "library default (colour order)",
             "seismograms_finite": finite, "cpu_baseline": cpu,
             "reference_fortran_cpu": {"value": 7.16e6, "unit": "GLL-point updates/s", "cores": 1,
                                       "kind": "reference",
@@ -300,7 +297,7 @@ def homogeneous_box_measurement(args) -> dict:
 def cpml_example_measurement(args) -> dict:
     """The reference example CPML_examples/homogeneous_halfspace_HEX8_elastic_absorbing_CPML_5sides
     (36 x 36 x 16 irregular elements, 1,366,625 points, 9036 C-PML elements, 2400 steps) with the
-    library defaults (FMA kernels, element-order sums), and its seismograms against the example's
+    library defaults (FMA kernels, colour-order sums), and its seismograms against the example's
     REF_SEIS."""
     import ctypes as C
     import numpy as np
@@ -626,19 +623,16 @@ def main():
     args = ap.parse_args()
 
     if args.kernel_probe:
-        # short fixed sequence for PMC counter runs: 4 batched steps of the 32-shot workload with
-        # each batched kernel variant, then 6 single-shot steps with colour-order sums
+        # short fixed sequence for PMC counter runs: 4 batched steps of the 32-shot workload, then 6
+        # single-shot steps with colour-order sums
         from specfem3d_amd import workloads as W
         from specfem3d_amd.batch import BatchSolver
         from specfem3d_amd.solver import GPUSolver
         w = W.gradient_shots_box(scale=args.batch_scale, nshots=32)
         w.shots = [(s_, r_, min(n_, 40)) for s_, r_, n_ in w.shots]
         b = BatchSolver(w.db, w.shots, exact=False, shots_per_group=8, assembly=3)
-        for ov in (0, 1):
-            b.set_tuning("lds_overlay", ov)
-            b.reset()
-            b.run(4, graph_steps=1)
-            log(f"[bench] kernel probe: 4 batched steps, lds_overlay {ov}")
+        b.run(4, graph_steps=1)
+        log("[bench] kernel probe: 4 batched steps")
         b.close()
         src, rec, _ = w.shots[0]
         g = GPUSolver(w.db, src, rec, nstep=6, exact=False, assembly=2)

@@ -343,7 +343,8 @@ void transfer_swf_data_tohost_(long* p1, int* p2, int* p3, realw* p4, realw* p5,
 /* exact = 1: element kernels without fused multiply-add (the CPU solver's rounding);
    assembly: order of a point's sums of element contributions, which the stiffness stores and the next
    update adds up. 1: element order (the CPU solver's); 2: the colour order of a greedy element
-   colouring; 0: any (element order). All are deterministic. */
+   colouring; 0: any (element order); -1, the default: 2 for a solid without attenuation, else 0. All are
+   deterministic, and reading a field between steps changes no bit. */
 void sf_set_options(long* Mesh_pointer, int exact, int assembly);
 /* tuning switch by name: "att_variant" 0..4 = scheduling of the attenuation state in the point
    stiffness kernel (same results; 4, the default, loads it straight into LDS);
@@ -406,10 +407,10 @@ int sf_norm_noalloc(const realw* field, long long npts, int ncomp, realw* out, v
 void sf_batch_reset(long batch);
 void sf_batch_time(long batch, int nsteps, double* stiffness_ms, double* step_ms);
 void sf_batch_destroy(long batch);
-/* host only: per-local-point flags of the fused batched mode for elements elems[q] of colour color[q]
+/* host only: per-local-point flags of a scatter colour by colour for elements elems[q] of colour color[q]
    (colours run in increasing order) and the points Stacey or sources add to before the colours
-   (forced[g] != 0): 1 = first writer, 2 = finisher of the Newmark update, 4 = finisher clears the
-   acceleration; 125 entries per element of ibool0; returns -1 if two elements of a colour share a
+   (forced[g] != 0): 1 = first writer, 2 = last writer, 4 = a point that is added to before the
+   colours; 125 entries per element of ibool0; returns -1 if two elements of a colour share a
    point */
 int sf_batch_point_flags(int nglob, int nelem, const int* ibool0, const int* elems, const int* color,
                          const unsigned char* forced, unsigned char* flags);

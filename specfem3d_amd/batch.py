@@ -6,7 +6,7 @@ re-runs the whole loop per shot. ``BatchSolver`` prepares the mesh once through 
 wavefields (``csrc/batch.hip``). The shots have their own sources, receivers and record lengths.
 Shots-per-workgroup and the assembly mode come from the library's autotuner, and time steps are
 replayed from captured hipGraphs. Each shot's seismograms are bit-identical to a single-shot
-``GPUSolver`` run with the same options. Meshes with fluid elements (coupled to the solid) step each
+``GPUSolver`` run with ``assembly=2`` (without FMA contraction, or under assembly 2). Meshes with fluid elements (coupled to the solid) step each
 shot's potentials too; sources and receivers lie in the solid.
 """
 from __future__ import annotations
@@ -23,7 +23,8 @@ class BatchSolver:
     def __init__(self, db, shots, exact: bool = False, device: int = 0, shots_per_group: int | None = None,
                  assembly: int | None = None, attenuation=None):
         """``shots``: list of (SourceSet, ReceiverSet, nstep), one per shot. ``assembly``
-        (0, 2, 3) is stored and has no effect: every shot's sums run in the colour order of the mesh.
+        0, 2 or 3: every shot's sums run in the colour order of the mesh; FMA builds use fused
+        multiply-adds in the Newmark update under 3 (``autotune`` sets 2 or 3 by the batch's size).
         ``attenuation``: 3-SLS set-up of the mesh (each shot then carries its own memory variables)."""
         if not shots:
             raise ValueError("no shots")

@@ -717,8 +717,8 @@ bool element_is_elastic(Mesh* m, int e) {
 
 // Greedy first-fit colouring of an element list (in list order): an element takes the lowest
 // colour not yet used by any element sharing one of its global points. The colours give an order of
-// a point's sums that does not depend on the launch. Elements keep their list order inside a colour. At most 32 colours (a bit mask per global point); a structured hexahedral
-// mesh needs 8.
+// a point's sums that does not depend on the launch. Elements keep their list order inside a colour. At most
+// 32 colours (a bit mask per global point); a structured hexahedral mesh needs 8.
 static int color_elements(int nglob, int nelem, const int* ibool0, const int* elems, int* col) {
   std::vector<uint32_t> used((size_t)nglob, 0u);
   int ncolor = 0;
@@ -1324,7 +1324,7 @@ extern "C" void FC_FUNC_(prepare_cleanup_device, PREPARE_CLEANUP_DEVICE)(long* M
 // exact = 1: element kernels without fused multiply-add (the CPU reference's rounding);
 // assembly: the order in which a global point's element contributions are summed. 1 = element order
 // (the reference's serial order), 2 = the colour order of a greedy element colouring, 0 = any order
-// (element order as well). All of them store
+// (element order as well), -1 (the default) = 2 for a solid without attenuation, else 0. All of them store
 // the local forces and sum them in the next update (k_gather_update).
 extern "C" void sf_set_options(long* Mesh_pointer, int exact, int assembly) {
   Mesh* m = from_handle(Mesh_pointer);

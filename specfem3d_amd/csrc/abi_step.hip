@@ -8,7 +8,7 @@
 // kernel_3 (mass division + corrector) is deferred: the next update_displacement on the same
 // field runs it fused with the predictor (one pass over u, v, a instead of two). Any entry
 // point that reads v or a (or writes the field) runs a pending corrector first, so results
-// are identical to the eager order.
+// are identical to the eager order, in FMA builds too: the passes round every operation.
 #include <algorithm>
 #include <cstring>
 #include <vector>
@@ -273,8 +273,8 @@ extern "C" void FC_FUNC_(update_displacement_cuda, UPDATE_DISPLACMENT_CUDA)(long
     m->pml_t1 = *deltatover2_F * (1.0f - 2.0f * 0.125f);
     m->pml_t2 = *deltatsqover2_F * (1.0f - 0.125f);
     if (!m->pending_k3_el[f])
-      launch_pml_store_old(m->stream, m->pml_npts, m->pml_pts, w.displ, w.veloc, w.accel, m->rmass, 0, 0.f,
-                           m->pml_t1, m->pml_t2, m->pml_old);
+      launch_pml_store_old(m->stream, m->pml_npts, m->pml_pts, w.displ, w.veloc, w.accel, m->pml_t1,
+                           m->pml_t2, m->pml_old);
   }
   if (m->pending_gather_el[f]) {
     GatherArgs a = gather_args(m, f);
@@ -1080,7 +1080,7 @@ extern "C" void FC_FUNC_(transfer_kernels_ac_to_host, TRANSFER_KERNELS_AC_TO_HOS
 
 // ---------------------------------------------------------------- library extensions (no reference counterpart)
 // sf_set_options: exact = 1 runs the element kernels without fused multiply-add (the CPU
-// reference's rounding); assembly = 1 sums element contributions in element order, 2 colours.
+// reference's rounding); assembly: order of the sums of element contributions, see its definition.
 extern "C" void sf_set_options(long* Mesh_pointer, int exact, int assembly);
 extern "C" void sf_synchronize(long* Mesh_pointer) {
   Mesh* m = from_handle(Mesh_pointer);

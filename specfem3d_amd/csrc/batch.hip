@@ -18,7 +18,8 @@
 //     counter, so a group of steps is captured once into a hipGraph and replayed;
 //   * the per-point arithmetic and the order of every sum equal the single-shot path (same
 //     kernels' expressions, same colour order, same order of faces), so each shot of a batch is
-//     bit-identical to its single-shot run in the colour order (assembly = 2).
+//     bit-identical to its single-shot run under assembly = 2 (assembly 3 differs in the rounding of the
+//     update in FMA builds, see newmark).
 // Shots-per-workgroup are chosen by an autotuner that times each candidate for a few steps from rest
 // and then resets the batch.
 #include <algorithm>
@@ -548,9 +549,10 @@ static void zero_state(Batch* b) {
   SF_CHECK(hipStreamSynchronize(m->stream));
 }
 
-// Point flags of the fused mode: for each global point, the element of its lowest colour writes
-// first (unless Stacey or a source adds to the point before the colours), the element of its
-// highest colour finishes the Newmark update and clears `a` where those passes add.
+// First and last writers of each point when the colours run one after the other, for callers of
+// sf_batch_point_flags: the element of a point's lowest colour writes first (unless Stacey or a source adds
+// to the point before the colours), the element of its highest colour last. The engine sums per point and
+// does not use them.
 static int point_flags(int nglob, int nelem, const int* ibool0, const int* elems, const int* color,
                        const unsigned char* forced, unsigned char* flags) {
   std::vector<int> cmin((size_t)nglob, 1 << 30), cmax((size_t)nglob, -1), nlast((size_t)nglob, 0);
@@ -1042,8 +1044,8 @@ extern "C" void sf_batch_set_options(long h, int shots_per_group, int assembly) 
 }
 
 // "local_groups": groups of eight shots whose local forces are held at a time (at most all of them, the
-// default where the card has the room; fewer save 24 B per local point and shot and take an extra pass
-// over accel; same results). "lds_overlay" 0/1 is accepted and read back without effect: the elastic
+// default where the card has the room; fewer save 24 B per local point and shot, 8 B in the fluid, and take
+// an extra pass over accel; same bits). "lds_overlay" 0/1 is accepted and read back without effect: the elastic
 // kernel's rows always share their LDS with the stress products. Unknown names are fatal.
 extern "C" void sf_batch_set_tuning(long h, const char* name, int value) {
   Batch* b = batch_of(h);
@@ -1227,11 +1229,11 @@ extern "C" void sf_batch_destroy(long h) {
   delete b;
 }
 
-// Host-only (no device needed): the fused mode's per-local-point flags for elements elems[q] of
+// Host-only (no device needed): per-local-point flags of a scatter colour by colour for elements elems[q] of
 // colour color[q] (colours run in increasing order) and the points that Stacey or sources add to
-// before the colours (forced[g] != 0): bit 1 first writer, bit 2 finisher, bit 4 cleared by the
-// finisher. flags has 125 entries per element of ibool0. Returns 0, or -1 if two elements of one
-// colour share a point.
+// before the colours (forced[g] != 0): bit 1 first writer, bit 2 last writer, bit 4 a point that is
+// added to before the colours. flags has 125 entries per element of ibool0. Returns 0, or -1 if two
+// elements of one colour share a point.
 extern "C" int sf_batch_point_flags(int nglob, int nelem, const int* ibool0, const int* elems, const int* color,
                                     const unsigned char* forced, unsigned char* flags) {
   return point_flags(nglob, nelem, ibool0, elems, color, forced, flags);

@@ -6,8 +6,9 @@
 // holes in the rows of the others. A workgroup takes one element and SC
 // shots (SC = 4 or 8): the element's ibool, moduli and Jacobian terms are loaded once for them, and
 // the workgroups of one element's shots are adjacent in the grid, so they share those. The per-point
-// arithmetic is elastic_point.h, the same code as the single-shot kernel, so a batched shot reproduces
-// its single-shot run.
+// arithmetic is elastic_point.h, the same code as the single-shot kernel, so a batched shot has the bits of
+// its single-shot run in the same order of sums (under assembly 3 in exact builds alone, see newmark in
+// batch.hip).
 //
 // Shots are stored in decreasing order of record length; a shot is live at step `it` while
 // nstep[s] >= it, and a group whose first shot has finished exits at once (uneven record
@@ -15,7 +16,7 @@
 // of the step can be replayed.
 //
 // The stiffness stores the local forces, and the update that starts the next step sums them per point
-// (k_batch_gather in batch.hip), in the element order of the single-shot run.
+// (k_batch_gather in batch.hip), in the colour order of a single-shot run under assembly = 2.
 //
 // Compiled twice like k_elastic.hip: SF_EXACT=1 without FMA contraction, SF_EXACT=0 with it.
 #include "elastic_point.h"
@@ -232,7 +233,9 @@ __device__ __forceinline__ int64_t eb_idx(int64_t e, int c, int p, int64_t S, in
 template <int NQ>
 __global__ void __launch_bounds__(128 * NQ) k_visco_batch(BatchArgs B, GLLk G) {
   constexpr int SC = 4 * NQ;
-  constexpr int PST = 132;                        // see k_elastic_batch
+  // LDS rows (component or product, shot) of PST floats, point fastest: the rows of a lane's two quads
+  // start 16 banks apart, so 16 consecutive points of two quads read 32 different banks
+  constexpr int PST = 132;
   constexpr int CPL = SC * PST;
   __shared__ realw sBuf[9 * CPL];
   realw* const sT = sBuf;                         // stress products [m][s][p]
@@ -404,7 +407,7 @@ __global__ void __launch_bounds__(128 * NQ) k_visco_batch(BatchArgs B, GLLk G) {
 
 // Batched acoustic stiffness (compute_forces_acoustic.F90:35-726; the arithmetic of k_acoustic per
 // point and shot): chi'' -= div((1/rho) grad chi) for SC = 4 NQ shots of one element per
-// workgroup. Lane = (GLL point p, quad of 4 consecutive shots) as in k_elastic_batch; the
+// workgroup. Lane = (GLL point p, quad of 4 consecutive shots) as in k_visco_batch; the
 // potential tile and the three products (rho^-1 jacobian grad chi . grad xi, eta, gamma) go through
 // LDS, one row of PST floats per (plane, shot). Every sum runs in k_acoustic's order (the gamma
 // contraction reads the same values the column kernel holds in registers), so a batched shot

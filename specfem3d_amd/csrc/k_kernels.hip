@@ -1,4 +1,4 @@
-// k_kernels.hip -- sensitivity-kernel accumulation, ordered assembly gather, max-norm.
+// k_kernels.hip -- sensitivity-kernel accumulation, receivers in fluid elements, max-norm.
 // Built with -ffp-contract=off (reference rounding).
 #include "kernels.h"
 

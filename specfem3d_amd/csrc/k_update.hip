@@ -95,25 +95,16 @@ __global__ void k_corrector_predictor(int64_t n4, int64_t n, realw* __restrict__
 
 // PML_displ_old (update_displ_elastic_PML, update_displacement_scheme.f90:417-455) at the global points
 // of the C-PML elements, from the field before the predictor: u + t1 v + t2 a with
-// t1 = deltatover2 (1 - 2 theta), t2 = deltatsqover2 (1 - theta). With a corrector still pending (it
-// is fused into the predictor that follows), the corrected v and a are formed first with the
-// corrector's own expressions.
+// t1 = deltatover2 (1 - 2 theta), t2 = deltatsqover2 (1 - theta). Where a corrector is pending, the pass
+// that runs it with the predictor stores the same for every point (OLD).
 __global__ void k_pml_store_old(int n, const int* __restrict__ pts, const realw* __restrict__ u,
-                                const realw* __restrict__ v, const realw* __restrict__ a,
-                                const realw* __restrict__ rm, int pending, realw dt2p, realw t1, realw t2,
+                                const realw* __restrict__ v, const realw* __restrict__ a, realw t1, realw t2,
                                 realw* __restrict__ old) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t g = pts[t];
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
-    realw ac = a[3 * g + c], vc = v[3 * g + c];
-    if (pending) {
-      ac = ac * rm[3 * g + c];
-      vc = vc + dt2p * ac;
-    }
-    old[3 * g + c] = u[3 * g + c] + t1 * vc + t2 * ac;
-  }
+  for (int c = 0; c < 3; c++) old[3 * g + c] = u[3 * g + c] + t1 * v[3 * g + c] + t2 * a[3 * g + c];
 }
 
 // Dirichlet condition on the outer faces of the C-PML layers (pml_impose_boundary_condition_elastic)
@@ -301,10 +292,9 @@ void launch_corrector_predictor(hipStream_t s, int64_t n, realw* u, realw* v, re
 }
 
 void launch_pml_store_old(hipStream_t s, int n, const int* pts, const realw* u, const realw* v, const realw* a,
-                          const realw* rmass, int pending, realw dt2p, realw t1, realw t2, realw* old) {
+                          realw t1, realw t2, realw* old) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_pml_store_old, grid_for(n, 256), dim3(256), 0, s, n, pts, u, v, a, rmass, pending, dt2p, t1,
-                     t2, old);
+  hipLaunchKernelGGL(k_pml_store_old, grid_for(n, 256), dim3(256), 0, s, n, pts, u, v, a, t1, t2, old);
   SF_LAUNCH_CHECK("k_pml_store_old");
 }
 

@@ -194,10 +194,9 @@ struct PmlArgs {
   int eb, pos0;            // ... pos0: launch position of the first listed element
 };
 void launch_elastic_pml(hipStream_t s, const PmlArgs& a, bool exact);
-// PML_displ_old at the listed points: u + t1 v + t2 a, with the pending corrector (a *= rmass,
-// v += dt2p a) applied first when dt2p_pending != 0
+// PML_displ_old at the listed points: u + t1 v + t2 a
 void launch_pml_store_old(hipStream_t s, int n, const int* pts, const realw* u, const realw* v, const realw* a,
-                          const realw* rmass, int pending, realw dt2p, realw t1, realw t2, realw* old);
+                          realw t1, realw t2, realw* old);
 // zero u, v, a at the listed points (Dirichlet condition of the C-PML outer faces)
 void launch_zero_points(hipStream_t s, int n, const int* pts, realw* u, realw* v, realw* a);
 
@@ -243,7 +242,7 @@ struct BatchArgs {
   int64_t nloc;
   realw alpha[3], beta[3], gamma[3];
 };
-// per-local-point flags of sf_batch_point_flags
+// per-local-point flags of sf_batch_point_flags (for its callers: the engine has no use for them)
 enum : unsigned char { BF_FIRST = 1, BF_LAST = 2, BF_ZERO = 4 };
 // sc = shots per workgroup (4, 8)
 void launch_elastic_batch(hipStream_t s, const BatchArgs& a, int sc, bool exact);
