@@ -356,7 +356,7 @@ def cpml_example_measurement(args) -> dict:
             "roofline": {"kernel": "k_elastic_pml (C-PML elements)", "bound": "hbm", "achieved": round(achieved, 1),
                          "peak": 8000.0, "unit": "GB/s", "frac": round(achieved / 8000.0, 4),
                          "bytes_per_launch": nbytes, "avg_launch_ms": pml_ms,
-                         "traffic": 400.6e6, "traffic_source": "profiles/k_elastic_pml_cpml5_example.md"},
+                         "traffic": 356.9e6, "traffic_source": "profiles/k_elastic_pml_cpml5_example.md"},
             "cpu_baseline": cpu}
 
 

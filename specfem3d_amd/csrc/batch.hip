@@ -18,8 +18,9 @@
 //     counter, so a group of steps is captured once into a hipGraph and replayed;
 //   * the per-point arithmetic and the order of every sum equal the single-shot path (same
 //     kernels' expressions, same colour order, same order of faces), so each shot of a batch is
-//     bit-identical to its single-shot run under assembly = 2 (assembly 3 differs in the rounding of the
-//     update in FMA builds, see newmark).
+//     bit-identical to its single-shot run under assembly = 2 (FMA builds: under assembly 2 without
+//     attenuation; 3 rounds the update another way, see newmark, and k_visco_batch fuses other products
+//     than k_elastic_pt).
 // Shots-per-workgroup are chosen by an autotuner that times each candidate for a few steps from rest
 // and then resets the batch.
 #include <algorithm>
@@ -166,8 +167,8 @@ __global__ void __launch_bounds__(256) k_batch_update(int64_t nrow, const int* _
 // the element pass without its arithmetic took 7.3 of 7.4 ms, of which the stores 4.4 ms (9.5 GB, 2.2
 // TB/s), and the shared points' u was read once per colour (6.3 instead of 3.3 GB). Here both passes
 // store whole lines, the element pass is bound by its arithmetic (3.45 ms there: VALU 2.4 ms, HBM 2.1,
-// LDS 1.6) and this one by HBM (3.96 ms, 19.3 GB, 4.9 TB/s). Steps before and after: 32x32x16 x 16
-// shots 598 -> 500 us, 64x64x32 x 32 8.53 -> 7.56 ms, viscoelastic 18x18x12 x 8 319 -> 233 us and
+// LDS 1.6) and this one by HBM (3.97 ms, 20.7 GB, 5.2 TB/s). Steps before and after: 32x32x16 x 16
+// shots 598 -> 473 us, 64x64x32 x 32 8.53 -> 7.28 ms, viscoelastic 18x18x12 x 8 319 -> 233 us and
 // 40x40x20 x 16 4.02 -> 3.41 ms.
 struct BatchGatherArgs {
   int64_t g0, n, nrow;           // global points [g0, g0 + n), rows of a group

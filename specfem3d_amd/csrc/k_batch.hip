@@ -7,7 +7,7 @@
 // shots (SC = 4 or 8): the element's ibool, moduli and Jacobian terms are loaded once for them, and
 // the workgroups of one element's shots are adjacent in the grid, so they share those. The per-point
 // arithmetic is elastic_point.h, the same code as the single-shot kernel, so a batched shot has the bits of
-// its single-shot run in the same order of sums (under assembly 3 in exact builds alone, see newmark in
+// its single-shot run in the same order of sums (FMA builds: without attenuation and under assembly 2, see
 // batch.hip).
 //
 // Shots are stored in decreasing order of record length; a shot is live at step `it` while

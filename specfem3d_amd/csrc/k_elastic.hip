@@ -244,7 +244,7 @@ k_elastic_pt(ElasticArgs A, GLLk G) {
 // same for eta) are reused in place: a row is read and written by one lane, and a point's values are
 // read and replaced by the lane of its column; only the xi derivatives need a barrier before they
 // replace u. 15 KB of LDS per workgroup, 61 to 80 VGPRs, 5 waves per SIMD. Per launch against
-// k_elastic_pt storing the same forces: 64x64x32 elements 187 -> 100 us (0.50 GB: the rate of a large
+// k_elastic_pt storing the same forces: 64x64x32 elements 187 -> 105 us (0.52 GB: the rate of a large
 // copy), 20x20x20 14.3 -> 12.5, 24^3 with strain 22.2 -> 19.5, irregular 43x37x29 89 -> 87 (its 40 B of
 // Jacobian terms per point were already the limit).
 // REG: the regular elements of a mesh (FMA build: the mapping is folded into the tables, so that a regular
