@@ -7,8 +7,8 @@ wavefields (``csrc/batch.hip``). The shots have their own sources, receivers and
 Shots-per-workgroup and the assembly mode come from the library's autotuner, and time steps are
 replayed from captured hipGraphs. Each shot's seismograms are bit-identical to a single-shot
 ``GPUSolver`` run with ``assembly=2, element_order="morton"`` (exact builds; FMA builds under
-assembly 2 and without attenuation, to rounding otherwise). Meshes with fluid elements (coupled to the solid) step each
-shot's potentials too; sources and receivers lie in the solid.
+assembly 2 and without attenuation, to rounding otherwise). Meshes with fluid elements (coupled to
+the solid) step each shot's potentials too; sources and receivers lie in the solid.
 """
 from __future__ import annotations
 
